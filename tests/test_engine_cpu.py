@@ -105,7 +105,7 @@ int main(void) {
 '''
 
 
-@pytest.mark.skipif(not os.path.isdir(REF_TREE), reason="reference headers not mounted")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF_TREE, "art")), reason="reference headers not mounted")
 def test_header_layouts_equal_reference(tmp_path):
     src = tmp_path / "probe.c"
     src.write_text(_probe_source())
@@ -183,7 +183,7 @@ def test_hip_module_table_and_config_on_own_core():
 
 
 @needs_ref
-@pytest.mark.skipif(not os.path.isdir(REF_TREE), reason="reference headers not mounted")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF_TREE, "art")), reason="reference headers not mounted")
 def test_hip_module_built_against_nart_headers_plugs_into_reference_runtime():
     """The drop-in claim, CPU part: compile the module against the reference's OWN headers, load it into the
     reference's OWN libart and drive op lookup, settings and shape inference through it."""
