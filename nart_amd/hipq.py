@@ -127,12 +127,18 @@ def quant_scale(x, bits):
 
 
 def _stream():
+    """The current HIP stream as an address (the void * of the C ABI).  The first call replaces this function by torch's own
+    two accessors: they take 0.1 us where building the torch.cuda.current_stream() object took 2.7 of a plan call's 6.6 us."""
     import torch
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    global _stream
+    torch.cuda.current_stream()  # initialises the device, and fails with torch's own message where there is none
+    device, raw = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+    _stream = lambda: raw(device())  # noqa: E731
+    return _stream()
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
+    return t.data_ptr() if t is not None else None
 
 
 def conv_out_dim(i, pad, k, stride):
