@@ -103,6 +103,15 @@ __device__ static __forceinline__ uint32_t ashr_sat_u8x4(int32_t v0, int32_t v1,
     return o;
 }
 
+// the same with a shift of its own in every lane
+__device__ static __forceinline__ uint32_t ashr_sat_u8x4_lanes(int32_t v0, int32_t v1, int32_t v2, int32_t v3, int32_t s)
+{
+    uint32_t o;
+    asm("v_ashr_pk_u8_i32 %0, %1, %2, %3" : "=v"(o) : "v"(v0), "v"(v1), "v"(s));
+    asm("v_ashr_pk_u8_i32 %0, %1, %2, %3 op_sel:[0,0,0,1]" : "+v"(o) : "v"(v2), "v"(v3), "v"(s));
+    return o;
+}
+
 template <bool FAST>
 __device__ static __forceinline__ uint32_t add_dword(uint32_t a, uint32_t b, const AddParams &p)
 {

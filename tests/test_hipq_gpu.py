@@ -1231,3 +1231,22 @@ def test_two_group_kernel_matches_the_oracle():
     w = rng.integers(0, 256, (64, 256, 3, 3), dtype=np.uint8)
     plan = hipq.Conv2d(x.shape, w, None, 1, 1, 1, 0.02, 7, 0.005, 100, 0.05, 3)
     assert not plan.kernel.endswith("_k2"), plan.kernel
+
+
+@pytest.mark.parametrize("shape,k,pad,st,method,ceil_mode", [
+    ((2, 16, 9, 7), 3, 1, 1, 1, False), ((1, 40, 10, 11), 3, 1, 2, 1, True), ((2, 32, 8, 8), 2, 0, 2, 1, False),
+    ((1, 24, 30, 30), 11, 5, 3, 1, True), ((1, 24, 30, 30), 12, 5, 3, 1, True),      # 121 and 144 pixels: either side of the packed form
+    ((1, 16, 33, 35), None, 0, 1, 1, False), ((3, 192, 35, 35), None, 0, 1, 1, False), ((2, 2048, 7, 7), None, 0, 1, 1, False),
+    ((1, 17, 160, 130), None, 0, 1, 1, False), ((300, 16, 4, 4), None, 0, 1, 1, False), ((3, 40, 9, 7), 3, 1, 2, 0, True)],
+    ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_pooling_of_sixteen_channels_per_lane(shape, k, pad, st, method, ceil_mode):
+    """Average windows clipped and hanging over the edge, global averages with few and with many pixels per thread."""
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(0, 256, shape, dtype=np.uint8)
+    N, Cc, H, W = shape
+    kk = (H, W) if k is None else (k, k)
+    for q in ((0.02, 0, 0.013, 5), (0.03, 131, 0.05, 120)):
+        want = orc.pool_u8(x, kk, pad, st, method, ceil_mode, *q)
+        y = torch.zeros((N, want.shape[2], want.shape[3], hipq.channel_stride(Cc)), dtype=torch.uint8, device="cuda")
+        hipq.pool_u8(hipq.to_device_nhwc(x), y, Cc, kk, pad, st, method, *q)
+        assert np.array_equal(hipq.from_device_nhwc(y, Cc), want)
