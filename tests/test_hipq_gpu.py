@@ -1250,3 +1250,16 @@ def test_pooling_of_sixteen_channels_per_lane(shape, k, pad, st, method, ceil_mo
         y = torch.zeros((N, want.shape[2], want.shape[3], hipq.channel_stride(Cc)), dtype=torch.uint8, device="cuda")
         hipq.pool_u8(hipq.to_device_nhwc(x), y, Cc, kk, pad, st, method, *q)
         assert np.array_equal(hipq.from_device_nhwc(y, Cc), want)
+
+
+@pytest.mark.parametrize("chans", [(16, 16), (17, 31), (83, 34, 5), (192, 100), (20, 24, 40, 16, 33)], ids=str)
+def test_concat_of_sixteen_channels_per_lane(chans):
+    rng = np.random.default_rng(sum(chans))
+    ins = [rng.integers(0, 256, (3, c, 5, 7), dtype=np.uint8) for c in chans]
+    ia, iz = [0.01 * (j + 1.5) for j in range(len(chans))], [(37 * j) % 256 for j in range(len(chans))]
+    want = orc.concat_u8(ins, ia, iz, 0.025, 9)
+    cs = hipq.channel_stride(sum(chans))
+    y = torch.full((3, 5, 7, cs), 255, dtype=torch.uint8, device="cuda")
+    hipq.concat_u8([hipq.to_device_nhwc(a) for a in ins], chans, y, ia, iz, 0.025, 9)
+    assert np.array_equal(hipq.from_device_nhwc(y, sum(chans)), want)
+    assert not y[..., sum(chans):].any()  # pad channels are zeros
