@@ -1263,3 +1263,14 @@ def test_concat_of_sixteen_channels_per_lane(chans):
     hipq.concat_u8([hipq.to_device_nhwc(a) for a in ins], chans, y, ia, iz, 0.025, 9)
     assert np.array_equal(hipq.from_device_nhwc(y, sum(chans)), want)
     assert not y[..., sum(chans):].any()  # pad channels are zeros
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 1, 1), (5, 81, 7, 9), (2, 16, 40, 41), (3, 1000, 1, 1), (2, 4099, 3, 3), (1, 41000, 1, 2)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_softmax_rows_in_lds(shape):
+    rng = np.random.default_rng(sum(shape))
+    x = rng.integers(0, 256, shape, dtype=np.uint8)
+    for q in ((0.06, 128, 1 / 256.0, 0), (0.5, 255, 0.004, 3), (3.0, 255, 0.004, 3)):
+        xd = hipq.to_device_nhwc(x)
+        got = hipq.from_device_nhwc(hipq.softmax_u8(xd, torch.full_like(xd, 9), shape[1], *q), shape[1])
+        assert np.array_equal(got, orc.softmax_u8(x, 1, *q)), q
