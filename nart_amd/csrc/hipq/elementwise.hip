@@ -150,10 +150,14 @@ __device__ static inline uint32_t relu_one(uint32_t x, const ReluArgs &p)
     return (uint32_t)sat_hi((int32_t)(rshift_rn((int64_t)pr, p.shift) + p.oz), p.hi);
 }
 
+// WORD: shift <= 31.  The multiplier has 23 bits, so difference * mult + 2^(shift - 1) stays below 2^32: one 24-bit
+// multiply-add and a shift per byte instead of a 64-bit product (3 instead of 11 vector instructions).
+template <bool WORD>
 __global__ __launch_bounds__(256) void relu_u8_kernel(const ReluArgs p)
 {
     const size_t nvec = p.count / 16;
     const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x, nthr = (size_t)gridDim.x * blockDim.x;
+    const uint32_t radd = WORD ? 1u << (p.shift - 1) : 0;
     for (size_t i = tid; i < nvec; i += nthr) {
         const u32x4 v = reinterpret_cast<const u32x4 *>(p.x)[i];
         u32x4 o;
@@ -161,8 +165,15 @@ __global__ __launch_bounds__(256) void relu_u8_kernel(const ReluArgs p)
         for (int d = 0; d < 4; d++) {
             uint32_t w = 0;
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                w |= relu_one((v[d] >> (8 * e)) & 255, p) << (8 * e);
+            for (int e = 0; e < 4; e++) {
+                const uint32_t x = (v[d] >> (8 * e)) & 255;
+                if (WORD) {
+                    const uint32_t dx = (uint32_t)(max((int)x, p.iz) - p.iz);
+                    w |= (uint32_t)min((int)((__umul24(dx, p.mult) + radd) >> p.shift) + p.oz, p.hi) << (8 * e);
+                } else {
+                    w |= relu_one(x, p) << (8 * e);
+                }
+            }
             o[d] = w;
         }
         reinterpret_cast<u32x4 *>(p.y)[i] = o;
@@ -934,7 +945,10 @@ extern "C" int hipq_relu_u8(const void *x, void *y, size_t count, float ia, int 
     HIPQ_REQUIRE(valid_shift(p.shift), "hipq_relu_u8: scale out of the fixed-point range");
     p.x = static_cast<const uint8_t *>(x), p.y = static_cast<uint8_t *>(y), p.count = count;
     p.iz = iz, p.oz = oz, p.hi = (1 << obits) - 1;
-    hipLaunchKernelGGL(relu_u8_kernel, dim3(grid_for(count / 16)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    if (p.shift <= 31)
+        hipLaunchKernelGGL(relu_u8_kernel<true>, dim3(grid_for(count / 16)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    else
+        hipLaunchKernelGGL(relu_u8_kernel<false>, dim3(grid_for(count / 16)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return launch_status("relu_u8_kernel");
 }
 

@@ -1274,3 +1274,12 @@ def test_softmax_rows_in_lds(shape):
         xd = hipq.to_device_nhwc(x)
         got = hipq.from_device_nhwc(hipq.softmax_u8(xd, torch.full_like(xd, 9), shape[1], *q), shape[1])
         assert np.array_equal(got, orc.softmax_u8(x, 1, *q)), q
+
+
+@pytest.mark.parametrize("ratio", [1.0, 1.9, 0.011, 3.0e-3, 1.0e-6])  # the last two beyond a 31-bit shift
+def test_relu_word_and_wide_forms(ratio):
+    x = np.arange(256 * 5 + 3, dtype=np.int64).astype(np.uint8)
+    for iz, oz, obits in ((0, 0, 8), (119, 7, 8), (255, 3, 6)):
+        xd = torch.from_numpy(x).cuda()
+        got = hipq.relu_u8(xd, torch.zeros_like(xd), ratio * 0.02, iz, 0.02, oz, obits).cpu().numpy()
+        assert np.array_equal(got, orc.relu_u8(x, ratio * 0.02, iz, 0.02, oz, obits)), (iz, oz, obits)
