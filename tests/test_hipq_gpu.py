@@ -1233,6 +1233,27 @@ def test_two_group_kernel_matches_the_oracle():
     assert not plan.kernel.endswith("_k2"), plan.kernel
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 5, 5), (3, 3, 13, 17), (2, 4, 1, 3), (2, 2, 7, 4), (2, 16, 8, 9), (3, 21, 6, 5), (1, 21, 31, 33),
+                                   (2, 33, 5, 8), (2, 40, 4, 7), (70, 5, 1, 1)], ids=lambda s: "x".join(map(str, s)))
+def test_layout_and_float_conversions_at_ragged_sizes(shape):
+    """Planes <-> pixels at the edges of the vector kernels' ranges: pixel counts that are no multiple of 4, of a wave or of a
+    work-group, channel counts on both sides of a 16-channel piece."""
+    rng = np.random.default_rng(sum(shape))
+    N, Cc, H, W = shape
+    x = (rng.standard_normal(shape) * 2).astype(np.float32)
+    b = rng.integers(0, 256, shape, dtype=np.uint8)
+    assert np.array_equal(hipq.from_device_nhwc(hipq.to_device_nhwc(b), Cc), b)
+    y = torch.full((N, H, W, hipq.channel_stride(Cc)), 7, dtype=torch.uint8, device="cuda")
+    assert np.array_equal(hipq.from_device_nhwc(hipq.quantize_u8(torch.from_numpy(x).cuda(), y, 0.019, 117), Cc), orc.quantize_u8(x, 0.019, 117))
+    got = hipq.from_device_nhwc(hipq.quantize_i8(torch.from_numpy(x).cuda(), y, 0.03), Cc).view(np.int8)
+    assert np.array_equal(got, orc.quantize_i8(x, 0.03))
+    f = torch.empty(shape, device="cuda")
+    hipq.dequantize_u8(hipq.to_device_nhwc(b), f, 0.11, 97)
+    assert np.array_equal(f.cpu().numpy().view(np.uint32), orc.dequantize_u8(b, 0.11, 97).view(np.uint32))
+    hipq.dequantize_i8(hipq.to_device_nhwc(b), f, 0.11)
+    assert np.array_equal(f.cpu().numpy().view(np.uint32), orc.dequantize_i8(b.view(np.int8), 0.11).view(np.uint32))
+
+
 @pytest.mark.parametrize("shape,k,pad,st,method,ceil_mode", [
     ((2, 16, 9, 7), 3, 1, 1, 1, False), ((1, 40, 10, 11), 3, 1, 2, 1, True), ((2, 32, 8, 8), 2, 0, 2, 1, False),
     ((1, 24, 30, 30), 11, 5, 3, 1, True), ((1, 24, 30, 30), 12, 5, 3, 1, True),      # 121 and 144 pixels: either side of the packed form
