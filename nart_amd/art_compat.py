@@ -135,6 +135,18 @@ class Parade:
         self._outputs = {t.ptr.contents.name.decode(): t for t in self._p.outputs()}
         self._by_name = dict(self._inputs)
         self._by_name.update(self._outputs)
+        # hip_mem_write: an array into a memory of the `hip` module and on its way to the device in one pass over it
+        self._write = next((f for f in (getattr(lib, "hip_mem_write", None) for lib in self._ctx._rt.libs) if f is not None), None)
+        if self._write is not None:
+            self._write.restype, self._write.argtypes = C.c_bool, [C.c_void_p, C.c_void_p, C.c_size_t]
+        self._io_in = [self._io(n, t) for n, t in self._inputs.items()]
+        self._io_out = [self._io(n, t) for n, t in self._outputs.items()]
+
+    @staticmethod
+    def _io(name, t):
+        """What run() needs of an input or output, looked up once per set of shapes: name, shape, dtype, memory, mem_cpu_data."""
+        c = t.ptr.contents
+        return (name, tuple(t.shape), numpy.dtype(_DTYPE_NAME[c.dtype]), c.mem, c.mem.contents.tp.contents.cpu_data_func)
 
     # ---- shapes and dtypes ------------------------------------------------------------------------------
     def input_shapes(self):
@@ -186,35 +198,38 @@ class Parade:
         if not self._core.parade_apply_reshape(self._p.ptr):
             return False
         self._core.parade_prepare(self._p.ptr)
+        self._collect()
         return True
 
     @staticmethod
-    def _check(kind, t, arr):
-        s = t.ptr.contents.shape
-        if s.dim_size != arr.ndim:
+    def _check(kind, shape, dtype, arr):
+        if len(shape) != arr.ndim:
             raise ValueError("%s dim size not match" % kind)
-        if tuple(int(s.dim[i]) for i in range(s.dim_size)) != tuple(arr.shape):
+        if shape != arr.shape:
             raise ValueError("%s shape not match" % kind)
-        if _DTYPE_NAME[t.ptr.contents.dtype] != str(arr.dtype):
+        if dtype != arr.dtype:
             raise ValueError("%s dtype not match" % kind)
 
     def run(self, inputs, outputs):
-        for name, t in self._inputs.items():
+        for name, shape, dtype, _, _ in self._io_in:
             assert name in inputs, "some input not given when calling parade.run"
-            self._check("input", t, numpy.asarray(inputs[name]))
-        for name, t in self._outputs.items():
+            self._check("input", shape, dtype, numpy.asarray(inputs[name]))
+        for name, shape, dtype, _, _ in self._io_out:
             assert name in outputs, "some output not given when calling parade.run"
-            self._check("output", t, outputs[name])
-        for name, t in self._inputs.items():
+            self._check("output", shape, dtype, outputs[name])
+        write = self._write
+        for name, _, _, mem, cpu_data in self._io_in:
             a = numpy.ascontiguousarray(inputs[name])
-            C.memmove(t._host(), a.ctypes.data, a.nbytes)
-        self.forward()
-        for name, t in self._outputs.items():
+            data = a.__array_interface__["data"][0]
+            if write is None or not write(mem, data, a.nbytes):
+                C.memmove(cpu_data(mem), data, a.nbytes)
+        self._core.parade_run(self._p.ptr)
+        for name, _, _, mem, cpu_data in self._io_out:
             out = outputs[name]
-            if out.flags["C_CONTIGUOUS"]:
-                C.memmove(out.ctypes.data, t._host(), out.nbytes)
+            if out.flags.c_contiguous:
+                C.memmove(out.__array_interface__["data"][0], cpu_data(mem), out.nbytes)
             else:
-                out[...] = t.numpy()
+                out[...] = self._outputs[name].numpy()
         return True
 
     def __del__(self):

@@ -95,7 +95,26 @@ struct hip_mem_t {
     // host, another workspace, a re-run - makes the hook launch the plain convolution into `dev` (hip_mem_settle).
     void (*pending)(void *ctx);
     void *pending_ctx;
+    // The mirror is being filled from the device by work queued on prod_stream (a recorded pass ends with that): whoever
+    // wants it waits for that stream.  host_read: the host has asked for device-written contents before.
+    bool down_issued, host_read;
+    // A float input whose reader is a uint8 quantize operator (quantize_prepare fills q_*).  hip_mem_write quantizes the
+    // values while it copies them into the mirror, a quarter of the bytes to bring to the device; q_valid: qhost (pinned) and,
+    // for what is not read from there directly, qdev hold the bytes of what the mirror holds.
+    const void *q_op;
+    float q_alpha;
+    int q_zp, q_bits;
+    uint8_t *qhost, *qdev;
+    size_t qhost_cap, qdev_cap;
+    bool q_valid;
 };
+
+// Up to this size a kernel reads or writes pinned host memory itself; above it the copy engine moves the bytes first.
+// The engine's copies cost a hand-over between two queues on each side and 9 us apiece beside their bytes; a kernel streams over
+// the host link at about the engine's rate.  (A pass of MobileNetV2 at batch 8, 1.2 MB in: 344 us with the line at 1 MB, 324 at
+// 4 MB; batch 24, 3.6 MB: 462 and 444; 9.6 MB gain nothing from a line at 16 MB, and there the engine overlaps with the
+// threads that copy into the pinned mirror.)
+constexpr size_t kHostDirect = 4 << 20;
 
 // make the device contents current: run the deferred producer, if any
 static inline void hip_mem_settle(hip_mem_t *m)
@@ -123,6 +142,10 @@ const void *hip_mem_dev_in(mem_t *m, hipStream_t st);
 void *hip_mem_dev_out(mem_t *m, hipStream_t st);
 // Host pointer with current contents (downloads / converts if the device is the newer side); read-only use.
 const void *hip_mem_host_in(mem_t *m);
+// May the next upload of this memory be a kernel that reads the pinned mirror?
+bool hip_mem_uploads_direct(const hip_mem_t *m);
+// Queues the device -> host copy of the contents on the stream that wrote them, without waiting.
+void hip_mem_start_download(hip_mem_t *m);
 static inline hip_mem_t *as_hip(mem_t *m) { return reinterpret_cast<hip_mem_t *>(m); }
 static inline bool is_hip_mem(const mem_t *m) { return m->tp == &hip_mem_tp_st; }
 

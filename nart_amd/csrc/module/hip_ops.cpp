@@ -79,8 +79,8 @@ op_t *alloc_op(workspace_t *)
 void dealloc_op(op_t *op)
 {
     // forget what the operator read (the registry of the convolution + add fusion, below)
-    forget_reader(op);
-    free(op);
+    if (forget_reader(op))
+        free(op);
 }
 void destroy_nothing(op_t *) {}
 
@@ -119,6 +119,9 @@ void require_hip_u8(op_t *op, size_t n_act, bool allow_i8 = false)
         }
         HIPM_CHECK(is_hip_mem(op->input_tensors[i]->mem));
         hip_mem_tag(op->input_tensors[i]);
+        hip_mem_t *m = as_hip(op->input_tensors[i]->mem);
+        if (!m->up_pending)
+            m->up_stream = op_stream(op); // where hip_mem_write sends what it brings to the device
         readers_of(op)[op->input_tensors[i]->mem].insert(op);
     }
 }
@@ -1130,6 +1133,15 @@ void quantize_run(op_t *op)
     int d[4];
     dims4(op->input_tensors[0], d);
     const hip_mem_t *y = as_hip(op->output_tensors[0].mem);
+    hip_mem_t *x = as_hip(op->input_tensors[0]->mem);
+    if (x->q_valid && x->q_op == op) { // quantized on its way in (hip_mem_write): what is left is the layout
+        const bool direct = x->size / 4 <= kHostDirect;
+        if (x->up_pending && x->up_stream != op_stream(op))
+            HIPM_HIP(hipStreamSynchronize(x->up_stream));
+        HIPM_HIPQ(hipq_nchw_to_nhwc_u8(direct ? x->qhost : x->qdev, out_ptr(op), d[0], d[1], d[2], d[3], y->cs, op_stream(op)));
+        x->up_pending = true, x->up_stream = op_stream(op);
+        return;
+    }
     if (op->output_tensors[0].dtype == dtINT8)
         HIPM_HIPQ(hipq_quantize_i8(static_cast<const float *>(in_ptr(op, 0)), out_ptr(op), d[0], d[1], d[2], d[3], y->cs,
                                    q->q.alpha[0], q->q.bits[0], op_stream(op)));
@@ -1163,6 +1175,12 @@ void quantize_prepare(op_t *op)
     hip_mem_tag(op->input_tensors[0]);
     alloc_and_tag(op);
     op->run_func = quantize_run;
+    hip_mem_t *x = as_hip(op->input_tensors[0]->mem);
+    x->q_valid = false;
+    x->q_op = row == 1 && op->output_tensors[0].mem != op->input_tensors[0]->mem ? op : nullptr;
+    x->q_alpha = q->q.alpha[0], x->q_zp = q->q.zp[0], x->q_bits = q->q.bits[0];
+    if (!x->up_pending)
+        x->up_stream = op_stream(op);
 }
 
 void dequantize_config(op_t *op)

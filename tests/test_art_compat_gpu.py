@@ -13,7 +13,7 @@ torch = pytest.importorskip("torch")
 
 from nart_amd import art_compat as art  # noqa: E402  (the one line a NART user changes)
 from nart_amd import cases, engine  # noqa: E402
-from oracle import casecpu  # noqa: E402  (checker only)
+from oracle import casecpu, orc  # noqa: E402  (checkers only)
 
 
 def _write(tmp_path, case):
@@ -93,3 +93,36 @@ def test_float_network_ends_and_missing_modules(tmp_path):
     assert np.array_equal(outputs[case.output.name].view(np.uint32), want.view(np.uint32))
     ctx2 = art.create_context_for_target("hip")
     assert ctx2.loaded_workspaces == ["hip"]
+
+
+@pytest.mark.parametrize("shape", [(1, 3, 5, 7), (3, 3, 70, 67), (2, 3, 431, 433), (5, 3, 640, 641)])
+def test_arrays_of_every_size_reach_the_device(shape):
+    """Parade.run's way of an array to the GPU: below and above the sizes at which helper threads copy, the copy engine is used
+    and the copies are cut; values quantized on the way in, values that are not (a misaligned array) and bytes."""
+    rng = np.random.default_rng(shape[2])
+    for kind in ("f32", "misaligned", "u8"):
+        c = cases.Case("write", 0)
+        if kind == "u8":
+            c.dequantize(c.input_u8(shape, 0.25, 7))
+        else:
+            c.dequantize(c.quantize(c.input_f32(shape), 0.0186, 114))
+        parade = art.Parade(engine.write_engine(c), art.create_context_for_target("hip"))
+        _, outputs = art.get_empty_io(parade)
+        for k in range(3):
+            print(shape, kind, k, flush=True)
+            if kind == "u8":
+                x = rng.integers(0, 256, shape, dtype=np.uint8)
+                q, alpha, zp = x, 0.25, 7
+            else:
+                x = (rng.standard_normal(shape) * 2.0).astype(np.float32)
+                x.reshape(-1)[:8] = [np.nan, np.inf, -np.inf, 0.0, 0.0093, -2.1204, 2.6226, 1e30]
+                x.reshape(-1)[-8:] = np.float32(0.0186) * (np.arange(8, dtype=np.float32) + 0.5)
+                if kind == "misaligned":
+                    raw = np.zeros(x.nbytes + 1, np.uint8)
+                    raw[1:] = x.reshape(-1).view(np.uint8)
+                    x = raw[1:].view(np.float32).reshape(shape)
+                q, alpha, zp = orc.quantize_u8(np.array(x), 0.0186, 114), 0.0186, 114
+            parade.run({c.input.name: x}, outputs)
+            want = orc.dequantize_u8(q, alpha, zp)
+            assert np.array_equal(outputs[c.output.name].view(np.uint32), want.reshape(outputs[c.output.name].shape).view(np.uint32)), (kind, k)
+            assert np.array_equal(parade._inputs[c.input.name].numpy().view(np.uint8), np.array(x).view(np.uint8))
