@@ -532,12 +532,43 @@ ART_PUBLIC bool workspace_support_op(workspace_t *ws, uint64_t code, bool strict
 }
 
 /* ---- parade (parade.c, parade_impl.h:23-32) ------------------------------------------------------------------ */
+/* A module may take over whole passes: parade_run offers it the operator list of a parade that lives on one of its
+ * workspaces (run returns false to have the operators run one by one; *state is the module's, given back through drop). */
+struct pass_runner {
+    const module_t *module;
+    bool (*run)(void **state, op_t *const *ops, size_t n);
+    void (*drop)(void *state);
+};
+static struct pass_runner g_runners[8];
+
+ART_PUBLIC void art_set_pass_runner(const module_t *module, bool (*run)(void **, op_t *const *, size_t), void (*drop)(void *))
+{
+    for (size_t i = 0; i < sizeof g_runners / sizeof g_runners[0]; ++i)
+        if (g_runners[i].module == NULL || g_runners[i].module == module) {
+            g_runners[i] = (struct pass_runner){module, run, drop};
+            return;
+        }
+}
+
+static const struct pass_runner *find_runner(const parade_t *p)
+{
+    for (size_t i = 1; i < p->op_count; ++i)
+        if (p->ops[i]->workspace != p->ops[0]->workspace)
+            return NULL;
+    for (size_t i = 0; p->op_count > 0 && i < sizeof g_runners / sizeof g_runners[0]; ++i)
+        if (g_runners[i].module != NULL && g_runners[i].module == p->ops[0]->workspace->module_type)
+            return &g_runners[i];
+    return NULL;
+}
+
 ART_PUBLIC parade_t *parade_new(void) { return (parade_t *)calloc(1, sizeof(parade_t)); }
 
 ART_PUBLIC void parade_delete(parade_t *p)
 {
     if (p == NULL)
         return;
+    if (p->pass != NULL)
+        p->runner->drop(p->pass);
     for (size_t i = 0; i < p->op_count; ++i)
         op_delete(p->ops[i]);
     for (size_t i = 0; i < p->input_tensor_count; ++i)
@@ -573,7 +604,15 @@ ART_PUBLIC void parade_prepare(parade_t *p)
 
 ART_PUBLIC void parade_run(parade_t *p)
 {
-    for (size_t i = 0; p != NULL && i < p->op_count; ++i)
+    if (p == NULL)
+        return;
+    if (!p->runner_sought) {
+        p->runner = find_runner(p);
+        p->runner_sought = true;
+    }
+    if (p->runner != NULL && p->runner->run(&p->pass, p->ops, p->op_count))
+        return;
+    for (size_t i = 0; i < p->op_count; ++i)
         op_run(p->ops[i]);
 }
 

@@ -13,6 +13,10 @@ struct _parade_t {
     tensor_t **weight_tensors;
     size_t output_tensor_count;
     tensor_t **output_tensors;
+    /* the module that may run the whole list as one pass, and what it keeps for that (art_set_pass_runner) */
+    const struct pass_runner *runner;
+    bool runner_sought;
+    void *pass;
 };
 
 void parade_push_op(parade_t *p, op_t *op);

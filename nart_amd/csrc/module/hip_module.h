@@ -62,6 +62,7 @@ struct hip_workspace_t {
     int dev_id;
     hipStream_t stream; // every kernel of this workspace is launched here
     bool own_stream;
+    uint64_t epoch; // counts prepare and destroy calls of this workspace's operators (a recorded pass is good for one value)
 };
 
 // ---- device memory with a host mirror -------------------------------------------------------------------
@@ -150,6 +151,18 @@ static inline hip_mem_t *as_hip(mem_t *m) { return reinterpret_cast<hip_mem_t *>
 static inline bool is_hip_mem(const mem_t *m) { return m->tp == &hip_mem_tp_st; }
 
 static inline hipStream_t op_stream(const op_t *op) { return reinterpret_cast<hip_workspace_t *>(op->workspace)->stream; }
+
+// ---- recorded passes (hip_pass.cpp) ----------------------------------------------------------------------------------
+// One pass over a parade whose operators all live on one `hip` workspace, as a HIP graph.  Fits parade_run's hook of the host
+// core (art_set_pass_runner); a runtime without that hook runs the operators one by one.
+bool hip_pass_run(void **state, op_t *const *ops, size_t n);
+void hip_pass_drop(void *state);
+// how many fused launches of each kind have been counted so far (hip_module_fused_*): a replayed pass counts what the
+// recorded one did
+constexpr int kHipCounters = 7;
+long *const *hip_counters(void);
+// the inputs that an operator's run() reads (the rest are weights, packed at prepare)
+size_t hip_op_activations(const op_t *op);
 
 extern "C" {
 extern const op_tp_t op_hip_quantize_tp, op_hip_dequantize_tp;

@@ -56,8 +56,12 @@ void same_shape_and_geometry(const op_t *op, const tensor_t *t)
     }
 }
 
+// an operator of this workspace was prepared or is going away: a recorded pass that names it is no longer good
+void touch(op_t *op) { ++reinterpret_cast<hip_workspace_t *>(op->workspace)->epoch; }
+
 void alloc_and_tag(op_t *op)
 {
+    touch(op);
     for (size_t i = 0; i < op->input_size; ++i) {
         tensor_alloc(op->input_tensors[i]);
     }
@@ -67,7 +71,7 @@ void alloc_and_tag(op_t *op)
     }
 }
 
-void forget_reader(op_t *op);
+bool forget_reader(op_t *op); // false: the workspace is gone already
 
 template <class T>
 op_t *alloc_op(workspace_t *)
@@ -80,7 +84,8 @@ void dealloc_op(op_t *op)
 {
     // forget what the operator read (the registry of the convolution + add fusion, below)
     if (forget_reader(op))
-        free(op);
+        touch(op);
+    free(op);
 }
 void destroy_nothing(op_t *) {}
 
@@ -98,12 +103,14 @@ long g_fused_blocks = 0, g_fused_tails = 0; // whole bottleneck blocks / blocks 
 
 reader_map &readers_of(op_t *op) { return g_readers[op->workspace]; }
 
-void forget_reader(op_t *op)
+bool forget_reader(op_t *op)
 {
     const auto it = g_readers.find(op->workspace);
-    if (it != g_readers.end())
-        for (auto &kv : it->second)
-            kv.second.erase(op);
+    if (it == g_readers.end())
+        return false;
+    for (auto &kv : it->second)
+        kv.second.erase(op);
+    return true;
 }
 
 // allow_i8: conv_2d, ip and dequantize also exist for int8 symmetric tensors (conv_2d.c:120-141, ip.cpp:312-331,
@@ -1099,6 +1106,7 @@ void reshape_config(op_t *) {}
 void reshape_run(op_t *) {}
 void reshape_prepare(op_t *op)
 {
+    touch(op);
     for (size_t i = 0; i < op->input_size; ++i)
         tensor_alloc(op->input_tensors[i]);
     op->run_func = reshape_run;
@@ -1233,6 +1241,25 @@ void dequantize_prepare(op_t *op)
     op->run_func = dequantize_run;
 }
 
+} // namespace
+
+long *const *hip_counters(void)
+{
+    static long *const c[kHipCounters] = {&g_fused_adds,     &g_fused_relus,  &g_fused_pools, &g_chained_convs,
+                                          &g_fused_dequants, &g_fused_blocks, &g_fused_tails};
+    return c;
+}
+
+size_t hip_op_activations(const op_t *op)
+{
+    return op->entry->tp == &op_conv_2d_tp || op->entry->tp == &op_ip_tp ? 1 : op->input_size;
+}
+
+// the host core's hook for whole passes; a runtime that has none (the reference's own) leaves it null
+extern "C" void art_set_pass_runner(const module_t *, bool (*)(void **, op_t *const *, size_t), void (*)(void *)) __attribute__((weak));
+
+namespace {
+
 // ---- workspace ------------------------------------------------------------------------------------------------------------
 int g_ws_count = 0;
 
@@ -1281,6 +1308,8 @@ static workspace_t *ws_new(const setting_entry_t *settings)
     HIPM_HIP(hipStreamCreateWithFlags(&ws->stream, hipStreamNonBlocking)); // default priority
     ws->own_stream = true;
     hip_stream_register(ws->stream);
+    if (art_set_pass_runner != nullptr)
+        art_set_pass_runner(&hip_module_tp, hip_pass_run, hip_pass_drop);
     return &ws->ws;
 }
 

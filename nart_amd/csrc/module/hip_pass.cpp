@@ -1,0 +1,232 @@
+// A pass over a parade as a HIP graph.  Launched one by one the operators of a pass cost the host 2.8 us a kernel and as much
+// again beside it, about what the small ones take on the GPU: MobileNetV2 at batch 6 spent 179 us launching 54 kernels that
+// take 235 us back to back and 275 us when each waits for its launch.  The kernels, their order and their arguments are the
+// same at every pass, so the second pass is recorded while the operators run (their run functions do not know) and the later
+// ones replay the record: one launch.  (It takes 18 - 25 us until its first kernel starts, an ordinary one 3; launching the
+// first four kernels the ordinary way in front of the graph, to hide that, gained nothing: 131.3 against 130.3 us for
+// ResNet-18 at batch 1.)
+//
+// The first pass runs eagerly: it allocates the tensors, and a program that runs once pays nothing.  What a pass does
+// beside launching - which side of a memory is current, which launches were left to a reader - is recorded as well, as the
+// state it leaves behind, and restored by a replay.  A record is dropped when an operator of the workspace is prepared or
+// destroyed, the workspace's stream changes, or a buffer it names has moved.
+#include <set>
+#include <vector>
+
+#include "hip_module.h"
+
+namespace {
+
+constexpr size_t kShortest = 8; // fewer kernels start sooner one by one (10 take 32 us as a graph, 54 one by one; 5 take 35 and 23)
+constexpr int kMaxRecords = 16; // a program that prepares or reallocates before every pass would record every second one for nothing
+
+// an input of the pass, as the record found it
+struct PassInput {
+    hip_mem_t *m;
+    enum { kDevice, kMirror, kQuantized } from; // the device side; the pinned mirror (the record uploads it); quantized bytes
+    const void *src, *dev;
+};
+
+// a memory that the pass writes, and the state it leaves behind
+struct PassOutput {
+    hip_mem_t *m;
+    void *dev, *host;
+    bool dev_valid, host_valid, down_issued;
+    void (*pending)(void *);
+    void *pending_ctx;
+};
+
+struct Pass {
+    uint64_t epoch = 0;
+    hipStream_t st = nullptr;
+    int runs = 0, records = 0;
+    hipGraphExec_t exec = nullptr;
+    std::vector<PassInput> in;
+    std::vector<PassOutput> out;
+    long counted[kHipCounters] = {};
+
+    void forget()
+    {
+        if (exec) {
+            HIPM_HIP(hipDeviceSynchronize()); // a replay may be under way, on a stream that may be gone
+            (void)hipGraphExecDestroy(exec);
+        }
+        exec = nullptr;
+        runs = 0;
+        in.clear();
+        out.clear();
+    }
+};
+
+bool capturing(hipStream_t st)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+
+// The inputs of the pass: memories that an operator reads before any has written them.  One that the host has just written and
+// that a kernel uploads is uploaded by the record.  false: not a pass that can be recorded.
+bool collect_inputs(Pass &p, op_t *const *ops, size_t n)
+{
+    std::set<const mem_t *> written, seen;
+    for (size_t i = 0; i < n; ++i) {
+        for (size_t k = 0; k < hip_op_activations(ops[i]); ++k) {
+            mem_t *mm = ops[i]->input_tensors[k]->mem;
+            if (written.count(mm))
+                continue;
+            if (!is_hip_mem(mm))
+                return false;
+            hip_mem_t *m = as_hip(mm);
+            if (!seen.insert(mm).second) {
+                for (const PassInput &in : p.in)
+                    if (in.m == m && in.from == PassInput::kQuantized && m->q_op != ops[i])
+                        return false; // read as values too: not worth a record's trouble
+                continue;
+            }
+            hip_mem_settle(m);
+            PassInput in = {m, PassInput::kDevice, nullptr, nullptr};
+            if (m->q_valid && m->q_op == ops[i]) {
+                in.from = PassInput::kQuantized;
+                in.src = m->qhost, in.dev = m->qdev;
+            } else if (m->host_valid && !m->dev_valid && m->host != nullptr && m->dev != nullptr && hip_mem_uploads_direct(m)) {
+                in.from = PassInput::kMirror;
+                in.src = m->host, in.dev = m->dev;
+            } else {
+                in.dev = hip_mem_dev_in(mm, p.st);
+            }
+            p.in.push_back(in);
+        }
+        for (size_t k = 0; k < ops[i]->output_size; ++k) {
+            mem_t *mm = ops[i]->output_tensors[k].mem;
+            if (!is_hip_mem(mm) || seen.count(mm)) // an operator writes what an earlier one reads: a view of an input
+                return false;
+            written.insert(mm);
+        }
+    }
+    return true;
+}
+
+void collect_outputs(Pass &p, op_t *const *ops, size_t n)
+{
+    std::set<hip_mem_t *> seen;
+    for (size_t i = 0; i < n; ++i)
+        for (size_t k = 0; k < ops[i]->output_size; ++k) {
+            hip_mem_t *m = as_hip(ops[i]->output_tensors[k].mem);
+            if (!seen.insert(m).second)
+                continue;
+            // what the host has fetched after an earlier pass it will fetch again: the record ends with the copy
+            if (m->host_read && m->host != nullptr && m->host_cap >= m->size && m->dev_valid && !m->host_valid && !m->pending
+                && !m->down_issued && m->size <= kHostDirect)
+                hip_mem_start_download(m);
+            p.out.push_back({m, m->dev, m->host, m->dev_valid, m->host_valid, m->down_issued, m->pending, m->pending_ctx});
+        }
+}
+
+bool record(Pass &p, op_t *const *ops, size_t n)
+{
+    if (!collect_inputs(p, ops, n))
+        return false;
+    std::vector<hip_mem_t> before_in;
+    for (const PassInput &in : p.in)
+        before_in.push_back(*in.m);
+    long before[kHipCounters];
+    for (int c = 0; c < kHipCounters; ++c)
+        before[c] = *hip_counters()[c];
+    if (hipStreamBeginCapture(p.st, hipStreamCaptureModeThreadLocal) != hipSuccess)
+        return false;
+    for (size_t i = 0; i < n; ++i)
+        op_run(ops[i]);
+    collect_outputs(p, ops, n);
+    hipGraph_t g = nullptr;
+    size_t nodes = 0;
+    bool ok = hipStreamEndCapture(p.st, &g) == hipSuccess && g != nullptr;
+    ok = ok && hipGraphGetNodes(g, nullptr, &nodes) == hipSuccess && nodes >= kShortest;
+    ok = ok && hipGraphInstantiate(&p.exec, g, nullptr, nullptr, 0) == hipSuccess;
+    if (g)
+        (void)hipGraphDestroy(g);
+    for (int c = 0; c < kHipCounters; ++c) {
+        p.counted[c] = *hip_counters()[c] - before[c];
+        *hip_counters()[c] = before[c];
+    }
+    if (!ok) { // nothing of it ran: the inputs are as they were, the operators write their outputs' state again
+        p.exec = nullptr;
+        for (size_t i = 0; i < p.in.size(); ++i)
+            *p.in[i].m = before_in[i];
+    }
+    return ok;
+}
+
+// everything the record names is where it was, and the inputs' contents are where it reads them
+bool still_good(const Pass &p)
+{
+    for (const PassInput &in : p.in) {
+        hip_mem_t *m = in.m;
+        hip_mem_settle(m);
+        if (in.from == PassInput::kQuantized) {
+            if (!m->q_valid || m->qhost != in.src || m->qdev != in.dev || (m->up_pending && m->up_stream != p.st))
+                return false;
+        } else if (in.from == PassInput::kMirror) {
+            if (!m->host_valid || m->host != in.src || m->dev != in.dev)
+                return false;
+        } else if (hip_mem_dev_in(&m->m, p.st) != in.dev) {
+            return false;
+        }
+    }
+    for (const PassOutput &o : p.out)
+        if (o.m->dev != o.dev || (o.down_issued && o.m->host != o.host))
+            return false;
+    return true;
+}
+
+} // namespace
+
+bool hip_pass_run(void **state, op_t *const *ops, size_t n)
+{
+    static const bool off = getenv("NART_HIP_NO_GRAPH") != nullptr;
+    hip_workspace_t *ws = reinterpret_cast<hip_workspace_t *>(ops[0]->workspace);
+    if (off || capturing(ws->stream))
+        return false;
+    if (*state == nullptr)
+        *state = new Pass;
+    Pass &p = *static_cast<Pass *>(*state);
+    if (p.epoch != ws->epoch || p.st != ws->stream) {
+        p.forget();
+        p.epoch = ws->epoch, p.st = ws->stream;
+    }
+    if (p.exec == nullptr) {
+        if (++p.runs < 2 || p.records >= kMaxRecords)
+            return false;
+        ++p.records;
+        if (!record(p, ops, n)) {
+            p.forget();
+            p.records = kMaxRecords;
+            return false;
+        }
+    } else if (!still_good(p)) {
+        p.forget();
+        return false;
+    }
+    HIPM_HIP(hipGraphLaunch(p.exec, p.st));
+    for (int c = 0; c < kHipCounters; ++c)
+        *hip_counters()[c] += p.counted[c];
+    for (const PassInput &in : p.in) {
+        if (in.from == PassInput::kDevice)
+            continue;
+        in.m->up_pending = true, in.m->up_stream = p.st; // the pass reads pinned memory
+        if (in.from == PassInput::kMirror)
+            in.m->dev_valid = true, in.m->down_issued = false, in.m->prod_stream = p.st;
+    }
+    for (const PassOutput &o : p.out) {
+        o.m->dev_valid = o.dev_valid, o.m->host_valid = o.host_valid, o.m->down_issued = o.down_issued, o.m->q_valid = false;
+        o.m->pending = o.pending, o.m->pending_ctx = o.pending_ctx;
+        o.m->prod_stream = p.st;
+    }
+    return true;
+}
+
+void hip_pass_drop(void *state)
+{
+    Pass *p = static_cast<Pass *>(state);
+    p->forget();
+    delete p;
+}

@@ -95,6 +95,33 @@ def test_float_network_ends_and_missing_modules(tmp_path):
     assert ctx2.loaded_workspaces == ["hip"]
 
 
+@pytest.mark.parametrize("build", [lambda: cases.resnet18(N=2, hw=96), lambda: cases.mobilenet_v2(N=1, hw=70), lambda: cases.resnet50(N=2, hw=64)])
+def test_recorded_passes_follow_their_inputs(tmp_path, build):
+    """The first pass runs operator by operator, the second is recorded, later ones replay the record: every one on new
+    inputs, with other GPU work and synchronisations between, with and without a new input, before and after a reshape."""
+    case = build()
+    ctx = art.create_context_for_target("hip")
+    parade = art.Parade(engine.write_engine(case), ctx)
+    inputs, outputs = art.get_empty_io(parade)
+    name, out = case.input.name, case.output.name
+    noise = torch.zeros(1 << 20, device="cuda")
+    for k in range(6):
+        print("pass", k, case.name, flush=True)
+        x = casecpu.random_input(case, k)
+        want = casecpu.run_case(case, x)[out].reshape(outputs[out].shape)
+        parade.run({name: x}, outputs)
+        assert np.array_equal(outputs[out].view(np.uint8), want.view(np.uint8)), k
+        noise.add_(1.0)
+        if k % 2:
+            torch.cuda.synchronize()
+        if k in (0, 3):  # the same input again, and what the input memory holds
+            parade.forward()
+            assert np.array_equal(parade._outputs[out].numpy().view(np.uint8), want.view(np.uint8)), k
+            assert np.array_equal(parade._inputs[name].numpy().view(np.uint8), x.view(np.uint8))
+        if k == 4:
+            assert parade.reshape({name: list(case.input.shape)}) is True
+
+
 @pytest.mark.parametrize("shape", [(1, 3, 5, 7), (3, 3, 70, 67), (2, 3, 431, 433), (5, 3, 640, 641)])
 def test_arrays_of_every_size_reach_the_device(shape):
     """Parade.run's way of an array to the GPU: below and above the sizes at which helper threads copy, the copy engine is used
