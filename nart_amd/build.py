@@ -1,6 +1,7 @@
 """Builds the native libraries of the package in-tree (no GPU needed: hipcc cross-compiles gfx950).
 
   nart_amd/lib/libhipq.so             HIP kernels + their C ABI (include/hipq.h)
+  nart_amd/lib/hipq_calls.so          the CPython extension behind hipq.py's per-call functions
   nart_amd/lib/libart.so              the minimal host core implementing the art C API (include/art/)
   nart_amd/lib/libart_module_hip.so   the `hip` case module (exports hip_module_tp)
 
@@ -161,6 +162,17 @@ def build_module(force=False, nart_tree=None, out_name="libart_module_hip.so"):
     return [out]
 
 
+def build_python(force=False):
+    """hipq_calls, the CPython extension behind hipq.py's per-call functions."""
+    import sysconfig
+    src = _glob("python", (".c",))
+    out = os.path.join(LIB, "hipq_calls.so")
+    if src and (force or not _newer(out, src + [os.path.join(INC, "hipq.h")])):
+        _run(["gcc", "-O2", "-std=gnu11", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_paths()["include"], "-I" + INC, "-o", out]
+             + src + ["-L" + LIB, "-lhipq", "-Wl,-rpath,$ORIGIN"])
+    return [out] if src else []
+
+
 def build_tools(force=False):
     """nart_promark, the command-line runner (counterpart of the reference's tools/promark.cpp); finds libart.so and
     the case modules next to itself."""
@@ -173,7 +185,7 @@ def build_tools(force=False):
 
 
 def build_all(force=False):
-    return [build_hipq(force)] + build_art(force) + build_tools(force)
+    return [build_hipq(force)] + build_python(force) + build_art(force) + build_tools(force)
 
 
 if __name__ == "__main__":

@@ -137,6 +137,28 @@ def _stream():
     return _stream()
 
 
+_CALLS = None
+
+
+def _calls():
+    """The extension nart_amd/csrc/python/hipq_calls.c, which takes tensors to the C ABI without ctypes."""
+    global _CALLS
+    if _CALLS is None:
+        import importlib.util
+        import torch
+        lib()
+        path = os.path.join(os.path.dirname(LIB_PATH), "hipq_calls.so")
+        if not os.path.exists(path):
+            raise HipqError("%s is missing: build it with `python -m nart_amd.build`" % path)
+        torch.cuda.current_stream()  # initialises the device, and fails with torch's own message where there is none
+        spec = importlib.util.spec_from_file_location("hipq_calls", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.init(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+        _CALLS = mod
+    return _CALLS
+
+
 def _ptr(t):
     return t.data_ptr() if t is not None else None
 
@@ -200,6 +222,7 @@ class Conv2d:
             check(lib().hipq_conv2d_plan_create_per_channel(C.byref(d), C.c_void_p(w.ctypes.data), bp,
                                                             C.c_void_p(wa_pc.ctypes.data), C.byref(h)))
         self.handle = h
+        self._address = h.value
         self.kernel = lib().hipq_conv2d_plan_kernel(h).decode()
         m = re.match(r"conv_mfma_i8_(\d+x\d+)", self.kernel)
         self._tile0 = TILE_INDEX.get(m.group(1), -1) if m else -1  # the built-in choice, for the tuner to return to
@@ -248,7 +271,9 @@ class Conv2d:
     def __call__(self, x, y=None, acc=None):
         if y is None:
             y = self.empty_output()
-        check(lib().hipq_conv2d_run(self.handle, _ptr(x), _ptr(y), _ptr(acc), _stream()))
+        rc = (_CALLS or _calls()).conv2d_run(self._address, x, y, acc)
+        if rc:
+            check(rc)
         return y
 
     def run_relu(self, x, y=None):
@@ -301,7 +326,7 @@ class Conv2d:
     def close(self):
         if self.handle:
             lib().hipq_conv2d_plan_destroy(self.handle)
-            self.handle = None
+            self.handle, self._address = None, 0
 
     def __del__(self):
         try:
@@ -363,72 +388,65 @@ def bottleneck_tail_run(mid, widen, x, residual, residual_first, res_alpha, res_
 
 
 def add_u8(a, b, y, ialpha0, izp0, ialpha1, izp1, oalpha, ozp, obits=8):
-    check(lib().hipq_add_u8(_ptr(a), _ptr(b), _ptr(y), a.numel(), ialpha0, izp0, ialpha1, izp1, oalpha, ozp, obits,
-                            _stream()))
+    rc = (_CALLS or _calls()).add_u8(a, b, y, ialpha0, izp0, ialpha1, izp1, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def eltwise_u8(ins, y, ialpha, izp, oalpha, ozp, operation=1, coeff=None, obits=8):
-    n = len(ins)
-    ptrs = (C.c_void_p * n)(*[t.data_ptr() for t in ins])
-    ia = np.ascontiguousarray(ialpha, np.float32)
-    iz = np.ascontiguousarray(izp, np.uint8)
-    cf = None if coeff is None else np.ascontiguousarray(coeff, np.float32)
-    check(lib().hipq_eltwise_u8(ptrs, n, C.c_void_p(cf.ctypes.data) if cf is not None else None,
-                                C.c_void_p(ia.ctypes.data), C.c_void_p(iz.ctypes.data), _ptr(y), y.numel(),
-                                operation, oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).eltwise_u8(ins, y, ialpha, izp, oalpha, ozp, operation, coeff, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def relu_u8(x, y, ialpha, izp, oalpha, ozp, obits=8):
-    check(lib().hipq_relu_u8(_ptr(x), _ptr(y), x.numel(), ialpha, izp, oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).relu_u8(x, y, ialpha, izp, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def concat_u8(ins, channels, y, ialpha, izp, oalpha, ozp, obits=8):
-    n = len(ins)
-    ptrs = (C.c_void_p * n)(*[t.data_ptr() for t in ins])
-    ch = np.ascontiguousarray(channels, np.int32)
-    ia = np.ascontiguousarray(ialpha, np.float32)
-    iz = np.ascontiguousarray(izp, np.uint8)
-    N, H, W, _ = y.shape
-    check(lib().hipq_concat_u8(ptrs, n, C.c_void_p(ch.ctypes.data), C.c_void_p(ia.ctypes.data), C.c_void_p(iz.ctypes.data),
-                               _ptr(y), N * H * W, oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).concat_u8(ins, channels, y, ialpha, izp, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def softmax_u8(x, y, Cc, ialpha, izp, oalpha, ozp, obits=8):
-    N, H, W, cs = x.shape
-    check(lib().hipq_softmax_u8(_ptr(x), _ptr(y), N * H * W, Cc, cs, ialpha, izp, oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).softmax_u8(x, y, Cc, ialpha, izp, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def pool_u8(x, y, Cc, kernel, pad, stride, method, ialpha, izp, oalpha, ozp, obits=8):
-    N, H, W, cs = x.shape
-    _, OH, OW, _ = y.shape
-    (kh, kw) = (kernel, kernel) if np.isscalar(kernel) else kernel
-    (ph, pw) = (pad, pad) if np.isscalar(pad) else pad
-    (sh, sw) = (stride, stride) if np.isscalar(stride) else stride
-    check(lib().hipq_pool_u8(_ptr(x), _ptr(y), N, Cc, H, W, OH, OW, cs, kh, kw, ph, pw, sh, sw, method, ialpha, izp,
-                             oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).pool_u8(x, y, Cc, kernel, pad, stride, method, ialpha, izp, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def quantize_u8(x_nchw, y, oalpha, ozp, obits=8):
-    N, Cc, H, W = x_nchw.shape
-    check(lib().hipq_quantize_u8(_ptr(x_nchw), _ptr(y), N, Cc, H, W, y.shape[-1], oalpha, ozp, obits, _stream()))
+    rc = (_CALLS or _calls()).quantize_u8(x_nchw, y, oalpha, ozp, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def quantize_i8(x_nchw, y, oalpha, obits=8):
-    N, Cc, H, W = x_nchw.shape
-    check(lib().hipq_quantize_i8(_ptr(x_nchw), _ptr(y), N, Cc, H, W, y.shape[-1], oalpha, obits, _stream()))
+    rc = (_CALLS or _calls()).quantize_i8(x_nchw, y, oalpha, obits)
+    if rc:
+        check(rc)
     return y
 
 
 def dequantize_i8(x, y_nchw, ialpha):
-    N, Cc, H, W = y_nchw.shape
-    check(lib().hipq_dequantize_i8(_ptr(x), _ptr(y_nchw), N, Cc, H, W, x.shape[-1], ialpha, _stream()))
+    rc = (_CALLS or _calls()).dequantize_i8(x, y_nchw, ialpha)
+    if rc:
+        check(rc)
     return y_nchw
 
 
@@ -440,6 +458,7 @@ def dequantize_i32(acc, y_nchw, alpha):
 
 
 def dequantize_u8(x, y_nchw, ialpha, izp):
-    N, Cc, H, W = y_nchw.shape
-    check(lib().hipq_dequantize_u8(_ptr(x), _ptr(y_nchw), N, Cc, H, W, x.shape[-1], ialpha, izp, _stream()))
+    rc = (_CALLS or _calls()).dequantize_u8(x, y_nchw, ialpha, izp)
+    if rc:
+        check(rc)
     return y_nchw
