@@ -57,6 +57,7 @@
 #include "conv_expand.h"
 #include "conv_dw.h"
 #include "conv_rows.h"
+#include "conv_stream.h"
 #include "conv_wreg.h"
 
 namespace hipq {
@@ -1027,214 +1028,6 @@ __global__ __launch_bounds__(256) void conv_mfma_pointwise_kernel(const ConvArgs
 }
 
 // ------------------------------------------------------------------------------------------------
-// Fully-connected layers and other 1x1 / stride 1 layers over a few hundred pixels at most (op_quant_ip_u8xu8_run,
-// art/modules/quant/src/op/ip.cpp:133-209, with the batch as the pixels).  Such a layer is a weight stream: every weight
-// byte is used once per pixel row and the weights are many times larger than the activations, so the time is the time
-// it takes to pull the weights out of HBM, and that takes every CU.  The tile kernels cannot give every CU a share (a
-// 128-row by 4096-column problem has 32 of their tiles); this kernel cuts the output into narrow column strips instead:
-//   * a work-group owns 16*NB output channels of 16*MB pixel rows and the whole reduction, on v_mfma_i32_16x16x64_i8:
-//     a weight fragment (16 rows of a 64-byte slab, 1 KB of the packed weights) is used by MB multiplies, a pixel
-//     fragment by NB, all of one wave;
-//   * the NW waves split the reduction in chunks of 128 bytes of k (two slabs: whole cache lines of the pixel rows), and
-//     each wave streams ITS chunks through LDS stages of its own, R deep, with the load unit (global_load_lds_dwordx4,
-//     eight lanes per 128-byte line: loading the MFMA operand straight into registers would make neighbouring lanes ask
-//     for 16 bytes of sixteen different rows, a quarter of the L1 rate).  No barrier in the loop: a wave waits for its
-//     own loads (vmcnt) and refills a stage once its own reads of it have returned (lgkmcnt);
-//   * 16-byte piece c of pixel row r sits at piece c ^ (r & 7) of its 128-byte LDS row, the blocks of eight rows are
-//     spaced so that rows r and r + 8 start in different halves of the banks, the weights keep their packed order: the
-//     fragment reads are free of bank conflicts;
-//   * the waves' partial sums meet once, in LDS, and the waves share the epilogue.
-// Requires in_cs % 128 == 0, weight zero point 128 (or int8), no fused residual: the host checks.
-template <int MB, int NB>
-struct StreamCfg {
-    static constexpr int ROWS = 16 * MB;
-    static constexpr int XI = ROWS / 8;            // pixel loads per chunk: 8 rows of 128 bytes each
-    static constexpr int PER = XI + 2 * NB;        // loads per chunk
-    // block j of 8 pixel rows sits at j * 1024 + ((j + 1) >> 1) * 128: the two blocks of a 16-row fragment start in
-    // different halves of the banks
-    static constexpr int XBYTES = XI * 1024 + (XI / 2 + 1) * 128;
-    static constexpr int STAGE = XBYTES + 2 * NB * 1024;
-    static constexpr int R0 = (160 * 1024) / (4 * STAGE);
-    static constexpr int R = R0 > 4 ? 4 : R0;      // stages per wave (four waves)
-    static_assert(R >= 2 && (R - 1) * PER <= 63, "stage count / vmcnt range");
-};
-
-// CONVX: any kernel size, stride and padding (a convolution over few pixels - the last stages of a network at batch 1 -
-// is the same weight stream): chunk c of a pixel's reduction is 128 bytes of the channels of ONE tap, read from the
-// neighbouring pixel that tap points at, or from the pad source where it points outside the image.
-template <int MB, int NB, bool CONVX>
-__global__ __launch_bounds__(256) void conv_mfma_stream_kernel(const ConvArgs a, const int mtiles)
-{
-    using Cfg = StreamCfg<MB, NB>;
-    constexpr int NW = 4, NT = MB * NB, R = Cfg::R, STAGE = Cfg::STAGE, PER = Cfg::PER, XI = Cfg::XI;
-    constexpr int WOFF = Cfg::XBYTES; // the weight slabs follow the pixel rows in a stage
-    static_assert(NW * R * STAGE >= NW * NT * 1024, "the stages double as the reduction buffer");
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[NW * R * STAGE];
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, q = lane >> 4;
-    // Work-groups go to the 8 XCDs in turn; the m-tiles of one column strip get consecutive numbers inside one XCD, so
-    // that the second reader of a strip's weights finds them in that XCD's L2.
-    const int idx = (int)blockIdx.x >> 3;
-    const int nt = (idx / mtiles) * 8 + ((int)blockIdx.x & 7), mt = idx % mtiles;
-    const int n0 = nt * (16 * NB), m0 = mt * (16 * MB);
-    if (n0 >= a.out_cs)
-        return;
-
-    const int nch = a.nslab >> 1;                                // chunks of two slabs
-    const int cnt = wave < nch ? (nch - wave + NW - 1) / NW : 0; // chunks of this wave
-    // Every work-group reads the same pixel rows: each starts the reduction at a different chunk, so that they do not
-    // all ask for the same lines at the same time (the order of an exact integer sum is free).
-    const int rot = (nt * 7 + mt * 3) % nch;
-    auto chunk_of = [&](int t) {
-        int c = wave + NW * t + rot;
-        return c >= nch ? c - nch : c;
-    };
-    uint8_t *const wl = lds + wave * (R * STAGE);
-    // load lane l of pixel instruction j: row 8 j + (l >> 3), LDS piece l & 7 = logical piece (l & 7) ^ (row & 7)
-    const int xrow = lane >> 3, xoff = ((lane & 7) ^ xrow) << 4;
-    const uint8_t *wsrc = a.wpack + (size_t)n0 * 64 + lane * 16;
-    const size_t wslab = (size_t)a.kout_pad * 64;
-    // CONVX: this lane's pixel of load j - first input row and column of its window, pixel index of its image's origin
-    int wih[CONVX ? XI : 1], wiw[CONVX ? XI : 1], wpix[CONVX ? XI : 1];
-    if (CONVX) {
-        const int ohw = a.OH * a.OW;
-#pragma unroll
-        for (int j = 0; j < XI; j++) {
-            const int m = min(m0 + 8 * j + xrow, a.P - 1);
-            const int n = fast_div(m, ohw, a.inv_ohw), rem = m - n * ohw;
-            const int oh = fast_div(rem, a.OW, a.inv_ow), ow = rem - oh * a.OW;
-            wih[j] = oh * a.stride_h - a.pad_h, wiw[j] = ow * a.stride_w - a.pad_w, wpix[j] = n * a.H * a.W;
-        }
-    }
-    const int cpt = a.in_cs >> 7; // chunks per tap
-    auto issue = [&](int t) {
-        const int chunk = chunk_of(t);
-        uint8_t *st = wl + (t % R) * STAGE;
-        if (CONVX) {
-            const int tap = chunk / cpt, coff = (chunk - tap * cpt) * 128 + xoff;
-            const int kr = tap / a.S, ks = tap - kr * a.S;
-#pragma unroll
-            for (int j = 0; j < XI; j++) {
-                const int ih = wih[j] + kr, iw = wiw[j] + ks;
-                const bool ok = (unsigned)ih < (unsigned)a.H && (unsigned)iw < (unsigned)a.W;
-                const uint8_t *src = ok ? a.x + (uint32_t)((wpix[j] + ih * a.W + iw) * a.in_cs + coff) : a.padbuf + (xoff & 48);
-                __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(st + j * 1024 + ((j + 1) >> 1) * 128), 16, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < XI; j++) {
-                const int m = min(m0 + 8 * j + xrow, a.P - 1); // rows beyond the last pixel repeat it; their results are dropped
-                const uint8_t *src = a.x + (uint32_t)(m * a.in_cs + chunk * 128 + xoff);
-                __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(st + j * 1024 + ((j + 1) >> 1) * 128), 16, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-                __builtin_amdgcn_global_load_lds((gptr_t)(wsrc + (size_t)(2 * chunk + h) * wslab + nb * 1024),
-                                                 (lptr_t)(st + WOFF + (h * NB + nb) * 1024), 16, 0, 0);
-    };
-
-    v4i acc[MB][NB];
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-            acc[mb][nb] = v4i{0, 0, 0, 0};
-
-    for (int u = 0; u < R - 1 && u < cnt; u++)
-        issue(u);
-    // fragment addresses inside a stage: weights in packed order; pixel row 16 mb + r lives in block 2 mb + (r >> 3)
-    // (rows r and r + 8 fall into different halves of the banks), piece (4 h + q) of the row at piece ^ (r & 7)
-    const int wfo = WOFF + r * 64 + ((q ^ ((r >> 2) & 3)) << 4);
-    const int xfo = (r >> 3) * 1152 + (r & 7) * 128; // + 2176 per 16-row fragment
-    for (int t = 0; t < cnt; t++) {
-        // this wave's fragment reads of chunk t - 1 have returned (the load unit's LDS writes are not ordered against
-        // pending reads), then its stage is refilled
-        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
-        if (t + R - 1 < cnt)
-            issue(t + R - 1);
-        const int ahead = min(R - 1, cnt - 1 - t); // chunks younger than t in flight
-        if (ahead >= 3)
-            wait_vmcnt<3 * PER>();
-        else if (ahead == 2)
-            wait_vmcnt<(R > 2 ? 2 : 0) * PER>();
-        else if (ahead == 1)
-            wait_vmcnt<PER>();
-        else
-            wait_vmcnt<0>();
-        const uint8_t *st = wl + (t % R) * STAGE;
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            v4i wf[NB];
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-                wf[nb] = *reinterpret_cast<const v4i *>(st + wfo + (h * NB + nb) * 1024);
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                const v4i xs = *reinterpret_cast<const v4i *>(st + mb * 2176 + xfo + (((4 * h + q) ^ (r & 7)) << 4)) ^ (int)a.xmask;
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    acc[mb][nb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wf[nb], xs, acc[mb][nb], 0, 0, 0);
-            }
-        }
-    }
-
-    // ---- the waves' partial sums meet in LDS; wave w finishes the tiles w, w + NW, ...
-    __syncthreads(); // every wave is done with its stages; no load is in flight any more
-    int32_t *red = reinterpret_cast<int32_t *>(lds); // [wave][tile][register][lane]
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                red[((wave * NT + mb * NB + nb) * 4 + v) * 64 + lane] = acc[mb][nb][v];
-    __syncthreads();
-#pragma unroll
-    for (int tl = 0; tl < (NT + NW - 1) / NW; tl++) {
-        const int tile = wave + tl * NW;
-        if (tile >= NT)
-            break;
-        const int mb = tile / NB, nb = tile % NB;
-        const int m = m0 + mb * 16 + r, ko = n0 + nb * 16 + 4 * q; // this lane: 4 consecutive channels of one pixel
-        const v4i bias = *reinterpret_cast<const v4i *>(a.bias2 + ko);
-        int32_t v[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            uint32_t s = (uint32_t)bias[e];
-#pragma unroll
-            for (int w = 0; w < NW; w++)
-                s += (uint32_t)red[((w * NT + tile) * 4 + e) * 64 + lane];
-            v[e] = (int32_t)s;
-        }
-        if (m >= a.P || ko >= a.out_cs)
-            continue;
-        if (a.acc_out != nullptr)
-            *reinterpret_cast<v4i *>(a.acc_out + (size_t)m * a.out_cs + ko) = v4i{v[0], v[1], v[2], v[3]};
-        int32_t rq[4];
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            rq[e] = a.qmult ? conv_requant_ch(a, v[e], ko + e) : a.fastq ? conv_requant<true>(a, v[e]) : conv_requant<false>(a, v[e]);
-        if (a.deq_out != nullptr) { // fused dequantize (op_dequantize_run_u8, art/modules/quant/src/op/dequantize.c:111-123)
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (ko + e < a.K)
-                    a.deq_out[(size_t)m * a.K + ko + e] = __fmul_rn((float)(rq[e] - a.q.zp), a.deq_alpha);
-            continue;
-        }
-        uint32_t packed = pack_low_bytes(rq[0], rq[1], rq[2], rq[3]);
-        if (a.res) { // fused residual add: exactly what the add operator computes from the convolution's stored bytes
-            const uint32_t rv = *reinterpret_cast<const uint32_t *>(a.res + (size_t)m * a.out_cs + ko);
-            packed = a.res_first ? add_dword<false>(rv, packed, a.addq) : add_dword<false>(packed, rv, a.addq);
-        }
-        *reinterpret_cast<uint32_t *>(a.y + (size_t)m * a.out_cs + ko) = packed;
-    }
-}
-
-// ------------------------------------------------------------------------------------------------
 // Depthwise 3x3 (group == C == K, stride 1 or 2): HBM-bound on paper (16 bytes in, 16 bytes out per output pixel and
 // 16 channels), in practice bounded by vector ALU work, so the kernel is written for instruction count.
 // One thread owns 4 channels (one dword of the channels-last tensors) of a strip of 4 output pixels along W; a
@@ -1502,11 +1295,6 @@ struct TileShape {
 static const TileShape kTiles[] = {{128, 128}, {256, 64}, {128, 64}, {64, 128}, {64, 64}};
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// conv_mfma_stream_kernel: a work-group's share is 16 * mb pixel rows by 16 * nb output channels, nw waves
-struct StreamShape {
-    int mb, nb, nw;
-};
-
 struct hipq_conv2d_plan {
     hipq_conv2d_desc d;
     ConvArgs args;
@@ -1550,43 +1338,66 @@ static bool pointwise_applies(const hipq_conv2d_plan *p)
 constexpr int kCUs = 256;
 static bool k2_applies(const hipq_conv2d_plan *p);
 
-// conv_mfma_stream_kernel: layers over at most 256 pixels (fully-connected layers: the pixels are the batch; the last
-// stages of a network at batch 1) whose pixels are whole 128-byte lines, weight zero point 128 (or int8).  Shape of a work-group's share: 16 * mb
-// pixel rows by 16 * nb output channels.  A strip that holds every pixel row reads each weight byte once; two m-tiles
-// per strip halve the pixel bytes a CU pulls through its L1 (what bounds the kernel once the weights stream at full
-// rate) and read the weights twice, the second time from L2.
+// Microseconds that the tile kernels take on a plan, as fitted to layers over 6 to 6 272 pixels: a launch, and a step per slab
+// of the reduction whose length is a round trip and hardly depends on how many of the CUs have a tile; from one tile per CU
+// on, the steps of a CU's tiles overlap in part.  The two-group kernel walks two slabs a step.
+static double tile_cost(const hipq_conv2d_plan *p)
+{
+    const ConvArgs &a = p->args;
+    const TileShape &t = kTiles[p->tile];
+    const double per_cu = (double)a.nbm * a.nbn / kCUs, crowd = per_cu > 1 ? 1 + 0.6 * (per_cu - 1) : 1;
+    if (k2_applies(p))
+        return 2.9 + 0.17 * a.nslab * crowd;
+    const double step = t.bm + t.bn <= 128 ? 0.22 : t.bm + t.bn <= 192 ? 0.31 : 0.5;
+    return 2.6 + (p->has_wzp ? 1.4 : 1.0) * step * a.nslab * crowd;
+}
+
+// The streaming kernel's, for one shape of its work-groups: LDS holds one work-group per CU, each round starts anew (1.5 us), pulls
+// (16 mb + 16 nb) rows of the reduction through the CU's L1 at 42 KB/us and ends with
+// an epilogue (0.8 us for the largest shape).
+static double stream_cost(const hipq_conv2d_plan *p, const StreamShape &c)
+{
+    const ConvArgs &a = p->args;
+    const long long wgs = (long long)((a.P + 16 * c.mb - 1) / (16 * c.mb)) * ((a.out_cs + 16 * c.nb - 1) / (16 * c.nb));
+    const double kb = 16.0 * (c.mb + c.nb) * a.nslab * 64 / 1000;
+    return 1.2 + (double)((wgs + kCUs - 1) / kCUs) * (1.5 + kb / 42 + 0.0125 * c.mb * c.nb * c.mb * c.nb);
+}
+
+// conv_mfma_stream_kernel: layers that the tile kernels would walk with a few tiles in many steps - fully-connected layers, the
+// last stages of a network at a small batch, layers with few output channels.  It takes what the two costs above say.  (Both
+// within 15 % on the layers they were fitted to; up to 256 pixels whatever the layer and up to 1024 with a reduction of 512
+// bytes, the rule before, was 12.1 against 6 us on 512 -> 2048 channels over 539 pixels and left 230 -> 24 channels, 3x3, over
+// 1568 to the tile kernels: 11.5 us, now 8.7.)
 static bool stream_applies(const hipq_conv2d_plan *p, StreamShape *shape = nullptr)
 {
-    const hipq_conv2d_desc &d = p->d;
-    const ConvArgs &a = p->args;
-    // up to 256 pixels whatever the layer; up to 1024 where the reduction is at least 512 bytes long (measured against the
-    // tile kernels: 3x3 on 784 pixels 4.8 against 7.0 us at 128 channels, 6.2 against 10.7 at 256, 12.3 against 18.4 at
-    // 512; 1x1 1024 -> 256 on 784 pixels 3.9 against 6.3; behind from 1568 pixels on, and at 256 -> 1024 from 392)
-    if (!(p->special && !p->tile_selected && p->variant == kMfma && !p->has_wzp && d.in_cs % 128 == 0
-          && (a.P <= 256 || (a.P <= 1024 && d.R * d.S * d.in_cs >= 512)) && (long long)d.N * d.H * d.W * d.in_cs < (1ll << 31)))
+    if (!(p->special && !p->tile_selected && p->variant == kMfma && p->args.R * p->args.S <= 255 && p->args.Ktot < (1 << 22)))
         return false;
-    if (shape) {
-        if (p->stream.mb) {
+    // Where the tile kernels' aligned addressing and the two-group kernel serve a layer well - 3x3 layers on 64-byte lines with a
+    // short reduction, 1x1 layers on an image whose last slab is partial - they keep it.
+    const ConvArgs &a = p->args;
+    const bool point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
+    if (!p->has_wzp && !fc
+        && (point ? a.in_cs % 64 != 0 && a.nslab % 2 == 0 && a.nslab >= 8 : a.in_cs % 128 == 64 && a.nslab <= 16))
+        return false;
+    if (p->stream.mb) { // named by the caller
+        if (shape)
             *shape = p->stream;
-            return true;
-        }
-        // What a CU pulls through its L1 bounds the kernel once the weights stream at full rate: per work-group
-        // (16 mb + 16 nb) rows of k bytes, times the rounds of work-groups the chip needs.  The smallest product wins,
-        // more work-groups on a tie (measured: 128 x 4096 x 4096 takes 8.6 us as 64 x 32, 11.3 as 128 x 16, 10.1 as
-        // 32 x 32; 64 x 2048 x 1000 takes 3.5 us as 16 x 16, 4.7 as 64 x 16).
-        static const StreamShape cand[] = {{8, 1, 4}, {4, 2, 4}, {4, 1, 4}, {2, 2, 4}, {2, 1, 4}, {1, 2, 4}, {1, 1, 4}};
-        const int rows = (a.P + 15) / 16;
-        long long best = -1, best_wgs = 0;
-        for (const StreamShape &c : cand) {
-            if (c.mb > 1 && c.mb / 2 >= rows)
-                continue; // half of the rows would be padding
-            const long long wgs = (long long)((rows + c.mb - 1) / c.mb) * ((a.out_cs + 16 * c.nb - 1) / (16 * c.nb));
-            const long long cost = ((wgs + kCUs - 1) / kCUs) * (c.mb + c.nb);
-            if (best < 0 || cost < best || (cost == best && wgs > best_wgs))
-                best = cost, best_wgs = wgs, *shape = c;
+        return true;
+    }
+    static const StreamShape cand[] = {{8, 1, 4}, {4, 2, 4}, {4, 1, 4}, {2, 2, 4}, {2, 1, 4}, {1, 2, 4}, {1, 1, 4}};
+    const int rows = (p->args.P + 15) / 16;
+    double best = 1e9;
+    for (const StreamShape &c : cand) {
+        if (c.mb > 1 && c.mb / 2 >= rows)
+            continue; // half of the rows would be padding
+        const double cost = stream_cost(p, c);
+        if (cost < best - 1e-9) {
+            best = cost;
+            if (shape)
+                *shape = c;
         }
     }
-    return true;
+    return best < 0.95 * tile_cost(p);
 }
 
 // conv_mfma_expand_kernel (conv_expand.hip): a 1x1 layer that widens the channels, for this launch's arguments (with a
@@ -1783,7 +1594,9 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
         // weights: [slab][kout_pad][64 bytes]; chunk c of row ko is stored at chunk c ^ ((ko >> 2) & 3),
         // the order the kernel keeps in LDS.  Rows of pad output channels stay zero (their outputs are
         // don't-care bytes in the pad channels of y).
-        wbuf.assign((size_t)a.nslab * a.kout_pad * 64, 0);
+        // An odd number of slabs is followed by one of padding slots: the streaming kernel takes two at a time.
+        const int packed = (a.nslab + 1) / 2 * 2;
+        wbuf.assign((size_t)packed * a.kout_pad * 64, 0);
         bbuf.assign((size_t)a.kout_pad, 0);
         for (int ko = 0; ko < d.K; ko++) {
             long long wsum = 0;
@@ -1804,6 +1617,8 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
                 const int slab = kp >> 6, chunk = ((kp >> 4) & 3) ^ ((ko >> 2) & 3);
                 wbuf[((size_t)slab * a.kout_pad + ko) * 64 + chunk * 16 + (kp & 15)] = (uint8_t)(int8_t)ws;
             }
+            if (packed > a.nslab)
+                memset(&wbuf[((size_t)a.nslab * a.kout_pad + ko) * 64], (uint8_t)(int8_t)-boff, 64);
             const long long c0 = (bias ? (long long)bias[ko] : 0) + (long long)aoff * wsum
                 + (long long)a.nslab * 64 * aoff * boff;
             bbuf[ko] = (int32_t)(uint32_t)(unsigned long long)c0;
@@ -2130,28 +1945,8 @@ static void launch_mfma(const hipq_conv2d_plan *p, const ConvArgs &a, hipStream_
     if (p->variant == kMfma && !streams && launch_halo<BM, BN, WM, WN>(p, a, grid, st))
         return;
     if (streams) {
-        const bool fc = a.R == 1 && a.S == 1 && a.stride_h == 1 && a.stride_w == 1 && a.pad_h == 0 && a.pad_w == 0;
-        const int mtiles = (a.P + 16 * ss.mb - 1) / (16 * ss.mb), ntiles = (a.out_cs + 16 * ss.nb - 1) / (16 * ss.nb);
-        const dim3 sgrid((ntiles + 7) / 8 * 8 * mtiles);
-        const int key = ss.mb * 100 + ss.nb * 10 + ss.nw;
-        switch (key) {
-#define HIPQ_STREAM_CASE(MB_, NB_)                                                                                       \
-    case MB_ * 100 + NB_ * 10 + 4:                                                                                      \
-        if (fc)                                                                                                         \
-            hipLaunchKernelGGL((conv_mfma_stream_kernel<MB_, NB_, false>), sgrid, dim3(256), 0, st, a, mtiles);         \
-        else                                                                                                            \
-            hipLaunchKernelGGL((conv_mfma_stream_kernel<MB_, NB_, true>), sgrid, dim3(256), 0, st, a, mtiles);          \
-        return;
-            HIPQ_STREAM_CASE(8, 1)
-            HIPQ_STREAM_CASE(4, 2)
-            HIPQ_STREAM_CASE(4, 1)
-            HIPQ_STREAM_CASE(2, 2)
-            HIPQ_STREAM_CASE(2, 1)
-            HIPQ_STREAM_CASE(1, 2)
-            HIPQ_STREAM_CASE(1, 1)
-#undef HIPQ_STREAM_CASE
-        default: break; // an unknown forced shape: the tile kernels below
-        }
+        if (launch_conv_stream(a, ss, st))
+            return; // an unknown forced shape: the tile kernels below
     }
     if (pointwise_applies(p) && a.acc_out == nullptr && a.res == nullptr) {
         // persistent work-groups (four waves, a strip of 32 pixels each per turn), five to a CU

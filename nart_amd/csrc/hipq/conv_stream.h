@@ -1,0 +1,16 @@
+// Convolutions over few pixels as a weight stream (conv_stream.hip).
+#pragma once
+
+#include "conv_shared.h"
+
+namespace hipq {
+
+// a work-group's share: 16 * mb pixels by 16 * nb output channels, nw waves
+struct StreamShape {
+    int mb, nb, nw;
+};
+
+// false: no instantiation for this shape, nothing launched
+bool launch_conv_stream(const ConvArgs &a, const StreamShape &s, hipStream_t st);
+
+} // namespace hipq

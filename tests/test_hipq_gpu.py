@@ -439,6 +439,35 @@ def test_streaming_kernel_on_convolutions_over_few_pixels():
         assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), conv), (i, plan.kernel)
 
 
+@pytest.mark.parametrize("wzp", [128, 101])
+def test_streaming_kernel_on_any_channel_count(wzp):
+    """Channel strides that are no multiple of 128 bytes (pieces that straddle two taps' chunks, a last chunk that is half or one
+    sixteenth full, an odd number of slabs), column strips fewer than XCDs, weight zero points other than 128, int8."""
+    rng = np.random.default_rng(wzp)
+    cases = [  # N, C, H, W, K, R, pad, stride
+        (6, 7307, 1, 1, 11, 1, 0, 1), (33, 1190, 1, 1, 300, 1, 0, 1), (3, 260, 1, 1, 1000, 1, 0, 1), (1, 529, 7, 8, 38, 3, 1, 2),
+        (10, 230, 20, 15, 24, 3, 1, 1), (16, 48, 14, 14, 64, 3, 1, 1), (4, 200, 14, 13, 300, 3, 1, 1), (2, 64, 28, 28, 64, 5, 2, 1),
+        (1, 150, 9, 9, 17, 3, 0, 1), (2, 130, 6, 7, 40, 5, 2, 2),
+    ]
+    seen = set()
+    for i, (N, C, H, W, K, R, pad, st) in enumerate(cases):
+        print("case", i, N, C, H, W, K, R, flush=True)
+        x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+        w = rng.integers(0, 256, (K, C, R, R), dtype=np.uint8)
+        b = rng.integers(-30000, 30000, K).astype(np.int32)
+        ia, wa = rand_q(rng), rand_q(rng)
+        q = (ia, int(rng.integers(0, 256)), wa, wzp, float(np.float32(ia * wa * np.sqrt(C * R * R) * 40.0)), int(rng.integers(0, 256)))
+        kern = check_conv(x, w, b, pad, st, 1, q, tag="any channels %d" % i)
+        assert "_stream_" in kern, kern
+        seen.add(kern)
+        if wzp == 128:
+            xs, ws = x.view(np.int8), w.view(np.int8)
+            p8 = hipq.Conv2d(x.shape, ws, b, pad, st, 1, q[0], 0, q[2], 0, q[4], 0, obits=7, dtype=hipq.DTYPE_I8)
+            want8 = orc.conv2d_i8(xs, ws, b, pad, st, 1, q[0], q[2], q[4], 7)
+            assert np.array_equal(hipq.from_device_nhwc(p8(hipq.to_device_nhwc(xs)), K).view(np.int8), want8), i
+    assert len(seen) >= 3, seen
+
+
 def test_output_stride_wider_than_the_channels():
     """A caller may write a convolution's output into a buffer with a wider channel stride than the layout rule gives
     (hipq_conv2d_desc.out_cs): the packed weights and folded constants cover every output-channel tile of that stride."""
