@@ -56,6 +56,7 @@
 #include "conv_block.h"
 #include "conv_expand.h"
 #include "conv_dw.h"
+#include "conv_hreg.h"
 #include "conv_rows.h"
 #include "conv_stream.h"
 #include "conv_wreg.h"
@@ -1347,7 +1348,7 @@ static double tile_cost(const hipq_conv2d_plan *p)
     const TileShape &t = kTiles[p->tile];
     const double per_cu = (double)a.nbm * a.nbn / kCUs, crowd = per_cu > 1 ? 1 + 0.6 * (per_cu - 1) : 1;
     if (k2_applies(p))
-        return 2.9 + 0.17 * a.nslab * crowd;
+        return 2.9 + (t.bm + t.bn <= 128 ? 0.17 : t.bm + t.bn <= 192 ? 0.22 : 0.42) * a.nslab * crowd;
     const double step = t.bm + t.bn <= 128 ? 0.22 : t.bm + t.bn <= 192 ? 0.31 : 0.5;
     return 2.6 + (p->has_wzp ? 1.4 : 1.0) * step * a.nslab * crowd;
 }
@@ -1428,9 +1429,27 @@ static bool wreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
     // on the other 1x1 layers and on larger images
     if (a.P > 16384 || a.P <= 1024)
         return false;
-    if (a.R == 3)
-        return true;
+    if (a.R == 3) // the patches of a ragged image must not be half empty
+        return 2 * a.OH * a.OW >= ((a.OH + 6) / 7) * ((a.OW + 6) / 7) * 49;
     return a.res == nullptr && a.stride_h == 1 && a.in_cs >= 4 * a.out_cs;
+}
+
+// conv_hreg_kernel (conv_hreg.hip): 3x3 / stride 1 / pad 1 with the pixels in LDS and the weights in registers, any image size.
+// Over more than 512 pixels it is ahead of the register-fed kernel's patches (256 -> 256 at 14x14, batch 64: 12.7 -> 11.2 us)
+// and, by the fitted costs, of the tile and streaming kernels (13x13, batch 11: 9.2 -> 5.3 us).  64-channel layers keep their
+// resident rows but for 32 000 to 90 000 pixels (56x56, batch 12, with the add: 7.4 -> 6.6 us; level at 100 000, 24 against
+// 15 us at 200 000, where the halo of a tile outweighs its nine steps), and up to 4 096 pixels the halo kernel.
+static bool hreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
+{
+    double us = 0;
+    if (!(p->variant == kMfma && p->special == 1 && !p->tile_selected && !p->has_wzp && a.P > 512 && conv_hreg_applies(a, &us)))
+        return false;
+    if (a.in_cs == 64 && (a.P <= 4096 || (rows_applies(p, a) && (a.P < 32000 || a.P > 90000))))
+        return false;
+    if (wreg_applies(p, a))
+        return true;
+    StreamShape s;
+    return us < 0.9 * (stream_applies(p, &s) ? stream_cost(p, s) : tile_cost(p));
 }
 
 // conv_stem3x3_kernel (conv_stem.hip): 3x3 / stride 2 from an image with at most 4 channels to at most 32
@@ -1443,7 +1462,9 @@ static void set_mfma_name(hipq_conv2d_plan *p, bool smallc)
 {
     char nm[96];
     StreamShape ss;
-    if (!smallc && wreg_applies(p, p->args))
+    if (!smallc && hreg_applies(p, p->args))
+        snprintf(nm, sizeof nm, "conv_mfma_i8_hreg3x3");
+    else if (!smallc && wreg_applies(p, p->args))
         snprintf(nm, sizeof nm, "conv_mfma_i8_wreg");
     else if (!smallc && stream_applies(p, &ss))
         snprintf(nm, sizeof nm, "conv_mfma_i8_stream_%dx%d%s", 16 * ss.mb, 16 * ss.nb, p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
@@ -1761,7 +1782,9 @@ extern "C" const char *hipq_conv2d_plan_kernel_add(const hipq_conv2d_plan *p)
     a.addq.hi = 255;  // to 8 bits
     char buf[96];
     StreamShape ss;
-    if (wreg_applies(p, a))
+    if (hreg_applies(p, a))
+        snprintf(buf, sizeof buf, "conv_mfma_i8_hreg3x3+add");
+    else if (wreg_applies(p, a))
         snprintf(buf, sizeof buf, "conv_mfma_i8_wreg+add");
     else if (stream_applies(p, &ss))
         snprintf(buf, sizeof buf, "conv_mfma_i8_stream_%dx%d%s+add", 16 * ss.mb, 16 * ss.nb, p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
@@ -2108,6 +2131,15 @@ extern "C" int hipq_conv2d_run_add_conv(const hipq_conv2d_plan *p, const void *x
     HIPQ_REQUIRE(hipq_conv2d_add_conv_fusable(p, residual_is_input0, res_alpha, res_zp, oalpha, ozp, obits, next),
                  "hipq_conv2d_run_add_conv: these two plans (%s, then %s) do not run as one kernel: run hipq_conv2d_run_add and "
                  "hipq_conv2d_run", p->name.c_str(), next->name.c_str());
+    // A work-group takes 128 pixels through all of both layers, 9 us and more for 64 -> 256 -> 64 and 17 for 128 -> 512 -> 128
+    // however few there are; the two layers on their own spread over the chip.  Level at 20 000 pixels; 6 900 pixels of the
+    // latter: 17.7 us as one launch, 9.6 as two.  (Mode 2 asks for the kernel wherever it applies.)
+    if (p->args.P < 20000 && p->special != 2) {
+        const int rc = hipq_conv2d_run_add(p, x, residual, residual_is_input0, res_alpha, res_zp, oalpha, ozp, obits, y, stream);
+        if (rc != 0)
+            return rc;
+        return next_relu ? hipq_conv2d_run_relu(next, y, y_next, stream) : hipq_conv2d_run(next, y, y_next, nullptr, stream);
+    }
     ConvArgs a, a2 = next->args;
     add_args(p, residual_is_input0, res_alpha, res_zp, oalpha, ozp, obits, &a);
     a.x = static_cast<const uint8_t *>(x);
@@ -2387,6 +2419,10 @@ static int run_conv(const hipq_conv2d_plan *p, ConvArgs &a, hipStream_t st)
     switch (p->variant) {
     case kMfma:
     case kMfmaSmallC:
+        if (hreg_applies(p, a)) {
+            launch_conv_hreg(a, st); // 3x3, any image size: the pixels in LDS once, weight operands straight into registers
+            break;
+        }
         if (wreg_applies(p, a)) {
             launch_conv_wreg(a, st); // few pixels: the pixel operand in LDS once, weight operands straight into registers
             break;

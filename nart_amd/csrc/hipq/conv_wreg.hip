@@ -20,7 +20,7 @@
 //     stores 16 bytes.
 // Requirements (checked by the host): uint8 tensors, weight zero point 128, per-tensor scale, one-multiply
 // requantisation, dense channel strides, input channels a multiple of 64 (1x1: 256, 512, 1024 or 2048; 3x3: 128, 256 or
-// 512), output channels a multiple of 128; 3x3: pad 1, output height and width multiples of 7.
+// 512), output channels a multiple of 128; 3x3: pad 1.
 #include "conv_wreg.h"
 
 #include <algorithm>
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256, 2) void conv_wreg_kernel(const ConvArgs a, con
         const int q = 32 * t + p;
         if (TAPS == 9) {
             const int qq = min(q, kWregPatch * kWregPatch - 1), py = (qq * 37) >> 8, px = qq - py * kWregPatch; // qq / 7 for qq < 49
-            valid[t] = q < kWregPatch * kWregPatch;
+            valid[t] = q < kWregPatch * kWregPatch && y0 + py < a.OH && x0 + px < a.OW; // patches may reach beyond the image
             prow[t] = S * py * GW + S * px;
             pix[t] = (size_t)((n * a.OH + y0 + py) * a.OW + x0 + px);
         } else {
@@ -303,7 +303,7 @@ bool conv_wreg_applies(const ConvArgs &a)
     if (a.R == 1 && a.S == 1)
         return a.pad_h == 0 && a.pad_w == 0 && (cpt == 4 || cpt == 8 || cpt == 16 || cpt == 32);
     return a.R == 3 && a.S == 3 && a.pad_h == 1 && a.pad_w == 1 && (cpt == 2 || cpt == 4 || cpt == 8) && a.res == nullptr
-        && a.OH % kWregPatch == 0 && a.OW % kWregPatch == 0;
+        && (long long)a.N * a.H * a.W * a.in_cs < (1ll << 31);
 }
 
 template <int CPT, int TAPS, int S>
@@ -311,7 +311,7 @@ static void launch_wreg(const ConvArgs &a, hipStream_t st)
 {
     WregGeom geo;
     geo.nnb = a.out_cs / 128, geo.nbpw = 1;
-    geo.PY = a.OH / kWregPatch, geo.PX = a.OW / kWregPatch;
+    geo.PY = (a.OH + kWregPatch - 1) / kWregPatch, geo.PX = (a.OW + kWregPatch - 1) / kWregPatch;
     geo.npg = TAPS == 9 ? a.N * geo.PY * geo.PX : (a.P + 63) / 64;
     const dim3 grid((unsigned)((geo.npg * geo.nnb + 7) / 8 * 8)), block(256);
     if constexpr (TAPS == 1) {

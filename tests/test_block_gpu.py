@@ -338,6 +338,62 @@ def test_register_fed_convolution(case):
                 assert np.array_equal(gota, wanta), (case, "add", res_first, int((gota != wanta).sum()))
 
 
+HREG_CASES = [  # N, C, H, W, K
+    (11, 256, 13, 13, 256), (3, 128, 17, 29, 200), (2, 512, 17, 19, 200), (1, 64, 70, 71, 48), (5, 64, 101, 9, 144), (25, 64, 40, 40, 64),
+    (900, 512, 1, 1, 256), (20, 256, 2, 40, 128), (64, 256, 14, 14, 256), (40, 128, 25, 26, 128), (1, 128, 90, 91, 128),
+]
+
+
+@pytest.mark.parametrize("case", HREG_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_register_fed_convolution_on_any_image(case):
+    """conv_hreg_kernel against the oracle's convolution and convolution + add: tiles of 32, 64 and 128 pixels that end inside an
+    image, a row or behind the last pixel, images of one pixel, one or two rows, taps that must not leak across borders,
+    channel groups that are partly outside the output, both operand orders of the add, a ReLU."""
+    N, C, H, W, K = case
+    rng = np.random.default_rng(sum(case))
+    x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (K, C, 3, 3), dtype=np.uint8)
+    sigma = 74.0 * 74.0 * math.sqrt(C * 9)
+    b = rng.integers(-int(sigma), int(sigma) + 1, K).astype(np.int32)
+    ia, oa = 0.03, float(np.float32(0.03 * rng.uniform(0.75, 1.35)))
+    q = (ia, int(rng.integers(0, 256)), float(np.float32(oa * 40.0 / (ia * sigma))), 128, oa, int(rng.integers(0, 200)))
+    relu = bool(sum(case) & 1)
+    plan = hipq.Conv2d(x.shape, w, b, 1, 1, 1, *q, relu=relu)
+    print("any image", case, relu, plan.kernel, flush=True)
+    assert "hreg3x3" in plan.kernel and "hreg3x3" in plan.kernel_add, (plan.kernel, plan.kernel_add)
+    want = orc.conv2d_u8(x, w, b, 1, 1, 1, *q)
+    if relu:
+        want = np.maximum(want, q[5]).astype(np.uint8)
+    xd = hipq.to_device_nhwc(x)
+    got = hipq.from_device_nhwc(plan(xd), K)
+    assert np.array_equal(got, want), (case, int((got != want).sum()), np.argwhere(got != want)[:8].tolist())
+    res = rng.integers(0, 256, want.shape, dtype=np.uint8)
+    ra, rz = float(np.float32(oa * rng.uniform(0.6, 1.6))), int(rng.integers(0, 256))
+    sa, sz = float(np.float32(math.hypot(oa, ra) * 1.1)), int(rng.integers(0, 40))
+    for res_first in (False, True):
+        wanta = orc.add_u8(res, want, ra, rz, q[4], q[5], sa, sz) if res_first else orc.add_u8(want, res, q[4], q[5], ra, rz, sa, sz)
+        ya = plan.run_add(xd, hipq.to_device_nhwc(res), res_first, ra, rz, sa, sz, plan.empty_output())
+        gota = hipq.from_device_nhwc(ya, K)
+        assert np.array_equal(gota, wanta), (case, "add", res_first, int((gota != wanta).sum()))
+
+
+@pytest.mark.parametrize("case", [(3, 256, 25, 25, 256), (5, 128, 37, 29, 128), (12, 512, 9, 11, 512)], ids=lambda c: "x".join(map(str, c)))
+def test_register_fed_stride_2_on_ragged_images(case):
+    """conv_wreg_kernel's 7x7 output patches on images whose output is no multiple of 7."""
+    N, C, H, W, K = case
+    rng = np.random.default_rng(sum(case))
+    x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (K, C, 3, 3), dtype=np.uint8)
+    b = rng.integers(-50000, 50000, K).astype(np.int32)
+    q = (0.03, int(rng.integers(0, 256)), 0.004, 128, float(np.float32(0.03 * 0.004 * 74.0 * 74.0 * math.sqrt(C * 9) / 40.0)), 17)
+    plan = hipq.Conv2d(x.shape, w, b, 1, 2, 1, *q).special(3)
+    assert plan.kernel == "conv_mfma_i8_wreg", plan.kernel
+    want = orc.conv2d_u8(x, w, b, 1, 2, 1, *q)
+    y = torch.full_like(plan.empty_output(), 99)
+    got = hipq.from_device_nhwc(plan(hipq.to_device_nhwc(x), y), K)
+    assert np.array_equal(got, want), (case, int((got != want).sum()))
+
+
 ADD2_CASES = [  # N, C (widening layer's input channels), output H, W, K, the shortcut's stride
     (2, 256, 14, 14, 1024, 2), (3, 512, 7, 7, 2048, 2), (1, 256, 9, 13, 384, 1), (2, 512, 14, 7, 1024, 1),
 ]

@@ -271,6 +271,24 @@ def test_fused_add_chained_with_the_next_1x1_convolution():
                 assert not plan.add_conv_fusable(res_first, ra, rz, oa, oz, nxt)
 
 
+def test_chained_convolution_in_one_and_in_two_launches():
+    """hipq_conv2d_run_add_conv runs as two launches on few pixels; mode 2 asks for the one kernel there: the same bytes."""
+    rng = np.random.default_rng(80)
+    for N, C, H, W, K, mid in ((2, 64, 28, 28, 256, 64), (1, 128, 40, 30, 512, 128), (3, 64, 27, 13, 256, 128)):
+        x, res = (torch.from_numpy(rng.integers(0, 256, (N, H, W, c), dtype=np.uint8)).cuda() for c in (C, K))
+        b, b2 = (rng.integers(-30000, 30000, k).astype(np.int32) for k in (K, mid))
+        w, w2 = rng.integers(0, 256, (K, C, 1, 1), dtype=np.uint8), rng.integers(0, 256, (mid, K, 1, 1), dtype=np.uint8)
+        for relu in (False, True):
+            got = []
+            for mode in (1, 2):
+                plan = hipq.Conv2d((N, C, H, W), w, b, 0, 1, 1, 0.02, 100, 0.005, 128, 0.11, 90).special(mode)
+                nxt = hipq.Conv2d((N, K, H, W), w2, b2, 0, 1, 1, 0.15, 30, 0.004, 128, 0.9, 60)
+                y, y2 = plan.empty_output(), nxt.empty_output()
+                plan.run_add_conv(x, res, False, 0.1, 80, 0.15, 30, y, nxt, y2, next_relu=relu)
+                got.append((y.cpu().numpy(), y2.cpu().numpy()))
+            assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1]), (C, K, mid, relu)
+
+
 def test_conv_grouped_and_depthwise():
     rng = np.random.default_rng(13)
     kerns = set()
