@@ -275,6 +275,23 @@ int hipq_bottleneck_run_conv(const hipq_conv2d_plan *reduce, const hipq_conv2d_p
                              const hipq_conv2d_plan *next, int next_relu, void *y_next, void *stream);
 
 /*
+ * An inverted residual block in one launch: y = project(depthwise(expand(x))) and, when add != 0, y = add(that, x) -
+ * bit-identical to hipq_conv2d_run (or hipq_conv2d_run_relu where bit 0 / bit 1 of `relus` is set for expand / depthwise) three
+ * times and hipq_add_u8: op_conv_2d_u8xu8_run (src/op/conv_2d_uint8_impl.c:39-165), then op_quant_add_run (src/op/add.c:83-148);
+ * the tensors in between never travel to memory.  `expand`: 1x1 / stride 1, at most 160 input channels; `depthwise`: 3x3 / pad 1 / stride 1 or 2; `project`:
+ * 1x1 / stride 1, at most 160 output channels; uint8 tensors, weight zero points 128, per-tensor weight scales, each layer
+ * reading its input with the scale and zero point it is written with.  The residual is x itself, read with expand's input
+ * scale and zero point; residual_is_input0, oalpha, ozp and obits (8) as in hipq_bottleneck_run.  y must not be x.
+ * hipq_inverted_residual_fusable answers (1 / 0) whether the plans run this way (by rule where it is faster;
+ * hipq_conv2d_plan_special(project, 2): wherever it can); hipq_inverted_residual_run fails with an error otherwise.
+ */
+int hipq_inverted_residual_fusable(const hipq_conv2d_plan *expand, const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *project,
+                                   int add, int residual_is_input0, float oalpha, int ozp, int obits);
+int hipq_inverted_residual_run(const hipq_conv2d_plan *expand, const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *project,
+                               const void *x, int relus, int add, int residual_is_input0, float oalpha, int ozp, int obits, void *y,
+                               void *stream);
+
+/*
  * The rest of a bottleneck block in one launch, from its 3x3 convolution on: y = add(widen(mid(x)), residual) and, when
  * `next` is not NULL, y_next = next(y) - bit-identical to hipq_conv2d_run(mid, x, t), hipq_conv2d_run_add(widen, t,
  * residual, ...) and hipq_conv2d_run(next, y, y_next): op_conv_2d_u8xu8_run (src/op/conv_2d_uint8_impl.c:39-165), then

@@ -57,6 +57,7 @@
 #include "conv_expand.h"
 #include "conv_dw.h"
 #include "conv_hreg.h"
+#include "conv_invres.h"
 #include "conv_rows.h"
 #include "conv_stream.h"
 #include "conv_wreg.h"
@@ -1598,6 +1599,7 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
     std::vector<uint8_t> wbuf;
     std::vector<int32_t> bbuf;
     size_t pad_off = 0, frag_off = 0;
+    bool frag_whole = false;
     if (d.group == 1 && (d.in_cs % 16 == 0 || d.in_cs == 4)) {
         const bool smallc = d.in_cs == 4;
         p->variant = smallc ? kMfmaSmallC : kMfma;
@@ -1648,10 +1650,11 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
         wbuf.resize(pad_off + 64, (uint8_t)pad_byte); // source of out-of-image taps
         // the same weights in fragment order (ConvArgs::wfrag) for the kernels whose waves load their MFMA weight
         // operands straight from memory: layers of a bottleneck block
-        if (!smallc && boff == 0 && d.in_cs % 64 == 0 && d.in_cs <= 2048 && d.out_cs <= 2048 && d.C == d.in_cs
-            && ((d.R == 1 && d.S == 1) || (d.R == 3 && d.S == 3))) {
+        const bool whole = d.in_cs % 64 == 0 && d.C == d.in_cs;
+        if (!smallc && boff == 0 && d.in_cs <= 2048 && d.out_cs <= 2048 && ((d.R == 1 && d.S == 1) || (d.R == 3 && d.S == 3 && whole))) {
+            frag_whole = whole;
             frag_off = (wbuf.size() + 255) / 256 * 256;
-            wbuf.resize(frag_off + pad_off, 0);
+            wbuf.resize(frag_off + (size_t)a.nslab * a.kout_pad * 64, 0);
             for (int sl = 0; sl < a.nslab; sl++)
                 for (int T = 0; T < a.kout_pad / 32; T++)
                     for (int kk = 0; kk < 2; kk++)
@@ -1727,8 +1730,9 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
     a.wpack = static_cast<const uint8_t *>(p->d_w);
     a.bias2 = static_cast<const int32_t *>(p->d_bias);
     a.padbuf = a.wpack + pad_off;
-    a.wfrag = frag_off ? a.wpack + frag_off : nullptr;
-    if (frag_off)
+    a.wfrag1 = frag_off && d.R == 1 ? a.wpack + frag_off : nullptr;
+    a.wfrag = frag_whole ? a.wpack + frag_off : nullptr;
+    if (frag_whole)
         set_mfma_name(p, false); // the register-fed kernel's rule looks at the fragment-order copy
     if (p->d_q) {
         a.qmult = static_cast<const uint32_t *>(p->d_q);
@@ -2204,6 +2208,58 @@ extern "C" int hipq_bottleneck_run(const hipq_conv2d_plan *p1, const hipq_conv2d
     a3.y = static_cast<uint8_t *>(y);
     launch_conv_block(a1, a2, a3, nullptr, static_cast<hipStream_t>(stream));
     return launch_status("conv_bottleneck_kernel");
+}
+
+// the launch arguments of an inverted residual block (hipq_inverted_residual_run); false if the add's scales are outside the
+// fixed-point range or a layer does not read what the one before it writes
+static bool invres_args(const hipq_conv2d_plan *pe, const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, int relus, int add,
+                        int residual_is_input0, float oalpha, int ozp, int obits, ConvArgs *ae, ConvArgs *ad, ConvArgs *ap)
+{
+    auto follows = [](const hipq_conv2d_plan *q, const hipq_conv2d_plan *p) { return q->d.izp == p->d.ozp && q->d.ialpha == p->d.oalpha; };
+    if (!follows(pp, pd) || !follows(pd, pe))
+        return false;
+    *ae = pe->args, *ad = pd->args, *ap = pp->args;
+    if (add && (obits != 8 || ozp < 0 || ozp > 255 || !add_args(pp, residual_is_input0, pe->d.ialpha, pe->d.izp, oalpha, ozp, obits, ap)))
+        return false;
+    // the ReLU clamps, as in hipq_conv2d_run_relu
+    if (relus & 1)
+        ae->lo = std::min(pe->d.ozp, ae->q.hi);
+    if (relus & 2)
+        ad->lo = std::min(pd->d.ozp, ad->q.hi);
+    return true;
+}
+
+extern "C" int hipq_inverted_residual_fusable(const hipq_conv2d_plan *pe, const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, int add,
+                                              int residual_is_input0, float oalpha, int ozp, int obits)
+{
+    for (const hipq_conv2d_plan *p : {pe, pd, pp})
+        if (!p || p->d.dtype != HIPQ_DTYPE_U8 || p->d.obits != 8
+            || (p == pd ? p->variant != kDepthwise3x3 : p->variant != kMfma || !p->special || p->tile_selected))
+            return 0;
+    ConvArgs ae, ad, ap;
+    if (!invres_args(pe, pd, pp, 0, add, residual_is_input0, oalpha, ozp, obits, &ae, &ad, &ap))
+        return 0;
+    return conv_invres_applies(ae, ad, ap) && (pp->special == 2 || conv_invres_preferred(ae, ad, ap)) ? 1 : 0;
+}
+
+extern "C" int hipq_inverted_residual_run(const hipq_conv2d_plan *pe, const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, const void *x,
+                                          int relus, int add, int residual_is_input0, float oalpha, int ozp, int obits, void *y, void *stream)
+{
+    clear_error();
+    HIPQ_REQUIRE(pe && pd && pp && x && y, "hipq_inverted_residual_run: null argument");
+    HIPQ_REQUIRE(x != y, "hipq_inverted_residual_run: the output cannot overwrite the block's input (neighbouring patches read it)");
+    HIPQ_REQUIRE(relus >= 0 && relus <= 3, "hipq_inverted_residual_run: relus %d", relus);
+    HIPQ_REQUIRE(hipq_inverted_residual_fusable(pe, pd, pp, add, residual_is_input0, oalpha, ozp, obits),
+                 "hipq_inverted_residual_run: these plans (%s, %s, %s) do not run as one kernel: run the operators separately",
+                 pe->name.c_str(), pd->name.c_str(), pp->name.c_str());
+    ConvArgs ae, ad, ap;
+    invres_args(pe, pd, pp, relus, add, residual_is_input0, oalpha, ozp, obits, &ae, &ad, &ap);
+    const uint8_t *in = static_cast<const uint8_t *>(x);
+    ae.x = in;
+    ap.res = add ? in : nullptr;
+    ap.y = static_cast<uint8_t *>(y);
+    launch_conv_invres(ae, ad, ap, static_cast<hipStream_t>(stream));
+    return launch_status("conv_invres_kernel");
 }
 
 extern "C" int hipq_bottleneck_conv_fusable(const hipq_conv2d_plan *p1, const hipq_conv2d_plan *p2, const hipq_conv2d_plan *p3,

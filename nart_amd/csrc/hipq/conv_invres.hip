@@ -1,0 +1,440 @@
+// An inverted residual block of a mobile network in ONE kernel: the 1x1 convolution that widens the channels, the depthwise
+// 3x3 convolution, the 1x1 convolution that narrows them again and, where there is one, the residual add.  gfx950 only.
+//
+// Reproduces, bit for bit, op_conv_2d_u8xu8_run (art/modules/quant/src/op/conv_2d_uint8_impl.c:39-165) three times and
+// op_quant_add_run (art/modules/quant/src/op/add.c:83-148): every intermediate value is requantised, clamped and re-read exactly
+// as if it had travelled through memory.
+//
+// Why: the hidden tensor is six times as wide as the block's input and output, is written and read twice, and the three layers
+// are three launches.  Here a work-group owns a patch of output pixels of ONE image, and its waves take the hidden channels in
+// slices of 32.  A wave takes a slice through all three layers on its own, without a barrier:
+//   * expand: the patch's input region, which lies re-centred in LDS, times the slice's weights, pixels as the ROWS of the
+//     multiply and channels as its columns: the 16 accumulators of a lane are four runs of four consecutive pixels of ONE
+//     channel, so a requantised run is a dword that the depthwise layer can use as it is;
+//   * depthwise: v_dot4_i32_i8 of such a dword with {w0, w1, w2, 0} and {0, w0, w1, w2} gives two neighbouring outputs (at stride
+//     2 one), the runs in between are v_alignbyte of two dwords: no byte transposes;
+//   * project: the slice's bytes, written to LDS as pixel rows, are one k-step of every output channel tile's reduction, whose
+//     accumulators a wave keeps over its slices.
+// Positions outside the image hold the depthwise layer's pad byte; the border of a patch is expanded again by its neighbours,
+// which costs vector instructions (the requantisation), not memory.
+// Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch and add their partial sums up
+// in LDS.  Many patches and few slices: every wave has a patch of its own and takes all slices through it, so that no barrier
+// and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
+// 65 us at 56x56, batch 64, against 32.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
+// instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice).
+// What bounds it is vector issue: some 650 instructions per slice of 8x8 outputs at stride 1, 70 of them per 32 expanded
+// positions; with few patches the chain launch - region - slices - sum.
+// Measured, the three launches -> this one (batch 64): 16 -> 96 -> 24 at 112x112, stride 2: 58 -> 34 us; 24 -> 144 -> 24 at 56x56:
+// 42 -> 32; 32 -> 192 -> 32 at 28x28: 21 -> 15.4; 64 -> 384 -> 64 at 14x14: 15 -> 11.8; batch 1: 10 -> 4.6 .. 6.4.
+// Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
+// requantisations, at most 160 input and output channels.
+#include "conv_invres.h"
+
+#include <algorithm>
+#include <cmath>
+
+#include "conv_frag.h"
+
+namespace hipq {
+
+using namespace frag;
+
+namespace {
+
+// waves of a work-group: three per SIMD leave each 168 registers, where that is enough for a shape's accumulators
+constexpr int max_waves(int PT, int CT) { return PT > 1 || CT > 4 ? 8 : 12; }
+
+struct InvresGeom {
+    int PY, PX; // patches per image
+    int nT;     // slices of 32 hidden channels
+    int nk, ct; // k-steps of the expanding layer, channel tiles of the projecting one
+    int xrow;   // bytes of a pixel row of the input region in LDS
+    int region; // bytes of an input region with its masks in LDS
+    int wave_bytes; // bytes of a wave's own buffers
+};
+
+// S: stride, PH x PW: output pixels of a patch (PW a multiple of 4).  Rows and columns of the input region, columns in whole
+// runs of four; tiles of 32 positions; pixel tiles of 32 outputs.
+template <int S, int PH_, int PW_>
+struct Patch {
+    static constexpr int PH = PH_, PW = PW_, RH = S * (PH - 1) + 3, QW = (S * (PW - 1) + 3 + 3) / 4, RW = 4 * QW;
+    static constexpr int NQ = RH * QW, TILES = (NQ + 7) / 8, PT = (PH * PW + 31) / 32;
+    static constexpr int E_BYTES = TILES * 8 * 128, D_BYTES = PT * 1024, MASK_BYTES = TILES * 8 * 4;
+};
+
+__device__ static __forceinline__ void lds_order()
+{
+    // a wave's LDS instructions execute in the order they are issued; this keeps the compiler to it
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ static __forceinline__ int32_t dot4(uint32_t a, int b, int32_t c)
+{
+    return __builtin_amdgcn_sdot4((int)a, b, c, false);
+}
+
+// dot(a, b) + c into a new register: the compiler's own choice for this is a copy of c followed by the accumulating form
+__device__ static __forceinline__ int32_t dot4_from(uint32_t a, int32_t b, int32_t c)
+{
+    int32_t d;
+    asm("v_dot4_i32_i8 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+    return d;
+}
+
+} // namespace
+
+// NK: k-steps of 32 input channels; CT: tiles of 32 output channels (both may be more than the layer has: the weights are zeros
+// there).  OWN: every wave has a patch of its own and takes all slices through it; otherwise the waves
+// of a work-group split the slices of one patch.
+template <int S, int PH, int PW, int NK, int CT, bool OWN>
+__global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT)) void conv_invres_kernel(const ConvArgs e, const ConvArgs d, const ConvArgs pr,
+                                                                                const InvresGeom geo)
+{
+    using G = Patch<S, PH, PW>;
+    constexpr int RH = G::RH, QW = G::QW, NQ = G::NQ, TILES = G::TILES, RW = G::RW, PT = G::PT;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int p = lane & 31, h = lane >> 5;
+    const int ch = 16 * ((p >> 2) & 1) + 4 * (p >> 3) + (p & 3); // the channel of a slice that this lane's column stands for
+    // work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of the patches
+    const int ppi = geo.PY * geo.PX;
+    int gid = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    if (OWN)
+        gid = gid * nw + wave;
+    if (gid >= ppi * d.N)
+        return;
+    const int n = gid / ppi, pi = gid - n * ppi, py = pi / geo.PX;
+    const int oy0 = py * PH, ox0 = (pi - py * geo.PX) * PW;
+    const int iy0 = S * oy0 - 1, ix0 = S * ox0 - 1; // the region's first row and column
+    const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + RH <= e.H && ix0 + RW <= e.W; // no position to replace
+    uint8_t *const xbuf = lds + (OWN ? wave * (geo.region + geo.wave_bytes) : 0);
+    uint32_t *const masks = reinterpret_cast<uint32_t *>(xbuf + geo.region - G::MASK_BYTES); // which bytes of a run lie inside the image
+    uint8_t *const ebuf = xbuf + geo.region + (OWN ? 0 : wave * geo.wave_bytes), *const dbuf = ebuf + G::E_BYTES;
+
+    // ---- a slice's weights and constants, each loaded as soon as the slice before has used its own
+    v4i we[NK], wp[CT];
+    int ebias, dbias, wa[3], wb[3];
+    auto load_e = [&](int T) {
+        ebias = e.bias2[32 * T + ch];
+#pragma unroll
+        for (int kk = 0; kk < NK; kk++)
+            we[kk] = kk == 0 || kk < geo.nk ? ldg128(e.wfrag1 + ((size_t)((kk >> 1) * (e.kout_pad >> 5) + T) * 2 + (kk & 1)) * 1024 + lane * 16)
+                                            : v4i{0, 0, 0, 0};
+    };
+    auto load_d = [&](int T) {
+        const int cd = min(32 * T + ch, d.in_cs - 1); // the last slice may be half empty; its products meet zero weights
+        dbias = d.bias2[cd];
+        const int *wt = reinterpret_cast<const int *>(d.wpack) + cd;
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            wa[r] = wt[(r * 2 + 0) * d.in_cs];
+            if (S == 1)
+                wb[r] = wt[(r * 2 + 1) * d.in_cs];
+        }
+    };
+    auto load_p = [&](int T) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+            wp[ct] = ct == 0 || ct < geo.ct ? ldg128(pr.wfrag1 + ((size_t)((T >> 1) * (pr.kout_pad >> 5) + ct) * 2 + (T & 1)) * 1024 + lane * 16)
+                                            : v4i{0, 0, 0, 0};
+    };
+    int T = OWN ? 0 : wave;
+    const int dT = OWN ? 1 : nw; // never more waves than slices
+
+    // ---- the input region -> LDS, re-centred; positions outside the image are never used (the masks below)
+    {
+        const int tid = OWN ? lane : (int)threadIdx.x, nthr = OWN ? 64 : (int)blockDim.x;
+        const int pieces = e.in_cs >> 4, inv = 65536 / pieces + 1; // id / pieces == (id * inv) >> 16: id < 4096, pieces <= 10
+        for (int id = tid; id < RH * RW * pieces; id += nthr) {
+            const int px = (id * inv) >> 16, c = id - px * pieces, ry = px / RW, rx = px - ry * RW;
+            const int iy = iy0 + ry, ix = ix0 + rx;
+            if ((unsigned)iy < (unsigned)e.H && (unsigned)ix < (unsigned)e.W)
+                *reinterpret_cast<v4i *>(xbuf + px * geo.xrow + c * 16)
+                    = ldg128(e.x + (uint32_t)(((n * e.H + iy) * e.W + ix) * e.in_cs + c * 16)) ^ (int)0x80808080;
+        }
+        if (!inside)
+            for (int q = tid; q < TILES * 8; q += nthr) {
+                const int ry = q / QW, rx = (q - ry * QW) * 4, iy = iy0 + ry;
+                uint32_t m = 0;
+                if (q < NQ && (unsigned)iy < (unsigned)e.H)
+                    for (int b = 0; b < 4; b++)
+                        m |= (unsigned)(ix0 + rx + b) < (unsigned)e.W ? 0xffu << (8 * b) : 0u;
+                masks[q] = m;
+            }
+    }
+    load_e(T);
+    load_d(T);
+    load_p(T);
+    v16i acc[CT][PT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int t = 0; t < PT; t++) {
+            // OWN: the accumulators start at the folded bias of the lane's 16 consecutive channels
+            init_acc(acc[ct][t], pr.bias2 + 32 * (ct < geo.ct ? ct : 0) + 16 * h, !OWN);
+        }
+    const uint32_t epad = d.padword ^ 0x80808080u;
+    if (OWN)
+        lds_order();
+    else
+        __syncthreads(); // the region and the masks are in LDS
+
+    for (; T < geo.nT; T += dT) {
+        const int Tn = min(T + dT, geo.nT - 1); // past the end: harmless loads
+        // ---- expand
+        auto expand = [&](auto whole) {
+#pragma unroll (TILES <= 4 ? TILES : 2)
+            for (int t = 0; t < TILES; t++) {
+                v16i a;
+                const uint8_t *row = xbuf + (32 * t + p) * geo.xrow + 16 * h;
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    a[i] = ebias;
+#pragma unroll
+                for (int kk = 0; kk < NK; kk++)
+                    a = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(row + 32 * kk), we[kk], a, 0, 0, 0);
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const int q = 8 * t + 2 * g + h;
+                    uint32_t v = conv_requant4<false>(e, a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]) ^ 0x80808080u;
+                    if (!decltype(whole)::value) {
+                        const uint32_t m = masks[q];
+                        v = (v & m) | (epad & ~m);
+                    }
+                    *reinterpret_cast<uint32_t *>(ebuf + (q * 32 + p) * 4) = v;
+                }
+            }
+        };
+        if (inside)
+            expand(std::true_type{});
+        else
+            expand(std::false_type{});
+        load_e(Tn);
+        lds_order();
+        // ---- depthwise: half h of the wave takes PH / 2 output rows of this lane's channel
+        constexpr int HR = PH / 2, IR = S * (HR - 1) + 3;
+        int32_t o[HR][PW];
+#pragma unroll
+        for (int ir = 0; ir < IR; ir++) {
+            const uint8_t *er = ebuf + ((S * HR * h + ir) * QW * 32 + p) * 4;
+            uint32_t q[QW];
+#pragma unroll
+            for (int i = 0; i < QW; i++)
+                q[i] = *reinterpret_cast<const uint32_t *>(er + i * 128);
+            uint32_t mid[QW - 1]; // bytes 2, 3 of run i and 0, 1 of run i + 1
+#pragma unroll
+            for (int i = 0; i + 1 < QW; i++)
+                mid[i] = __builtin_amdgcn_alignbyte(q[i + 1], q[i], 2);
+#pragma unroll
+            for (int r = 0; r < HR; r++) {
+                const int kr = ir - S * r;
+                if (kr < 0 || kr > 2)
+                    continue;
+#pragma unroll
+                for (int x = 0; x < PW; x++) {
+                    const uint32_t v = S == 1 ? ((x & 2) ? mid[x >> 2] : q[x >> 2]) : ((x & 1) ? mid[x >> 1] : q[x >> 1]);
+                    const int w = S == 1 && (x & 1) ? wb[kr] : wa[kr];
+                    o[r][x] = kr == 0 ? dot4_from(v, w, dbias) : dot4(v, w, o[r][x]);
+                }
+            }
+        }
+        load_d(Tn);
+        // this lane's channel of its outputs, as bytes of the pixel rows that the last layer multiplies
+#pragma unroll
+        for (int r = 0; r < HR; r++)
+#pragma unroll
+            for (int x4 = 0; x4 < PW; x4 += 4) {
+                const uint32_t v = conv_requant4<false>(d, o[r][x4], o[r][x4 + 1], o[r][x4 + 2], o[r][x4 + 3]) ^ 0x80808080u;
+                uint8_t *to = dbuf + (((HR * h + r) * PW + x4) * 32) + ch;
+                to[0] = (uint8_t)v, to[32] = (uint8_t)(v >> 8), to[64] = (uint8_t)(v >> 16), to[96] = (uint8_t)(v >> 24);
+            }
+        lds_order();
+        // ---- project: one k-step of every channel tile (rows past the patch, where it has fewer than 32 pixels, are never stored)
+        v4i b[PT];
+#pragma unroll
+        for (int t = 0; t < PT; t++)
+            b[t] = *reinterpret_cast<const v4i *>(dbuf + (32 * t + p) * 32 + 16 * h);
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int t = 0; t < PT; t++)
+                acc[ct][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wp[ct], b[t], acc[ct][t], 0, 0, 0);
+        load_p(Tn);
+        lds_order();
+    }
+
+    auto store = [&](int ct, int t, const v16i &s) {
+        const int m = 32 * t + p, oy = oy0 + m / PW, ox = ox0 + m % PW, c0 = 32 * ct + 16 * h;
+        if (m >= PH * PW || oy >= pr.OH || ox >= pr.OW || c0 >= pr.out_cs)
+            return;
+        const size_t at = (size_t)((n * pr.OH + oy) * pr.OW + ox) * pr.out_cs + c0;
+        const v4i v = pr.res != nullptr ? requant_add16(pr, s, ldg128(pr.res + at)) : requant16(pr, s, 0);
+        *reinterpret_cast<v4i *>(pr.y + at) = v;
+    };
+    if (OWN) {
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int t = 0; t < PT; t++)
+                store(ct, t, acc[ct][t]);
+        return;
+    }
+    // ---- the waves' partial sums meet in LDS (where the region was), over the folded bias
+    __syncthreads();
+    int32_t *const red = reinterpret_cast<int32_t *>(lds);
+    for (int i = threadIdx.x; i < CT * PT * 1024; i += blockDim.x) {
+        const int l = i & 63, r = (i >> 6) & 15, ct = (i >> 10) / PT;
+        red[i] = pr.bias2[32 * min(ct, geo.ct - 1) + 16 * (l >> 5) + r];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int t = 0; t < PT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                atomicAdd(&red[((ct * PT + t) * 16 + r) * 64 + lane], acc[ct][t][r]);
+    __syncthreads();
+    for (int i = wave; i < CT * PT; i += nw) {
+        v16i s;
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+            s[r] = red[(i * 16 + r) * 64 + lane];
+        store(i / PT, i % PT, s);
+    }
+}
+
+namespace {
+
+template <int S, int PH, int PW, int NK, int CT, bool OWN>
+void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+{
+    using G = Patch<S, PH, PW>;
+    InvresGeom geo;
+    geo.PY = (p.OH + PH - 1) / PH, geo.PX = (p.OW + PW - 1) / PW;
+    geo.nT = (d.in_cs + 31) / 32;
+    geo.nk = (e.in_cs + 31) / 32, geo.ct = (p.out_cs + 31) / 32;
+    // rows of 16 bytes (the other half of a k-step meets zero weights) and of 32 read without bank conflicts as they are, longer
+    // ones 16 bytes apart
+    geo.xrow = e.in_cs == 16 ? 16 : NK == 1 ? 32 : 32 * NK + 16;
+    geo.region = (G::TILES * 32 * geo.xrow + 16 + G::MASK_BYTES + 15) / 16 * 16;
+    geo.wave_bytes = G::E_BYTES + G::D_BYTES;
+    const long long patches = (long long)d.N * geo.PY * geo.PX;
+    int nw = 4;
+    unsigned lds;
+    if (OWN) {
+        lds = (unsigned)(nw * (geo.region + geo.wave_bytes));
+    } else {
+        nw = std::min(geo.nT, max_waves(G::PT, CT));
+        while (geo.region + nw * geo.wave_bytes > 160 * 1024)
+            nw--; // one wave needs at most 14 KB beside 63 KB of pixels
+        const int rounds = (geo.nT + nw - 1) / nw;
+        nw = (geo.nT + rounds - 1) / rounds; // the same rounds with fewer waves
+        lds = (unsigned)std::max(geo.region + nw * geo.wave_bytes, CT * G::PT * 4096);
+    }
+    const long long wgs = OWN ? (patches + nw - 1) / nw : patches;
+    hipLaunchKernelGGL((conv_invres_kernel<S, PH, PW, NK, CT, OWN>), dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(64 * nw), lds, st, e, d, p, geo);
+}
+
+// ---- the shapes, and what each takes
+enum Shape { k2x4, k4x8, k8x8, kOwn, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2
+
+// Time by shape, in us, fitted to 80 measured blocks (1 to 64 images of 3x3 to 130x130, the channel counts of a mobile network;
+// within 20 % of each) - linear in the rounds of slices a wave takes one after the other, alone and per channel tile of 32, the
+// slices per SIMD of the chip, the channel tiles, and the work-groups per CU, as a quotient and rounded up.
+double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
+{
+    static const double kCost[2][kShapes][7] = {
+        {{2.49, 0, 0, 1.031, 1.281, 0, 0}, {0.515, 1.774, 0, 0.75, 1.394, 0, 1.631}, {0, 2.022, 0.665, 0.097, 0, 0.23, 4.513}, {0.654, 1.918, 0.192, 0, 0, 0, 1.112}},
+        {{2.937, 0, 0, 1.084, 1.108, 0, 0}, {4.668, 0, 0.643, 0.981, 0.187, 0, 0.469}, {}, {0.346, 2.266, 0, 0, 0.938, 0.51, 0.363}}};
+    const int s = d.stride_h, ph = shape == k2x4 ? 2 : shape == k8x8 || (shape == kOwn && s == 1) ? 8 : 4, pw = shape == k2x4 ? 4 : 8;
+    const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32, nT = (d.in_cs + 31) / 32;
+    if ((shape == kOwn && (nk > 2 || ct > 2)) || (shape == k8x8 && (s == 2 || ct > 3)))
+        return 1e30; // not built: the accumulators or the region would be too much for a wave
+    const double patches = (double)d.N * ((p.OH + ph - 1) / ph) * ((p.OW + pw - 1) / pw);
+    const int nw = shape == kOwn ? 1 : std::min(nT, max_waves((ph * pw + 31) / 32, ct)), rounds = (nT + nw - 1) / nw;
+    const double v[7] = {1, (double)rounds, (double)rounds * ct, patches * nT / 1024, (double)ct, patches / 256, std::ceil(patches / 256)};
+    double t = 0;
+    for (int i = 0; i < 7; i++)
+        t += kCost[s - 1][shape][i] * v[i];
+    return t;
+}
+
+int choose_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, double *us)
+{
+    int best = k2x4;
+    *us = shape_cost(e, d, p, best);
+    for (int sh = k4x8; sh < kShapes; sh++)
+        if (const double t = shape_cost(e, d, p, sh); t < *us)
+            *us = t, best = sh;
+    return best;
+}
+
+template <int S, int NK, int CT>
+void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+{
+    double us;
+    const int shape = choose_shape(e, d, p, &us);
+    if constexpr (NK <= 2 && CT <= 2)
+        if (shape == kOwn)
+            return launch_shape<S, S == 1 ? 8 : 4, 8, NK, CT, true>(e, d, p, st);
+    if constexpr (S == 1 && CT <= 3)
+        if (shape == k8x8)
+            return launch_shape<S, 8, 8, NK, CT, false>(e, d, p, st);
+    if (shape == k4x8)
+        return launch_shape<S, 4, 8, NK, CT, false>(e, d, p, st);
+    launch_shape<S, 2, 4, NK, CT, false>(e, d, p, st);
+}
+
+template <int S>
+void launch_stride(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+{
+    const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32;
+    if (nk == 1 && ct <= 2)
+        ct == 1 ? launch_tiles<S, 1, 1>(e, d, p, st) : launch_tiles<S, 1, 2>(e, d, p, st);
+    else if (nk <= 2 && ct <= 3)
+        ct <= 2 ? launch_tiles<S, 2, 2>(e, d, p, st) : launch_tiles<S, 2, 3>(e, d, p, st);
+    else if (nk <= 3)
+        ct <= 3 ? launch_tiles<S, 3, 3>(e, d, p, st) : launch_tiles<S, 3, 5>(e, d, p, st);
+    else
+        launch_tiles<S, 5, 5>(e, d, p, st);
+}
+
+bool plain(const ConvArgs &a) { return a.bwz == 0 && a.xmask != 0 && a.lo >= 0 && a.fastq && a.qmult == nullptr; }
+
+bool point(const ConvArgs &a)
+{
+    return plain(a) && a.group == 1 && a.R == 1 && a.S == 1 && a.pad_h == 0 && a.pad_w == 0 && a.stride_h == 1 && a.stride_w == 1
+        && a.wfrag1 != nullptr && a.in_cs % 16 == 0 && a.out_cs % 16 == 0;
+}
+
+} // namespace
+
+bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
+{
+    return plain(d) && d.group == d.C && d.R == 3 && d.S == 3 && d.pad_h == 1 && d.pad_w == 1 && d.stride_h == d.stride_w
+        && (d.stride_h == 1 || d.stride_h == 2) && d.in_cs == d.out_cs && d.in_cs % 16 == 0 && point(p) && p.in_cs == d.in_cs && p.N == d.N
+        && p.H == d.OH && p.W == d.OW && (long long)p.P * p.out_cs < (1ll << 31) && p.out_cs <= 160
+        && (p.res == nullptr || (p.addq.fast && p.addq.hi == 255)) && point(e) && e.out_cs == d.in_cs && e.in_cs <= 160
+        && e.N == d.N && e.OH == d.H && e.OW == d.W && (long long)e.P * e.in_cs < (1ll << 31);
+}
+
+// The three launches: their latencies, the hidden tensor's bytes at both resolutions, the expanding layer's products (fitted to
+// the same blocks, within 11 %).
+bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
+{
+    const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
+    const double apart = d.stride_h == 1 ? 9.25 + 1.007 * wide + 0.00548 * wide * e.in_cs : 9.32 + 1.996 * narrow + 0.00451 * wide * e.in_cs;
+    double us;
+    choose_shape(e, d, p, &us);
+    return us < 0.95 * apart;
+}
+
+void launch_conv_invres(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+{
+    d.stride_h == 1 ? launch_stride<1>(e, d, p, st) : launch_stride<2>(e, d, p, st);
+}
+
+} // namespace hipq

@@ -99,7 +99,7 @@ typedef std::map<const mem_t *, std::set<const op_t *>> reader_map;
 // keyed by workspace (the runtime is single-threaded, art/include/art/workspace.h has no locking either)
 std::map<const workspace_t *, reader_map> g_readers;
 long g_fused_adds = 0, g_fused_relus = 0, g_fused_pools = 0, g_chained_convs = 0, g_fused_dequants = 0; // fused launches so far (hip_module_fused_*)
-long g_fused_blocks = 0, g_fused_tails = 0; // whole bottleneck blocks / blocks from their 3x3 layer on, as one launch
+long g_fused_blocks = 0, g_fused_inverted = 0, g_fused_tails = 0; // whole bottleneck / inverted residual blocks, blocks from their 3x3 layer on, as one launch
 
 reader_map &readers_of(op_t *op) { return g_readers[op->workspace]; }
 
@@ -146,6 +146,11 @@ struct conv_op_t {
     // A convolution that heads a bottleneck block (1x1, then 3x3, then 1x1 and the add with the block's input) which
     // hipq_bottleneck_run computes in one launch: the block's 3x3 convolution and its add (else null).
     const op_t *blk_next, *blk_add;
+    // An expanding, a depthwise and a projecting convolution that hipq_inverted_residual_run computes in one launch, with the
+    // relus behind the first two and the add with the block's input where there are: set for all three by the first one's run().
+    op_t *ir_project;                             // the chain's last convolution (in all three; else null)
+    op_t *ir_expand, *ir_dw;                      // in the last one
+    const op_t *ir_relu1, *ir_relu2, *ir_add;     // in the last one; null: none
     // this pass's output has already been written by the kernel of the pooling operator whose output this convolution
     // reads (hipq_conv2d_run_maxpool_conv): run() has nothing left to do
     bool computed_ahead;
@@ -304,6 +309,61 @@ bool conv_continues_block(op_t *op, const op_t *r)
     return false;
 }
 
+// ---- inverted residual blocks ----------------------------------------------------------------------------------------
+// 1x1 [-> relu] -> depthwise 3x3 [-> relu] -> 1x1 [-> add(., block input)], every intermediate tensor read by its successor only:
+// the first two convolutions and their relus leave hooks, and the run() of the last convolution (or of the add, to which it
+// leaves its own) launches hipq_inverted_residual_run.
+op_t *only_reader_mut(const op_t *op) { return const_cast<op_t *>(only_reader(op)); }
+
+// r is the relu behind convolution c that c's own clamp computes
+bool relu_clamps(const op_t *r, const conv_op_t *c);
+
+bool conv_heads_inverted_residual(op_t *op)
+{
+    static const bool off = getenv("NART_HIP_NO_FUSION") != nullptr;
+    conv_op_t *e = reinterpret_cast<conv_op_t *>(op);
+    if (off || op->entry->tp != &op_conv_2d_tp || e->desc.dtype != HIPQ_DTYPE_U8 || e->kernel_h != 1)
+        return false;
+    const op_t *relu[2] = {nullptr, nullptr};
+    op_t *conv[3] = {op, nullptr, nullptr};
+    for (int k = 0; k < 2; ++k) {
+        op_t *r = only_reader_mut(conv[k]);
+        if (r != nullptr && r->entry->tp == &op_relu_tp) {
+            if (!relu_clamps(r, reinterpret_cast<const conv_op_t *>(conv[k])))
+                return false;
+            relu[k] = r;
+            r = only_reader_mut(r);
+        }
+        if (r == nullptr || r->entry->tp != &op_conv_2d_tp || reinterpret_cast<conv_op_t *>(r)->plan == nullptr)
+            return false;
+        conv[k + 1] = r;
+    }
+    conv_op_t *d = reinterpret_cast<conv_op_t *>(conv[1]), *p = reinterpret_cast<conv_op_t *>(conv[2]);
+    int i = 0;
+    const op_t *a = add_reading(conv[2], &i);
+    bool ok;
+    if (a != nullptr && a->input_tensors[1 - i]->mem == op->input_tensors[0]->mem) {
+        const QSet &qi = add_inputs(a), &qo = add_output(a);
+        ok = qi.alpha[1 - i] == e->desc.ialpha && qi.zp[1 - i] == e->desc.izp
+            && hipq_inverted_residual_fusable(e->plan, d->plan, p->plan, 1, i == 1, qo.alpha[0], qo.zp[0], qo.bits[0]);
+    } else {
+        // where the projecting layer leaves its launch to another operator, that one decides
+        const op_t *r = only_reader(conv[2]);
+        a = nullptr;
+        ok = (r == nullptr || r->entry->tp == &op_conv_2d_tp) && hipq_inverted_residual_fusable(e->plan, d->plan, p->plan, 0, 0, 1.0f, 0, 8);
+    }
+    if (!ok)
+        return false;
+    e->ir_project = d->ir_project = p->ir_project = conv[2];
+    p->ir_expand = op, p->ir_dw = conv[1];
+    p->ir_relu1 = relu[0], p->ir_relu2 = relu[1], p->ir_add = a;
+    return true;
+}
+
+// The block that ends in convolution `pop` (and the add `add`, null: none) as one launch into y; false: nothing launched, run
+// the operators
+bool inverted_residual_launch(op_t *pop, const op_t *add, void *y);
+
 // 1: the only reader of the convolution's output is an add or a relu of this workspace that can take over the launch
 bool sole_reader_fuses(op_t *op)
 {
@@ -339,7 +399,7 @@ void conv_run(op_t *op)
         return;
     }
     if (c->defer == 0)
-        c->defer = sole_reader_fuses(op) ? 1 : -1;
+        c->defer = conv_heads_inverted_residual(op) || (c->ir_project != nullptr && c->ir_project != op) || sole_reader_fuses(op) ? 1 : -1;
     if (c->defer == 1) {
         hip_mem_t *ym = as_hip(op->output_tensors[0].mem);
         (void)out_ptr(op); // the buffer exists and the device side is the current one - once the hook has run
@@ -347,7 +407,7 @@ void conv_run(op_t *op)
         ym->pending_ctx = op;
         return;
     }
-    if (conv_run_chained(op, out_ptr(op), 0))
+    if (inverted_residual_launch(op, nullptr, out_ptr(op)) || conv_run_chained(op, out_ptr(op), 0))
         return;
     HIPM_HIPQ(hipq_conv2d_run(c->plan, in_ptr(op, 0), out_ptr(op), nullptr, op_stream(op)));
 }
@@ -371,6 +431,7 @@ void build_plan(op_t *op, const hipq_conv2d_desc &d, const uint8_t *w, const voi
 {
     conv_op_t *c = reinterpret_cast<conv_op_t *>(op);
     c->defer = 0; // decided at the next run, when every operator of the pass has been prepared
+    c->ir_project = nullptr;
     const float *wa_pc = per_channel_walpha(c);
     uint64_t pc_id = 0;
     if (wa_pc) {
@@ -607,7 +668,7 @@ bool run_fused_into_convolution(op_t *op, void *y)
         return false;
     op_t *cop = static_cast<op_t *>(as_hip(op->input_tensors[i]->mem)->pending_ctx);
     conv_op_t *c = reinterpret_cast<conv_op_t *>(cop);
-    if (block_launch(op, cop, i, y, nullptr, 0, nullptr))
+    if (inverted_residual_launch(cop, op, y) || block_launch(op, cop, i, y, nullptr, 0, nullptr))
         return true;
     const int o = 1 - i;
     const void *res = in_ptr(op, o); // settles the other input if it is deferred as well
@@ -676,7 +737,7 @@ bool add_defers(op_t *op)
         const int o = 1 - i;
         const reader_map &rm = readers_of(op);
         const auto it = rm.find(op->output_tensors[0].mem);
-        if (!off && it != rm.end())
+        if (!off && c->ir_add != op && it != rm.end())
             for (const op_t *r : it->second) {
                 if (r->workspace != op->workspace || r->entry->tp != &op_conv_2d_tp)
                     continue;
@@ -822,6 +883,8 @@ bool relu_is_clamp_of(const ew_op_t *e, const conv_op_t *c)
         && e->qo.zp[0] == c->desc.ozp && e->qo.bits[0] == c->desc.obits;
 }
 
+bool relu_clamps(const op_t *r, const conv_op_t *c) { return relu_is_clamp_of(reinterpret_cast<const ew_op_t *>(r), c); }
+
 // convolution + relu as one launch into the relu's output memory `y`; false: not possible, run the relu plainly
 bool relu_launch_into(op_t *op, void *y)
 {
@@ -851,6 +914,40 @@ void relu_launch_deferred(void *ctx)
                                e->qo.bits[0], op_stream(op)));
 }
 
+bool inverted_residual_launch(op_t *pop, const op_t *add, void *y)
+{
+    conv_op_t *p = reinterpret_cast<conv_op_t *>(pop);
+    if (p->ir_project != pop || p->ir_add != add)
+        return false;
+    conv_op_t *e = reinterpret_cast<conv_op_t *>(p->ir_expand), *d = reinterpret_cast<conv_op_t *>(p->ir_dw);
+    // every launch of the chain is still this one's to make
+    auto left = [](const tensor_t *t, void (*hook)(void *), const void *ctx) {
+        const hip_mem_t *m = as_hip(t->mem);
+        return m->pending == hook && m->pending_ctx == ctx;
+    };
+    if (!left(&p->ir_expand->output_tensors[0], conv_launch_plain, e) || !left(&p->ir_dw->output_tensors[0], conv_launch_plain, d)
+        || (p->ir_relu1 && !left(&p->ir_relu1->output_tensors[0], relu_launch_deferred, p->ir_relu1))
+        || (p->ir_relu2 && !left(&p->ir_relu2->output_tensors[0], relu_launch_deferred, p->ir_relu2)))
+        return false;
+    const void *x = in_ptr(p->ir_expand, 0);
+    if (x == y)
+        return false;
+    int first = 0, zp = 0, bits = 8;
+    float alpha = 1.0f;
+    if (add != nullptr) {
+        const ew_op_t *a = reinterpret_cast<const ew_op_t *>(add);
+        first = add->input_tensors[0]->mem == p->ir_expand->input_tensors[0]->mem;
+        alpha = a->qo.alpha[0], zp = a->qo.zp[0], bits = a->qo.bits[0];
+    }
+    if (hipq_inverted_residual_run(e->plan, d->plan, p->plan, x, (p->ir_relu1 ? 1 : 0) | (p->ir_relu2 ? 2 : 0), add != nullptr, first, alpha, zp,
+                                   bits, y, op_stream(pop)) != 0)
+        return false;
+    g_fused_relus += (p->ir_relu1 != nullptr) + (p->ir_relu2 != nullptr);
+    g_fused_adds += add != nullptr;
+    ++g_fused_inverted;
+    return true; // the tensors in between stay unwritten; their hooks stay for whoever asks
+}
+
 void relu_run(op_t *op)
 {
     ew_op_t *e = reinterpret_cast<ew_op_t *>(op);
@@ -865,7 +962,10 @@ void relu_run(op_t *op)
             const auto it = rm.find(op->output_tensors[0].mem);
             if (!off && it != rm.end() && it->second.size() == 1) {
                 const op_t *r = *it->second.begin();
-                if (r->workspace == op->workspace && r->entry->tp == &op_pool_tp
+                const op_t *block = reinterpret_cast<conv_op_t *>(m->pending_ctx)->ir_project;
+                if (block != nullptr && block != m->pending_ctx)
+                    e->defer = 1; // within an inverted residual block: its last operator launches
+                else if (r->workspace == op->workspace && r->entry->tp == &op_pool_tp
                     && pool_fuses_with(r, reinterpret_cast<conv_op_t *>(m->pending_ctx)->plan))
                     e->defer = 1;
             }
@@ -1246,7 +1346,7 @@ void dequantize_prepare(op_t *op)
 long *const *hip_counters(void)
 {
     static long *const c[kHipCounters] = {&g_fused_adds,     &g_fused_relus,  &g_fused_pools, &g_chained_convs,
-                                          &g_fused_dequants, &g_fused_blocks, &g_fused_tails};
+                                          &g_fused_dequants, &g_fused_blocks, &g_fused_inverted, &g_fused_tails};
     return c;
 }
 
@@ -1321,6 +1421,7 @@ ART_PUBLIC long hip_module_fused_pools(void) { return g_fused_pools; }
 ART_PUBLIC long hip_module_chained_convs(void) { return g_chained_convs; }
 ART_PUBLIC long hip_module_fused_dequants(void) { return g_fused_dequants; }
 ART_PUBLIC long hip_module_fused_blocks(void) { return g_fused_blocks; }
+ART_PUBLIC long hip_module_fused_inverted(void) { return g_fused_inverted; }
 ART_PUBLIC long hip_module_fused_tails(void) { return g_fused_tails; }
 
 ART_PUBLIC void *hip_workspace_stream(workspace_t *w) { return reinterpret_cast<hip_workspace_t *>(w)->stream; }

@@ -66,6 +66,9 @@ _SIGS = {
                                            C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
     "hipq_bottleneck_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int,
                                       C.c_void_p, C.c_void_p]),
+    "hipq_inverted_residual_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_int, C.c_int]),
+    "hipq_inverted_residual_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_float, C.c_int,
+                                             C.c_int, C.c_void_p, C.c_void_p]),
     "hipq_bottleneck_tail_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int, C.c_int,
                                                C.c_void_p]),
     "hipq_bottleneck_tail_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float,
@@ -356,6 +359,22 @@ def bottleneck_run(reduce, mid, widen, x, residual_first, oalpha, ozp, y, obits=
     """y = add(widen(mid(reduce(x))), x) in one launch (include/hipq.h: hipq_bottleneck_run)."""
     check(lib().hipq_bottleneck_run(reduce.handle, mid.handle, widen.handle, _ptr(x), int(bool(residual_first)), oalpha, ozp,
                                     obits, _ptr(y), _stream()))
+    return y
+
+
+def inverted_residual_fusable(expand, depthwise, project, add=None, obits=8):
+    """Can expand -> depthwise -> project [-> add(., x)] run as one kernel (include/hipq.h)?  add: None or
+    (residual first?, scale of the sum, its zero point)."""
+    rf, oa, oz = add if add is not None else (False, 1.0, 0)
+    return bool(lib().hipq_inverted_residual_fusable(expand.handle, depthwise.handle, project.handle,
+                                                     int(add is not None), int(bool(rf)), oa, oz, obits))
+
+
+def inverted_residual_run(expand, depthwise, project, x, y, add=None, relus=0, obits=8):
+    """y = project(depthwise(expand(x))) [+ x] in one launch (include/hipq.h: hipq_inverted_residual_run)."""
+    rf, oa, oz = add if add is not None else (False, 1.0, 0)
+    check(lib().hipq_inverted_residual_run(expand.handle, depthwise.handle, project.handle, _ptr(x), relus,
+                                           int(add is not None), int(bool(rf)), oa, oz, obits, _ptr(y), _stream()))
     return y
 
 

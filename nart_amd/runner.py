@@ -37,6 +37,7 @@ class HipqExecutor:
                     self.fused[node.output] = u[0]  # launched at the add's position: both operands exist by then
         self.pooled = {}     # conv output name -> the max-pooling node computed inside the convolution's kernel
         self.blocks = {}     # id(add node) -> (reduce, mid, widen conv nodes) of an identity bottleneck block run as one kernel
+        self.invres = {}     # id(add or projecting conv node) -> (expand, depthwise, project conv nodes) run as one kernel
         self.in_block = {}   # id(conv node) -> the add node of its block
         self.tails = {}      # id(add node) -> (mid, widen, next or None): the block from its 3x3 layer on as one kernel
         self.duals = {}      # id(add node) -> (widen, shortcut): both 1x1 convolutions and the add as one kernel
@@ -88,6 +89,16 @@ class HipqExecutor:
             elif node.kind == "conv" and id(node) in self.in_block:
                 self.buf.pop(y.name, None)  # computed inside the block's kernel, never materialised
                 continue
+            elif id(node) in self.invres:
+                convs = self.invres[id(node)]
+                plans = [self._early.pop(id(c)) for c in convs]
+                self.plans += plans
+                xin = convs[0].inputs[0]
+                add = (node.inputs[0] == xin, y.alpha, y.zp) if node.kind == "add" else None
+                nb = int(np.prod(T[xin].shape)) + int(np.prod(y.shape)) + sum(case.weights[c.attrs["w"]].size + 4 * c.attrs["K"] for c in convs)
+                fn = (lambda ps=plans, i=self.buf[xin], o=out, add=add: hipq.inverted_residual_run(ps[0], ps[1], ps[2], i, o, add))
+                self.steps.append({"label": node.output, "kind": "inverted residual", "fn": fn, "ops": sum(p.ops for p in plans), "bytes": nb,
+                                   "kernel": "conv_mfma_i8_inverted_residual" + ("+add" if add else "")})
             elif node.kind == "add" and id(node) in self.blocks:
                 c1, c2, c3 = self.blocks[id(node)]
                 plans = [self._early.pop(id(c)) for c in (c1, c2, c3)]
@@ -321,6 +332,7 @@ class HipqExecutor:
                     or n.attrs["relu"] or len(uses.get(name, [])) != 1 or name == case.output.name):
                 return None
             return n
+        self._find_inverted_residuals(conv_plan, prod, uses)
         for add in case.nodes:
             if add.kind != "add" or len(add.inputs) != 2 or add.inputs[0] == add.inputs[1]:
                 continue
@@ -343,7 +355,7 @@ class HipqExecutor:
                     break
                 for c, p in zip((c1, c2, c3), plans):
                     self._early.setdefault(id(c), p)  # keep the plans for the operators' own turns
-            if id(add) in self.blocks:
+            if id(add) in self.blocks or id(add) in self.invres:
                 continue
             # a block with a projection shortcut: both inputs of the add are 1x1 convolutions read by nobody else
             pair = [prod.get(i) for i in add.inputs]
@@ -392,6 +404,46 @@ class HipqExecutor:
                 self._early.setdefault(id(c2), p2)
                 self._early.setdefault(id(c3), p3)
 
+    def _find_inverted_residuals(self, conv_plan, prod, uses):
+        """1x1, depthwise 3x3, 1x1 [and the add with the first one's input] that hipq_inverted_residual_run computes in one launch."""
+        case = self.case
+        T = case.tensors
+
+        def only_use(name):
+            u = uses.get(name, [])
+            return u[0] if len(u) == 1 and name != case.output.name else None
+
+        def is_conv(n, k):
+            return n is not None and n.kind == "conv" and n.attrs["k"] == k and n.attrs["pad"] == k // 2
+        for d in case.nodes:
+            if not is_conv(d, 3) or d.attrs["group"] != T[d.inputs[0]].shape[1] or d.attrs["group"] == 1:
+                continue
+            e, p = prod.get(d.inputs[0]), only_use(d.output)
+            if (not is_conv(e, 1) or only_use(e.output) is not d or not is_conv(p, 1) or T[e.inputs[0]].dtype != "u8"
+                    or any(n.attrs["group"] != 1 or n.attrs["stride"] != 1 for n in (e, p))):
+                continue
+            add = only_use(p.output)
+            if (add is None or add.kind != "add" or sorted(add.inputs) != sorted([p.output, e.inputs[0]]) or p.attrs["relu"]
+                    or p.output == e.inputs[0]):
+                add = None
+            plans = [conv_plan(n)[0] for n in (e, d, p)]
+            for n, pl in zip((e, d, p), plans):
+                self._early[id(n)] = pl
+            if self.share is not None:
+                # a part of a batch fuses exactly where the whole did: the tensors in between exist there or they do not
+                if self.share[0].buf.get(d.output) is not None:
+                    continue
+                plans[2].special(2)
+            st = T[add.output] if add is not None else None
+            if not hipq.inverted_residual_fusable(*plans, (add.inputs[0] == e.inputs[0], st.alpha, st.zp) if add is not None else None):
+                continue
+            last = add if add is not None else p
+            self.invres[id(last)] = (e, d, p)
+            for n in (e, d) + ((p,) if add is not None else ()):
+                self.in_block[id(n)] = last
+            if add is None:
+                self.fused.pop(p.output, None)
+
     def _tensor(self, t):
         N, C, H, W = t.shape
         if self.share is not None:
@@ -410,7 +462,7 @@ class HipqExecutor:
     @property
     def elided(self):
         """Names of the tensors that are never materialised (absorbed into a fused kernel)."""
-        return set(self.fused) | set(self.pooled) | set(self.dequantized) | {c.output for cs in self.blocks.values() for c in cs} | {c.output for cs in self.tails.values() for c in cs[:2]} | {c.output for cs in self.duals.values() for c in cs}
+        return set(self.fused) | {c.output for cs in self.invres.values() for c in cs[:2]} | set(self.pooled) | set(self.dequantized) | {c.output for cs in self.blocks.values() for c in cs} | {c.output for cs in self.tails.values() for c in cs[:2]} | {c.output for cs in self.duals.values() for c in cs}
 
     def set_input(self, x):
         inp = self.case.input

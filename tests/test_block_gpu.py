@@ -528,3 +528,51 @@ if __name__ == "__main__":
     for N, CW, HW in ((64, 1024, 14), (64, 512, 28), (64, 256, 56)):
         time_tail(N, CW, HW)
     time_layers()
+
+
+INVRES_CASES = [  # N, CIN, HIDDEN, COUT, H, W, stride
+    (1, 16, 96, 24, 20, 33, 2), (1, 24, 144, 24, 14, 9, 1), (2, 32, 192, 64, 7, 7, 2), (3, 64, 384, 64, 5, 6, 1), (1, 160, 960, 160, 7, 7, 1),
+    (2, 96, 576, 96, 14, 14, 1), (2, 96, 80, 160, 3, 50, 2), (1, 48, 40, 72, 1, 1, 1), (1, 30, 33, 10, 2, 1, 2), (4, 128, 256, 40, 17, 19, 1),
+    (40, 24, 144, 24, 33, 31, 1), (40, 24, 144, 32, 33, 31, 1), (64, 16, 96, 24, 56, 56, 2), (64, 40, 100, 60, 29, 28, 2),
+    (64, 64, 384, 96, 14, 14, 1), (30, 32, 64, 32, 31, 34, 1), (12, 96, 200, 130, 40, 40, 1),
+]
+
+
+@pytest.mark.parametrize("case", INVRES_CASES, ids=lambda c: "x".join(map(str, c)))
+def test_inverted_residual_block(case):
+    """conv_invres_kernel against the oracle's convolutions and add: patches of 2x4, 4x8 and 8x8 outputs and one wave per patch, all
+    partly outside the image, images of one pixel, slices and tiles that are partly empty, both strides, ReLUs in the plan and at
+    the launch, with and without the add in both operand orders."""
+    N, CI, CH, CO, H, W, st = case
+    rng = np.random.default_rng(sum(case))
+    x = rng.integers(0, 256, (N, CI, H, W), dtype=np.uint8)
+    late = bool(sum(case) & 1)  # the ReLUs as flags of the launch instead of the plans
+    t, a, z, plans, cur = x, 0.03, int(rng.integers(0, 256)), [], None
+    qx = (a, z)
+    for k, (C, K, R, s, group) in enumerate(((CI, CH, 1, 1, 1), (CH, CH, 3, st, CH), (CH, CO, 1, 1, 1))):
+        w = rng.integers(1, 256, (K, C // group, R, R), dtype=np.uint8)
+        sigma = 74.0 * 74.0 * math.sqrt(w[0].size) * (0.7 if k else 1.0)
+        b = rng.integers(-int(sigma), int(sigma) + 1, K).astype(np.int32)
+        oa = float(np.float32(0.03 * rng.uniform(0.75, 1.35)))
+        q = (a, z, float(np.float32(oa * 45.0 / (a * sigma))), 128, oa, int(rng.integers(0, 60)) if k < 2 else int(rng.integers(90, 160)))
+        plans.append(hipq.Conv2d(t.shape, w, b, R // 2, s, group, *q, relu=k < 2 and not late))
+        t = orc.conv2d_u8(t, w, b, R // 2, s, group, *q)
+        if k < 2:
+            t = np.maximum(t, q[5]).astype(np.uint8)
+        a, z = q[4], q[5]
+    plans[2].special(2)
+    xd = hipq.to_device_nhwc(x)
+    relus = 3 if late else 0
+    assert hipq.inverted_residual_fusable(*plans), case
+    print("inverted residual", case, late, flush=True)
+    got = hipq.from_device_nhwc(hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), relus=relus), CO)
+    assert len(np.unique(t)) > min(8, t.size // 2)
+    assert np.array_equal(got, t), (case, int((got != t).sum()), np.argwhere(got != t)[:8].tolist())
+    if CI != CO or st != 1:
+        return
+    sa, sz = float(np.float32(math.hypot(a, qx[0]) * 1.1)), int(rng.integers(0, 60))
+    for first in (False, True):
+        want = orc.add_u8(x, t, *qx, a, z, sa, sz) if first else orc.add_u8(t, x, a, z, *qx, sa, sz)
+        y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (first, sa, sz), relus)
+        got = hipq.from_device_nhwc(y, CO)
+        assert np.array_equal(got, want), (case, "add", first, int((got != want).sum()))

@@ -358,6 +358,59 @@ def test_whole_bottleneck_block_runs_as_one_kernel(own_rt):
     ws.delete()
 
 
+@pytest.mark.parametrize("relus", [False, True])
+def test_inverted_residual_block_runs_as_one_kernel(own_rt, relus):
+    """conv_2d (24 -> 144, 1x1) -> depthwise 3x3 -> conv_2d (144 -> 24) -> add with the block's input, with relus as operators of
+    their own or none: the launches are left to the add, whose run() launches hipq_inverted_residual_run.  A host that reads a
+    tensor in between gets the operators one by one; every tensor can still be read afterwards, pass after pass."""
+    import ctypes as C
+    from oracle import orc
+    blocks = own_rt.libs[1].hip_module_fused_inverted
+    blocks.restype = C.c_long
+    ws = own_rt.workspace("hip")
+    rng = np.random.default_rng(41)
+    x = rng.integers(0, 256, (2, 24, 15, 17), dtype=np.uint8)
+    shapes = ((144, 24, 1, 1), (144, 1, 3, 144), (24, 144, 1, 1))
+    ws_w = [rng.integers(1, 256, (K, Cc, k, k), dtype=np.uint8) for K, Cc, k, _ in shapes]
+    bs = [rng.integers(-9000, 9000, s[0]).astype(np.int32) for s in shapes]
+    qs = [dict(ialpha=0.05, izp=9, walpha=0.0018, wzp=128, oalpha=0.06, ozp=30),
+          dict(ialpha=0.06, izp=30, walpha=0.0026, wzp=128, oalpha=0.055, ozp=40),
+          dict(ialpha=0.055, izp=40, walpha=0.0012, wzp=128, oalpha=0.07, ozp=121)]
+    t, wants = x, []
+    for w, b, q, (K, Cc, k, g) in zip(ws_w, bs, qs, shapes):
+        t = orc.conv2d_u8(t, w, b, k // 2, 1, g, q["ialpha"], q["izp"], q["walpha"], 128, q["oalpha"], q["ozp"])
+        wants.append(t)
+        if relus and K == 144:
+            t = np.maximum(t, q["ozp"]).astype(np.uint8)
+            wants.append(t)
+    want = orc.add_u8(x, t, 0.05, 9, 0.07, 121, 0.09, 10)
+    assert len(np.unique(want)) > 32
+    for peek in (None, 0, 1, 2):
+        tx = ws.tensor(x)
+        ops, cur = [], tx
+        for w, b, q, (K, Cc, k, g) in zip(ws_w, bs, qs, shapes):
+            ops.append(ws.conv2d(cur, ws.tensor(w), ws.tensor(b), k // 2, 1, g, q).prepare())
+            cur = ops[-1].output(0)
+            if relus and K == 144:
+                ops.append(ws.relu(cur, dict(ialpha=q["oalpha"], izp=q["ozp"], oalpha=q["oalpha"], ozp=q["ozp"])).prepare())
+                cur = ops[-1].output(0)
+        add = ws.add(tx, cur, dict(ialpha=[0.05, 0.07], izp=[9, 121], oalpha=0.09, ozp=10)).prepare()
+        for rep in range(2):
+            n0 = blocks()
+            for j, o in enumerate(ops):
+                o.run()
+                if peek == j:
+                    assert same_bits(o.output(0).numpy(), wants[j]), (peek, rep)
+            add.run()
+            assert same_bits(add.output(0).numpy(), want), (peek, rep)
+            assert blocks() == n0 + (1 if peek is None else 0), (peek, rep, blocks() - n0)
+        for j, o in enumerate(ops):
+            assert same_bits(o.output(0).numpy(), wants[j]), (peek, j)
+        for o in [add] + ops[::-1]:
+            o.delete()
+    ws.delete()
+
+
 def test_whole_block_and_the_next_stage_first_layer_run_as_one_kernel(own_rt):
     """The same block followed by conv_2d (1024 -> 512, 1x1) that reads the sum: the add leaves its launch to that
     convolution, whose run() launches hipq_bottleneck_run_conv for all five operators; the sum is written as well.  A host
