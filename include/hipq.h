@@ -281,7 +281,8 @@ int hipq_bottleneck_run_conv(const hipq_conv2d_plan *reduce, const hipq_conv2d_p
  * the tensors in between never travel to memory.  `expand`: 1x1 / stride 1, at most 160 input channels; `depthwise`: 3x3 / pad 1 / stride 1 or 2; `project`:
  * 1x1 / stride 1, at most 160 output channels; uint8 tensors, weight zero points 128, per-tensor weight scales, each layer
  * reading its input with the scale and zero point it is written with.  The residual is x itself, read with expand's input
- * scale and zero point; residual_is_input0, oalpha, ozp and obits (8) as in hipq_bottleneck_run.  y must not be x.
+ * scale and zero point, so the add needs stride 1 and as many output as input channels; residual_is_input0, oalpha, ozp and
+ * obits (8) as in hipq_bottleneck_run.  y must not be x.
  * hipq_inverted_residual_fusable answers (1 / 0) whether the plans run this way (by rule where it is faster;
  * hipq_conv2d_plan_special(project, 2): wherever it can); hipq_inverted_residual_run fails with an error otherwise.
  */

@@ -414,10 +414,12 @@ bool point(const ConvArgs &a)
 
 bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
+    // the residual is the block's input, which the kernel reads with the output's geometry: it has to be a tensor of that shape
+    const bool same = d.stride_h == 1 && e.C == p.K && e.in_cs == p.out_cs;
     return plain(d) && d.group == d.C && d.R == 3 && d.S == 3 && d.pad_h == 1 && d.pad_w == 1 && d.stride_h == d.stride_w
         && (d.stride_h == 1 || d.stride_h == 2) && d.in_cs == d.out_cs && d.in_cs % 16 == 0 && point(p) && p.in_cs == d.in_cs && p.N == d.N
         && p.H == d.OH && p.W == d.OW && (long long)p.P * p.out_cs < (1ll << 31) && p.out_cs <= 160
-        && (p.res == nullptr || (p.addq.fast && p.addq.hi == 255)) && point(e) && e.out_cs == d.in_cs && e.in_cs <= 160
+        && (p.res == nullptr || (p.addq.fast && p.addq.hi == 255 && same)) && point(e) && e.out_cs == d.in_cs && e.in_cs <= 160
         && e.N == d.N && e.OH == d.H && e.OW == d.W && (long long)e.P * e.in_cs < (1ll << 31);
 }
 

@@ -1,0 +1,61 @@
+"""Host-side logic of the compiled libraries without a GPU: every case runs in a process of its own in which tests/hip_stub.c
+stands in for the HIP runtime (streams, graphs and copies keep their order, kernels do nothing)."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+# ---- the cases, each in its own process --------------------------------------------------------------------------------------
+def inverted_residual_add_needs_equal_shapes():
+    """The residual of hipq_inverted_residual_run is the block's input, read with the output's geometry: an add is taken only
+    where the two are the same tensor shape, at stride 1 and with equal channels.  (The shapes without an add stay accepted.)"""
+    import numpy as np
+    from nart_amd import hipq
+
+    def block(ci, ch, co, hw, stride):
+        plans = []
+        for C_, K, R, s, g, H in ((ci, ch, 1, 1, 1, hw), (ch, ch, 3, stride, ch, hw), (ch, co, 1, 1, 1, (hw - 1) // stride + 1)):
+            w = np.full((K, C_ // g, R, R), 129, np.uint8)
+            plans.append(hipq.Conv2d((1, C_, H, H), w, None, R // 2, s, g, 0.05, 9, 0.002, 128, 0.05, 9))
+        plans[2].special(2)
+        return plans
+    x, y = np.zeros(1 << 16, np.uint8), np.zeros(1 << 16, np.uint8)  # never touched
+    kernels = C.c_long.in_dll(STUB, "stub_kernels")
+    for ci, ch, co, stride, same in ((24, 144, 24, 1, True), (16, 96, 24, 1, False), (24, 144, 16, 1, False), (24, 144, 24, 2, False),
+                                     (30, 64, 32, 1, False), (32, 64, 30, 1, False)):
+        plans = block(ci, ch, co, 14, stride)
+        assert hipq.inverted_residual_fusable(*plans), (ci, ch, co, stride)
+        for first in (False, True):
+            assert hipq.inverted_residual_fusable(*plans, add=(first, 0.09, 10)) is same, (ci, ch, co, stride, first)
+            before = kernels.value
+            rc = hipq.lib().hipq_inverted_residual_run(*[p.handle for p in plans], x.ctypes.data, 0, 1, int(first), 0.09, 10, 8, y.ctypes.data,
+                                                       None)
+            assert (rc == 0) is same and kernels.value == before + same, (ci, ch, co, stride, first)
+
+
+CASES = [inverted_residual_add_needs_equal_shapes]
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "hip_stub.so")
+    subprocess.check_call(["gcc", "-O1", "-std=gnu11", "-Wall", "-Werror", "-fPIC", "-shared", os.path.join(ROOT, "tests", "hip_stub.c"), "-o", so])
+    return so
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: c.__name__)
+def test_host_side(case, stub):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), stub, case.__name__], cwd=ROOT, stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-4000:]
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    STUB = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+    globals()[sys.argv[2]]()
