@@ -937,6 +937,10 @@ bool inverted_residual_launch(op_t *pop, const op_t *add, void *y)
     if (add != nullptr) {
         const ew_op_t *a = reinterpret_cast<const ew_op_t *>(add);
         first = add->input_tensors[0]->mem == p->ir_expand->input_tensors[0]->mem;
+        // the kernel reads the residual as the expanding layer reads it; either operator may have been prepared again since
+        const int o = first ? 0 : 1;
+        if (a->qi.alpha[o] != e->desc.ialpha || a->qi.zp[o] != e->desc.izp)
+            return false;
         alpha = a->qo.alpha[0], zp = a->qo.zp[0], bits = a->qo.bits[0];
     }
     if (hipq_inverted_residual_run(e->plan, d->plan, p->plan, x, (p->ir_relu1 ? 1 : 0) | (p->ir_relu2 ? 2 : 0), add != nullptr, first, alpha, zp,

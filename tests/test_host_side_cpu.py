@@ -38,7 +38,45 @@ def inverted_residual_add_needs_equal_shapes():
             assert (rc == 0) is same and kernels.value == before + same, (ci, ch, co, stride, first)
 
 
-CASES = [inverted_residual_add_needs_equal_shapes]
+def runtime():
+    from nart_amd import art
+    lib = os.path.join(ROOT, "nart_amd", "lib")
+    return art.Runtime(os.path.join(lib, "libart.so"), [os.path.join(lib, "libart_module_hip.so")])
+
+
+def fused_block_follows_the_scales_of_its_operators():
+    """An inverted residual block that ran as one launch, then one operator alone gets another input scale and is prepared again -
+    the add for its residual, or the first convolution: the two no longer read the block's input alike, so the block runs
+    operator by operator until they do again."""
+    import numpy as np
+    rt = runtime()
+    ws = rt.workspace("hip")
+    fused = rt.libs[1].hip_module_fused_inverted
+    fused.restype = C.c_long
+    x = ws.tensor(np.zeros((2, 24, 15, 17), np.uint8))
+    ops, cur = [], x
+    for K, c, k, g, q in ((144, 24, 1, 1, dict(ialpha=0.05, izp=9, walpha=0.0018, wzp=128, oalpha=0.06, ozp=30)),
+                          (144, 1, 3, 144, dict(ialpha=0.06, izp=30, walpha=0.0026, wzp=128, oalpha=0.055, ozp=40)),
+                          (24, 144, 1, 1, dict(ialpha=0.055, izp=40, walpha=0.0012, wzp=128, oalpha=0.07, ozp=121))):
+        ops.append(ws.conv2d(cur, ws.tensor(np.full((K, c, k, k), 130, np.uint8)), None, k // 2, 1, g, q).prepare())
+        cur = ops[-1].output(0)
+    ops.append(ws.add(x, cur, dict(ialpha=[0.05, 0.07], izp=[9, 121], oalpha=0.09, ozp=10)).prepare())
+
+    def taken():
+        before = fused()
+        for o in ops:
+            o.run()
+        return fused() - before
+    assert taken() == 1 and taken() == 1
+    for ialpha, izp, want in ((0.04, 9, 0), (0.05, 9, 1), (0.05, 11, 0), (0.05, 9, 1)):
+        ops[3].set_quant(ialpha=[ialpha, 0.07], izp=[izp, 121]).config().prepare()
+        assert taken() == want, ("add", ialpha, izp)
+    for ialpha, izp, want in ((0.04, 9, 0), (0.05, 9, 1), (0.05, 11, 0), (0.05, 9, 1)):
+        ops[0].set_quant(ialpha=ialpha, izp=izp).config().prepare()
+        assert taken() == want, ("expanding convolution", ialpha, izp)
+
+
+CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators]
 
 
 @pytest.fixture(scope="module")

@@ -411,6 +411,41 @@ def test_inverted_residual_block_runs_as_one_kernel(own_rt, relus):
     ws.delete()
 
 
+def test_inverted_residual_block_with_changed_scales(own_rt):
+    """The add of a fused block gets another scale for its residual and is prepared again, alone, then the first convolution does:
+    the bytes are the oracle's for the scales that each operator has now."""
+    from oracle import orc
+    ws = own_rt.workspace("hip")
+    rng = np.random.default_rng(42)
+    x = rng.integers(0, 256, (2, 24, 15, 17), dtype=np.uint8)
+    shapes = ((144, 24, 1, 1), (144, 1, 3, 144), (24, 144, 1, 1))
+    ws_w = [rng.integers(1, 256, (K, Cc, k, k), dtype=np.uint8) for K, Cc, k, _ in shapes]
+    qs = [dict(ialpha=0.05, izp=9, walpha=0.0018, wzp=128, oalpha=0.06, ozp=30),
+          dict(ialpha=0.06, izp=30, walpha=0.0026, wzp=128, oalpha=0.055, ozp=40),
+          dict(ialpha=0.055, izp=40, walpha=0.0012, wzp=128, oalpha=0.07, ozp=121)]
+    tx = ws.tensor(x)
+    ops, cur = [], tx
+    for w, q, (K, Cc, k, g) in zip(ws_w, qs, shapes):
+        ops.append(ws.conv2d(cur, ws.tensor(w), None, k // 2, 1, g, q).prepare())
+        cur = ops[-1].output(0)
+    add = ws.add(tx, cur, dict(ialpha=[0.05, 0.07], izp=[9, 121], oalpha=0.09, ozp=10)).prepare()
+    for head, residual in ((0.05, 0.05), (0.05, 0.031), (0.062, 0.031), (0.062, 0.062)):
+        if qs[0]["ialpha"] != head:
+            qs[0]["ialpha"] = head
+            ops[0].set_quant(ialpha=head, izp=9).config().prepare()
+        add.set_quant(ialpha=[residual, 0.07], izp=[9, 121]).config().prepare()
+        t = x
+        for w, q, (K, Cc, k, g) in zip(ws_w, qs, shapes):
+            t = orc.conv2d_u8(t, w, None, k // 2, 1, g, q["ialpha"], q["izp"], q["walpha"], 128, q["oalpha"], q["ozp"])
+        want = orc.add_u8(x, t, residual, 9, 0.07, 121, 0.09, 10)
+        for o in ops + [add]:
+            o.run()
+        assert len(np.unique(want)) > 32 and same_bits(add.output(0).numpy(), want), (head, residual)
+    for o in [add] + ops[::-1]:
+        o.delete()
+    ws.delete()
+
+
 def test_whole_block_and_the_next_stage_first_layer_run_as_one_kernel(own_rt):
     """The same block followed by conv_2d (1024 -> 512, 1x1) that reads the sum: the add leaves its launch to that
     convolution, whose run() launches hipq_bottleneck_run_conv for all five operators; the sum is written as well.  A host
