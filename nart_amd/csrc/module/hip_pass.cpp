@@ -20,6 +20,14 @@ namespace {
 constexpr size_t kShortest = 8; // fewer kernels start sooner one by one (10 take 32 us as a graph, 54 one by one; 5 take 35 and 23)
 constexpr int kMaxRecords = 16; // a program that prepares or reallocates before every pass would record every second one for nothing
 
+// A HIP call that may fail here without harm: its error does not stay behind for the next launch's check.
+bool worked(hipError_t e)
+{
+    if (e != hipSuccess)
+        (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
 // an input of the pass, as the record found it
 struct PassInput {
     hip_mem_t *m;
@@ -49,7 +57,7 @@ struct Pass {
     {
         if (exec) {
             HIPM_HIP(hipDeviceSynchronize()); // a replay may be under way, on a stream that may be gone
-            (void)hipGraphExecDestroy(exec);
+            (void)worked(hipGraphExecDestroy(exec));
         }
         exec = nullptr;
         runs = 0;
@@ -58,10 +66,11 @@ struct Pass {
     }
 };
 
-bool capturing(hipStream_t st)
+// The null stream cannot be captured; a stream whose owner is capturing it takes the operators into that graph.
+bool recordable(hipStream_t st)
 {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(st, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+    return st != nullptr && worked(hipStreamIsCapturing(st, &s)) && s == hipStreamCaptureStatusNone;
 }
 
 // The inputs of the pass: memories that an operator reads before any has written them.  One that the host has just written and
@@ -132,18 +141,18 @@ bool record(Pass &p, op_t *const *ops, size_t n)
     long before[kHipCounters];
     for (int c = 0; c < kHipCounters; ++c)
         before[c] = *hip_counters()[c];
-    if (hipStreamBeginCapture(p.st, hipStreamCaptureModeThreadLocal) != hipSuccess)
+    if (!worked(hipStreamBeginCapture(p.st, hipStreamCaptureModeThreadLocal)))
         return false;
     for (size_t i = 0; i < n; ++i)
         op_run(ops[i]);
     collect_outputs(p, ops, n);
     hipGraph_t g = nullptr;
     size_t nodes = 0;
-    bool ok = hipStreamEndCapture(p.st, &g) == hipSuccess && g != nullptr;
-    ok = ok && hipGraphGetNodes(g, nullptr, &nodes) == hipSuccess && nodes >= kShortest;
-    ok = ok && hipGraphInstantiate(&p.exec, g, nullptr, nullptr, 0) == hipSuccess;
+    bool ok = worked(hipStreamEndCapture(p.st, &g)) && g != nullptr;
+    ok = ok && worked(hipGraphGetNodes(g, nullptr, &nodes)) && nodes >= kShortest;
+    ok = ok && worked(hipGraphInstantiate(&p.exec, g, nullptr, nullptr, 0));
     if (g)
-        (void)hipGraphDestroy(g);
+        (void)worked(hipGraphDestroy(g));
     for (int c = 0; c < kHipCounters; ++c) {
         p.counted[c] = *hip_counters()[c] - before[c];
         *hip_counters()[c] = before[c];
@@ -184,7 +193,7 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
 {
     static const bool off = getenv("NART_HIP_NO_GRAPH") != nullptr;
     hip_workspace_t *ws = reinterpret_cast<hip_workspace_t *>(ops[0]->workspace);
-    if (off || capturing(ws->stream))
+    if (off || !recordable(ws->stream))
         return false;
     if (*state == nullptr)
         *state = new Pass;

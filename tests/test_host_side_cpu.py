@@ -76,7 +76,48 @@ def fused_block_follows_the_scales_of_its_operators():
         assert taken() == want, ("expanding convolution", ialpha, izp)
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators]
+def small_parade(rt, ws, hw=64):
+    """An engine file whose pass is long enough to be recorded, and one pass over it: one() returns what that pass did."""
+    import numpy as np
+    from nart_amd import cases, engine
+    case = cases.resnet18(N=1, hw=hw)
+    p = engine.Parade(rt, engine.write_engine(case), [ws])
+    x = np.zeros(case.input.shape, np.float32)
+    count = {n: C.c_long.in_dll(STUB, "stub_" + n) for n in ("kernels", "captures", "graph_launches")}
+
+    def one(read=True):
+        before = {n: c.value for n, c in count.items()}
+        p.inputs()[0].write(x)
+        p.run()
+        if read:
+            p.outputs()[0].numpy()
+        did = {n: c.value - before[n] for n, c in count.items()}
+        return "recorded" if did["captures"] else "replayed" if did["graph_launches"] else "eager" if did["kernels"] else "nothing"
+    return p, one
+
+
+def a_pass_that_cannot_be_recorded_runs_its_operators():
+    """On the null stream, which cannot be captured, and where the runtime refuses the graph: every pass runs operator by
+    operator, and no error stays behind for the next launch to find."""
+    rt = runtime()
+    ws = rt.workspace("hip")
+    rt.libs[1].hip_workspace_set_stream.argtypes = [C.c_void_p, C.c_void_p]
+    rt.libs[1].hip_workspace_set_stream(ws.ptr, None)
+    p, one = small_parade(rt, ws)
+    assert [one() for _ in range(5)] == ["eager"] * 5 and STUB.stub_error() == 0
+    p.delete()
+    ws.delete()
+    fail = C.c_long.in_dll(STUB, "stub_fail_instantiate")
+    fail.value = 1
+    ws = rt.workspace("hip")
+    p, one = small_parade(rt, ws)
+    for i in range(4):
+        assert one() == ("recorded" if i == 1 else "eager") and STUB.stub_error() == 0, i  # pass 1: tried, refused, then run
+    p.delete()
+
+
+CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
+         a_pass_that_cannot_be_recorded_runs_its_operators]
 
 
 @pytest.fixture(scope="module")

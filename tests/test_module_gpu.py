@@ -56,6 +56,27 @@ def test_engine_file_runs_on_hip_workspace(own_rt):
     ws.delete()
 
 
+@pytest.mark.parametrize("stream", ["null", "own", "torch"])
+def test_passes_on_the_streams_of_a_workspace(own_rt, stream):
+    """Five passes over one engine file on the null stream (never recorded), on the workspace's own stream and on a caller's: the
+    first runs operator by operator, the second may be recorded, later ones replayed; every one gives the oracle's bytes."""
+    import ctypes as C
+    set_stream = own_rt.libs[1].hip_workspace_set_stream
+    set_stream.argtypes = [C.c_void_p, C.c_void_p]
+    ws = own_rt.workspace("hip")
+    theirs = torch.cuda.Stream()
+    if stream != "own":
+        set_stream(ws.ptr, theirs.cuda_stream if stream == "torch" else None)
+    case = cases.resnet18(N=1, hw=64)
+    p = engine.Parade(own_rt, engine.write_engine(case), [ws])
+    for seed in range(5):
+        x = casecpu.random_input(case, seed)
+        got = p.forward(x).reshape(case.output.shape)
+        assert same_bits(got, casecpu.run_case(case, x)[case.output.name]), (stream, seed)
+    p.delete()
+    ws.delete()
+
+
 def test_version2_engine_file(own_rt):
     """Version-2 engine files (an optional pre-processing block after every input declaration) load on the repo's core
     and run on the hip workspace; the block is handed back unchanged."""
