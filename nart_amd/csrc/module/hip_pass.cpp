@@ -10,6 +10,7 @@
 // beside launching - which side of a memory is current, which launches were left to a reader - is recorded as well, as the
 // state it leaves behind, and restored by a replay.  A record is dropped when an operator of the workspace is prepared or
 // destroyed, the workspace's stream changes, or a buffer it names has moved.
+#include <algorithm>
 #include <set>
 #include <vector>
 
@@ -18,7 +19,8 @@
 namespace {
 
 constexpr size_t kShortest = 8; // fewer kernels start sooner one by one (10 take 32 us as a graph, 54 one by one; 5 take 35 and 23)
-constexpr int kMaxRecords = 16; // a program that prepares or reallocates before every pass would record every second one for nothing
+constexpr long kWorth = 16;     // replays after which a record has paid for itself
+constexpr int kMaxWait = 256;   // eager passes before the next record, at most
 
 // A HIP call that may fail here without harm: its error does not stay behind for the next launch's check.
 bool worked(hipError_t e)
@@ -47,20 +49,27 @@ struct PassOutput {
 struct Pass {
     uint64_t epoch = 0;
     hipStream_t st = nullptr;
-    int runs = 0, records = 0;
+    int runs = 0;    // passes run operator by operator since the last record
+    int wait = 1;    // how many of them before the next
+    long served = 0; // replays of the present record
     hipGraphExec_t exec = nullptr;
     std::vector<PassInput> in;
     std::vector<PassOutput> out;
     long counted[kHipCounters] = {};
 
-    void forget()
+    // A program that prepares or reallocates before every few passes would record for nothing: each record that has not served
+    // kWorth replays, or was refused, doubles the passes until the next attempt, one that has sets them back to one.
+    void forget(bool refused = false)
     {
         if (exec) {
             HIPM_HIP(hipDeviceSynchronize()); // a replay may be under way, on a stream that may be gone
             (void)worked(hipGraphExecDestroy(exec));
         }
+        if (exec || refused)
+            wait = served >= kWorth ? 1 : std::min(2 * wait, kMaxWait);
         exec = nullptr;
         runs = 0;
+        served = 0;
         in.clear();
         out.clear();
     }
@@ -202,18 +211,17 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
         p.forget();
         p.epoch = ws->epoch, p.st = ws->stream;
     }
+    if (p.exec != nullptr && !still_good(p))
+        p.forget();
     if (p.exec == nullptr) {
-        if (++p.runs < 2 || p.records >= kMaxRecords)
+        if (p.runs++ < p.wait)
             return false;
-        ++p.records;
         if (!record(p, ops, n)) {
-            p.forget();
-            p.records = kMaxRecords;
+            p.forget(true);
             return false;
         }
-    } else if (!still_good(p)) {
-        p.forget();
-        return false;
+    } else {
+        ++p.served;
     }
     HIPM_HIP(hipGraphLaunch(p.exec, p.st));
     for (int c = 0; c < kHipCounters; ++c)

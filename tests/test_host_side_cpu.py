@@ -116,8 +116,32 @@ def a_pass_that_cannot_be_recorded_runs_its_operators():
     p.delete()
 
 
+def records_are_taken_again_after_many_changes():
+    """A program that prepares its parade again before every third pass, or creates parades beside it, gets fewer and fewer
+    attempts to record; once it leaves the parade alone its passes are recorded and replayed again."""
+    rt = runtime()
+    ws = rt.workspace("hip")
+    p, one = small_parade(rt, ws)
+    did = []
+    for _ in range(40):
+        rt.core.parade_prepare(p.ptr)
+        did += [one(), one(), one()]
+    assert did[:3] == ["eager", "recorded", "replayed"] and did.count("recorded") <= 3
+    settled = [one() for _ in range(600)]
+    assert settled.count("recorded") == 1 and settled[-300:] == ["replayed"] * 300
+    rt.core.parade_prepare(p.ptr)  # a record that has served long: the next is taken at once
+    assert [one() for _ in range(3)] == ["eager", "recorded", "replayed"]
+    for _ in range(20):
+        small_parade(rt, ws)[0].delete()
+        one()
+    assert [one() for _ in range(600)][-300:] == ["replayed"] * 300
+    p.delete()
+    ws.delete()
+
+
 CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
-         a_pass_that_cannot_be_recorded_runs_its_operators]
+         a_pass_that_cannot_be_recorded_runs_its_operators,
+         records_are_taken_again_after_many_changes]
 
 
 @pytest.fixture(scope="module")
