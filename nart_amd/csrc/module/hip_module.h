@@ -97,7 +97,8 @@ struct hip_mem_t {
     void (*pending)(void *ctx);
     void *pending_ctx;
     // The mirror is being filled from the device by work queued on prod_stream (a recorded pass ends with that): whoever
-    // wants it waits for that stream.  host_read: the host has asked for device-written contents before.
+    // wants it waits for that stream.  host_read: the host has asked for device-written contents
+    // since a pass was last recorded.
     bool down_issued, host_read;
     // A float input whose reader is a uint8 quantize operator (quantize_prepare fills q_*).  hip_mem_write quantizes the
     // values while it copies them into the mirror, a quarter of the bytes to bring to the device; q_valid: qhost (pinned) and,

@@ -21,6 +21,7 @@ namespace {
 constexpr size_t kShortest = 8; // fewer kernels start sooner one by one (10 take 32 us as a graph, 54 one by one; 5 take 35 and 23)
 constexpr long kWorth = 16;     // replays after which a record has paid for itself
 constexpr int kMaxWait = 256;   // eager passes before the next record, at most
+constexpr int kUnread = 8;      // replays in a row that copied back an output nobody asked for
 
 // A HIP call that may fail here without harm: its error does not stay behind for the next launch's check.
 bool worked(hipError_t e)
@@ -52,6 +53,7 @@ struct Pass {
     int runs = 0;    // passes run operator by operator since the last record
     int wait = 1;    // how many of them before the next
     long served = 0; // replays of the present record
+    int unread = 0;  // the last of them after which an output that the record copies back was not read
     hipGraphExec_t exec = nullptr;
     std::vector<PassInput> in;
     std::vector<PassOutput> out;
@@ -59,17 +61,17 @@ struct Pass {
 
     // A program that prepares or reallocates before every few passes would record for nothing: each record that has not served
     // kWorth replays, or was refused, doubles the passes until the next attempt, one that has sets them back to one.
-    void forget(bool refused = false)
+    void forget(bool refused = false, bool for_less = false)
     {
         if (exec) {
             HIPM_HIP(hipDeviceSynchronize()); // a replay may be under way, on a stream that may be gone
             (void)worked(hipGraphExecDestroy(exec));
         }
-        if (exec || refused)
+        if ((exec || refused) && !for_less)
             wait = served >= kWorth ? 1 : std::min(2 * wait, kMaxWait);
         exec = nullptr;
         runs = 0;
-        served = 0;
+        served = unread = 0;
         in.clear();
         out.clear();
     }
@@ -132,8 +134,10 @@ void collect_outputs(Pass &p, op_t *const *ops, size_t n)
             hip_mem_t *m = as_hip(ops[i]->output_tensors[k].mem);
             if (!seen.insert(m).second)
                 continue;
-            // what the host has fetched after an earlier pass it will fetch again: the record ends with the copy
-            if (m->host_read && m->host != nullptr && m->host_cap >= m->size && m->dev_valid && !m->host_valid && !m->pending
+            // what the host has fetched since the last record it will fetch again: the record ends with the copy
+            const bool wanted = m->host_read;
+            m->host_read = false;
+            if (wanted && m->host != nullptr && m->host_cap >= m->size && m->dev_valid && !m->host_valid && !m->pending
                 && !m->down_issued && m->size <= kHostDirect)
                 hip_mem_start_download(m);
             p.out.push_back({m, m->dev, m->host, m->dev_valid, m->host_valid, m->down_issued, m->pending, m->pending_ctx});
@@ -213,6 +217,14 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
     }
     if (p.exec != nullptr && !still_good(p))
         p.forget();
+    if (p.exec != nullptr) {
+        bool unread = false;
+        for (const PassOutput &o : p.out)
+            unread = unread || (o.down_issued && o.m->down_issued);
+        p.unread = unread ? p.unread + 1 : 0;
+        if (p.unread > kUnread)
+            p.forget(false, true); // the next record copies back what has been read by then
+    }
     if (p.exec == nullptr) {
         if (p.runs++ < p.wait)
             return false;
