@@ -451,6 +451,10 @@ extern "C" __attribute__((visibility("default"))) bool hip_mem_write(mem_t *mm, 
         return false;
     hip_mem_t *m = as_hip(mm);
     m->pending = nullptr; // about to be overwritten, all of it
+    if (m->down_issued) { // the device is still writing the mirror
+        wait_stream(m->prod_stream);
+        m->down_issued = false;
+    }
     ensure_host(m);
     finish_upload(m);
     const bool known = stream_known(m->up_stream);

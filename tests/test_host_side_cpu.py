@@ -174,9 +174,43 @@ def an_output_that_nobody_reads_is_not_copied_back():
     ws.delete()
 
 
+def a_write_waits_for_the_copy_back_that_fills_the_same_mirror():
+    """A replayed pass has queued the copy of its output into the host mirror; the program then writes an array of its own into that
+    tensor (hip_mem_write) and reads it: it gets its array, not what the copy brings later."""
+    import numpy as np
+    from nart_amd import cases, engine
+    rt = runtime()
+    ws = rt.workspace("hip")
+    # ten convolutions, then floats: their copy into the mirror is one of the runtime's own copies
+    c = cases.Case("chain", 3)
+    t = c.input_u8((1, 16, 8, 8), 0.05, 9)
+    for _ in range(10):
+        t = c.conv(t, 16, 3)
+    c.output = c.dequantize(t)
+    p = engine.Parade(rt, engine.write_engine(c), [ws])
+    out = p.outputs()[0]
+    write = rt.libs[1].hip_mem_write
+    write.argtypes, write.restype = [C.c_void_p, C.c_void_p, C.c_size_t], C.c_bool
+    replays = C.c_long.in_dll(STUB, "stub_graph_launches")
+    for i in range(4):
+        p.inputs()[0].write(np.zeros((1, 16, 8, 8), np.uint8))
+        p.run()
+        if i < 3:
+            out.numpy()
+    assert replays.value >= 2
+    mine = np.arange(out.numpy().size, dtype=np.float32).reshape(out.shape)
+    p.run()
+    assert write(out.ptr.contents.mem, mine.ctypes.data, mine.nbytes)
+    rt.libs[1].hip_workspace_synchronize(C.c_void_p(C.addressof(ws.ptr.contents)))
+    assert np.array_equal(out.numpy(), mine)
+    p.delete()
+    ws.delete()
+
+
 CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
          a_pass_that_cannot_be_recorded_runs_its_operators,
-         records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back]
+         records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
+         a_write_waits_for_the_copy_back_that_fills_the_same_mirror]
 
 
 @pytest.fixture(scope="module")
