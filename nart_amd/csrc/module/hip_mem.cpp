@@ -165,8 +165,24 @@ static void download(hip_mem_t *m)
 
 bool hip_mem_uploads_direct(const hip_mem_t *m) { return m->layout == HIP_LAYOUT_NHWC_U8 && m->size <= kHostDirect; }
 
+// the pinned memory is about to be handed out for writing: what still reads it must finish first
+static void finish_upload(hip_mem_t *m)
+{
+    if (m->up_pending) {
+        wait_stream(m->up_stream);
+        m->up_pending = false;
+    }
+}
+
+void hip_mem_read_on(hip_mem_t *m, hipStream_t st)
+{
+    if (m->up_stream != st)
+        finish_upload(m); // one stream is remembered: the one before has finished
+}
+
 static void upload(hip_mem_t *m, hipStream_t st)
 {
+    hip_mem_read_on(m, st);
     grow_dev(&m->dev, &m->dev_cap, dev_bytes(m));
     if (hip_mem_uploads_direct(m)) {
         HIPM_HIPQ(hipq_nchw_to_nhwc_u8(m->host, m->dev, m->N, m->C, m->H, m->W, m->cs, st));
@@ -182,15 +198,6 @@ static void upload(hip_mem_t *m, hipStream_t st)
     m->up_stream = st;
     m->prod_stream = st;
     m->down_issued = false;
-}
-
-// the mirror is about to be handed out for writing: an upload that still reads it must finish first
-static void finish_upload(hip_mem_t *m)
-{
-    if (m->up_pending) {
-        wait_stream(m->up_stream);
-        m->up_pending = false;
-    }
 }
 
 // mem_cpu_data(): the caller may read or WRITE through the pointer (the runtime fills inputs and weights this
@@ -227,8 +234,8 @@ const void *hip_mem_dev_in(mem_t *mm, hipStream_t st)
         ensure_host(m); // never-written memory reads as zeros
         m->host_valid = true;
         upload(m, st);
-    } else if (m->up_pending && m->up_stream != st) {
-        finish_upload(m); // brought here on another stream (hip_mem_write)
+    } else {
+        hip_mem_read_on(m, st); // it may be on its way here on another stream (hip_mem_write)
     }
     return m->dev;
 }

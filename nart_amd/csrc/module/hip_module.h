@@ -146,6 +146,8 @@ void *hip_mem_dev_out(mem_t *m, hipStream_t st);
 const void *hip_mem_host_in(mem_t *m);
 // May the next upload of this memory be a kernel that reads the pinned mirror?
 bool hip_mem_uploads_direct(const hip_mem_t *m);
+// Work on `st` is about to read the pinned memory (mirror or quantized bytes): waits for another stream that still does.
+void hip_mem_read_on(hip_mem_t *m, hipStream_t st);
 // Queues the device -> host copy of the contents on the stream that wrote them, without waiting.
 void hip_mem_start_download(hip_mem_t *m);
 static inline hip_mem_t *as_hip(mem_t *m) { return reinterpret_cast<hip_mem_t *>(m); }

@@ -1248,8 +1248,7 @@ void quantize_run(op_t *op)
     hip_mem_t *x = as_hip(op->input_tensors[0]->mem);
     if (x->q_valid && x->q_op == op) { // quantized on its way in (hip_mem_write): what is left is the layout
         const bool direct = x->size / 4 <= kHostDirect;
-        if (x->up_pending && x->up_stream != op_stream(op))
-            HIPM_HIP(hipStreamSynchronize(x->up_stream));
+        hip_mem_read_on(x, op_stream(op));
         HIPM_HIPQ(hipq_nchw_to_nhwc_u8(direct ? x->qhost : x->qdev, out_ptr(op), d[0], d[1], d[2], d[3], y->cs, op_stream(op)));
         x->up_pending = true, x->up_stream = op_stream(op);
         return;

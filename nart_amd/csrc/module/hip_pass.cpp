@@ -107,9 +107,11 @@ bool collect_inputs(Pass &p, op_t *const *ops, size_t n)
             PassInput in = {m, PassInput::kDevice, nullptr, nullptr};
             if (m->q_valid && m->q_op == ops[i]) {
                 in.from = PassInput::kQuantized;
+                hip_mem_read_on(m, p.st);
                 in.src = m->qhost, in.dev = m->qdev;
             } else if (m->host_valid && !m->dev_valid && m->host != nullptr && m->dev != nullptr && hip_mem_uploads_direct(m)) {
                 in.from = PassInput::kMirror;
+                hip_mem_read_on(m, p.st);
                 in.src = m->host, in.dev = m->dev;
             } else {
                 in.dev = hip_mem_dev_in(mm, p.st);
@@ -185,11 +187,13 @@ bool still_good(const Pass &p)
         hip_mem_t *m = in.m;
         hip_mem_settle(m);
         if (in.from == PassInput::kQuantized) {
-            if (!m->q_valid || m->qhost != in.src || m->qdev != in.dev || (m->up_pending && m->up_stream != p.st))
+            if (!m->q_valid || m->qhost != in.src || m->qdev != in.dev)
                 return false;
+            hip_mem_read_on(m, p.st);
         } else if (in.from == PassInput::kMirror) {
             if (!m->host_valid || m->host != in.src || m->dev != in.dev)
                 return false;
+            hip_mem_read_on(m, p.st);
         } else if (hip_mem_dev_in(&m->m, p.st) != in.dev) {
             return false;
         }

@@ -68,7 +68,13 @@ int hipDeviceSynchronize(void)
         drain(s);
     return kSuccess;
 }
-int hipMalloc(void **p, size_t n) { return *p = calloc(n ? n : 1, 1), kSuccess; }
+int hipMalloc(void **p, size_t n) /* whole pages, as the runtime gives */
+{
+    n = (n + 4096) / 4096 * 4096;
+    *p = aligned_alloc(4096, n);
+    memset(*p, 0, n);
+    return kSuccess;
+}
 int hipFree(void *p) { return hipDeviceSynchronize(), free(p), kSuccess; }
 int hipHostMalloc(void **p, size_t n, unsigned f) { return (void)f, hipMalloc(p, n); }
 int hipHostFree(void *p) { return hipFree(p); }

@@ -207,10 +207,62 @@ def a_write_waits_for_the_copy_back_that_fills_the_same_mirror():
     ws.delete()
 
 
+def a_write_waits_for_every_stream_that_reads_the_array():
+    """One float input, quantize operators on two workspaces: the one prepared last reads the quantized bytes in pinned memory, the
+    other the values.  The next array is written only when both streams have read the one before - also when one of the
+    workspaces replays a recorded pass."""
+    import numpy as np
+    rt = runtime()
+    write = rt.libs[1].hip_mem_write
+    write.argtypes, write.restype = [C.c_void_p, C.c_void_p, C.c_size_t], C.c_bool
+    stream_of = rt.libs[1].hip_workspace_stream
+    stream_of.argtypes, stream_of.restype = [C.c_void_p], C.c_void_p
+    STUB.stub_pending.argtypes, STUB.stub_pending.restype = [C.c_void_p], C.c_long
+    for n in (8, 2048):  # read by the kernels directly; above 4 MB of bytes (16 MB of values) brought to the device first
+        a = np.ones((1, 3, n, 1024 if n > 8 else n), np.float32)
+        two = [rt.workspace("hip"), rt.workspace("hip")]
+        streams = [stream_of(w.ptr) for w in two]
+        for order in ((0, 1), (1, 0)):
+            x = two[0].tensor(a)
+            ops = [w.quantize(x, 0.1, 3).prepare() for w in two]
+            for _ in range(3):
+                assert write(x.ptr.contents.mem, a.ctypes.data, a.nbytes)
+                for k in order:
+                    ops[k].run()
+                assert max(STUB.stub_pending(s) for s in streams) > 0
+                assert write(x.ptr.contents.mem, a.ctypes.data, a.nbytes)
+                pending = [STUB.stub_pending(s) for s in streams]  # above the line: the new array's own copies, on one stream
+                assert pending == [0, 0] if n == 8 else 0 in pending, (n, order, pending)
+                for o in ops:
+                    o.run()
+            for o in ops:
+                o.delete()
+    # a recorded pass on the first workspace, the values read by an operator on the second
+    from nart_amd import cases, engine
+    c = cases.Case("chain", 3)
+    t = c.quantize(c.input_f32((1, 16, 8, 8)), 0.05, 9)
+    for _ in range(10):
+        t = c.conv(t, 16, 3)
+    c.output = t
+    a = np.ones((1, 16, 8, 8), np.float32)
+    p = engine.Parade(rt, engine.write_engine(c), [two[0]])
+    x = p.inputs()[0]
+    replays, captures = (C.c_long.in_dll(STUB, "stub_" + k) for k in ("graph_launches", "captures"))
+    quantize = two[1].quantize(x, 0.07, 5).prepare()
+    for i in range(6):
+        assert write(x.ptr.contents.mem, a.ctypes.data, a.nbytes)
+        quantize.run()
+        p.run()
+        assert write(x.ptr.contents.mem, a.ctypes.data, a.nbytes)
+        assert [STUB.stub_pending(s) for s in streams] == [0, 0], i
+        p.run()
+    assert captures.value >= 1 and replays.value >= 3
+
+
 CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
-         a_write_waits_for_the_copy_back_that_fills_the_same_mirror]
+         a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array]
 
 
 @pytest.fixture(scope="module")
