@@ -12,7 +12,7 @@
 
 #include "hip_module.h"
 
-// The streams of the live `hip` workspaces.  A memory remembers the stream that last wrote its device side and the one
+// The streams of the live `hip` workspaces.  A memory remembers the stream that last used its device side and the one
 // that last read its host mirror, and may outlive the workspace that owned it: a stream that has been retired was
 // synchronised when its workspace went away, so there is nothing left to wait for (and nothing valid to wait on).
 static std::vector<hipStream_t> &live_streams()
@@ -180,9 +180,19 @@ void hip_mem_read_on(hip_mem_t *m, hipStream_t st)
         finish_upload(m); // one stream is remembered: the one before has finished
 }
 
+void hip_mem_use_on(hip_mem_t *m, hipStream_t st)
+{
+    if (m->prod_stream == st)
+        return;
+    if (m->dev)
+        wait_stream(m->prod_stream);
+    m->prod_stream = st;
+}
+
 static void upload(hip_mem_t *m, hipStream_t st)
 {
     hip_mem_read_on(m, st);
+    hip_mem_use_on(m, st);
     grow_dev(&m->dev, &m->dev_cap, dev_bytes(m));
     if (hip_mem_uploads_direct(m)) {
         HIPM_HIPQ(hipq_nchw_to_nhwc_u8(m->host, m->dev, m->N, m->C, m->H, m->W, m->cs, st));
@@ -196,7 +206,6 @@ static void upload(hip_mem_t *m, hipStream_t st)
     m->dev_valid = true;
     m->up_pending = true; // the copy still reads the mirror
     m->up_stream = st;
-    m->prod_stream = st;
     m->down_issued = false;
 }
 
@@ -235,7 +244,7 @@ const void *hip_mem_dev_in(mem_t *mm, hipStream_t st)
         m->host_valid = true;
         upload(m, st);
     } else {
-        hip_mem_read_on(m, st); // it may be on its way here on another stream (hip_mem_write)
+        hip_mem_use_on(m, st);
     }
     return m->dev;
 }
@@ -244,7 +253,7 @@ void *hip_mem_dev_out(mem_t *mm, hipStream_t st)
 {
     hip_mem_t *m = as_hip(mm);
     m->pending = nullptr; // about to be overwritten: a deferred producer's result is dead
-    m->prod_stream = st;  // whoever reads the contents from outside that stream waits for it first
+    hip_mem_use_on(m, st);
     grow_dev(&m->dev, &m->dev_cap, dev_bytes(m));
     m->dev_valid = true;
     m->host_valid = m->down_issued = m->q_valid = false;
@@ -482,6 +491,8 @@ extern "C" __attribute__((visibility("default"))) bool hip_mem_write(mem_t *mm, 
     uint8_t *to = nullptr;
     const uint8_t *from = quant ? m->qhost : static_cast<const uint8_t *>(m->host);
     if (known && dbytes > kHostDirect) {
+        if (!quant)
+            hip_mem_use_on(m, m->up_stream);
         if (quant) {
             grow_dev(reinterpret_cast<void **>(&m->qdev), &m->qdev_cap, dbytes);
             to = m->qdev;
@@ -527,7 +538,6 @@ extern "C" __attribute__((visibility("default"))) bool hip_mem_write(mem_t *mm, 
             if (m->layout == HIP_LAYOUT_NHWC_U8)
                 HIPM_HIPQ(hipq_nchw_to_nhwc_u8(m->stage, m->dev, m->N, m->C, m->H, m->W, m->cs, m->up_stream));
             m->dev_valid = true;
-            m->prod_stream = m->up_stream;
         }
         m->up_pending = true;
     }

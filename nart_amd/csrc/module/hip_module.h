@@ -88,8 +88,8 @@ struct hip_mem_t {
     // once that copy has finished.
     bool up_pending;
     hipStream_t up_stream;
-    // The stream whose work last wrote `dev` (a workspace's, or the null stream for an upload on behalf of foreign code):
-    // a reader outside that stream waits for it, and for nothing else.
+    // The stream whose work last used `dev` (a workspace's, or the null stream on behalf of foreign code); what others did to
+    // it before has finished.  Whoever uses it on another stream, or wants the contents, waits for this one, and for nothing else.
     hipStream_t prod_stream;
     // Deferred producer.  A convolution whose only reader is an add does not launch at its own run(): it leaves this
     // hook, and the add runs both as one fused kernel (hip_ops.cpp).  Whoever else asks for the contents first - the
@@ -146,6 +146,8 @@ void *hip_mem_dev_out(mem_t *m, hipStream_t st);
 const void *hip_mem_host_in(mem_t *m);
 // May the next upload of this memory be a kernel that reads the pinned mirror?
 bool hip_mem_uploads_direct(const hip_mem_t *m);
+// Work on `st` is about to read or write the device side: waits for another stream that still uses it.
+void hip_mem_use_on(hip_mem_t *m, hipStream_t st);
 // Work on `st` is about to read the pinned memory (mirror or quantized bytes): waits for another stream that still does.
 void hip_mem_read_on(hip_mem_t *m, hipStream_t st);
 // Queues the device -> host copy of the contents on the stream that wrote them, without waiting.

@@ -112,6 +112,7 @@ bool collect_inputs(Pass &p, op_t *const *ops, size_t n)
             } else if (m->host_valid && !m->dev_valid && m->host != nullptr && m->dev != nullptr && hip_mem_uploads_direct(m)) {
                 in.from = PassInput::kMirror;
                 hip_mem_read_on(m, p.st);
+                hip_mem_use_on(m, p.st);
                 in.src = m->host, in.dev = m->dev;
             } else {
                 in.dev = hip_mem_dev_in(mm, p.st);
@@ -122,6 +123,7 @@ bool collect_inputs(Pass &p, op_t *const *ops, size_t n)
             mem_t *mm = ops[i]->output_tensors[k].mem;
             if (!is_hip_mem(mm) || seen.count(mm)) // an operator writes what an earlier one reads: a view of an input
                 return false;
+            hip_mem_use_on(as_hip(mm), p.st); // another workspace's operators may be reading what the pass before left there
             written.insert(mm);
         }
     }
@@ -194,13 +196,16 @@ bool still_good(const Pass &p)
             if (!m->host_valid || m->host != in.src || m->dev != in.dev)
                 return false;
             hip_mem_read_on(m, p.st);
+            hip_mem_use_on(m, p.st);
         } else if (hip_mem_dev_in(&m->m, p.st) != in.dev) {
             return false;
         }
     }
-    for (const PassOutput &o : p.out)
+    for (const PassOutput &o : p.out) {
         if (o.m->dev != o.dev || (o.down_issued && o.m->host != o.host))
             return false;
+        hip_mem_use_on(o.m, p.st);
+    }
     return true;
 }
 
@@ -247,12 +252,11 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
             continue;
         in.m->up_pending = true, in.m->up_stream = p.st; // the pass reads pinned memory
         if (in.from == PassInput::kMirror)
-            in.m->dev_valid = true, in.m->down_issued = false, in.m->prod_stream = p.st;
+            in.m->dev_valid = true, in.m->down_issued = false;
     }
     for (const PassOutput &o : p.out) {
         o.m->dev_valid = o.dev_valid, o.m->host_valid = o.host_valid, o.m->down_issued = o.down_issued, o.m->q_valid = false;
         o.m->pending = o.pending, o.m->pending_ctx = o.pending_ctx;
-        o.m->prod_stream = p.st;
     }
     return true;
 }

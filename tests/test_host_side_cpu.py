@@ -259,10 +259,54 @@ def a_write_waits_for_every_stream_that_reads_the_array():
     assert captures.value >= 1 and replays.value >= 3
 
 
+def operators_of_two_workspaces_wait_for_each_other():
+    """One workspace's operator reads what another's writes: it is queued when that has finished, and the writer runs again when the
+    reader has finished - operator by operator, and as recorded passes whose input or output the other workspace uses."""
+    import numpy as np
+    from nart_amd import cases, engine
+    rt = runtime()
+    stream_of = rt.libs[1].hip_workspace_stream
+    stream_of.argtypes, stream_of.restype = [C.c_void_p], C.c_void_p
+    STUB.stub_pending.argtypes, STUB.stub_pending.restype = [C.c_void_p], C.c_long
+    two = [rt.workspace("hip"), rt.workspace("hip")]
+    first, second = [stream_of(w.ptr) for w in two]
+    q = dict(ialpha=0.1, izp=3, oalpha=0.2, ozp=4)
+    writer = two[0].relu(two[0].tensor(np.ones((1, 16, 8, 8), np.uint8)), q).prepare()
+    reader = two[1].relu(writer.output(0), q).prepare()
+    for _ in range(3):
+        writer.run()
+        assert STUB.stub_pending(second) == 0 and STUB.stub_pending(first) > 0
+        reader.run()
+        assert STUB.stub_pending(first) == 0 and STUB.stub_pending(second) > 0
+    c = cases.Case("chain", 3)
+    t = c.input_u8((1, 16, 8, 8), 0.05, 9)
+    for _ in range(10):
+        t = c.conv(t, 16, 3)
+    c.output = t
+    p = engine.Parade(rt, engine.write_engine(c), [two[0]])
+    reader = two[1].relu(p.outputs()[0], q).prepare()
+    replays = C.c_long.in_dll(STUB, "stub_graph_launches")
+    x = p.inputs()[0]
+    beside = two[1].relu(x, q).prepare()
+    x.write(np.ones((1, 16, 8, 8), np.uint8))
+    rt.libs[1].hip_workspace_synchronize(C.c_void_p(C.addressof(two[1].ptr.contents)))
+    for i in range(6):
+        p.run()
+        assert STUB.stub_pending(second) == 0 and STUB.stub_pending(first) > 0, i
+        (reader if i % 2 else beside).run()
+        assert STUB.stub_pending(first) == 0 and STUB.stub_pending(second) > 0, i
+    x.write(np.ones((1, 16, 8, 8), np.uint8))  # waits for whoever reads the pinned side; the pass brings the values in again
+    beside.run()
+    p.run()
+    assert STUB.stub_pending(second) == 0
+    assert replays.value >= 4
+
+
 CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
-         a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array]
+         a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
+         operators_of_two_workspaces_wait_for_each_other]
 
 
 @pytest.fixture(scope="module")
