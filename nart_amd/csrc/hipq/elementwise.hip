@@ -771,19 +771,20 @@ __global__ __launch_bounds__(256) void quantize_u8_c4_kernel(const QuantArgs p)
 }
 
 // More channels (stride a multiple of 16): a thread converts 16 channels (blockIdx.z) of one pixel; the 64 lanes of a wave read
-// 64 consecutive pixels of a plane per load and every lane writes one 128-bit piece.
+// 64 consecutive pixels of a plane per load and every lane writes one 128-bit piece.  The grid covers the whole stride: pieces of
+// pad channels alone are written as zeros.
 template <bool SIGNED>
 __global__ __launch_bounds__(256) void quantize_u8_c16_kernel(const QuantArgs p)
 {
     const int hw = p.H * p.W, n = blockIdx.y, c0 = blockIdx.z * 16;
-    const int last = p.C - 1 - c0; // channels beyond it read that plane again and store zeros: no load waits for a branch
-    const float *xn = p.x + ((size_t)n * p.C + c0) * hw;
+    const int last = p.C - 1 - c0; // channels beyond it read plane C - 1 again and store zeros: no load waits for a branch
+    const float *xn = p.x + (size_t)n * p.C * hw;
     uint8_t *yn = p.y + (size_t)n * hw * p.cs + c0;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < hw; i += gridDim.x * 256) {
         float v[16];
 #pragma unroll
         for (int c = 0; c < 16; c++)
-            v[c] = xn[(size_t)min(c, last) * hw + i];
+            v[c] = xn[(size_t)min(c0 + c, p.C - 1) * hw + i];
         u32x4 o = {0, 0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 16; c++)
@@ -1207,7 +1208,7 @@ static int launch_quantize(const char *who, bool sgn, const float *x, void *y, i
         return launch_status(sgn ? "quantize_i8_c4_kernel" : "quantize_u8_c4_kernel");
     }
     if (image16(hw, N, cs) && aligned16(y)) {
-        const dim3 grid((unsigned)std::min<size_t>((hw + 255) / 256, 1024), N, (C + 15) / 16);
+        const dim3 grid((unsigned)std::min<size_t>((hw + 255) / 256, 1024), N, cs / 16);
         if (sgn)
             hipLaunchKernelGGL(quantize_u8_c16_kernel<true>, grid, dim3(256), 0, st, p);
         else

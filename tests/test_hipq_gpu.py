@@ -754,6 +754,24 @@ def test_quantize_dequantize():
         assert np.array_equal(fd.cpu().numpy().view(np.uint32), orc.dequantize_u8(want, oa, oz).view(np.uint32))
 
 
+@pytest.mark.parametrize("C, HW, cs", [(16, 9, 48), (3, 8, 32), (17, 7, 64), (33, 3, 80), (40, 64, 112)])
+def test_quantize_writes_every_pad_byte(C, HW, cs):
+    """A channel stride wider than the channels need: the pad channels are written as zeros, also whole 16-byte pieces of them
+    (C x HW x HW images from 9 to 4096 pixels: both kernels)."""
+    rng = np.random.default_rng(C)
+    x = rng.standard_normal((2, C, HW, HW)).astype(np.float32)
+    for signed in (False, True):
+        y = torch.full((2, HW, HW, cs), 99, dtype=torch.uint8, device="cuda")
+        want = np.zeros((2, HW, HW, cs), np.uint8)
+        if signed:
+            hipq.quantize_i8(torch.from_numpy(x).cuda(), y, 0.02)
+            want[..., :C] = orc.quantize_i8(x, 0.02).transpose(0, 2, 3, 1).view(np.uint8)
+        else:
+            hipq.quantize_u8(torch.from_numpy(x).cuda(), y, 0.02, 120)
+            want[..., :C] = orc.quantize_u8(x, 0.02, 120).transpose(0, 2, 3, 1)
+        assert np.array_equal(y.cpu().numpy(), want), (C, HW, cs, signed)
+
+
 def test_dequantize_of_int32_accumulators():
     """hipq_dequantize_i32 (no counterpart in the reference, which dequantizes bytes only): a convolution's accumulator
     dump times ialpha * walpha, against the oracle's closed form, plus values where int32 -> fp32 rounds."""
