@@ -101,13 +101,6 @@ __global__ __launch_bounds__(256) void conv_mfma_stream_kernel(const ConvArgs a,
             wih[j] = oh * a.stride_h - a.pad_h, wiw[j] = ow * a.stride_w - a.pad_w, wpix[j] = n * a.H * a.W;
         }
     }
-    // otherwise: where this lane's row of load j starts (rows beyond the last pixel repeat it; their results are dropped)
-    int xat[CONVX ? 1 : XI];
-    if (!CONVX) {
-#pragma unroll
-        for (int j = 0; j < XI; j++)
-            xat[j] = min(m0 + 8 * j + xrow, a.P - 1) * a.in_cs;
-    }
     auto issue = [&](int t) {
         const int chunk = chunk_of(t);
         uint8_t *st = wl + (t % R) * STAGE;
@@ -137,8 +130,12 @@ __global__ __launch_bounds__(256) void conv_mfma_stream_kernel(const ConvArgs a,
             // a piece beyond the pixel's channels meets weights that add nothing: any bytes of the tensor will do
             const int k = chunk * 128 + xoff, off = WHOLE || k < a.in_cs ? k : 0;
 #pragma unroll
-            for (int j = 0; j < XI; j++)
-                __builtin_amdgcn_global_load_lds((gptr_t)(a.x + (uint32_t)(xat[j] + off)), (lptr_t)(st + j * 1024 + ((j + 1) >> 1) * 128), 16, 0, 0);
+            for (int j = 0; j < XI; j++) {
+                // rows beyond the last pixel repeat it, their results are dropped; formed here and not kept over the loop, which
+                // took 128 x 4096 x 4096 from 9.05 to 9.31 us
+                const int m = min(m0 + 8 * j + xrow, a.P - 1);
+                __builtin_amdgcn_global_load_lds((gptr_t)(a.x + (uint32_t)(m * a.in_cs + off)), (lptr_t)(st + j * 1024 + ((j + 1) >> 1) * 128), 16, 0, 0);
+            }
         }
 #pragma unroll
         for (int h = 0; h < 2; h++)
