@@ -1,7 +1,7 @@
 """Builds the native libraries of the package in-tree (no GPU needed: hipcc cross-compiles gfx950).
 
   nart_amd/lib/libhipq.so             HIP kernels + their C ABI (include/hipq.h)
-  nart_amd/lib/hipq_calls.so          the CPython extension behind hipq.py's per-call functions
+  nart_amd/lib/hipq_calls.<abi>.so    the CPython extension behind hipq.py's per-call functions
   nart_amd/lib/libart.so              the minimal host core implementing the art C API (include/art/)
   nart_amd/lib/libart_module_hip.so   the `hip` case module (exports hip_module_tp)
 
@@ -163,10 +163,11 @@ def build_module(force=False, nart_tree=None, out_name="libart_module_hip.so"):
 
 
 def build_python(force=False):
-    """hipq_calls, the CPython extension behind hipq.py's per-call functions."""
+    """hipq_calls, the CPython extension behind hipq.py's per-call functions.  Its name carries the interpreter's ABI tag:
+    another interpreter builds (and hipq.py loads) a file of its own."""
     import sysconfig
     src = _glob("python", (".c",))
-    out = os.path.join(LIB, "hipq_calls.so")
+    out = os.path.join(LIB, "hipq_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
     if src and (force or not _newer(out, src + [os.path.join(INC, "hipq.h")])):
         _run(["gcc", "-O2", "-std=gnu11", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_paths()["include"], "-I" + INC, "-o", out]
              + src + ["-L" + LIB, "-lhipq", "-Wl,-rpath,$ORIGIN"])

@@ -148,11 +148,12 @@ def _calls():
     global _CALLS
     if _CALLS is None:
         import importlib.util
+        import sysconfig
         import torch
         lib()
-        path = os.path.join(os.path.dirname(LIB_PATH), "hipq_calls.so")
+        path = os.path.join(os.path.dirname(LIB_PATH), "hipq_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
         if not os.path.exists(path):
-            raise HipqError("%s is missing: build it with `python -m nart_amd.build`" % path)
+            raise HipqError("%s is missing: build it with `python -m nart_amd.build` under this interpreter" % path)
         torch.cuda.current_stream()  # initialises the device, and fails with torch's own message where there is none
         spec = importlib.util.spec_from_file_location("hipq_calls", path)
         mod = importlib.util.module_from_spec(spec)

@@ -92,3 +92,20 @@ def test_no_kernel_uses_scratch_memory():
     assert all(v["scratch"] == 0 for v in usage.values())
     tiles = {k: v for k, v in usage.items() if "conv_mfma_dma_kernel" in k}
     assert tiles and all(v["vgprs"] <= 168 for v in tiles.values())  # three waves per SIMD at least
+
+
+def test_the_extension_belongs_to_one_interpreter(monkeypatch):
+    """hipq_calls carries the interpreter's ABI tag: another interpreter neither loads this one's file nor takes it for built."""
+    import sysconfig
+    from nart_amd import build
+    (here,) = build.build_python()
+    assert here.endswith("hipq_calls" + sysconfig.get_config_var("EXT_SUFFIX")) and "cpython-3" in here and os.path.exists(here)
+    real = sysconfig.get_config_var
+    monkeypatch.setattr(sysconfig, "get_config_var", lambda n: ".cpython-999-other.so" if n == "EXT_SUFFIX" else real(n))
+    commands = []
+    monkeypatch.setattr(build, "_run", commands.append)
+    (there,) = build.build_python()
+    assert there != here and len(commands) == 1 and there in commands[0]
+    monkeypatch.setattr(hipq, "_CALLS", None)
+    with pytest.raises(hipq.HipqError, match="cpython-999"):
+        hipq._calls()
