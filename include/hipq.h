@@ -212,10 +212,11 @@ int hipq_conv2d_run_add(const hipq_conv2d_plan *plan, const void *x, const void 
                         float res_alpha, int res_zp, float oalpha, int ozp, int obits, void *y, void *stream);
 
 /*
- * hipq_conv2d_run_add followed, in the same kernel, by the 1x1 convolution `next` that reads the sum (the last layer of
- * one bottleneck block, its residual add, and the first layer of the next block): y = add(conv(x), residual) and
- * y_next = next(y), bit-identical to hipq_conv2d_run_add followed by hipq_conv2d_run(next, y, y_next).  The sum is
- * written once and never read back.  Serves uint8 plans where `plan` is a 1x1 convolution from 64 or 128 to a multiple
+ * hipq_conv2d_run_add followed by the 1x1 convolution `next` that reads the sum (the last layer of one bottleneck block, its
+ * residual add, and the first layer of the next block): y = add(conv(x), residual) and y_next = next(y), bit-identical to
+ * hipq_conv2d_run_add followed by hipq_conv2d_run(next, y, y_next).  From 20 000 pixels on (hipq_conv2d_plan_special(plan, 2):
+ * whatever their number) this is one kernel, the sum written once and never read back; on fewer pixels, where the two
+ * layers spread over more CUs by themselves, it is those two launches (hipq_conv2d_add_conv_kernel says which).  Serves uint8 plans where `plan` is a 1x1 convolution from 64 or 128 to a multiple
  * of 64 (at most 1024) channels over at least 1024 pixels that the widening kernel computes, and `next` a 1x1 / stride 1
  * convolution of the same pixels to 64 or 128 channels (channel stride equal to that) whose input scale and zero point
  * are the sum's oalpha / ozp, obits 8, weight zero points 128, per-tensor weight scales.
@@ -228,6 +229,9 @@ int hipq_conv2d_add_conv_fusable(const hipq_conv2d_plan *plan, int residual_is_i
 int hipq_conv2d_run_add_conv(const hipq_conv2d_plan *plan, const void *x, const void *residual, int residual_is_input0,
                              float res_alpha, int res_zp, float oalpha, int ozp, int obits, void *y,
                              const hipq_conv2d_plan *next, int next_relu, void *y_next, void *stream);
+/* Name of the kernel, or of the two, separated by a comma, that hipq_conv2d_run_add_conv launches for plans it serves.  The
+ * string is valid until the calling thread's next call. */
+const char *hipq_conv2d_add_conv_kernel(const hipq_conv2d_plan *plan, const hipq_conv2d_plan *next);
 
 /*
  * The last layer of a bottleneck block with a projection shortcut, in one launch: y = add(plan(x), shortcut(x_shortcut)),

@@ -2126,6 +2126,20 @@ extern "C" int hipq_conv2d_add_conv_fusable(const hipq_conv2d_plan *p, int resid
     return conv_expand_chain_applies(a, next->args) ? 1 : 0;
 }
 
+// A work-group of the chained kernel takes 128 pixels through all of both layers, 9 us and more for 64 -> 256 -> 64 and 17 for
+// 128 -> 512 -> 128 however few there are; the two layers on their own spread over the chip.  Level at 20 000 pixels; 6 900 pixels
+// of the latter: 17.7 us as one launch, 9.6 as two.  (Mode 2 asks for the kernel wherever it applies.)
+static bool add_conv_is_one_kernel(const hipq_conv2d_plan *p) { return p->args.P >= 20000 || p->special == 2; }
+
+extern "C" const char *hipq_conv2d_add_conv_kernel(const hipq_conv2d_plan *p, const hipq_conv2d_plan *next)
+{
+    static thread_local std::string nm;
+    if (!p || !next)
+        return "";
+    nm = add_conv_is_one_kernel(p) ? "conv_mfma_i8_expand+add+conv" : std::string(hipq_conv2d_plan_kernel_add(p)) + ", " + next->name;
+    return nm.c_str();
+}
+
 extern "C" int hipq_conv2d_run_add_conv(const hipq_conv2d_plan *p, const void *x, const void *residual, int residual_is_input0,
                                         float res_alpha, int res_zp, float oalpha, int ozp, int obits, void *y,
                                         const hipq_conv2d_plan *next, int next_relu, void *y_next, void *stream)
@@ -2135,10 +2149,7 @@ extern "C" int hipq_conv2d_run_add_conv(const hipq_conv2d_plan *p, const void *x
     HIPQ_REQUIRE(hipq_conv2d_add_conv_fusable(p, residual_is_input0, res_alpha, res_zp, oalpha, ozp, obits, next),
                  "hipq_conv2d_run_add_conv: these two plans (%s, then %s) do not run as one kernel: run hipq_conv2d_run_add and "
                  "hipq_conv2d_run", p->name.c_str(), next->name.c_str());
-    // A work-group takes 128 pixels through all of both layers, 9 us and more for 64 -> 256 -> 64 and 17 for 128 -> 512 -> 128
-    // however few there are; the two layers on their own spread over the chip.  Level at 20 000 pixels; 6 900 pixels of the
-    // latter: 17.7 us as one launch, 9.6 as two.  (Mode 2 asks for the kernel wherever it applies.)
-    if (p->args.P < 20000 && p->special != 2) {
+    if (!add_conv_is_one_kernel(p)) {
         const int rc = hipq_conv2d_run_add(p, x, residual, residual_is_input0, res_alpha, res_zp, oalpha, ozp, obits, y, stream);
         if (rc != 0)
             return rc;

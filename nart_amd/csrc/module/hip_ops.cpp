@@ -99,6 +99,7 @@ typedef std::map<const mem_t *, std::set<const op_t *>> reader_map;
 // keyed by workspace (the runtime is single-threaded, art/include/art/workspace.h has no locking either)
 std::map<const workspace_t *, reader_map> g_readers;
 long g_fused_adds = 0, g_fused_relus = 0, g_fused_pools = 0, g_chained_convs = 0, g_fused_dequants = 0; // fused launches so far (hip_module_fused_*)
+// (g_chained_convs: convolutions launched by another operator's call, which on few pixels is two kernels)
 long g_fused_blocks = 0, g_fused_inverted = 0, g_fused_tails = 0; // whole bottleneck / inverted residual blocks, blocks from their 3x3 layer on, as one launch
 
 reader_map &readers_of(op_t *op) { return g_readers[op->workspace]; }
@@ -218,7 +219,7 @@ bool conv_continues_block(op_t *op, const op_t *r);
 bool dequantize_fuses_with(const op_t *deq_op, const hipq_conv2d_plan *plan);
 // a max pooling that the stem convolution's kernel can compute as well (hipq_conv2d_maxpool_fusable)
 bool pool_fuses_with(const op_t *pool_op, const hipq_conv2d_plan *plan);
-// the convolution `op` as the tail of the kernel that computes the add it reads (hipq_conv2d_run_add_conv); y: where its
+// the convolution `op` in the call that computes the add it reads (hipq_conv2d_run_add_conv, or a whole block); y: where its
 // output goes, relu: with the ReLU clamp.  false: not possible, run it plainly
 bool conv_run_chained(op_t *op, void *y, int relu);
 
@@ -695,7 +696,7 @@ void add_plain_into(op_t *op, void *y)
                               e->qo.alpha[0], e->qo.zp[0], e->qo.bits[0], op_stream(op)));
 }
 
-// The hook an add leaves on its output when a 1x1 convolution that reads the sum can run in the same kernel
+// The hook an add leaves on its output when a 1x1 convolution that reads the sum can run in the same call
 // (add_defers): that convolution's run() launches hipq_conv2d_run_add_conv; whoever else asks for the sum first gets
 // the convolution + add launch (or the plain add).
 void add_launch_deferred(void *ctx)

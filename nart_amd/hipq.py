@@ -57,6 +57,7 @@ _SIGS = {
     "hipq_conv2d_add_conv_fusable": (C.c_int, [C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "hipq_conv2d_run_add_conv": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int,
                                            C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
+    "hipq_conv2d_add_conv_kernel": (C.c_char_p, [C.c_void_p, C.c_void_p]),
     "hipq_conv2d_add2_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_conv2d_run_add2": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int,
                                        C.c_void_p, C.c_void_p]),
@@ -294,12 +295,17 @@ class Conv2d:
         return y
 
     def add_conv_fusable(self, residual_first, res_alpha, res_zp, oalpha, ozp, nxt, obits=8):
-        """Can run_add and the 1x1 convolution `nxt` that reads the sum run as one kernel (include/hipq.h)?"""
+        """Does run_add_conv serve this plan, this add and the 1x1 convolution `nxt` that reads the sum (include/hipq.h)?"""
         return bool(lib().hipq_conv2d_add_conv_fusable(self.handle, int(bool(residual_first)), res_alpha, res_zp, oalpha, ozp,
                                                        obits, nxt.handle))
 
+    def add_conv_kernel(self, nxt):
+        """Names of the kernel or kernels that run_add_conv launches (include/hipq.h: hipq_conv2d_add_conv_kernel)."""
+        return lib().hipq_conv2d_add_conv_kernel(self.handle, nxt.handle).decode()
+
     def run_add_conv(self, x, residual, residual_first, res_alpha, res_zp, oalpha, ozp, y, nxt, y_next, obits=8, next_relu=False):
-        """y = add(conv(x), residual) and y_next = nxt(y) in one launch (include/hipq.h: hipq_conv2d_run_add_conv)."""
+        """y = add(conv(x), residual) and y_next = nxt(y) in one call - one launch, or two on few pixels (add_conv_kernel;
+        include/hipq.h: hipq_conv2d_run_add_conv)."""
         check(lib().hipq_conv2d_run_add_conv(self.handle, _ptr(x), _ptr(residual), int(bool(residual_first)), res_alpha, res_zp,
                                              oalpha, ozp, obits, _ptr(y), nxt.handle, int(bool(next_relu)), _ptr(y_next), _stream()))
         return y, y_next

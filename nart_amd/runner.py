@@ -300,7 +300,7 @@ class HipqExecutor:
                     done.add(id(nd))
                     fn = (lambda p=plan, i=xin, r=self.buf[other], rf=res_first, ot=ot, st=st, o=out, p2=p2, y2=y2:
                           p.run_add_conv(i, r, rf, ot.alpha, ot.zp, st.alpha, st.zp, o, p2, y2))
-                    self.steps.append({"label": node.output, "kind": "conv+add+conv", "kernel": "conv_mfma_i8_expand+add+conv",
+                    self.steps.append({"label": node.output, "kind": "conv+add+conv", "kernel": plan.add_conv_kernel(p2),
                                        "fn": fn, "ops": plan.ops + p2.ops, "bytes": nbytes + nb2 - int(np.prod(st.shape)),
                                        "plan": plan})
                     continue

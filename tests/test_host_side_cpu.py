@@ -38,6 +38,24 @@ def inverted_residual_add_needs_equal_shapes():
             assert (rc == 0) is same and kernels.value == before + same, (ci, ch, co, stride, first)
 
 
+def a_chained_add_names_its_kernels():
+    """hipq_conv2d_run_add_conv is one kernel from 20 000 pixels on, or where mode 2 asks for it, and two launches below that: the
+    name says which, and as many kernels are launched."""
+    import numpy as np
+    from nart_amd import hipq
+    kernels = C.c_long.in_dll(STUB, "stub_kernels")
+    x = np.zeros(64, np.uint8).ctypes.data  # never touched
+    for N, HW, mode, one in ((2, 24, 1, False), (2, 24, 2, True), (7, 56, 1, True), (6, 56, 1, False)):
+        wide = hipq.Conv2d((N, 64, HW, HW), np.full((256, 64, 1, 1), 129, np.uint8), None, 0, 1, 1, 0.05, 9, 0.002, 128, 0.05, 9).special(mode)
+        nxt = hipq.Conv2d((N, 256, HW, HW), np.full((64, 256, 1, 1), 129, np.uint8), None, 0, 1, 1, 0.09, 10, 0.002, 128, 0.05, 9)
+        assert wide.add_conv_fusable(False, 0.04, 3, 0.09, 10, nxt)
+        name = wide.add_conv_kernel(nxt)
+        assert name == ("conv_mfma_i8_expand+add+conv" if one else wide.kernel_add + ", " + nxt.kernel), (N, HW, mode, name)
+        before = kernels.value
+        hipq.check(hipq.lib().hipq_conv2d_run_add_conv(wide.handle, x, x, 0, 0.04, 3, 0.09, 10, 8, x, nxt.handle, 0, x, None))
+        assert kernels.value - before == (1 if one else 2), (N, HW, mode, name)
+
+
 def runtime():
     from nart_amd import art
     lib = os.path.join(ROOT, "nart_amd", "lib")
@@ -302,7 +320,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, fused_block_follows_the_scales_of_its_operators,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,

@@ -281,8 +281,8 @@ def test_plain_eltwise_sum_fuses_like_add(own_rt):
 
 def test_add_and_the_next_1x1_convolution_run_as_one_kernel(own_rt):
     """conv_2d (64 -> 256, 1x1) -> add -> conv_2d (256 -> 64, 1x1) [-> relu]: the first convolution defers to the add, the
-    add defers to the convolution that reads the sum, and that convolution (or the relu behind it) launches all of it as
-    one kernel; the sum is written as well, for its other readers.  A host that reads the sum before the second
+    add defers to the convolution that reads the sum, and that convolution (or the relu behind it) launches all of it in one
+    call (one kernel from 20 000 pixels on, two on the 1152 of this test); the sum is written as well, for its other readers.  A host that reads the sum before the second
     convolution runs gets convolution + add as one kernel and the second convolution on its own.  Same bytes as the
     operators run one by one, pass after pass."""
     import ctypes as C
