@@ -1305,6 +1305,7 @@ struct hipq_conv2d_plan {
     int stages = 0; // load stages of the DMA kernel; 0 = the built-in rule
     int special = 1; // the halo-tile and pointwise kernels: 0 never, 1 built-in rule, 2 wherever they apply
     bool tile_selected = false;     // hipq_conv2d_plan_select named a tile: the tile kernels, not the streaming kernel
+    int invres_shape = -1; // patch shape of the inverted residual block this plan projects (hipq_inverted_residual_select); -1: by cost
     StreamShape stream = {0, 0, 0}; // explicit shape of the streaming kernel (hipq_conv2d_plan_stream); mb = 0: built-in rule
     bool has_wzp;
     void *d_w = nullptr, *d_bias = nullptr, *d_q = nullptr;
@@ -2269,8 +2270,21 @@ extern "C" int hipq_inverted_residual_run(const hipq_conv2d_plan *pe, const hipq
     ae.x = in;
     ap.res = add ? in : nullptr;
     ap.y = static_cast<uint8_t *>(y);
-    launch_conv_invres(ae, ad, ap, static_cast<hipStream_t>(stream));
+    launch_conv_invres(ae, ad, ap, pp->invres_shape, static_cast<hipStream_t>(stream));
     return launch_status("conv_invres_kernel");
+}
+
+extern "C" int hipq_inverted_residual_select(hipq_conv2d_plan *pp, int shape)
+{
+    clear_error();
+    HIPQ_REQUIRE(pp && shape >= -1 && shape <= 3, "hipq_inverted_residual_select: null plan, or shape %d outside -1..3", shape);
+    pp->invres_shape = shape;
+    return 0;
+}
+
+extern "C" const char *hipq_inverted_residual_kernel(const hipq_conv2d_plan *pe, const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp)
+{
+    return hipq_inverted_residual_fusable(pe, pd, pp, 0, 0, 1.0f, 0, 8) ? conv_invres_name(pe->args, pd->args, pp->args, pp->invres_shape) : "";
 }
 
 extern "C" int hipq_bottleneck_conv_fusable(const hipq_conv2d_plan *p1, const hipq_conv2d_plan *p2, const hipq_conv2d_plan *p3,

@@ -362,8 +362,13 @@ double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
     return t;
 }
 
-int choose_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, double *us)
+// wanted: the caller's choice, where that shape is built for these channels; -1: the cheapest
+int choose_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted, double *us)
 {
+    if (wanted >= 0 && wanted < kShapes && shape_cost(e, d, p, wanted) < 1e30) {
+        *us = shape_cost(e, d, p, wanted);
+        return wanted;
+    }
     int best = k2x4;
     *us = shape_cost(e, d, p, best);
     for (int sh = k4x8; sh < kShapes; sh++)
@@ -373,10 +378,8 @@ int choose_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, double
 }
 
 template <int S, int NK, int CT>
-void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape, hipStream_t st)
 {
-    double us;
-    const int shape = choose_shape(e, d, p, &us);
     if constexpr (NK <= 2 && CT <= 2)
         if (shape == kOwn)
             return launch_shape<S, S == 1 ? 8 : 4, 8, NK, CT, true>(e, d, p, st);
@@ -388,18 +391,37 @@ void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipSt
     launch_shape<S, 2, 4, NK, CT, false>(e, d, p, st);
 }
 
-template <int S>
-void launch_stride(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+// the channel counts that are built: k-steps of the expanding layer and channel tiles of the projecting one, each at least what the
+// layers have
+struct Channels {
+    int nk, ct;
+};
+
+Channels channels_of(const ConvArgs &e, const ConvArgs &p)
 {
     const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32;
     if (nk == 1 && ct <= 2)
-        ct == 1 ? launch_tiles<S, 1, 1>(e, d, p, st) : launch_tiles<S, 1, 2>(e, d, p, st);
-    else if (nk <= 2 && ct <= 3)
-        ct <= 2 ? launch_tiles<S, 2, 2>(e, d, p, st) : launch_tiles<S, 2, 3>(e, d, p, st);
-    else if (nk <= 3)
-        ct <= 3 ? launch_tiles<S, 3, 3>(e, d, p, st) : launch_tiles<S, 3, 5>(e, d, p, st);
-    else
-        launch_tiles<S, 5, 5>(e, d, p, st);
+        return {1, ct};
+    if (nk <= 2 && ct <= 3)
+        return {2, ct <= 2 ? 2 : 3};
+    if (nk <= 3)
+        return {3, ct <= 3 ? 3 : 5};
+    return {5, 5};
+}
+
+template <int S>
+void launch_stride(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape, hipStream_t st)
+{
+    const Channels c = channels_of(e, p);
+    switch (c.nk * 10 + c.ct) {
+    case 11: launch_tiles<S, 1, 1>(e, d, p, shape, st); break;
+    case 12: launch_tiles<S, 1, 2>(e, d, p, shape, st); break;
+    case 22: launch_tiles<S, 2, 2>(e, d, p, shape, st); break;
+    case 23: launch_tiles<S, 2, 3>(e, d, p, shape, st); break;
+    case 33: launch_tiles<S, 3, 3>(e, d, p, shape, st); break;
+    case 35: launch_tiles<S, 3, 5>(e, d, p, shape, st); break;
+    default: launch_tiles<S, 5, 5>(e, d, p, shape, st); break;
+    }
 }
 
 bool plain(const ConvArgs &a) { return a.bwz == 0 && a.xmask != 0 && a.lo >= 0 && a.fastq && a.qmult == nullptr; }
@@ -430,13 +452,26 @@ bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs 
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
     const double apart = d.stride_h == 1 ? 9.25 + 1.007 * wide + 0.00548 * wide * e.in_cs : 9.32 + 1.996 * narrow + 0.00451 * wide * e.in_cs;
     double us;
-    choose_shape(e, d, p, &us);
+    choose_shape(e, d, p, -1, &us);
     return us < 0.95 * apart;
 }
 
-void launch_conv_invres(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted)
 {
-    d.stride_h == 1 ? launch_stride<1>(e, d, p, st) : launch_stride<2>(e, d, p, st);
+    static const char *const kPatch[kShapes] = {"2x4", "4x8", "8x8", "own"};
+    static thread_local char nm[48];
+    double us;
+    const int shape = choose_shape(e, d, p, wanted, &us);
+    const Channels c = channels_of(e, p);
+    snprintf(nm, sizeof nm, "conv_invres_s%d_%s_k%d_n%d", d.stride_h, kPatch[shape], c.nk, c.ct);
+    return nm;
+}
+
+void launch_conv_invres(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted, hipStream_t st)
+{
+    double us;
+    const int shape = choose_shape(e, d, p, wanted, &us);
+    d.stride_h == 1 ? launch_stride<1>(e, d, p, shape, st) : launch_stride<2>(e, d, p, shape, st);
 }
 
 } // namespace hipq

@@ -70,6 +70,8 @@ _SIGS = {
     "hipq_inverted_residual_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_inverted_residual_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_float, C.c_int,
                                              C.c_int, C.c_void_p, C.c_void_p]),
+    "hipq_inverted_residual_select": (C.c_int, [C.c_void_p, C.c_int]),
+    "hipq_inverted_residual_kernel": (C.c_char_p, [C.c_void_p, C.c_void_p, C.c_void_p]),
     "hipq_bottleneck_tail_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int, C.c_int,
                                                C.c_void_p]),
     "hipq_bottleneck_tail_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float,
@@ -375,6 +377,16 @@ def inverted_residual_fusable(expand, depthwise, project, add=None, obits=8):
     rf, oa, oz = add if add is not None else (False, 1.0, 0)
     return bool(lib().hipq_inverted_residual_fusable(expand.handle, depthwise.handle, project.handle,
                                                      int(add is not None), int(bool(rf)), oa, oz, obits))
+
+
+def inverted_residual_select(project, shape=-1):
+    """Tuning hook: the patch shape of the block that `project` closes, 0..3, -1 by cost (include/hipq.h)."""
+    check(lib().hipq_inverted_residual_select(project.handle, int(shape)))
+
+
+def inverted_residual_kernel(expand, depthwise, project):
+    """Name of the kernel that inverted_residual_run launches for these plans, "" where it does not."""
+    return lib().hipq_inverted_residual_kernel(expand.handle, depthwise.handle, project.handle).decode()
 
 
 def inverted_residual_run(expand, depthwise, project, x, y, add=None, relus=0, obits=8):

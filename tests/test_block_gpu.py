@@ -576,3 +576,46 @@ def test_inverted_residual_block(case):
         y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (first, sa, sz), relus)
         got = hipq.from_device_nhwc(y, CO)
         assert np.array_equal(got, want), (case, "add", first, int((got != want).sum()))
+
+
+INVRES_CHANNELS = [(1, 1, 16, 24), (1, 2, 24, 40), (2, 2, 40, 60), (2, 3, 64, 72), (3, 3, 96, 96), (3, 5, 80, 130), (5, 5, 160, 160)]
+# every kernel that is built: k-steps, channel tiles, their channel counts; stride; shape
+INVRES_SHAPES = [(nk, ct, ci, co, st, sh) for nk, ct, ci, co in INVRES_CHANNELS for st in (1, 2) for sh in range(4)
+                 if not (sh == 3 and (nk > 2 or ct > 2)) and not (sh == 2 and (st == 2 or ct > 3))]
+
+
+@pytest.mark.parametrize("case", INVRES_SHAPES, ids=lambda c: "s%d_%s_k%d_n%d" % (c[4], ("2x4", "4x8", "8x8", "own")[c[5]], c[0], c[1]))
+def test_inverted_residual_every_kernel(case):
+    """Each of the 39 instantiations of conv_invres_kernel by name, on an image whose patches overhang on two sides (13 x 11) and one
+    smaller than a patch, three slices of which the last is partial, against the oracle's convolutions; where input and output
+    have equal channels, the add as well."""
+    nk, ct, ci, co, st, sh = case
+    assert len(INVRES_SHAPES) == 39
+    ch = 80
+    for N, H, W in ((3, 13, 11), (1, 3, 2)):
+        rng = np.random.default_rng(ci + co + st + H)
+        x = rng.integers(0, 256, (N, ci, H, W), dtype=np.uint8)
+        t, a, z, plans = x, 0.03, 77, []
+        for k, (C, K, R, s, group) in enumerate(((ci, ch, 1, 1, 1), (ch, ch, 3, st, ch), (ch, co, 1, 1, 1))):
+            w = rng.integers(1, 256, (K, C // group, R, R), dtype=np.uint8)
+            sigma = 74.0 * 74.0 * math.sqrt(w[0].size) * (0.7 if k else 1.0)
+            b = rng.integers(-int(sigma), int(sigma) + 1, K).astype(np.int32)
+            oa = float(np.float32(0.03 * rng.uniform(0.75, 1.35)))
+            q = (a, z, float(np.float32(oa * 45.0 / (a * sigma))), 128, oa, 30 if k < 2 else 120)
+            plans.append(hipq.Conv2d(t.shape, w, b, R // 2, s, group, *q, relu=k < 2))
+            t = orc.conv2d_u8(t, w, b, R // 2, s, group, *q)
+            if k < 2:
+                t = np.maximum(t, q[5]).astype(np.uint8)
+            a, z = q[4], q[5]
+        plans[2].special(2)
+        hipq.inverted_residual_select(plans[2], sh)
+        name = hipq.inverted_residual_kernel(*plans)
+        assert name == "conv_invres_s%d_%s_k%d_n%d" % (st, ("2x4", "4x8", "8x8", "own")[sh], nk, ct), name
+        print(name, (N, H, W), flush=True)
+        xd = hipq.to_device_nhwc(x)
+        got = hipq.from_device_nhwc(hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99)), co)
+        assert np.array_equal(got, t), (name, int((got != t).sum()), np.argwhere(got != t)[:8].tolist())
+        if ci == co and st == 1:
+            want = orc.add_u8(t, x, a, z, 0.03, 77, 0.05, 20)
+            y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (False, 0.05, 20))
+            assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
