@@ -308,57 +308,103 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT
 
 namespace {
 
-template <int S, int PH, int PW, int NK, int CT, bool OWN>
-void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, hipStream_t st)
+// the channel counts that are built: k-steps of the expanding layer and channel tiles of the projecting one, each at least what the
+// layers have
+struct Channels {
+    int nk, ct;
+};
+
+Channels channels_of(const ConvArgs &e, const ConvArgs &p)
 {
-    using G = Patch<S, PH, PW>;
-    InvresGeom geo;
-    geo.PY = (p.OH + PH - 1) / PH, geo.PX = (p.OW + PW - 1) / PW;
-    geo.nT = (d.in_cs + 31) / 32;
-    geo.nk = (e.in_cs + 31) / 32, geo.ct = (p.out_cs + 31) / 32;
+    const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32;
+    if (nk == 1 && ct <= 2)
+        return {1, ct};
+    if (nk <= 2 && ct <= 3)
+        return {2, ct <= 2 ? 2 : 3};
+    if (nk <= 3)
+        return {3, ct <= 3 ? 3 : 5};
+    return {5, 5};
+}
+
+enum Shape { k2x4, k4x8, k8x8, kOwn, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2
+
+// how a launch divides the work
+struct Division {
+    int PY, PX, nT, xrow, region, wave_bytes;
+    int nw, rounds; // waves of a work-group; slices that one of them takes one after the other
+    unsigned lds;
+    long long wgs;
+};
+
+Division divide(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
+{
+    const Channels c = channels_of(e, p);
+    const int S = d.stride_h, ph = shape == k2x4 ? 2 : shape == k8x8 || (shape == kOwn && S == 1) ? 8 : 4, pw = shape == k2x4 ? 4 : 8;
+    const int tiles = ((S * (ph - 1) + 3) * ((S * (pw - 1) + 6) / 4) + 7) / 8, pt = (ph * pw + 31) / 32; // as in Patch
+    Division v;
+    v.PY = (p.OH + ph - 1) / ph, v.PX = (p.OW + pw - 1) / pw;
+    v.nT = (d.in_cs + 31) / 32;
     // rows of 16 bytes (the other half of a k-step meets zero weights) and of 32 read without bank conflicts as they are, longer
     // ones 16 bytes apart
-    geo.xrow = e.in_cs == 16 ? 16 : NK == 1 ? 32 : 32 * NK + 16;
-    geo.region = (G::TILES * 32 * geo.xrow + 16 + G::MASK_BYTES + 15) / 16 * 16;
-    geo.wave_bytes = G::E_BYTES + G::D_BYTES;
-    const long long patches = (long long)d.N * geo.PY * geo.PX;
-    int nw = 4;
-    unsigned lds;
-    if (OWN) {
-        lds = (unsigned)(nw * (geo.region + geo.wave_bytes));
+    v.xrow = e.in_cs == 16 ? 16 : c.nk == 1 ? 32 : 32 * c.nk + 16;
+    v.region = (tiles * 32 * v.xrow + 16 + tiles * 32 + 15) / 16 * 16;
+    v.wave_bytes = tiles * 1024 + pt * 1024;
+    const long long patches = (long long)d.N * v.PY * v.PX;
+    if (shape == kOwn) {
+        v.nw = 4, v.rounds = v.nT, v.wgs = (patches + 3) / 4;
+        v.lds = (unsigned)(4 * (v.region + v.wave_bytes));
     } else {
-        nw = std::min(geo.nT, max_waves(G::PT, CT));
-        while (geo.region + nw * geo.wave_bytes > 160 * 1024)
-            nw--; // one wave needs at most 14 KB beside 63 KB of pixels
-        const int rounds = (geo.nT + nw - 1) / nw;
-        nw = (geo.nT + rounds - 1) / rounds; // the same rounds with fewer waves
-        lds = (unsigned)std::max(geo.region + nw * geo.wave_bytes, CT * G::PT * 4096);
+        v.nw = std::min(v.nT, max_waves(pt, c.ct));
+        while (v.region + v.nw * v.wave_bytes > 160 * 1024)
+            v.nw--; // one wave needs at most 14 KB beside 63 KB of pixels
+        v.rounds = (v.nT + v.nw - 1) / v.nw;
+        v.nw = (v.nT + v.rounds - 1) / v.rounds; // the same rounds with fewer waves
+        v.wgs = patches;
+        v.lds = (unsigned)std::max(v.region + v.nw * v.wave_bytes, c.ct * pt * 4096);
     }
-    const long long wgs = OWN ? (patches + nw - 1) / nw : patches;
-    hipLaunchKernelGGL((conv_invres_kernel<S, PH, PW, NK, CT, OWN>), dim3((unsigned)((wgs + 7) / 8 * 8)), dim3(64 * nw), lds, st, e, d, p, geo);
+    return v;
+}
+
+template <int S, int PH, int PW, int NK, int CT, bool OWN>
+void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape, hipStream_t st)
+{
+    using G = Patch<S, PH, PW>;
+    const Division v = divide(e, d, p, shape);
+    InvresGeom geo;
+    geo.PY = v.PY, geo.PX = v.PX, geo.nT = v.nT, geo.xrow = v.xrow, geo.region = v.region, geo.wave_bytes = v.wave_bytes;
+    geo.nk = (e.in_cs + 31) / 32, geo.ct = (p.out_cs + 31) / 32;
+    static_assert(G::E_BYTES == G::TILES * 1024 && G::D_BYTES == G::PT * 1024 && G::MASK_BYTES == G::TILES * 32, "divide()");
+    hipLaunchKernelGGL((conv_invres_kernel<S, PH, PW, NK, CT, OWN>), dim3((unsigned)((v.wgs + 7) / 8 * 8)), dim3(64 * v.nw), v.lds, st, e, d, p, geo);
 }
 
 // ---- the shapes, and what each takes
-enum Shape { k2x4, k4x8, k8x8, kOwn, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2
 
-// Time by shape, in us, fitted to 80 measured blocks (1 to 64 images of 3x3 to 130x130, the channel counts of a mobile network;
-// within 20 % of each) - linear in the rounds of slices a wave takes one after the other, alone and per channel tile of 32, the
-// slices per SIMD of the chip, the channel tiles, and the work-groups per CU, as a quotient and rounded up.
+// Time by shape, in us, fitted to 160 blocks (1 to 128 images of 3x3 to 130x130, the channel counts of mobile networks; nine in ten
+// within 20 % of the fit, all within 33; every block's times are in profiles/inverted_residual_shapes_gfx950.md).  A launch; for every generation of
+// resident work-groups its start and end; for every slice that a wave then takes its chain, alone, per channel tile and per
+// k-step; and the slices per SIMD of the chip, which share the vector units.  How many work-groups a CU holds decides: the
+// fit before this one knew only patches per CU, which is right where nine small work-groups fit one, and picked shapes up to
+// 1.7 times slower than the three launches from 64 channels on (18 images of 20x103, 64 -> 384 -> 96: 34 against 25 us).
 double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    static const double kCost[2][kShapes][7] = {
-        {{2.49, 0, 0, 1.031, 1.281, 0, 0}, {0.515, 1.774, 0, 0.75, 1.394, 0, 1.631}, {0, 2.022, 0.665, 0.097, 0, 0.23, 4.513}, {0.654, 1.918, 0.192, 0, 0, 0, 1.112}},
-        {{2.937, 0, 0, 1.084, 1.108, 0, 0}, {4.668, 0, 0.643, 0.981, 0.187, 0, 0.469}, {}, {0.346, 2.266, 0, 0, 0.938, 0.51, 0.363}}};
-    const int s = d.stride_h, ph = shape == k2x4 ? 2 : shape == k8x8 || (shape == kOwn && s == 1) ? 8 : 4, pw = shape == k2x4 ? 4 : 8;
-    const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32, nT = (d.in_cs + 31) / 32;
-    if ((shape == kOwn && (nk > 2 || ct > 2)) || (shape == k8x8 && (s == 2 || ct > 3)))
+    // launch, slice, slice x channel tiles, slice x k-steps, slices per SIMD, generation
+    static const double kCost[2][kShapes][6] = {
+        {{2.87, 0, 0.323, 0, 0.473, 1.00}, {2.07, 0, 0.498, 0.016, 0.572, 2.71}, {2.45, 0.701, 0.825, 0.135, 0.225, 2.56}, {0, 1.362, 0.224, 0.117, 0.581, 3.26}},
+        {{2.17, 0, 0.368, 0.035, 0.394, 2.06}, {3.46, 0, 0.540, 0.268, 0.946, 1.75}, {}, {1.86, 1.663, 0.076, 0.302, 0.533, 1.00}}};
+    const int s = d.stride_h;
+    const Channels c = channels_of(e, p);
+    if ((shape == kOwn && (c.nk > 2 || c.ct > 2)) || (shape == k8x8 && (s == 2 || c.ct > 3)))
         return 1e30; // not built: the accumulators or the region would be too much for a wave
-    const double patches = (double)d.N * ((p.OH + ph - 1) / ph) * ((p.OW + pw - 1) / pw);
-    const int nw = shape == kOwn ? 1 : std::min(nT, max_waves((ph * pw + 31) / 32, ct)), rounds = (nT + nw - 1) / nw;
-    const double v[7] = {1, (double)rounds, (double)rounds * ct, patches * nT / 1024, (double)ct, patches / 256, std::ceil(patches / 256)};
+    const Division v = divide(e, d, p, shape);
+    // waves per SIMD that the registers allow
+    const int waves = shape == kOwn ? (s == 2 ? 4 : c.ct == 1 ? 3 : 2) : max_waves(shape == k8x8 ? 2 : 1, c.ct) / 4;
+    const int held = std::max(1, std::min((int)(160 * 1024 / v.lds), 4 * waves / v.nw)); // work-groups of a CU
+    const double gens = (double)((v.wgs + 256 * held - 1) / (256 * held)), steps = gens * v.rounds;
+    const double patches = (double)d.N * v.PY * v.PX;
+    const double f[6] = {1, steps, steps * c.ct, steps * c.nk, patches * v.nT / 1024, gens};
     double t = 0;
-    for (int i = 0; i < 7; i++)
-        t += kCost[s - 1][shape][i] * v[i];
+    for (int i = 0; i < 6; i++)
+        t += kCost[s - 1][shape][i] * f[i];
     return t;
 }
 
@@ -382,31 +428,13 @@ void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
 {
     if constexpr (NK <= 2 && CT <= 2)
         if (shape == kOwn)
-            return launch_shape<S, S == 1 ? 8 : 4, 8, NK, CT, true>(e, d, p, st);
+            return launch_shape<S, S == 1 ? 8 : 4, 8, NK, CT, true>(e, d, p, shape, st);
     if constexpr (S == 1 && CT <= 3)
         if (shape == k8x8)
-            return launch_shape<S, 8, 8, NK, CT, false>(e, d, p, st);
+            return launch_shape<S, 8, 8, NK, CT, false>(e, d, p, shape, st);
     if (shape == k4x8)
-        return launch_shape<S, 4, 8, NK, CT, false>(e, d, p, st);
-    launch_shape<S, 2, 4, NK, CT, false>(e, d, p, st);
-}
-
-// the channel counts that are built: k-steps of the expanding layer and channel tiles of the projecting one, each at least what the
-// layers have
-struct Channels {
-    int nk, ct;
-};
-
-Channels channels_of(const ConvArgs &e, const ConvArgs &p)
-{
-    const int nk = (e.in_cs + 31) / 32, ct = (p.out_cs + 31) / 32;
-    if (nk == 1 && ct <= 2)
-        return {1, ct};
-    if (nk <= 2 && ct <= 3)
-        return {2, ct <= 2 ? 2 : 3};
-    if (nk <= 3)
-        return {3, ct <= 3 ? 3 : 5};
-    return {5, 5};
+        return launch_shape<S, 4, 8, NK, CT, false>(e, d, p, shape, st);
+    launch_shape<S, 2, 4, NK, CT, false>(e, d, p, k2x4, st);
 }
 
 template <int S>
@@ -446,14 +474,15 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
 }
 
 // The three launches: their latencies, the hidden tensor's bytes at both resolutions, the expanding layer's products (fitted to
-// the same blocks, within 11 %).
+// the same blocks, within 20 %, one 24).  Chosen by this the 160 blocks take 0.6 % more than the best choice would on average, one
+// in twenty more than 3 %, the worst 31 %; by the fits before 3.0, 18 and 73 %.
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
-    const double apart = d.stride_h == 1 ? 9.25 + 1.007 * wide + 0.00548 * wide * e.in_cs : 9.32 + 1.996 * narrow + 0.00451 * wide * e.in_cs;
+    const double apart = d.stride_h == 1 ? 8.55 + 0.790 * wide + 0.00403 * wide * e.in_cs : 8.78 + 1.437 * narrow + 0.00502 * wide * e.in_cs;
     double us;
     choose_shape(e, d, p, -1, &us);
-    return us < 0.95 * apart;
+    return us < apart;
 }
 
 const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted)
