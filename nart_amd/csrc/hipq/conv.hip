@@ -1343,7 +1343,8 @@ static bool k2_applies(const hipq_conv2d_plan *p);
 
 // Microseconds that the tile kernels take on a plan, as fitted to layers over 6 to 6 272 pixels: a launch, and a step per slab
 // of the reduction whose length is a round trip and hardly depends on how many of the CUs have a tile; from one tile per CU
-// on, the steps of a CU's tiles overlap in part.  The two-group kernel walks two slabs a step.
+// on, the steps of a CU's tiles overlap in part.  The two-group kernel walks two slabs a step.  (56 layers of
+// profiles/convolution_costs_gfx950.md: 0.79 to 1.12 of the measured time, nine in ten 0.86 to 1.09.)
 static double tile_cost(const hipq_conv2d_plan *p)
 {
     const ConvArgs &a = p->args;
@@ -1357,7 +1358,7 @@ static double tile_cost(const hipq_conv2d_plan *p)
 
 // The streaming kernel's, for one shape of its work-groups: LDS holds one work-group per CU, each round starts anew (1.5 us), pulls
 // (16 mb + 16 nb) rows of the reduction through the CU's L1 at 42 KB/us and ends with
-// an epilogue (0.8 us for the largest shape).
+// an epilogue (0.8 us for the largest shape).  (The same layers: 0.86 to 1.23 of the measured time, nine in ten 0.91 to 1.16.)
 static double stream_cost(const hipq_conv2d_plan *p, const StreamShape &c)
 {
     const ConvArgs &a = p->args;
@@ -1367,16 +1368,19 @@ static double stream_cost(const hipq_conv2d_plan *p, const StreamShape &c)
 }
 
 // conv_mfma_stream_kernel: layers that the tile kernels would walk with a few tiles in many steps - fully-connected layers, the
-// last stages of a network at a small batch, layers with few output channels.  It takes what the two costs above say.  (Both
-// within 15 % on the layers they were fitted to; up to 256 pixels whatever the layer and up to 1024 with a reduction of 512
-// bytes, the rule before, was 12.1 against 6 us on 512 -> 2048 channels over 539 pixels and left 230 -> 24 channels, 3x3, over
-// 1568 to the tile kernels: 11.5 us, now 8.7.)
+// last stages of a network at a small batch, layers with few output channels.  It takes what the two costs above say: 0.4 % above the
+// better kernel on average over those 56 layers, 8 % at worst.  (Up to 256 pixels whatever the layer and up to 1024 with a
+// reduction of 512 bytes, the rule before, was 12.1 against 6 us on 512 -> 2048 channels over 539 pixels and left 230 -> 24
+// channels, 3x3, over 1568 to the tile kernels: 11.5 us, now 8.7.)
 static bool stream_applies(const hipq_conv2d_plan *p, StreamShape *shape = nullptr)
 {
     if (!(p->special && !p->tile_selected && p->variant == kMfma && p->args.R * p->args.S <= 255 && p->args.Ktot < (1 << 22)))
         return false;
-    // Where the tile kernels' aligned addressing and the two-group kernel serve a layer well - 3x3 layers on 64-byte lines with a
-    // short reduction, 1x1 layers on an image whose last slab is partial - they keep it.
+    // Two classes keep the kernels they had: 3x3 layers on 64 channels (resident rows, halo tiles) and 1x1 layers on an image whose
+    // last slab is partial (the two-group kernel).  Both sides measured (same file): the rows kernel is level (3.3 and 3.4 us either
+    // way at 49 and 196 pixels, 3.8 against 3.9 at 3136); the halo kernel takes 5.0 where streaming takes 3.4 to 4.4, the
+    // two-group kernel 3.9 to 7.8 where streaming takes 2.6 to 4.6, until some 6000 pixels x 256 channels (5.9 against 20, 5.2
+    // against 12).  What draws the line is the kernel that these layers are pinned to in the tests, not speed.
     const ConvArgs &a = p->args;
     const bool point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
     if (!p->has_wzp && !fc
@@ -1440,7 +1444,8 @@ static bool wreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
 // Over more than 512 pixels it is ahead of the register-fed kernel's patches (256 -> 256 at 14x14, batch 64: 12.7 -> 11.2 us)
 // and, by the fitted costs, of the tile and streaming kernels (13x13, batch 11: 9.2 -> 5.3 us).  64-channel layers keep their
 // resident rows but for 32 000 to 90 000 pixels (56x56, batch 12, with the add: 7.4 -> 6.6 us; level at 100 000, 24 against
-// 15 us at 200 000, where the halo of a tile outweighs its nine steps), and up to 4 096 pixels the halo kernel.
+// 15 us at 200 000, where the halo of a tile outweighs its nine steps), and up to 4 096 pixels the halo kernel, which they are
+// pinned to in the tests (5.2 us against 3.3 on 2400 pixels of 135 output channels).
 static bool hreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
 {
     double us = 0;

@@ -151,7 +151,8 @@ __device__ static inline uint32_t relu_one(uint32_t x, const ReluArgs &p)
 }
 
 // WORD: shift <= 31.  The multiplier has 23 bits, so difference * mult + 2^(shift - 1) stays below 2^32: one 24-bit
-// multiply-add and a shift per byte instead of a 64-bit product (3 instead of 11 vector instructions).
+// multiply-add and a shift per byte instead of a 64-bit product (3 instead of 11 vector instructions).  Bytes in and out, 64-bit ->
+// 24-bit form: 2 x 1 MB 2.03 -> 1.97 us (a launch), 2 x 10.2 MB 5.55 -> 4.76, 2 x 51.4 MB 19.4 -> 16.6 (6.2 TB/s).
 template <bool WORD>
 __global__ __launch_bounds__(256) void relu_u8_kernel(const ReluArgs p)
 {
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(256) void pool_u8_kernel(const PoolArgs p)
 // Pooling with a channel stride that is a multiple of 16: a thread owns 16 channels of one output pixel (128-bit
 // loads, one 128-bit store), 32-bit index arithmetic.  Maxima and sums are taken on the packed dwords (sums: bytes 0, 2 and
 // bytes 1, 3 as two 16-bit halves each; the host guarantees windows of at most 128 pixels).  Average pooling of 8 x 35 x 35 x 192,
-// 3x3 / stride 1: 7.4 us with four channels per thread -> 4.4.
+// 3x3 / stride 1: 6.75 us with four channels per thread -> 3.64.
 template <bool AVG>
 __global__ __launch_bounds__(256) void pool16_u8_kernel(const PoolArgs p, double inv_c16, double inv_ow, double inv_oh)
 {
@@ -343,7 +344,7 @@ __global__ __launch_bounds__(256) void pool16_u8_kernel(const PoolArgs p, double
 // NT / cpb thread groups; a thread sums its pixels on packed 16-bit lanes, unpacked every 256 of them, and the partial sums meet in
 // LDS in two steps.  What bounds it is one thread's list of pixels (a load latency per four), so the host takes the largest cpb
 // that still makes 1024 work-groups and 1024 threads where 256 would leave lists of more than four.  8 x 35 x 35 x 192:
-// 152 us with one thread per four channels and image -> 7.2 with 256 threads -> 4.6.
+// 150 us with one thread per four channels and image -> 7.2 with 256 threads -> 4.1.
 template <int NT>
 __global__ __launch_bounds__(NT) void pool_gavg16_u8_kernel(const PoolArgs p, uint32_t mult, int shift, int cpb_log2)
 {
@@ -469,7 +470,7 @@ struct __attribute__((packed)) unaligned_t { T v; };
 template <class T>
 __device__ static inline void store_unaligned(uint8_t *p, T v) { reinterpret_cast<unaligned_t<T> *>(p)->v = v; }
 
-// 8 x 35 x 35, 192 + 100 channels: 5.5 us with a thread per output dword -> 4.1
+// 8 x 35 x 35, 192 + 100 channels: 4.98 us with a thread per output dword -> 3.08
 __global__ __launch_bounds__(256) void concat16_u8_kernel(const ConcatArgs p)
 {
     const int j = blockIdx.y, ch = p.off[j + 1] - p.off[j], n16 = p.cs[j] >> 4, tail = ch & 15;
@@ -522,7 +523,7 @@ __global__ __launch_bounds__(256) void concat16_u8_kernel(const ConcatArgs p)
 // y = saturate_float_by_bits(e / sum / oalpha + ozp) with IEEE fp32 divisions.
 // A work-group stages the bytes of `rows` pixels in LDS (coalesced both ways), one thread per pixel walks its channels for the sum -
 // that order leaves no other parallelism - and all threads share the divisions, four channels at a time, writing the bytes back in
-// place.  A thread per pixel for everything took 31.5 us for 9800 pixels of 81 channels, this 5.1.
+// place.  A thread per pixel for everything took 31.0 us for 9800 pixels of 81 channels, this 4.6.
 struct SoftmaxArgs {
     const uint8_t *x;
     uint8_t *y;
@@ -818,7 +819,7 @@ __global__ __launch_bounds__(256) void dequantize_u8_kernel(const DequantArgs p)
 
 // Images: a thread converts VEC channels (16, or the 4 of a network input; blockIdx.z) of one pixel with one load; the 64 lanes
 // of a wave write 64 consecutive pixels of a plane per store.  The loop over single bytes above reads every line VEC
-// times over and divides twice per value: 64 x 21 x 56 x 56 took 12.2 us, this 5.6.
+// times over and divides twice per value: 64 x 21 x 56 x 56 took 11.8 us, this 4.6.
 template <int VEC>
 __global__ __launch_bounds__(256) void dequantize_planes_kernel(const DequantArgs p)
 {
