@@ -148,27 +148,33 @@ int hipq_conv2d_plan_select(hipq_conv2d_plan *plan, int tile, int stages);
  * 3x3 stem kernel (name "..._stem3x3"): 3x3 / stride 2 convolutions of an image with at most 4 channels (channel stride 4,
  * rows of at most 248 pixels, a multiple of 4) to at most 32 channels (stride 32), weight zero point 128: the input rows
  * of a work-group in LDS, two multiplies per 32 pixels, 128-bit stores straight from the accumulators; modes 1 and 2.
- * mode 1 (the default) uses them where they measured faster: the rows kernel wherever it applies, the halo kernel for
- * the other 64-channel inputs up to 63 pixels wide, the pointwise kernel wherever it applies, the two-group kernel for layers with at most one tile per CU (256),
+ * 3x3 kernel for any image (name "..._hreg3x3"): 3x3 / stride 1 / pad 1 convolutions from 64, 128, 256 or 512 channels (weight zero
+ * point 128, per-tensor scale, one-multiply requantisation), the pixels of a work-group in LDS once and the weights straight
+ * in registers, with or without the residual add; mode 1 only.  Register-fed kernel (name "..._wreg"): 1x1 and 3x3 layers
+ * of 14x14 and 7x7 images; modes 1 and 3.
+ * mode 1 (the default) uses them where they measured faster: the 3x3 kernel for any image over more than 512 pixels where its
+ * fitted cost is the smaller one (64 channels: from 4096 pixels, and 32 000 to 90 000 where the rows kernel applies), the rows
+ * kernel wherever else it applies, the halo kernel for the other 64-channel inputs up to 63 pixels wide, the pointwise kernel wherever it applies, the two-group kernel for layers with at most one tile per CU (256),
  * the widening kernel at 64 input channels with or without the add (from 150 000 pixels), with it at 128 (from 50 000)
  * and without it at 256 (from 20 000);
  * mode 2 the halo kernel instead of the rows kernel and also for 128, 256 and 512 channels (128-channel tiles, images up to 31 pixels wide), the
- * two-group kernel whatever the number of tiles and the widening kernel wherever it applies; mode 0 none of them.
+ * two-group kernel whatever the number of tiles and the widening kernel wherever it applies; mode 3 the register-fed kernel
+ * wherever it applies; mode 0 none of them.
  * Identical results in every mode.  Plans that do not run the MFMA kernel return an error.
  */
 int hipq_conv2d_plan_special(hipq_conv2d_plan *plan, int mode);
 /*
- * Tuning hook (no counterpart in the reference) for the streaming kernel (name "..._stream_<rows>x<cols>"): layers over
- * at most 256 output pixels (1024 where a pixel's reduction is at least 512 bytes long) whose input pixels are multiples
- * of 128 bytes (weight zero point 128, or int8) - the fully-connected layers, op_quant_ip_u8xu8_run
- * (src/op/ip.cpp:133-209), whose pixels are the batch, and convolutions of any kernel size, stride and padding over small
- * images (the late stages of a network at batch 1); hipq_conv2d_run_add fuses the residual add into it.  They
- * are bound by the weight stream, so the output is cut into strips of 16 or 32 channels, one work-group each, whose waves
- * split the reduction and stream their shares through LDS stages of their own into the 16x16x64 MFMA.  rows: pixel rows
- * per work-group (16, 32, 64 or 128), cols: 16 or 32 (128 x 32 does not exist), waves: 4; 0, 0, 0 returns to the built-in rule (one strip
- * shape that minimises what a CU pulls through its L1).  hipq_conv2d_plan_special(plan, 0) switches the kernel off, and so
- * does naming a tile with hipq_conv2d_plan_select.
- * Identical results for every choice.  Plans that the kernel does not serve return an error.
+ * Tuning hook (no counterpart in the reference) for the streaming kernel (name "..._stream_<rows>x<cols>"): layers that the tile
+ * kernels would walk with a few tiles in many steps - the fully-connected layers, op_quant_ip_u8xu8_run
+ * (src/op/ip.cpp:133-209), whose pixels are the batch, and convolutions of any kernel size, stride, padding, channel count and
+ * weight zero point over few pixels or to few channels; hipq_conv2d_run_add fuses the residual add into it.  The output is cut
+ * into strips of 16 or 32 channels, one work-group each, whose waves split the reduction and stream their shares through LDS
+ * stages of their own into the 16x16x64 MFMA.  The built-in rule takes it where a fitted cost says that it is faster than the
+ * tile kernels, in the shape with the smallest cost; 3x3 layers on 64 channels and 1x1 layers on an image whose last 64-byte
+ * slab is partial (an even number of at least 8 slabs) keep the kernels of hipq_conv2d_plan_special.  rows: pixel rows per
+ * work-group (16, 32, 64 or 128), cols: 16 or 32 (128 x 32 does not exist), waves: 4; 0, 0, 0 returns to the built-in rule.
+ * hipq_conv2d_plan_special(plan, 0) switches the kernel off, and so does naming a tile with hipq_conv2d_plan_select.
+ * Identical results for every choice.  Plans that do not run the kernel return an error.
  */
 int hipq_conv2d_plan_stream(hipq_conv2d_plan *plan, int rows, int cols, int waves);
 

@@ -41,6 +41,8 @@
 //     with its halo and the nine taps are read from LDS at shifted rows, instead of one slab per tap from memory.
 //   * 1x1 / stride 1 layers with at most 64 input and 256 output channels run conv_mfma_pointwise_kernel: a wave per
 //     strip of 32 pixels, pixel fragments straight from global memory, no LDS staging of activations, no barriers.
+//   * Layers over few pixels or to few channels are streamed (conv_stream.hip); 3x3 layers on any image keep their pixels in LDS
+//     and their weights in registers (conv_hreg.hip); whole blocks are one kernel (conv_block.hip, conv_invres.hip).
 //   * Other shapes: C <= 4 inputs (the RGB stem) use a register-staged variant of the same tile computation,
 //     depthwise 3x3 a dot-product kernel, remaining depthwise / grouped shapes plain per-output kernels.
 #include <algorithm>

@@ -20,18 +20,18 @@
 // Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch and add their partial sums up
 // in LDS.  Many patches and few slices: every wave has a patch of its own and takes all slices through it, so that no barrier
 // and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
-// 65 us at 56x56, batch 64, against 32.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
+// 64 us at 56x56, batch 64, against 32.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
 // instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice).
 // What bounds it is vector issue: some 650 instructions per slice of 8x8 outputs at stride 1, 70 of them per 32 expanded
 // positions; with few patches the chain launch - region - slices - sum.
-// Measured, the three launches -> this one (batch 64): 16 -> 96 -> 24 at 112x112, stride 2: 58 -> 34 us; 24 -> 144 -> 24 at 56x56:
-// 42 -> 32; 32 -> 192 -> 32 at 28x28: 21 -> 15.4; 64 -> 384 -> 64 at 14x14: 15 -> 11.8; batch 1: 10 -> 4.6 .. 6.4.
+// Measured, the three launches -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at 112x112, stride 2: 44 -> 33 us;
+// 24 -> 144 -> 24 at 56x56: 38 -> 32; 32 -> 192 -> 32 at 28x28: 16.4 -> 14.6; 64 -> 384 -> 64 at 14x14: 13.4 -> 11.2; batch 1:
+// 8.3 .. 9.6 -> 4.1 .. 6.0 (profiles/inverted_residual_shapes_gfx950.md).
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
-// requantisations, at most 160 input and output channels.
+// requantisations, at most 160 input and output channels; with the add stride 1 and as many output as input channels.
 #include "conv_invres.h"
 
 #include <algorithm>
-#include <cmath>
 
 #include "conv_frag.h"
 

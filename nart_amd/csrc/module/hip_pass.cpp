@@ -1,10 +1,11 @@
-// A pass over a parade as a HIP graph.  Launched one by one the operators of a pass cost the host 2.8 us a kernel and as much
-// again beside it, about what the small ones take on the GPU: MobileNetV2 at batch 6 spent 179 us launching 54 kernels that
-// take 235 us back to back and 275 us when each waits for its launch.  The kernels, their order and their arguments are the
-// same at every pass, so the second pass is recorded while the operators run (their run functions do not know) and the later
-// ones replay the record: one launch.  (It takes 18 - 25 us until its first kernel starts, an ordinary one 3; launching the
-// first four kernels the ordinary way in front of the graph, to hide that, gained nothing: 131.3 against 130.3 us for
-// ResNet-18 at batch 1.)
+// A pass over a parade as a HIP graph.  The kernels, their order and their arguments are the same at every pass, so the second
+// pass is recorded while the operators run (their run functions do not know) and the later ones replay the record: one launch.
+// What it gives is the host time of the launches where the host is the slower side, and the gaps between small kernels: from
+// host array to host array, operator by operator -> replayed: MobileNetV2 at batch 1 161 -> 151 us, at batch 6 and 160x160 186 ->
+// 179; ResNet-18 at batch 1 (129 -> 130) and ResNet-50 at batch 64 (1016 -> 1013) are level.  The second pass pays for it:
+// 135 to 260 us more than the ones around it.  (A graph takes 18 - 25 us until its first kernel starts, an ordinary launch 3;
+// launching the first four kernels the ordinary way in front of the graph, to hide that, gained nothing: 131.3 against 130.3 us
+// for ResNet-18 at batch 1.)
 //
 // The first pass runs eagerly: it allocates the tensors, and a program that runs once pays nothing.  What a pass does
 // beside launching - which side of a memory is current, which launches were left to a reader - is recorded as well, as the
@@ -19,7 +20,7 @@
 namespace {
 
 constexpr size_t kShortest = 8; // fewer kernels start sooner one by one (10 take 32 us as a graph, 54 one by one; 5 take 35 and 23)
-constexpr long kWorth = 16;     // replays after which a record has paid for itself
+constexpr long kWorth = 16;     // replays that pay for a record (155 us beside 10 a replay for MobileNetV2 at batch 1)
 constexpr int kMaxWait = 256;   // eager passes before the next record, at most
 constexpr int kUnread = 8;      // replays in a row that copied back an output nobody asked for
 
