@@ -65,8 +65,11 @@ static size_t dev_bytes(const hip_mem_t *m)
 
 static mem_t *hm_new(void)
 {
-    auto *m = static_cast<hip_mem_t *>(calloc(1, sizeof(hip_mem_t)));
-    return &m->m;
+    constexpr size_t bytes = (sizeof(hip_mem_t) + 63) / 64 * 64;
+    void *m = aligned_alloc(64, bytes); // whole cache lines
+    HIPM_CHECK(m != nullptr);
+    memset(m, 0, bytes);
+    return &static_cast<hip_mem_t *>(m)->m;
 }
 
 static void hm_free(mem_t *mm)

@@ -73,33 +73,35 @@ struct hip_workspace_t {
 enum hip_layout_t { HIP_LAYOUT_RAW = 0, HIP_LAYOUT_NHWC_U8 = 1 };
 
 struct hip_mem_t {
+    // What a pass looks at and restores comes first, 64 bytes: a replay visits every memory of the pass before its launch.
     mem_t m;            // must be first (art/include/art/mem.h:66-69)
-    size_t size;        // logical size in bytes (dense NCHW), as requested through mem_alloc
-    void *host;         // pinned host mirror, allocated on first mem_cpu_data()
-    size_t host_cap;
     void *dev;          // device buffer in `layout`
-    size_t dev_cap;
-    void *stage;        // device scratch for the dense side of a layout conversion
-    size_t stage_cap;
-    hip_layout_t layout;
-    int N, C, H, W, cs; // geometry for HIP_LAYOUT_NHWC_U8
-    bool host_valid, dev_valid;
-    // An upload reads the pinned mirror asynchronously on `up_stream`: the mirror may only be handed out for writing
-    // once that copy has finished.
-    bool up_pending;
-    hipStream_t up_stream;
+    void *host;         // pinned host mirror, allocated on first mem_cpu_data()
     // The stream whose work last used `dev` (a workspace's, or the null stream on behalf of foreign code); what others did to
     // it before has finished.  Whoever uses it on another stream, or wants the contents, waits for this one, and for nothing else.
     hipStream_t prod_stream;
+    // An upload reads the pinned mirror asynchronously on `up_stream`: the mirror may only be handed out for writing
+    // once that copy has finished (up_pending).
+    hipStream_t up_stream;
     // Deferred producer.  A convolution whose only reader is an add does not launch at its own run(): it leaves this
     // hook, and the add runs both as one fused kernel (hip_ops.cpp).  Whoever else asks for the contents first - the
     // host, another workspace, a re-run - makes the hook launch the plain convolution into `dev` (hip_mem_settle).
     void (*pending)(void *ctx);
     void *pending_ctx;
+    bool host_valid, dev_valid;
+    bool up_pending;
     // The mirror is being filled from the device by work queued on prod_stream (a recorded pass ends with that): whoever
-    // wants it waits for that stream.  host_read: the host has asked for device-written contents
-    // since a pass was last recorded.
+    // wants it waits for that stream.  host_read: the host has asked for device-written contents since a pass was last recorded.
     bool down_issued, host_read;
+    bool q_valid; // see q_op
+
+    size_t size;        // logical size in bytes (dense NCHW), as requested through mem_alloc
+    size_t host_cap;
+    size_t dev_cap;
+    void *stage;        // device scratch for the dense side of a layout conversion
+    size_t stage_cap;
+    hip_layout_t layout;
+    int N, C, H, W, cs; // geometry for HIP_LAYOUT_NHWC_U8
     // A float input whose reader is a uint8 quantize operator (quantize_prepare fills q_*).  hip_mem_write quantizes the
     // values while it copies them into the mirror, a quarter of the bytes to bring to the device; q_valid: qhost (pinned) and,
     // for what is not read from there directly, qdev hold the bytes of what the mirror holds.
@@ -108,7 +110,6 @@ struct hip_mem_t {
     int q_zp, q_bits;
     uint8_t *qhost, *qdev;
     size_t qhost_cap, qdev_cap;
-    bool q_valid;
 };
 
 // Up to this size a kernel reads or writes pinned host memory itself; above it the copy engine moves the bytes first.
