@@ -38,9 +38,9 @@ PEAK_HBM_GBS = 8000.0     # MI355X HBM3E, GB/s (published)
 # file that holds the counter readings and a digest of the kernel sources it was taken with: the line reports it only
 # for the default workload with default flags and only while the sources under nart_amd/csrc/hipq still have that digest
 # (traffic is null, with the reason, once a kernel has changed and the profile has not been taken again).
-TRAFFIC_FROM_PROFILE = {"workload": "resnet50", "batch": 64, "bytes_per_launch": 52.40e6,
+TRAFFIC_FROM_PROFILE = {"workload": "resnet50", "batch": 64, "bytes_per_launch": 52.39e6,
                         "source": "profiles/conv_mfma_i8_resnet50_n64.md",
-                        "sources_sha256": "7b2ea2a739053335"}
+                        "sources_sha256": "5737b64c37b498a3"}
 
 
 def kernel_sources_digest():
@@ -326,7 +326,7 @@ def module_path(build, batch, steps):
     if p.returncode != 0 or not m:
         return {"error": "nart_promark exit %d: %s" % (p.returncode, (p.stderr or p.stdout)[-300:])}
     ms = float(m.group(1))
-    return {"runner": "nart_promark -b %d -n %d (engine.bin on the hip workspace through hip_module_tp, eager launches, no host copies)" % (batch, steps),
+    return {"runner": "nart_promark -b %d -n %d (engine.bin on the hip workspace through hip_module_tp, passes recorded and replayed by parade_run, no host copies)" % (batch, steps),
             "ms_per_batch": round(ms, 4), "value": round(batch / (ms * 1e-3), 1)}
 
 

@@ -22,8 +22,9 @@
 // and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
 // 64 us at 56x56, batch 64, against 32.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
 // instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice).
-// What bounds it is vector issue: some 650 instructions per slice of 8x8 outputs at stride 1, 70 of them per 32 expanded
-// positions; with few patches the chain launch - region - slices - sum.
+// What bounds it: with a patch per wave vector issue - some 650 instructions per slice of 8x8 outputs at stride 1, 70 of them per 32
+// expanded positions, 55 to 64 % of a CU's busy time at batch 64; with a shared patch the chain launch - region - slices - sum
+// (vector issue 35 to 44 %).
 // Measured, the three launches -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at 112x112, stride 2: 44 -> 33 us;
 // 24 -> 144 -> 24 at 56x56: 38 -> 32; 32 -> 192 -> 32 at 28x28: 16.4 -> 14.6; 64 -> 384 -> 64 at 14x14: 13.4 -> 11.2; batch 1:
 // 8.3 .. 9.6 -> 4.1 .. 6.0 (profiles/inverted_residual_shapes_gfx950.md).
