@@ -1345,8 +1345,8 @@ static bool k2_applies(const hipq_conv2d_plan *p);
 
 // Microseconds that the tile kernels take on a plan, as fitted to layers over 6 to 6 272 pixels: a launch, and a step per slab
 // of the reduction whose length is a round trip and hardly depends on how many of the CUs have a tile; from one tile per CU
-// on, the steps of a CU's tiles overlap in part.  The two-group kernel walks two slabs a step.  (56 layers of
-// profiles/convolution_costs_gfx950.md: 0.79 to 1.12 of the measured time, nine in ten 0.86 to 1.09.)
+// on, the steps of a CU's tiles overlap in part.  The two-group kernel walks two slabs a step.  (On 56
+// random layers 0.79 to 1.12 of the measured time, nine in ten 0.86 to 1.09.)
 static double tile_cost(const hipq_conv2d_plan *p)
 {
     const ConvArgs &a = p->args;
@@ -1379,7 +1379,7 @@ static bool stream_applies(const hipq_conv2d_plan *p, StreamShape *shape = nullp
     if (!(p->special && !p->tile_selected && p->variant == kMfma && p->args.R * p->args.S <= 255 && p->args.Ktot < (1 << 22)))
         return false;
     // Two classes keep the kernels they had: 3x3 layers on 64 channels (resident rows, halo tiles) and 1x1 layers on an image whose
-    // last slab is partial (the two-group kernel).  Both sides measured (same file): the rows kernel is level (3.3 and 3.4 us either
+    // last slab is partial (the two-group kernel).  Both sides measured: the rows kernel is level (3.3 and 3.4 us either
     // way at 49 and 196 pixels, 3.8 against 3.9 at 3136); the halo kernel takes 5.0 where streaming takes 3.4 to 4.4, the
     // two-group kernel 3.9 to 7.8 where streaming takes 2.6 to 4.6, until some 6000 pixels x 256 channels (5.9 against 20, 5.2
     // against 12).  What draws the line is the kernel that these layers are pinned to in the tests, not speed.

@@ -133,8 +133,8 @@ int lds_bytes(const ConvArgs &a, const HregShape &s)
 }
 
 // Microseconds for one shape: 2.6 beside the reduction, a slab as long as the slower of its multiplies and its weight bytes,
-// once for every work-group that a CU gets.  (26 layers of profiles/convolution_costs_gfx950.md: 0.76 to 1.72 of the measured time over
-// all shapes, the middle half 0.90 to 1.18; the shape it picks is at most 14 % behind the best one, once 28 %.)
+// once for every work-group that a CU gets.  (On 26 layers 0.76 to 1.72 of the measured time over all shapes, the middle half 0.90
+// to 1.18; the shape it picks is at most 14 % behind the best one, once 28 %.)
 double shape_cost(const ConvArgs &a, const HregShape &s)
 {
     const double slab = std::max(0.031 * s.mt, 0.029 * s.nw) + 0.004 * s.mt;

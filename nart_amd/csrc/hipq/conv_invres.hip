@@ -27,7 +27,7 @@
 // (vector issue 35 to 44 %).
 // Measured, the three launches -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at 112x112, stride 2: 44 -> 33 us;
 // 24 -> 144 -> 24 at 56x56: 38 -> 32; 32 -> 192 -> 32 at 28x28: 16.4 -> 14.6; 64 -> 384 -> 64 at 14x14: 13.4 -> 11.2; batch 1:
-// 8.3 .. 9.6 -> 4.1 .. 6.0 (profiles/inverted_residual_shapes_gfx950.md).
+// 8.3 .. 9.6 -> 4.1 .. 6.0.
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
 // requantisations, at most 160 input and output channels; with the add stride 1 and as many output as input channels.
 #include "conv_invres.h"
@@ -381,11 +381,11 @@ void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
 // ---- the shapes, and what each takes
 
 // Time by shape, in us, fitted to 160 blocks (1 to 128 images of 3x3 to 130x130, the channel counts of mobile networks; nine in ten
-// within 20 % of the fit, all within 33; every block's times are in profiles/inverted_residual_shapes_gfx950.md).  A launch; for every generation of
-// resident work-groups its start and end; for every slice that a wave then takes its chain, alone, per channel tile and per
-// k-step; and the slices per SIMD of the chip, which share the vector units.  How many work-groups a CU holds decides: the
-// fit before this one knew only patches per CU, which is right where nine small work-groups fit one, and picked shapes up to
-// 1.7 times slower than the three launches from 64 channels on (18 images of 20x103, 64 -> 384 -> 96: 34 against 25 us).
+// within 21 % of the fit, all within 33).  A launch; for every generation of resident work-groups its start and end; for every
+// slice that a wave then takes its chain, alone, per channel tile and per k-step; and the slices per SIMD of the chip, which
+// share the vector units.  How many work-groups a CU holds decides: the fit before this one knew only patches per CU, which is
+// right where nine small work-groups fit one, and picked shapes up to 1.7 times slower than the three launches from 64 channels
+// on (18 images of 20x103, 64 -> 384 -> 96: 34 against 25 us).
 double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
     // launch, slice, slice x channel tiles, slice x k-steps, slices per SIMD, generation
@@ -476,7 +476,8 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
 
 // The three launches: their latencies, the hidden tensor's bytes at both resolutions, the expanding layer's products (fitted to
 // the same blocks, within 20 %, one 24).  Chosen by this the 160 blocks take 0.6 % more than the best choice would on average, one
-// in twenty more than 3 %, the worst 31 %; by the fits before 3.0, 18 and 73 %.
+// in twenty more than 3 %, the worst 31 % (3.0, 18 and 73 % by the fits before); 180 blocks that the fits have not seen 0.75, 4
+// and 22 % (1.5, 10 and 39 %).
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
