@@ -179,6 +179,16 @@ int hipq_conv2d_plan_special(hipq_conv2d_plan *plan, int mode);
 int hipq_conv2d_plan_stream(hipq_conv2d_plan *plan, int rows, int cols, int waves);
 
 /*
+ * Tuning: the shape of the kernel that keeps a layer's pixels in LDS and loads its weights straight into registers
+ * (conv_resident.hip).  pixels and channels: a wave's share, 16 x 16 to 128 x 32; channel_waves: waves of a work-group side by side
+ * over the output channels; reduction_waves: waves that share every reduction.  0, 0, 0, 0 returns to the built-in rule, which
+ * takes the kernel where a fitted cost says that it is faster than the tile and streaming kernels.  hipq_conv2d_plan_special
+ * (any mode but 1), naming a tile and naming a shape of the streaming kernel leave it to the caller's choice as well.
+ * Identical results for every choice.  Shapes that are not built, or whose pixels do not fit LDS, return an error.
+ */
+int hipq_conv2d_plan_resident(hipq_conv2d_plan *plan, int pixels, int channels, int channel_waves, int reduction_waves);
+
+/*
  * Run: op_conv_2d_u8xu8_run — src/op/conv_2d_uint8_impl.c:39-165 (im2col src/utils/im2col.cpp:487,
  * GEMM src/gemm/default/gemm.c:306).  x, y: device NHWC.  acc_out: optional device int32
  * [N*OH*OW, out_cs] that receives the raw accumulators (bias included), NULL to skip.

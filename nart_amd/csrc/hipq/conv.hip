@@ -60,6 +60,7 @@
 #include "conv_dw.h"
 #include "conv_hreg.h"
 #include "conv_invres.h"
+#include "conv_resident.h"
 #include "conv_rows.h"
 #include "conv_stream.h"
 #include "conv_wreg.h"
@@ -1308,6 +1309,8 @@ struct hipq_conv2d_plan {
     int special = 1; // the halo-tile and pointwise kernels: 0 never, 1 built-in rule, 2 wherever they apply
     bool tile_selected = false;     // hipq_conv2d_plan_select named a tile: the tile kernels, not the streaming kernel
     int invres_shape = -1; // patch shape of the inverted residual block this plan projects (hipq_inverted_residual_select); -1: by cost
+    ResidentShape resident = {0, 0, 0, 0}, resident_add = {0, 0, 0, 0}; // of conv_resident_kernel, without and with a residual; mb = 0: another kernel
+    bool resident_named = false;           // by the caller (hipq_conv2d_plan_resident)
     StreamShape stream = {0, 0, 0}; // explicit shape of the streaming kernel (hipq_conv2d_plan_stream); mb = 0: built-in rule
     bool has_wzp;
     void *d_w = nullptr, *d_bias = nullptr, *d_q = nullptr;
@@ -1467,11 +1470,83 @@ static bool stem3_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
     return p->variant == kMfmaSmallC && p->special >= 1 && !p->tile_selected && !p->has_wzp && conv_stem3x3_applies(a, a.rowb);
 }
 
+// conv_resident_kernel (conv_resident.hip): any layer whose pixels fit LDS.  Against what the tile and the streaming kernels take,
+// fitted to 820 layers of the range that its own cost is fitted to (nine in ten within 15 %).
+static double tile_us(const hipq_conv2d_plan *p)
+{
+    const ConvArgs &a = p->args;
+    const TileShape &t = kTiles[p->tile];
+    if (k2_applies(p))
+        return tile_cost(p);
+    const bool aligned = a.in_cs % 64 == 0 || (a.R == 1 && a.S == 1);
+    const double cu = std::max(1.0, (double)a.nbm * a.nbn / kCUs), step = (t.bm + t.bn) / 128.0, out = cu * t.bm * t.bn / 4096, pc = p->d_q ? out : 0;
+    if (p->has_wzp || !aligned)
+        return 2.67 + a.nslab * (0.112 + 0.213 * step + 0.109 * (cu - 1) * step + (p->has_wzp ? 0.039 * std::max(1.0, cu / 2) : 0)) + 0.384 * out + 0.586 * pc;
+    return 2.39 + a.nslab * step * (0.249 + 0.121 * (cu - 1)) + 0.45 * out + 0.57 * pc;
+}
+
+static double stream_us(const hipq_conv2d_plan *p, const StreamShape &s)
+{
+    const ConvArgs &a = p->args;
+    const bool point = a.R == 1 && a.S == 1;
+    const long long wgs = (long long)((a.P + 16 * s.mb - 1) / (16 * s.mb)) * ((a.out_cs + 16 * s.nb - 1) / (16 * s.nb));
+    return 2.56 + (double)((wgs + kCUs - 1) / kCUs) * ((point ? 0.0147 : 0.0233) * (s.mb + s.nb) * a.nslab + 0.193 * s.mb * s.nb + (point ? 0 : 0.34) + (p->d_q ? 0.32 : 0));
+}
+
+// Which shape, if any, the built-in rule takes it in.  The margins are what keeps layers from getting slower where both fits are a few
+// per cent off: with them 3 of 250 layers that changed kernel got more than 4 % slower (and the 250 a quarter faster), 9 with a twentieth
+// throughout.  Layers that have a kernel of their own keep it, and so do those that stream_applies keeps out for the
+// tests' sake.
+static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a)
+{
+    ResidentShape s = {0, 0, 0, 0};
+    double us;
+    if (!(p->variant == kMfma && p->special == 1 && !p->tile_selected && !p->stream.mb && conv_resident_applies(a)) || hreg_applies(p, a) || wreg_applies(p, a)
+        || rows_applies(p, a) || expand_applies(p, a) || pointwise_applies(p) || !conv_resident_choose(a, &s, &us))
+        return {0, 0, 0, 0};
+    StreamShape ss;
+    const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
+    // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.5 us streamed, 7.7 with resident rows; 128
+    // rows 10.5 against 9.1
+    if (streams && fc && ss.mb < 4)
+        return {0, 0, 0, 0};
+    // a 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 8.5 against 10.5 us
+    if (!streams && (halo_applies(p) || (point && (a.P > 8192 || a.stride_h > 1 || a.stride_w > 1 || (k2_applies(p) && (a.in_cs % 64 != 0 || a.P > 2048))))))
+        return {0, 0, 0, 0};
+    const double now = streams ? stream_us(p, ss) : tile_us(p);
+    const double margin = streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
+    return us < margin * now ? s : ResidentShape{0, 0, 0, 0};
+}
+
+// the arguments of a launch with a residual that ordinary scale ratios and 8 bits allow: which kernel it goes to hangs on these
+static ConvArgs with_residual(const hipq_conv2d_plan *p)
+{
+    ConvArgs a = p->args;
+    a.res = a.padbuf; // any non-null pointer
+    a.addq.fast = 1;  // the 32-bit form of the add
+    a.addq.hi = 255;
+    return a;
+}
+
+static void resident_name(const hipq_conv2d_plan *p, const ResidentShape &s, char *nm, size_t size, const char *behind)
+{
+    // "stream": the layers that are a stream of weights, whichever of the two kernels they run
+    StreamShape ss;
+    snprintf(nm, size, "conv_mfma_i8_%sresident_%dx%d%s%s%s", stream_applies(p, &ss) ? "stream_" : "", 16 * s.mb, 16 * s.nb * s.nwc,
+             p->has_wzp ? "_wzp" : "", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "", behind);
+}
+
 static void set_mfma_name(hipq_conv2d_plan *p, bool smallc)
 {
     char nm[96];
     StreamShape ss;
-    if (!smallc && hreg_applies(p, p->args))
+    if (!p->resident_named) {
+        p->resident = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, p->args);
+        p->resident_add = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, with_residual(p));
+    }
+    if (p->resident.mb)
+        resident_name(p, p->resident, nm, sizeof nm, "");
+    else if (!smallc && hreg_applies(p, p->args))
         snprintf(nm, sizeof nm, "conv_mfma_i8_hreg3x3");
     else if (!smallc && wreg_applies(p, p->args))
         snprintf(nm, sizeof nm, "conv_mfma_i8_wreg");
@@ -1740,11 +1815,12 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
     a.padbuf = a.wpack + pad_off;
     a.wfrag1 = frag_off && d.R == 1 ? a.wpack + frag_off : nullptr;
     a.wfrag = frag_whole ? a.wpack + frag_off : nullptr;
-    if (frag_whole)
+    if (p->variant == kMfma)
         set_mfma_name(p, false); // the register-fed kernel's rule looks at the fragment-order copy
     if (p->d_q) {
         a.qmult = static_cast<const uint32_t *>(p->d_q);
         a.qshift = reinterpret_cast<const int32_t *>(a.qmult + qbuf.size() / 2);
+        a.fastch = std::all_of(qbuf.begin() + qbuf.size() / 2, qbuf.end(), [](uint32_t sh) { return sh >= 33 && sh <= 52; });
         if (p->variant == kMfma || p->variant == kMfmaSmallC)
             set_mfma_name(p, p->variant == kMfmaSmallC); // the pointwise kernel does not serve per-channel scales
         else
@@ -1788,13 +1864,12 @@ extern "C" const char *hipq_conv2d_plan_kernel_add(const hipq_conv2d_plan *p)
     if (!p || (p->variant != kMfma && p->variant != kMfmaSmallC))
         return "";
     static thread_local std::string nm;
-    ConvArgs a = p->args;
-    a.res = a.padbuf; // any non-null pointer: the question is which kernel a launch with a residual goes to
-    a.addq.fast = 1;  // the 32-bit form of the add, which ordinary scale ratios allow
-    a.addq.hi = 255;  // to 8 bits
+    const ConvArgs a = with_residual(p);
     char buf[96];
     StreamShape ss;
-    if (hreg_applies(p, a))
+    if (p->resident_add.mb)
+        resident_name(p, p->resident_add, buf, sizeof buf, "+add");
+    else if (hreg_applies(p, a))
         snprintf(buf, sizeof buf, "conv_mfma_i8_hreg3x3+add");
     else if (wreg_applies(p, a))
         snprintf(buf, sizeof buf, "conv_mfma_i8_wreg+add");
@@ -1864,6 +1939,23 @@ extern "C" int hipq_conv2d_plan_stream(hipq_conv2d_plan *p, int rows, int cols, 
         HIPQ_REQUIRE(found, "hipq_conv2d_plan_stream: no instantiation for %d rows x %d columns with %d waves", rows, cols, waves);
         p->stream = {rows / 16, cols / 16, waves};
     }
+    set_mfma_name(p, false);
+    return 0;
+}
+
+extern "C" int hipq_conv2d_plan_resident(hipq_conv2d_plan *p, int pixels, int channels, int channel_waves, int reduction_waves)
+{
+    clear_error();
+    HIPQ_REQUIRE(p, "hipq_conv2d_plan_resident: null plan");
+    const ResidentShape s = {pixels / 16, channels / 16, channel_waves, reduction_waves};
+    double us;
+    const bool named = pixels != 0 || channels != 0 || channel_waves != 0 || reduction_waves != 0;
+    HIPQ_REQUIRE(!named || (p->variant == kMfma && pixels % 16 == 0 && channels % 16 == 0 && conv_resident_applies(p->args) && conv_resident_cost(p->args, s, &us)),
+                 "hipq_conv2d_plan_resident: %d pixels x %d channels a wave, %d x %d waves are not built for this plan (it runs %s)", pixels, channels, channel_waves,
+                 reduction_waves, p->name.c_str());
+    HIPQ_REQUIRE(p->variant == kMfma, "hipq_conv2d_plan_resident: only the MFMA kernels have variants (this plan runs %s)", p->name.c_str());
+    p->resident_named = named;
+    p->resident = p->resident_add = s;
     set_mfma_name(p, false);
     return 0;
 }
@@ -2507,6 +2599,10 @@ static int run_conv(const hipq_conv2d_plan *p, ConvArgs &a, hipStream_t st)
     switch (p->variant) {
     case kMfma:
     case kMfmaSmallC:
+        if (const ResidentShape &r = a.res != nullptr ? p->resident_add : p->resident; r.mb) {
+            launch_conv_resident(a, r, st); // any layer whose pixels fit LDS, weight operands straight into registers
+            break;
+        }
         if (hreg_applies(p, a)) {
             launch_conv_hreg(a, st); // 3x3, any image size: the pixels in LDS once, weight operands straight into registers
             break;

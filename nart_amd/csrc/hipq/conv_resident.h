@@ -1,0 +1,21 @@
+// Convolutions whose input pixels stay in LDS while the weights go straight into registers (conv_resident.hip).
+#pragma once
+
+#include "conv_shared.h"
+
+namespace hipq {
+
+// a work-group's share: 16 mb pixels by 16 nb nwc output channels; ks waves share every reduction, so it has nwc ks of them
+struct ResidentShape {
+    int mb, nb, nwc, ks;
+};
+
+// Can conv_resident_kernel compute a plan's launches?
+bool conv_resident_applies(const ConvArgs &a);
+// Can it in this shape?  *us: what it is expected to take.
+bool conv_resident_cost(const ConvArgs &a, const ResidentShape &s, double *us);
+// the cheapest shape; false: none
+bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us);
+void launch_conv_resident(const ConvArgs &a, const ResidentShape &s, hipStream_t st);
+
+} // namespace hipq

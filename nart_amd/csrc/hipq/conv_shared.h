@@ -52,6 +52,7 @@ struct ConvArgs {
     // nullptr = the per-tensor pair in q.  Such plans requantise with the 64-bit form, channel by channel.
     const uint32_t *qmult;
     const int32_t *qshift;
+    int fastch; // 1: the one-multiply requantisation is valid for every channel's shift
     const uint8_t *res; // fused residual add: the other operand (same layout as y), or nullptr
     int res_first;      // 1: the residual is input 0 of the add, the convolution's output input 1
     AddParams addq;

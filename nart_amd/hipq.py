@@ -50,6 +50,7 @@ _SIGS = {
     "hipq_conv2d_plan_select": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "hipq_conv2d_plan_special": (C.c_int, [C.c_void_p, C.c_int]),
     "hipq_conv2d_plan_stream": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int]),
+    "hipq_conv2d_plan_resident": (C.c_int, [C.c_void_p] + [C.c_int] * 4),
     "hipq_conv2d_run_relu": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "hipq_conv2d_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "hipq_conv2d_run_add": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int,
@@ -267,6 +268,12 @@ class Conv2d:
     def stream(self, rows=0, cols=0, waves=0):
         """Tuning hook: shape of the streaming (fully-connected) kernel's work-groups (include/hipq.h)."""
         check(lib().hipq_conv2d_plan_stream(self.handle, rows, cols, waves))
+        self.kernel = lib().hipq_conv2d_plan_kernel(self.handle).decode()
+        return self
+
+    def resident(self, pixels=0, channels=0, channel_waves=0, reduction_waves=0):
+        """Tuning hook: shape of the kernel that keeps a layer's pixels in LDS (include/hipq.h)."""
+        check(lib().hipq_conv2d_plan_resident(self.handle, pixels, channels, channel_waves, reduction_waves))
         self.kernel = lib().hipq_conv2d_plan_kernel(self.handle).decode()
         return self
 
