@@ -11,7 +11,7 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
 // Is it faster than the separate launches?
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p);
 // The launch and its name, conv_invres_s<stride>_<patch>_k<k-steps>_n<channel tiles>; wanted: 0 patches of 2x4 outputs, 1 4x8,
-// 2 8x8, 3 a patch per wave, -1 (or a shape that is not built for these channels) by cost
+// 2 8x8, 3 a patch per wave, 4 one of 4x8 at stride 1, -1 (or a shape that is not built for these channels) by cost
 void launch_conv_invres(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted, hipStream_t st);
 const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted);
 

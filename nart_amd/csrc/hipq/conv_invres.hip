@@ -8,26 +8,32 @@
 // Why: the hidden tensor is six times as wide as the block's input and output, is written and read twice, and the three layers
 // are three launches.  Here a work-group owns a patch of output pixels of ONE image, and its waves take the hidden channels in
 // slices of 32.  A wave takes a slice through all three layers on its own, without a barrier:
-//   * expand: the patch's input region, which lies re-centred in LDS, times the slice's weights, pixels as the ROWS of the
-//     multiply and channels as its columns: the 16 accumulators of a lane are four runs of four consecutive pixels of ONE
-//     channel, so a requantised run is a dword that the depthwise layer can use as it is;
-//   * depthwise: v_dot4_i32_i8 of such a dword with {w0, w1, w2, 0} and {0, w0, w1, w2} gives two neighbouring outputs (at stride
-//     2 one), the runs in between are v_alignbyte of two dwords: no byte transposes;
-//   * project: the slice's bytes, written to LDS as pixel rows, are one k-step of every output channel tile's reduction, whose
+//   * expand: the slice's weights, channels as the ROWS of the multiply, times the patch's input region, which lies re-centred in
+//     LDS: the 16 accumulators of a lane are 16 consecutive channels of one position, requantised to 16 bytes of its row in LDS;
+//   * depthwise, also on the matrix cores: for each of the nine taps a diagonal matrix of the slice's 32 weights, made from a dword by
+//     a byte permutation and four ANDs, times the rows at that tap.  31 of 32 products are with zeros, and still nine matrix
+//     instructions and 45 others replace the 130 dot products, byte alignments and LDS reads of 32 outputs of 32 channels: vector issue
+//     is what these kernels wait for, the matrix cores idle;
+//   * project: the requantised sums are, as they lie in the lanes, one k-step of every output channel tile's reduction, whose
 //     accumulators a wave keeps over its slices.
+// Patches of 2x4 outputs do not fill a multiply's 32 columns.  Theirs keeps the expanded pixels as rows (a lane has four runs of four
+// consecutive pixels of ONE channel), takes dot products of such a run with {w0, w1, w2, 0} and {0, w0, w1, w2} (two neighbouring
+// outputs; one at stride 2), and passes the result to the last layer through LDS.
 // Positions outside the image hold the depthwise layer's pad byte; the border of a patch is expanded again by its neighbours,
 // which costs vector instructions (the requantisation), not memory.
 // Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch and add their partial sums up
 // in LDS.  Many patches and few slices: every wave has a patch of its own and takes all slices through it, so that no barrier
 // and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
-// 64 us at 56x56, batch 64, against 32.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
-// instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice).
-// What bounds it: with a patch per wave vector issue - some 650 instructions per slice of 8x8 outputs at stride 1, 70 of them per 32
-// expanded positions, 55 to 64 % of a CU's busy time at batch 64; with a shared patch the chain launch - region - slices - sum
-// (vector issue 35 to 44 %).
-// Measured, the three launches -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at 112x112, stride 2: 44 -> 33 us;
-// 24 -> 144 -> 24 at 56x56: 38 -> 32; 32 -> 192 -> 32 at 28x28: 16.4 -> 14.6; 64 -> 384 -> 64 at 14x14: 13.4 -> 11.2; batch 1:
-// 8.3 .. 9.6 -> 4.1 .. 6.0.
+// 55 us at 56x56, batch 64, against 26.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
+// instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice; but a wave of 8x8 outputs
+// with a patch of its own holds 100 registers where one of 4x8 holds 60: 28.4 us against 26.2 for that block, 13.3 against 11.2 for
+// 32 -> 192 -> 32 at 28x28).
+// What bounds it: vector issue - with a patch per wave three quarters of a CU's busy time at batch 64, the requantisations first;
+// with a shared patch the chain launch - region - slices - sum as well.
+// Measured, the three launches -> the depthwise layer as dot products -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at
+// 112x112, stride 2: 60 -> 33 -> 27.6 us; 24 -> 144 -> 24 at 56x56: 39 -> 33 -> 26.2; 24 -> 144 -> 32, stride 2: 27 -> 20 -> 15.6;
+// 32 -> 192 -> 32 at 28x28: 19.5 -> 14.6 -> 11.2; 64 -> 384 -> 64 at 14x14: 14.9 -> 12 -> 10.3; 96 -> 576 -> 96: 18.3 -> 17.3 -> 14.4;
+// batch 1 (2x4): 8.3 .. 9.6 -> 4.1 .. 6.0.
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
 // requantisations, at most 160 input and output channels; with the add stride 1 and as many output as input channels.
 #include "conv_invres.h"
@@ -43,7 +49,7 @@ using namespace frag;
 namespace {
 
 // waves of a work-group: three per SIMD leave each 168 registers, where that is enough for a shape's accumulators
-constexpr int max_waves(int PT, int CT) { return PT > 1 || CT > 4 ? 8 : 12; }
+constexpr int max_waves(int TILES, int PT, int NK, int CT) { return PT > 1 || CT > 4 || (TILES > 1 && CT > 2 && (TILES > 4 || NK > 2)) ? 8 : 12; }
 
 struct InvresGeom {
     int PY, PX; // patches per image
@@ -54,13 +60,17 @@ struct InvresGeom {
     int wave_bytes; // bytes of a wave's own buffers
 };
 
-// S: stride, PH x PW: output pixels of a patch (PW a multiple of 4).  Rows and columns of the input region, columns in whole
-// runs of four; tiles of 32 positions; pixel tiles of 32 outputs.
+// S: stride, PH x PW: output pixels of a patch.  Rows and columns of the input region; tiles of 32 positions; pixel tiles of 32
+// outputs.
+// MATRIX: the depthwise layer as diagonal matrices, for patches that fill a multiply's 32 columns; otherwise as dot products, with the
+// region's rows in whole runs of four columns.
 template <int S, int PH_, int PW_>
 struct Patch {
-    static constexpr int PH = PH_, PW = PW_, RH = S * (PH - 1) + 3, QW = (S * (PW - 1) + 3 + 3) / 4, RW = 4 * QW;
-    static constexpr int NQ = RH * QW, TILES = (NQ + 7) / 8, PT = (PH * PW + 31) / 32;
-    static constexpr int E_BYTES = TILES * 8 * 128, D_BYTES = PT * 1024, MASK_BYTES = TILES * 8 * 4;
+    static constexpr int PH = PH_, PW = PW_;
+    static constexpr bool MATRIX = PH * PW >= 32;
+    static constexpr int QW = (S * (PW - 1) + 3 + 3) / 4, RH = S * (PH - 1) + 3, RW = MATRIX ? S * (PW - 1) + 3 : 4 * QW, NP = RH * RW;
+    static constexpr int TILES = (NP + 31) / 32, PT = (PH * PW + 31) / 32;
+    static constexpr int E_BYTES = TILES * 1024, D_BYTES = MATRIX ? 0 : PT * 1024, MASK_BYTES = MATRIX ? 0 : TILES * 32;
 };
 
 __device__ static __forceinline__ void lds_order()
@@ -83,17 +93,49 @@ __device__ static __forceinline__ int32_t dot4_from(uint32_t a, int32_t b, int32
     return d;
 }
 
+// 16 accumulators (16 consecutive channels of a position) -> their bytes, re-centred (XOR 0x80 = 128 less, as signed bytes).  The rounding
+// and the zero point ride along as the high word of a 64-bit multiply-add (v_mad_i64_i32 takes 4.4 clocks, v_mul_hi_i32 and the
+// addition 8 where few waves share a SIMD; the zero of the low word is hidden from the compiler, which would take the sum apart
+// again), and the last shift saturates to signed bytes, which have the 128 in the constants: 5 to 8 % of these kernels, which issue
+// vector instructions for three quarters of their time.
+__device__ static __forceinline__ v4i requant_centred(const ConvArgs &a, const v16i &s)
+{
+    uint32_t zero = 0;
+    asm("" : "+v"(zero));
+    const uint64_t add = (uint64_t)(uint32_t)(a.qadd - (128 << a.qt)) << 32 | zero;
+    const int32_t plo = (a.lo - 128) * (1 << a.qt), phi = ((a.q.hi - 127) * (1 << a.qt)) - 1;
+    v4i o;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        int32_t r[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            r[k] = (int32_t)(((uint64_t)((int64_t)s[4 * g + k] * (int)a.q.mult) + add) >> 32);
+            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r[k]) : "v"(r[k]), "s"(plo), "v"(phi));
+        }
+        uint32_t b;
+        asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(b) : "v"(r[0]), "v"(r[1]), "s"(a.qt));
+        asm("v_ashr_pk_i8_i32 %0, %1, %2, %3 op_sel:[0,0,0,1]" : "+v"(b) : "v"(r[2]), "v"(r[3]), "s"(a.qt));
+        o[g] = (int)b;
+    }
+    // a matrix instruction may read these next, two wait states behind the vector instruction that wrote them at the earliest: the
+    // compiler, which sees to that, does not see what the assembly above writes
+    asm("s_nop 1" : "+v"(o));
+    return o;
+}
+
 } // namespace
 
 // NK: k-steps of 32 input channels; CT: tiles of 32 output channels (both may be more than the layer has: the weights are zeros
 // there).  OWN: every wave has a patch of its own and takes all slices through it; otherwise the waves
 // of a work-group split the slices of one patch.
 template <int S, int PH, int PW, int NK, int CT, bool OWN>
-__global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT)) void conv_invres_kernel(const ConvArgs e, const ConvArgs d, const ConvArgs pr,
+__global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES, Patch<S, PH, PW>::PT, NK, CT)) void conv_invres_kernel(const ConvArgs e, const ConvArgs d, const ConvArgs pr,
                                                                                 const InvresGeom geo)
 {
     using G = Patch<S, PH, PW>;
-    constexpr int RH = G::RH, QW = G::QW, NQ = G::NQ, TILES = G::TILES, RW = G::RW, PT = G::PT;
+    constexpr int RH = G::RH, RW = G::RW, NP = G::NP, TILES = G::TILES, PT = G::PT, QW = G::QW;
+    constexpr bool MATRIX = G::MATRIX;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
@@ -111,27 +153,48 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT
     const int iy0 = S * oy0 - 1, ix0 = S * ox0 - 1; // the region's first row and column
     const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + RH <= e.H && ix0 + RW <= e.W; // no position to replace
     uint8_t *const xbuf = lds + (OWN ? wave * (geo.region + geo.wave_bytes) : 0);
-    uint32_t *const masks = reinterpret_cast<uint32_t *>(xbuf + geo.region - G::MASK_BYTES); // which bytes of a run lie inside the image
-    uint8_t *const ebuf = xbuf + geo.region + (OWN ? 0 : wave * geo.wave_bytes), *const dbuf = ebuf + G::E_BYTES;
+    uint32_t *const masks = reinterpret_cast<uint32_t *>(xbuf + geo.region - G::MASK_BYTES); // dot products: which bytes of a run lie inside the image
+    uint8_t *const ebuf = xbuf + geo.region + (OWN ? 0 : wave * geo.wave_bytes);
 
     // ---- a slice's weights and constants, each loaded as soon as the slice before has used its own
     v4i we[NK], wp[CT];
-    int ebias, dbias, wa[3], wb[3];
+    // MATRIX: the folded biases of the lane's 16 consecutive channels, and the depthwise weights of the channel that its row of a multiply
+    // stands for, a kernel row each; otherwise biases and weights of the channel that its column stands for, the weights in both
+    // alignments
+    v16i ebias, dbias;
+    int ebias1, dbias1, wd[3], wb[3];
     auto load_e = [&](int T) {
-        ebias = e.bias2[32 * T + ch];
+        if constexpr (MATRIX)
+            init_acc(ebias, e.bias2 + 32 * T + 16 * h, false);
+        else
+            ebias1 = e.bias2[32 * T + ch];
 #pragma unroll
         for (int kk = 0; kk < NK; kk++)
             we[kk] = kk == 0 || kk < geo.nk ? ldg128(e.wfrag1 + ((size_t)((kk >> 1) * (e.kout_pad >> 5) + T) * 2 + (kk & 1)) * 1024 + lane * 16)
                                             : v4i{0, 0, 0, 0};
     };
+    // the matrix of a tap is diagonal: the row's own channel's weight, where this lane's half of the columns has that channel
+    const bool diagonal = (ch >> 4) == h;
+    uint32_t sel[3], dm[4]; // byte s of a dword to the channel's place in its dword; which of the four dwords that is
+#pragma unroll
+    for (int s = 0; s < 3; s++)
+        sel[s] = 0x0c0c0c0cu ^ ((0x0cu ^ s) << (8 * (ch & 3)));
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        dm[j] = diagonal && ((ch & 15) >> 2) == j ? ~0u : 0u;
+        asm("" : "+v"(dm[j])); // masks in registers: an AND each, not a select
+    }
     auto load_d = [&](int T) {
-        const int cd = min(32 * T + ch, d.in_cs - 1); // the last slice may be half empty; its products meet zero weights
-        dbias = d.bias2[cd];
+        const int c0 = min(32 * T + 16 * h, d.in_cs - 16), cd = min(32 * T + ch, d.in_cs - 1); // the last slice may be half empty; its products meet zero weights
+        if constexpr (MATRIX)
+            init_acc(dbias, d.bias2 + c0, false);
+        else
+            dbias1 = d.bias2[cd];
         const int *wt = reinterpret_cast<const int *>(d.wpack) + cd;
 #pragma unroll
         for (int r = 0; r < 3; r++) {
-            wa[r] = wt[(r * 2 + 0) * d.in_cs];
-            if (S == 1)
+            wd[r] = wt[(r * 2 + 0) * d.in_cs];
+            if (!MATRIX && S == 1)
                 wb[r] = wt[(r * 2 + 1) * d.in_cs];
         }
     };
@@ -144,26 +207,39 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT
     int T = OWN ? 0 : wave;
     const int dT = OWN ? 1 : nw; // never more waves than slices
 
-    // ---- the input region -> LDS, re-centred; positions outside the image are never used (the masks below)
+    // ---- the input region -> LDS, re-centred; positions outside the image are never used (the mask below)
     {
         const int tid = OWN ? lane : (int)threadIdx.x, nthr = OWN ? 64 : (int)blockDim.x;
         const int pieces = e.in_cs >> 4, inv = 65536 / pieces + 1; // id / pieces == (id * inv) >> 16: id < 4096, pieces <= 10
-        for (int id = tid; id < RH * RW * pieces; id += nthr) {
+        for (int id = tid; id < NP * pieces; id += nthr) {
             const int px = (id * inv) >> 16, c = id - px * pieces, ry = px / RW, rx = px - ry * RW;
             const int iy = iy0 + ry, ix = ix0 + rx;
             if ((unsigned)iy < (unsigned)e.H && (unsigned)ix < (unsigned)e.W)
                 *reinterpret_cast<v4i *>(xbuf + px * geo.xrow + c * 16)
                     = ldg128(e.x + (uint32_t)(((n * e.H + iy) * e.W + ix) * e.in_cs + c * 16)) ^ (int)0x80808080;
         }
-        if (!inside)
-            for (int q = tid; q < TILES * 8; q += nthr) {
-                const int ry = q / QW, rx = (q - ry * QW) * 4, iy = iy0 + ry;
-                uint32_t m = 0;
-                if (q < NQ && (unsigned)iy < (unsigned)e.H)
-                    for (int b = 0; b < 4; b++)
-                        m |= (unsigned)(ix0 + rx + b) < (unsigned)e.W ? 0xffu << (8 * b) : 0u;
-                masks[q] = m;
-            }
+    }
+    if (!MATRIX && !inside)
+        for (int q = (OWN ? lane : (int)threadIdx.x); q < TILES * 8; q += OWN ? 64 : (int)blockDim.x) {
+            const int ry = q / QW, rx = (q - ry * QW) * 4, iy = iy0 + ry;
+            uint32_t m = 0;
+            if (q < RH * QW && (unsigned)iy < (unsigned)e.H)
+                for (int b = 0; b < 4; b++)
+                    m |= (unsigned)(ix0 + rx + b) < (unsigned)e.W ? 0xffu << (8 * b) : 0u;
+            masks[q] = m;
+        }
+    uint32_t outside = 0; // bit t: the lane's position of tile t lies outside the image
+    if (MATRIX && !inside)
+#pragma unroll
+        for (int t = 0; t < TILES; t++) {
+            const int pos = 32 * t + p, ry = pos / RW;
+            outside |= (unsigned)(iy0 + ry) < (unsigned)e.H && (unsigned)(ix0 + pos - ry * RW) < (unsigned)e.W ? 0u : 1u << t;
+        }
+    int first[PT]; // the lane's outputs 32 t + p: their first tap in the expanded region
+#pragma unroll
+    for (int t = 0; t < PT; t++) {
+        const int m = min(32 * t + p, PH * PW - 1);
+        first[t] = (S * (m / PW) * RW + S * (m % PW)) * 32 + 16 * h;
     }
     load_e(T);
     load_d(T);
@@ -176,7 +252,7 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT
             // OWN: the accumulators start at the folded bias of the lane's 16 consecutive channels
             init_acc(acc[ct][t], pr.bias2 + 32 * (ct < geo.ct ? ct : 0) + 16 * h, !OWN);
         }
-    const uint32_t epad = d.padword ^ 0x80808080u;
+    const int epad = (int)(d.padword ^ 0x80808080u);
     if (OWN)
         lds_order();
     else
@@ -184,79 +260,124 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::PT, CT
 
     for (; T < geo.nT; T += dT) {
         const int Tn = min(T + dT, geo.nT - 1); // past the end: harmless loads
-        // ---- expand
-        auto expand = [&](auto whole) {
+        v4i b[PT]; // the depthwise layer's bytes, as the last layer's pixel operand
+        if constexpr (MATRIX) {
+            // ---- expand: a lane's 16 channels of a position are 16 bytes of the position's row
+            auto expand = [&](auto whole) {
 #pragma unroll (TILES <= 4 ? TILES : 2)
-            for (int t = 0; t < TILES; t++) {
-                v16i a;
-                const uint8_t *row = xbuf + (32 * t + p) * geo.xrow + 16 * h;
+                for (int t = 0; t < TILES; t++) {
+                    v16i a = ebias;
+                    const uint8_t *row = xbuf + (32 * t + p) * geo.xrow + 16 * h;
 #pragma unroll
-                for (int i = 0; i < 16; i++)
-                    a[i] = ebias;
+                    for (int kk = 0; kk < NK; kk++)
+                        a = __builtin_amdgcn_mfma_i32_32x32x32_i8(we[kk], *reinterpret_cast<const v4i *>(row + 32 * kk), a, 0, 0, 0);
+                    v4i v = requant_centred(e, a);
+                    if (!decltype(whole)::value && (outside >> t & 1))
+                        v = v4i{epad, epad, epad, epad};
+                    *reinterpret_cast<v4i *>(ebuf + (32 * t + p) * 32 + 16 * h) = v;
+                }
+            };
+            if (inside)
+                expand(std::true_type{});
+            else
+                expand(std::false_type{});
+            load_e(Tn);
+            lds_order();
+            // ---- depthwise, on the matrix cores: tap by tap a diagonal matrix times the region's rows at that tap.  The requantised sums
+            // are the pixel operand of the last layer as they are
+            v16i o[PT];
 #pragma unroll
-                for (int kk = 0; kk < NK; kk++)
-                    a = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(row + 32 * kk), we[kk], a, 0, 0, 0);
+            for (int t = 0; t < PT; t++)
+                o[t] = dbias;
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int q = 8 * t + 2 * g + h;
-                    uint32_t v = conv_requant4<false>(e, a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]) ^ 0x80808080u;
-                    if (!decltype(whole)::value) {
-                        const uint32_t m = masks[q];
-                        v = (v & m) | (epad & ~m);
+            for (int r = 0; r < 3; r++)
+#pragma unroll
+                for (int s = 0; s < 3; s++) {
+                    const uint32_t w = __builtin_amdgcn_perm(0, (uint32_t)wd[r], sel[s]);
+                    const v4i m = {(int)(w & dm[0]), (int)(w & dm[1]), (int)(w & dm[2]), (int)(w & dm[3])};
+#pragma unroll
+                    for (int t = 0; t < PT; t++)
+                        o[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(m, *reinterpret_cast<const v4i *>(ebuf + first[t] + (r * RW + s) * 32), o[t], 0, 0, 0);
+                }
+            load_d(Tn);
+#pragma unroll
+            for (int t = 0; t < PT; t++)
+                b[t] = requant_centred(d, o[t]);
+        } else {
+            // ---- expand, pixels as the rows of the multiply: a lane's accumulators are four runs of four consecutive pixels of its channel
+            auto expand = [&](auto whole) {
+#pragma unroll
+                for (int t = 0; t < TILES; t++) {
+                    v16i a;
+                    const uint8_t *row = xbuf + (32 * t + p) * geo.xrow + 16 * h;
+#pragma unroll
+                    for (int i = 0; i < 16; i++)
+                        a[i] = ebias1;
+#pragma unroll
+                    for (int kk = 0; kk < NK; kk++)
+                        a = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(row + 32 * kk), we[kk], a, 0, 0, 0);
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int q = 8 * t + 2 * g + h;
+                        uint32_t v = conv_requant4<false>(e, a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]) ^ 0x80808080u;
+                        if (!decltype(whole)::value) {
+                            const uint32_t m = masks[q];
+                            v = (v & m) | ((uint32_t)epad & ~m);
+                        }
+                        *reinterpret_cast<uint32_t *>(ebuf + (q * 32 + p) * 4) = v;
                     }
-                    *reinterpret_cast<uint32_t *>(ebuf + (q * 32 + p) * 4) = v;
+                }
+            };
+            if (inside)
+                expand(std::true_type{});
+            else
+                expand(std::false_type{});
+            load_e(Tn);
+            lds_order();
+            // ---- depthwise: half h of the wave takes PH / 2 output rows of this lane's channel
+            constexpr int HR = PH / 2, IR = S * (HR - 1) + 3;
+            uint8_t *const dbuf = ebuf + G::E_BYTES;
+            int32_t o[HR][PW];
+#pragma unroll
+            for (int ir = 0; ir < IR; ir++) {
+                const uint8_t *er = ebuf + ((S * HR * h + ir) * QW * 32 + p) * 4;
+                uint32_t q[QW];
+#pragma unroll
+                for (int i = 0; i < QW; i++)
+                    q[i] = *reinterpret_cast<const uint32_t *>(er + i * 128);
+                uint32_t mid[QW - 1]; // bytes 2, 3 of run i and 0, 1 of run i + 1
+#pragma unroll
+                for (int i = 0; i + 1 < QW; i++)
+                    mid[i] = __builtin_amdgcn_alignbyte(q[i + 1], q[i], 2);
+#pragma unroll
+                for (int r = 0; r < HR; r++) {
+                    const int kr = ir - S * r;
+                    if (kr < 0 || kr > 2)
+                        continue;
+#pragma unroll
+                    for (int x = 0; x < PW; x++) {
+                        const uint32_t v = S == 1 ? ((x & 2) ? mid[x >> 2] : q[x >> 2]) : ((x & 1) ? mid[x >> 1] : q[x >> 1]);
+                        const int w = S == 1 && (x & 1) ? wb[kr] : wd[kr];
+                        o[r][x] = kr == 0 ? dot4_from(v, w, dbias1) : dot4(v, w, o[r][x]);
+                    }
                 }
             }
-        };
-        if (inside)
-            expand(std::true_type{});
-        else
-            expand(std::false_type{});
-        load_e(Tn);
-        lds_order();
-        // ---- depthwise: half h of the wave takes PH / 2 output rows of this lane's channel
-        constexpr int HR = PH / 2, IR = S * (HR - 1) + 3;
-        int32_t o[HR][PW];
+            load_d(Tn);
+            // this lane's channel of its outputs, as bytes of the pixel rows that the last layer multiplies
 #pragma unroll
-        for (int ir = 0; ir < IR; ir++) {
-            const uint8_t *er = ebuf + ((S * HR * h + ir) * QW * 32 + p) * 4;
-            uint32_t q[QW];
+            for (int r = 0; r < HR; r++)
 #pragma unroll
-            for (int i = 0; i < QW; i++)
-                q[i] = *reinterpret_cast<const uint32_t *>(er + i * 128);
-            uint32_t mid[QW - 1]; // bytes 2, 3 of run i and 0, 1 of run i + 1
-#pragma unroll
-            for (int i = 0; i + 1 < QW; i++)
-                mid[i] = __builtin_amdgcn_alignbyte(q[i + 1], q[i], 2);
-#pragma unroll
-            for (int r = 0; r < HR; r++) {
-                const int kr = ir - S * r;
-                if (kr < 0 || kr > 2)
-                    continue;
-#pragma unroll
-                for (int x = 0; x < PW; x++) {
-                    const uint32_t v = S == 1 ? ((x & 2) ? mid[x >> 2] : q[x >> 2]) : ((x & 1) ? mid[x >> 1] : q[x >> 1]);
-                    const int w = S == 1 && (x & 1) ? wb[kr] : wa[kr];
-                    o[r][x] = kr == 0 ? dot4_from(v, w, dbias) : dot4(v, w, o[r][x]);
+                for (int x4 = 0; x4 < PW; x4 += 4) {
+                    const uint32_t v = conv_requant4<false>(d, o[r][x4], o[r][x4 + 1], o[r][x4 + 2], o[r][x4 + 3]) ^ 0x80808080u;
+                    uint8_t *to = dbuf + (((HR * h + r) * PW + x4) * 32) + ch;
+                    to[0] = (uint8_t)v, to[32] = (uint8_t)(v >> 8), to[64] = (uint8_t)(v >> 16), to[96] = (uint8_t)(v >> 24);
                 }
-            }
+            lds_order();
+#pragma unroll
+            for (int t = 0; t < PT; t++)
+                b[t] = *reinterpret_cast<const v4i *>(dbuf + (32 * t + p) * 32 + 16 * h);
         }
-        load_d(Tn);
-        // this lane's channel of its outputs, as bytes of the pixel rows that the last layer multiplies
-#pragma unroll
-        for (int r = 0; r < HR; r++)
-#pragma unroll
-            for (int x4 = 0; x4 < PW; x4 += 4) {
-                const uint32_t v = conv_requant4<false>(d, o[r][x4], o[r][x4 + 1], o[r][x4 + 2], o[r][x4 + 3]) ^ 0x80808080u;
-                uint8_t *to = dbuf + (((HR * h + r) * PW + x4) * 32) + ch;
-                to[0] = (uint8_t)v, to[32] = (uint8_t)(v >> 8), to[64] = (uint8_t)(v >> 16), to[96] = (uint8_t)(v >> 24);
-            }
-        lds_order();
         // ---- project: one k-step of every channel tile (rows past the patch, where it has fewer than 32 pixels, are never stored)
-        v4i b[PT];
-#pragma unroll
-        for (int t = 0; t < PT; t++)
-            b[t] = *reinterpret_cast<const v4i *>(dbuf + (32 * t + p) * 32 + 16 * h);
 #pragma unroll
         for (int ct = 0; ct < CT; ct++)
 #pragma unroll
@@ -327,7 +448,7 @@ Channels channels_of(const ConvArgs &e, const ConvArgs &p)
     return {5, 5};
 }
 
-enum Shape { k2x4, k4x8, k8x8, kOwn, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2
+enum Shape { k2x4, k4x8, k8x8, kOwn, kOwn4, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2; kOwn4: 4x8 at stride 1
 
 // how a launch divides the work
 struct Division {
@@ -341,21 +462,22 @@ Division divide(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int sha
 {
     const Channels c = channels_of(e, p);
     const int S = d.stride_h, ph = shape == k2x4 ? 2 : shape == k8x8 || (shape == kOwn && S == 1) ? 8 : 4, pw = shape == k2x4 ? 4 : 8;
-    const int tiles = ((S * (ph - 1) + 3) * ((S * (pw - 1) + 6) / 4) + 7) / 8, pt = (ph * pw + 31) / 32; // as in Patch
+    const bool matrix = ph * pw >= 32; // these as in Patch
+    const int tiles = ((S * (ph - 1) + 3) * (matrix ? S * (pw - 1) + 3 : (S * (pw - 1) + 6) / 4 * 4) + 31) / 32, pt = (ph * pw + 31) / 32;
     Division v;
     v.PY = (p.OH + ph - 1) / ph, v.PX = (p.OW + pw - 1) / pw;
     v.nT = (d.in_cs + 31) / 32;
     // rows of 16 bytes (the other half of a k-step meets zero weights) and of 32 read without bank conflicts as they are, longer
     // ones 16 bytes apart
     v.xrow = e.in_cs == 16 ? 16 : c.nk == 1 ? 32 : 32 * c.nk + 16;
-    v.region = (tiles * 32 * v.xrow + 16 + tiles * 32 + 15) / 16 * 16;
-    v.wave_bytes = tiles * 1024 + pt * 1024;
+    v.region = (tiles * 32 * v.xrow + 16 + (matrix ? 0 : tiles * 32) + 15) / 16 * 16;
+    v.wave_bytes = tiles * 1024 + (matrix ? 0 : pt * 1024);
     const long long patches = (long long)d.N * v.PY * v.PX;
-    if (shape == kOwn) {
+    if (shape >= kOwn) {
         v.nw = 4, v.rounds = v.nT, v.wgs = (patches + 3) / 4;
         v.lds = (unsigned)(4 * (v.region + v.wave_bytes));
     } else {
-        v.nw = std::min(v.nT, max_waves(pt, c.ct));
+        v.nw = std::min(v.nT, max_waves(tiles, pt, c.nk, c.ct));
         while (v.region + v.nw * v.wave_bytes > 160 * 1024)
             v.nw--; // one wave needs at most 14 KB beside 63 KB of pixels
         v.rounds = (v.nT + v.nw - 1) / v.nw;
@@ -374,37 +496,37 @@ void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
     InvresGeom geo;
     geo.PY = v.PY, geo.PX = v.PX, geo.nT = v.nT, geo.xrow = v.xrow, geo.region = v.region, geo.wave_bytes = v.wave_bytes;
     geo.nk = (e.in_cs + 31) / 32, geo.ct = (p.out_cs + 31) / 32;
-    static_assert(G::E_BYTES == G::TILES * 1024 && G::D_BYTES == G::PT * 1024 && G::MASK_BYTES == G::TILES * 32, "divide()");
+    static_assert(G::E_BYTES == G::TILES * 1024, "divide()");
     hipLaunchKernelGGL((conv_invres_kernel<S, PH, PW, NK, CT, OWN>), dim3((unsigned)((v.wgs + 7) / 8 * 8)), dim3(64 * v.nw), v.lds, st, e, d, p, geo);
 }
 
 // ---- the shapes, and what each takes
 
-// Time by shape, in us, fitted to 160 blocks (1 to 128 images of 3x3 to 130x130, the channel counts of mobile networks; nine in ten
-// within 21 % of the fit, all within 33).  A launch; for every generation of resident work-groups its start and end; for every
-// slice that a wave then takes its chain, alone, per channel tile and per k-step; and the slices per SIMD of the chip, which
-// share the vector units.  How many work-groups a CU holds decides: the fit before this one knew only patches per CU, which is
-// right where nine small work-groups fit one, and picked shapes up to 1.7 times slower than the three launches from 64 channels
-// on (18 images of 20x103, 64 -> 384 -> 96: 34 against 25 us).
+// Time by shape, in us, fitted to 460 blocks (1 to 128 images of 3x3 to 130x130, the channel counts of mobile networks; nine in ten
+// within 20 % of the fit).  A launch; for every generation of resident work-groups its start and end; for every
+// slice that a wave then takes its chain, alone, per channel tile and per k-step; and per SIMD of the chip the slices and the patches,
+// which share the vector units.
 double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    // launch, slice, slice x channel tiles, slice x k-steps, slices per SIMD, generation
-    static const double kCost[2][kShapes][6] = {
-        {{2.87, 0, 0.323, 0, 0.473, 1.00}, {2.07, 0, 0.498, 0.016, 0.572, 2.71}, {2.45, 0.701, 0.825, 0.135, 0.225, 2.56}, {0, 1.362, 0.224, 0.117, 0.581, 3.26}},
-        {{2.17, 0, 0.368, 0.035, 0.394, 2.06}, {3.46, 0, 0.540, 0.268, 0.946, 1.75}, {}, {1.86, 1.663, 0.076, 0.302, 0.533, 1.00}}};
+    // launch, slice, slice x channel tiles, slice x k-steps, slices per SIMD, generation, patches per SIMD
+    static const double kCost[2][kShapes][7] = {
+        {{2.909, 0, 0.325, 0, 0.461, 1.071, 0}, {1.845, 0, 0.445, 0, 0.479, 2.666, 0}, {2.087, 0.323, 0.783, 0.128, 0.253, 2.985, 0},
+         {1.250, 1.240, 0.226, 0.058, 0.298, 2.046, 0.956}, {1.197, 0.605, 0.123, 0.129, 0.279, 1.566, 0.504}},
+        {{2.287, 0, 0.368, 0.016, 0.382, 1.932, 0}, {2.669, 0, 0.465, 0.148, 0.832, 2.360, 0}, {}, {2.845, 1.062, 0.146, 0.186, 0.096, 0.266, 1.780}, {}}};
     const int s = d.stride_h;
     const Channels c = channels_of(e, p);
-    if ((shape == kOwn && (c.nk > 2 || c.ct > 2)) || (shape == k8x8 && (s == 2 || c.ct > 3)))
+    if ((shape >= kOwn && (c.nk > 2 || c.ct > 2)) || (shape == kOwn4 && s == 2) || (shape == k8x8 && (s == 2 || c.ct > 3)))
         return 1e30; // not built: the accumulators or the region would be too much for a wave
     const Division v = divide(e, d, p, shape);
     // waves per SIMD that the registers allow
-    const int waves = shape == kOwn ? (s == 2 ? 4 : c.ct == 1 ? 3 : 2) : max_waves(shape == k8x8 ? 2 : 1, c.ct) / 4;
+    const int waves = shape == kOwn4 || (shape == kOwn && s == 2) ? (c.ct == 1 ? 4 : 3)
+        : shape == kOwn ? (c.ct == 1 ? 3 : 2) : max_waves(shape == k2x4 ? s : s == 1 ? 2 : 5, shape == k8x8 ? 2 : 1, c.nk, c.ct) / 4;
     const int held = std::max(1, std::min((int)(160 * 1024 / v.lds), 4 * waves / v.nw)); // work-groups of a CU
     const double gens = (double)((v.wgs + 256 * held - 1) / (256 * held)), steps = gens * v.rounds;
     const double patches = (double)d.N * v.PY * v.PX;
-    const double f[6] = {1, steps, steps * c.ct, steps * c.nk, patches * v.nT / 1024, gens};
+    const double f[7] = {1, steps, steps * c.ct, steps * c.nk, patches * v.nT / 1024, gens, patches / 1024};
     double t = 0;
-    for (int i = 0; i < 6; i++)
+    for (int i = 0; i < 7; i++)
         t += kCost[s - 1][shape][i] * f[i];
     return t;
 }
@@ -427,9 +549,13 @@ int choose_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wa
 template <int S, int NK, int CT>
 void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape, hipStream_t st)
 {
-    if constexpr (NK <= 2 && CT <= 2)
+    if constexpr (NK <= 2 && CT <= 2) {
         if (shape == kOwn)
             return launch_shape<S, S == 1 ? 8 : 4, 8, NK, CT, true>(e, d, p, shape, st);
+        if constexpr (S == 1)
+            if (shape == kOwn4)
+                return launch_shape<1, 4, 8, NK, CT, true>(e, d, p, shape, st);
+    }
     if constexpr (S == 1 && CT <= 3)
         if (shape == k8x8)
             return launch_shape<S, 8, 8, NK, CT, false>(e, d, p, shape, st);
@@ -474,14 +600,14 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
         && e.N == d.N && e.OH == d.H && e.OW == d.W && (long long)e.P * e.in_cs < (1ll << 31);
 }
 
-// The three launches: their latencies, the hidden tensor's bytes at both resolutions, the expanding layer's products (fitted to
-// the same blocks, within 20 %, one 24).  Chosen by this the 160 blocks take 0.6 % more than the best choice would on average, one
-// in twenty more than 3 %, the worst 31 % (3.0, 18 and 73 % by the fits before); 180 blocks that the fits have not seen 0.75, 4
-// and 22 % (1.5, 10 and 39 %).
+// The three launches: their latencies, the hidden tensor's bytes at the output's resolution, the products of both 1x1 layers (fitted to
+// the same blocks, nine in ten within 10 %).  Chosen by this the 460 blocks take 1.4 % more than the best choice would on average, one
+// in twenty more than 9 %, one in a hundred 23 %.
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
-    const double apart = d.stride_h == 1 ? 8.55 + 0.790 * wide + 0.00403 * wide * e.in_cs : 8.78 + 1.437 * narrow + 0.00502 * wide * e.in_cs;
+    const double apart = d.stride_h == 1 ? 8.40 + 0.953 * narrow + 0.00326 * wide * e.in_cs + 0.00191 * narrow * p.out_cs
+                                         : 8.74 + 2.163 * narrow + 0.00291 * wide * e.in_cs + 0.00176 * narrow * p.out_cs;
     double us;
     choose_shape(e, d, p, -1, &us);
     return us < apart;
@@ -489,7 +615,7 @@ bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs 
 
 const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted)
 {
-    static const char *const kPatch[kShapes] = {"2x4", "4x8", "8x8", "own"};
+    static const char *const kPatch[kShapes] = {"2x4", "4x8", "8x8", "own", "own4x8"};
     static thread_local char nm[48];
     double us;
     const int shape = choose_shape(e, d, p, wanted, &us);

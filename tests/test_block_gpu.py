@@ -619,3 +619,37 @@ def test_inverted_residual_every_kernel(case):
             want = orc.add_u8(t, x, a, z, 0.03, 77, 0.05, 20)
             y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (False, 0.05, 20))
             assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
+
+
+@pytest.mark.parametrize("hw", [(13, 11), (4, 8), (3, 2)], ids=lambda v: "%dx%d" % v)
+@pytest.mark.parametrize("case", [(1, 1, 24, 24), (1, 2, 24, 40), (2, 2, 40, 60)], ids=lambda c: "k%d_n%d" % c[:2])
+def test_inverted_residual_half_patch_per_wave(case, hw):
+    """A patch of 4x8 outputs per wave: overhanging on two sides, exactly one, smaller than one; 5 images, so that the last
+    work-group has idle waves; three slices, the last partial; with the add where the channels allow it."""
+    nk, ct, ci, co = case
+    rng = np.random.default_rng(ci + co + hw[0])
+    x = rng.integers(0, 256, (5, ci, *hw), dtype=np.uint8)
+    t, a, z, plans = x, 0.03, 77, []
+    for k, (C, K, R, group) in enumerate(((ci, 80, 1, 1), (80, 80, 3, 80), (80, co, 1, 1))):
+        w = rng.integers(1, 256, (K, C // group, R, R), dtype=np.uint8)
+        sigma = 74.0 * 74.0 * math.sqrt(w[0].size) * (0.7 if k else 1.0)
+        b = rng.integers(-int(sigma), int(sigma) + 1, K).astype(np.int32)
+        oa = float(np.float32(0.03 * rng.uniform(0.75, 1.35)))
+        q = (a, z, float(np.float32(oa * 45.0 / (a * sigma))), 128, oa, 30 if k < 2 else 120)
+        plans.append(hipq.Conv2d(t.shape, w, b, R // 2, 1, group, *q, relu=k < 2))
+        t = orc.conv2d_u8(t, w, b, R // 2, 1, group, *q)
+        if k < 2:
+            t = np.maximum(t, q[5]).astype(np.uint8)
+        a, z = q[4], q[5]
+    plans[2].special(2)
+    hipq.inverted_residual_select(plans[2], 4)
+    name = hipq.inverted_residual_kernel(*plans)
+    assert name == "conv_invres_s1_own4x8_k%d_n%d" % (nk, ct), name
+    print(name, hw, flush=True)
+    xd = hipq.to_device_nhwc(x)
+    got = hipq.from_device_nhwc(hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99)), co)
+    assert np.array_equal(got, t), (name, int((got != t).sum()))
+    if ci == co:
+        want = orc.add_u8(t, x, a, z, 0.03, 77, 0.05, 20)
+        y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (False, 0.05, 20))
+        assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
