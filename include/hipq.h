@@ -321,6 +321,27 @@ int hipq_inverted_residual_run(const hipq_conv2d_plan *expand, const hipq_conv2d
 int hipq_inverted_residual_select(hipq_conv2d_plan *project, int shape);
 const char *hipq_inverted_residual_kernel(const hipq_conv2d_plan *expand, const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *project);
 
+
+/*
+ * A depthwise 3x3 layer and the 1x1 / stride 1 layer that reads it in one launch, with the add behind them where `residual` is not
+ * null: bit-identical to hipq_conv2d_run (hipq_conv2d_run_relu where `relu` is set, for the depthwise layer) twice and hipq_add_u8
+ * (src/op/conv_2d_uint8_impl.c:39-165, src/op/add.c:83-148); the tensor in between never travels to memory.  The requirements
+ * on the layers are those of hipq_inverted_residual_run, for any number of channels; the residual (scale ralpha, zero point rzp)
+ * has the output's shape.  y must not be x; it may be the residual.
+ * hipq_depthwise_point_fusable answers (1 / 0) whether the plans run this way (by rule where it is faster;
+ * hipq_conv2d_plan_special(point, 2): wherever it can); hipq_depthwise_point_run fails with an error otherwise.
+ * hipq_depthwise_point_select: tuning hook, the division of the work by index, -1 by cost (also where that one is not built for the
+ * stride), with identical results; hipq_depthwise_point_kernel names what runs, conv_dwpoint_s<stride>_[narrow]<4 | 8>x8_n<channel
+ * tiles of a work-group>.
+ */
+int hipq_depthwise_point_fusable(const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *point, int add, int residual_is_input0,
+                                 float ralpha, int rzp, float oalpha, int ozp, int obits);
+int hipq_depthwise_point_run(const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *point, const void *x, int relu,
+                             const void *residual, int residual_is_input0, float ralpha, int rzp, float oalpha, int ozp, int obits,
+                             void *y, void *stream);
+int hipq_depthwise_point_select(hipq_conv2d_plan *point, int shape);
+const char *hipq_depthwise_point_kernel(const hipq_conv2d_plan *depthwise, const hipq_conv2d_plan *point);
+
 /*
  * The rest of a bottleneck block in one launch, from its 3x3 convolution on: y = add(widen(mid(x)), residual) and, when
  * `next` is not NULL, y_next = next(y) - bit-identical to hipq_conv2d_run(mid, x, t), hipq_conv2d_run_add(widen, t,

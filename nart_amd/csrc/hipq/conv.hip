@@ -59,6 +59,7 @@
 #include "conv_expand.h"
 #include "conv_dw.h"
 #include "conv_hreg.h"
+#include "conv_dwpoint.h"
 #include "conv_invres.h"
 #include "conv_resident.h"
 #include "conv_rows.h"
@@ -1308,6 +1309,7 @@ struct hipq_conv2d_plan {
     int stages = 0; // load stages of the DMA kernel; 0 = the built-in rule
     int special = 1; // the halo-tile and pointwise kernels: 0 never, 1 built-in rule, 2 wherever they apply
     bool tile_selected = false;     // hipq_conv2d_plan_select named a tile: the tile kernels, not the streaming kernel
+    int dwpoint_shape = -1; // the same of the depthwise layer and this plan as one kernel (hipq_depthwise_point_select)
     int invres_shape = -1; // patch shape of the inverted residual block this plan projects (hipq_inverted_residual_select); -1: by cost
     ResidentShape resident = {0, 0, 0, 0}, resident_add = {0, 0, 0, 0}; // of conv_resident_kernel, without and with a residual; mb = 0: another kernel
     bool resident_named = false;           // by the caller (hipq_conv2d_plan_resident)
@@ -2384,6 +2386,69 @@ extern "C" int hipq_inverted_residual_select(hipq_conv2d_plan *pp, int shape)
 extern "C" const char *hipq_inverted_residual_kernel(const hipq_conv2d_plan *pe, const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp)
 {
     return hipq_inverted_residual_fusable(pe, pd, pp, 0, 0, 1.0f, 0, 8) ? conv_invres_name(pe->args, pd->args, pp->args, pp->invres_shape) : "";
+}
+
+// the launch arguments of a depthwise layer and the 1x1 layer behind it (hipq_depthwise_point_run); false if the add's scales are
+// outside the fixed-point range or the second layer does not read what the first one writes
+static bool dwpoint_args(const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, int relu, int add, int residual_is_input0, float ralpha, int rzp,
+                         float oalpha, int ozp, int obits, ConvArgs *ad, ConvArgs *ap)
+{
+    if (pp->d.izp != pd->d.ozp || pp->d.ialpha != pd->d.oalpha)
+        return false;
+    *ad = pd->args, *ap = pp->args;
+    if (add
+        && (obits != 8 || ozp < 0 || ozp > 255 || rzp < 0 || rzp > 255
+            || !add_args(pp, residual_is_input0, ralpha, rzp, oalpha, ozp, obits, ap)))
+        return false;
+    if (relu) // the ReLU clamp, as in hipq_conv2d_run_relu
+        ad->lo = std::min(pd->d.ozp, ad->q.hi);
+    return true;
+}
+
+extern "C" int hipq_depthwise_point_fusable(const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, int add, int residual_is_input0, float ralpha,
+                                            int rzp, float oalpha, int ozp, int obits)
+{
+    for (const hipq_conv2d_plan *p : {pd, pp})
+        if (!p || p->d.dtype != HIPQ_DTYPE_U8 || p->d.obits != 8
+            || (p == pd ? p->variant != kDepthwise3x3 : p->variant != kMfma || !p->special || p->tile_selected))
+            return 0;
+    ConvArgs ad, ap;
+    if (!dwpoint_args(pd, pp, 0, add, residual_is_input0, ralpha, rzp, oalpha, ozp, obits, &ad, &ap))
+        return 0;
+    return conv_dwpoint_applies(ad, ap) && (pp->special == 2 || conv_dwpoint_us(ad, ap) < conv_dwpoint_apart_us(ad, ap)) ? 1 : 0;
+}
+
+extern "C" int hipq_depthwise_point_run(const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp, const void *x, int relu, const void *residual,
+                                        int residual_is_input0, float ralpha, int rzp, float oalpha, int ozp, int obits, void *y, void *stream)
+{
+    clear_error();
+    HIPQ_REQUIRE(pd && pp && x && y, "hipq_depthwise_point_run: null argument");
+    HIPQ_REQUIRE(x != y, "hipq_depthwise_point_run: the output cannot overwrite the input (neighbouring patches read it)");
+    const int add = residual != nullptr;
+    HIPQ_REQUIRE(hipq_depthwise_point_fusable(pd, pp, add, residual_is_input0, ralpha, rzp, oalpha, ozp, obits),
+                 "hipq_depthwise_point_run: these plans (%s, %s) do not run as one kernel: run the operators separately", pd->name.c_str(),
+                 pp->name.c_str());
+    ConvArgs ad, ap;
+    dwpoint_args(pd, pp, relu, add, residual_is_input0, ralpha, rzp, oalpha, ozp, obits, &ad, &ap);
+    ad.x = static_cast<const uint8_t *>(x);
+    ap.res = static_cast<const uint8_t *>(residual);
+    ap.y = static_cast<uint8_t *>(y);
+    launch_conv_dwpoint(ad, ap, pp->dwpoint_shape, static_cast<hipStream_t>(stream));
+    return launch_status("conv_dwpoint_kernel");
+}
+
+extern "C" int hipq_depthwise_point_select(hipq_conv2d_plan *pp, int shape)
+{
+    clear_error();
+    HIPQ_REQUIRE(pp && shape >= -1 && shape < conv_dwpoint_shapes(), "hipq_depthwise_point_select: null plan, or shape %d outside -1..%d", shape,
+                 conv_dwpoint_shapes() - 1);
+    pp->dwpoint_shape = shape;
+    return 0;
+}
+
+extern "C" const char *hipq_depthwise_point_kernel(const hipq_conv2d_plan *pd, const hipq_conv2d_plan *pp)
+{
+    return hipq_depthwise_point_fusable(pd, pp, 0, 0, 1.0f, 0, 1.0f, 0, 8) ? conv_dwpoint_name(pd->args, pp->args, pp->dwpoint_shape) : "";
 }
 
 extern "C" int hipq_bottleneck_conv_fusable(const hipq_conv2d_plan *p1, const hipq_conv2d_plan *p2, const hipq_conv2d_plan *p3,

@@ -40,7 +40,8 @@
 
 #include <algorithm>
 
-#include "conv_frag.h"
+#include "conv_dw_frag.h"
+#include "conv_dwpoint.h"
 
 namespace hipq {
 
@@ -73,13 +74,6 @@ struct Patch {
     static constexpr int E_BYTES = TILES * 1024, D_BYTES = MATRIX ? 0 : PT * 1024, MASK_BYTES = MATRIX ? 0 : TILES * 32;
 };
 
-__device__ static __forceinline__ void lds_order()
-{
-    // a wave's LDS instructions execute in the order they are issued; this keeps the compiler to it
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __device__ static __forceinline__ int32_t dot4(uint32_t a, int b, int32_t c)
 {
     return __builtin_amdgcn_sdot4((int)a, b, c, false);
@@ -91,37 +85,6 @@ __device__ static __forceinline__ int32_t dot4_from(uint32_t a, int32_t b, int32
     int32_t d;
     asm("v_dot4_i32_i8 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
     return d;
-}
-
-// 16 accumulators (16 consecutive channels of a position) -> their bytes, re-centred (XOR 0x80 = 128 less, as signed bytes).  The rounding
-// and the zero point ride along as the high word of a 64-bit multiply-add (v_mad_i64_i32 takes 4.4 clocks, v_mul_hi_i32 and the
-// addition 8 where few waves share a SIMD; the zero of the low word is hidden from the compiler, which would take the sum apart
-// again), and the last shift saturates to signed bytes, which have the 128 in the constants: 5 to 8 % of these kernels, which issue
-// vector instructions for three quarters of their time.
-__device__ static __forceinline__ v4i requant_centred(const ConvArgs &a, const v16i &s)
-{
-    uint32_t zero = 0;
-    asm("" : "+v"(zero));
-    const uint64_t add = (uint64_t)(uint32_t)(a.qadd - (128 << a.qt)) << 32 | zero;
-    const int32_t plo = (a.lo - 128) * (1 << a.qt), phi = ((a.q.hi - 127) * (1 << a.qt)) - 1;
-    v4i o;
-#pragma unroll
-    for (int g = 0; g < 4; g++) {
-        int32_t r[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            r[k] = (int32_t)(((uint64_t)((int64_t)s[4 * g + k] * (int)a.q.mult) + add) >> 32);
-            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r[k]) : "v"(r[k]), "s"(plo), "v"(phi));
-        }
-        uint32_t b;
-        asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(b) : "v"(r[0]), "v"(r[1]), "s"(a.qt));
-        asm("v_ashr_pk_i8_i32 %0, %1, %2, %3 op_sel:[0,0,0,1]" : "+v"(b) : "v"(r[2]), "v"(r[3]), "s"(a.qt));
-        o[g] = (int)b;
-    }
-    // a matrix instruction may read these next, two wait states behind the vector instruction that wrote them at the earliest: the
-    // compiler, which sees to that, does not see what the assembly above writes
-    asm("s_nop 1" : "+v"(o));
-    return o;
 }
 
 } // namespace
@@ -140,7 +103,7 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int p = lane & 31, h = lane >> 5;
-    const int ch = 16 * ((p >> 2) & 1) + 4 * (p >> 3) + (p & 3); // the channel of a slice that this lane's column stands for
+    const int ch = slice_channel(p); // the channel of a slice that this lane's column stands for
     // work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of the patches
     const int ppi = geo.PY * geo.PX;
     int gid = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
@@ -173,17 +136,7 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
             we[kk] = kk == 0 || kk < geo.nk ? ldg128(e.wfrag1 + ((size_t)((kk >> 1) * (e.kout_pad >> 5) + T) * 2 + (kk & 1)) * 1024 + lane * 16)
                                             : v4i{0, 0, 0, 0};
     };
-    // the matrix of a tap is diagonal: the row's own channel's weight, where this lane's half of the columns has that channel
-    const bool diagonal = (ch >> 4) == h;
-    uint32_t sel[3], dm[4]; // byte s of a dword to the channel's place in its dword; which of the four dwords that is
-#pragma unroll
-    for (int s = 0; s < 3; s++)
-        sel[s] = 0x0c0c0c0cu ^ ((0x0cu ^ s) << (8 * (ch & 3)));
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        dm[j] = diagonal && ((ch & 15) >> 2) == j ? ~0u : 0u;
-        asm("" : "+v"(dm[j])); // masks in registers: an AND each, not a select
-    }
+    const DiagonalTap taps(lane);
     auto load_d = [&](int T) {
         const int c0 = min(32 * T + 16 * h, d.in_cs - 16), cd = min(32 * T + ch, d.in_cs - 1); // the last slice may be half empty; its products meet zero weights
         if constexpr (MATRIX)
@@ -293,8 +246,7 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
             for (int r = 0; r < 3; r++)
 #pragma unroll
                 for (int s = 0; s < 3; s++) {
-                    const uint32_t w = __builtin_amdgcn_perm(0, (uint32_t)wd[r], sel[s]);
-                    const v4i m = {(int)(w & dm[0]), (int)(w & dm[1]), (int)(w & dm[2]), (int)(w & dm[3])};
+                    const v4i m = taps.matrix(wd[r], s);
 #pragma unroll
                     for (int t = 0; t < PT; t++)
                         o[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(m, *reinterpret_cast<const v4i *>(ebuf + first[t] + (r * RW + s) * 32), o[t], 0, 0, 0);
@@ -606,8 +558,10 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
-    const double apart = d.stride_h == 1 ? 8.40 + 0.953 * narrow + 0.00326 * wide * e.in_cs + 0.00191 * narrow * p.out_cs
+    double apart = d.stride_h == 1 ? 8.40 + 0.953 * narrow + 0.00326 * wide * e.in_cs + 0.00191 * narrow * p.out_cs
                                          : 8.74 + 2.163 * narrow + 0.00291 * wide * e.in_cs + 0.00176 * narrow * p.out_cs;
+    if (conv_dwpoint_applies(d, p)) // the last two layers are one launch where that is faster
+        apart -= std::max(0.0, conv_dwpoint_apart_us(d, p) - conv_dwpoint_us(d, p));
     double us;
     choose_shape(e, d, p, -1, &us);
     return us < apart;

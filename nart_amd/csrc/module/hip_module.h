@@ -165,7 +165,7 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n);
 void hip_pass_drop(void *state);
 // how many fused launches of each kind have been counted so far (hip_module_fused_*): a replayed pass counts what the
 // recorded one did
-constexpr int kHipCounters = 8;
+constexpr int kHipCounters = 9;
 long *const *hip_counters(void);
 // the inputs that an operator's run() reads (the rest are weights, packed at prepare)
 size_t hip_op_activations(const op_t *op);

@@ -100,7 +100,7 @@ typedef std::map<const mem_t *, std::set<const op_t *>> reader_map;
 std::map<const workspace_t *, reader_map> g_readers;
 long g_fused_adds = 0, g_fused_relus = 0, g_fused_pools = 0, g_chained_convs = 0, g_fused_dequants = 0; // fused launches so far (hip_module_fused_*)
 // (g_chained_convs: convolutions launched by another operator's call, which on few pixels is two kernels)
-long g_fused_blocks = 0, g_fused_inverted = 0, g_fused_tails = 0; // whole bottleneck / inverted residual blocks, blocks from their 3x3 layer on, as one launch
+long g_fused_blocks = 0, g_fused_inverted = 0, g_fused_pairs = 0, g_fused_tails = 0; // whole bottleneck / inverted residual blocks, blocks from their 3x3 layer on, as one launch
 
 reader_map &readers_of(op_t *op) { return g_readers[op->workspace]; }
 
@@ -149,8 +149,9 @@ struct conv_op_t {
     const op_t *blk_next, *blk_add;
     // An expanding, a depthwise and a projecting convolution that hipq_inverted_residual_run computes in one launch, with the
     // relus behind the first two and the add with the block's input where there are: set for all three by the first one's run().
+    // Or only the last two, with any add, for hipq_depthwise_point_run.
     op_t *ir_project;                             // the chain's last convolution (in all three; else null)
-    op_t *ir_expand, *ir_dw;                      // in the last one
+    op_t *ir_expand, *ir_dw;                      // in the last one; no ir_expand: the depthwise convolution is the first
     const op_t *ir_relu1, *ir_relu2, *ir_add;     // in the last one; null: none
     // this pass's output has already been written by the kernel of the pooling operator whose output this convolution
     // reads (hipq_conv2d_run_maxpool_conv): run() has nothing left to do
@@ -361,6 +362,40 @@ bool conv_heads_inverted_residual(op_t *op)
     return true;
 }
 
+// What is left of such a block where the first layer stays a launch of its own, or there is none: depthwise 3x3 [-> relu] -> 1x1
+// [-> add], which hipq_depthwise_point_run computes
+bool conv_heads_depthwise_point(op_t *op)
+{
+    static const bool off = getenv("NART_HIP_NO_FUSION") != nullptr;
+    conv_op_t *d = reinterpret_cast<conv_op_t *>(op);
+    if (off || op->entry->tp != &op_conv_2d_tp || d->desc.dtype != HIPQ_DTYPE_U8 || d->kernel_h != 3 || d->ir_project != nullptr)
+        return false;
+    const op_t *relu = nullptr;
+    op_t *r = only_reader_mut(op);
+    if (r != nullptr && r->entry->tp == &op_relu_tp) {
+        if (!relu_clamps(r, d))
+            return false;
+        relu = r;
+        r = only_reader_mut(r);
+    }
+    if (r == nullptr || r->entry->tp != &op_conv_2d_tp || reinterpret_cast<conv_op_t *>(r)->plan == nullptr)
+        return false;
+    conv_op_t *p = reinterpret_cast<conv_op_t *>(r);
+    int i = 0;
+    const op_t *a = add_reading(r, &i), *next = only_reader(r);
+    if (a != nullptr) {
+        const QSet &qi = add_inputs(a), &qo = add_output(a);
+        if (!hipq_depthwise_point_fusable(d->plan, p->plan, 1, i == 1, qi.alpha[1 - i], qi.zp[1 - i], qo.alpha[0], qo.zp[0], qo.bits[0]))
+            return false;
+    } else if ((next != nullptr && next->entry->tp != &op_conv_2d_tp) // where the 1x1 layer leaves its launch to another operator, that one decides
+               || !hipq_depthwise_point_fusable(d->plan, p->plan, 0, 0, 1.0f, 0, 1.0f, 0, 8))
+        return false;
+    d->ir_project = p->ir_project = r;
+    p->ir_expand = nullptr, p->ir_dw = op;
+    p->ir_relu1 = nullptr, p->ir_relu2 = relu, p->ir_add = a;
+    return true;
+}
+
 // The block that ends in convolution `pop` (and the add `add`, null: none) as one launch into y; false: nothing launched, run
 // the operators
 bool inverted_residual_launch(op_t *pop, const op_t *add, void *y);
@@ -400,7 +435,10 @@ void conv_run(op_t *op)
         return;
     }
     if (c->defer == 0)
-        c->defer = conv_heads_inverted_residual(op) || (c->ir_project != nullptr && c->ir_project != op) || sole_reader_fuses(op) ? 1 : -1;
+        c->defer = (c->ir_project != op && conv_heads_inverted_residual(op)) || (c->ir_project != nullptr && c->ir_project != op)
+                || conv_heads_depthwise_point(op) || sole_reader_fuses(op)
+            ? 1
+            : -1;
     if (c->defer == 1) {
         hip_mem_t *ym = as_hip(op->output_tensors[0].mem);
         (void)out_ptr(op); // the buffer exists and the device side is the current one - once the hook has run
@@ -921,25 +959,40 @@ bool inverted_residual_launch(op_t *pop, const op_t *add, void *y)
     if (p->ir_project != pop || p->ir_add != add)
         return false;
     conv_op_t *e = reinterpret_cast<conv_op_t *>(p->ir_expand), *d = reinterpret_cast<conv_op_t *>(p->ir_dw);
+    op_t *const head = e != nullptr ? p->ir_expand : p->ir_dw;
+    // without an expanding layer the residual is any tensor, whose own launch may be due
+    const int o = add != nullptr && add->input_tensors[0]->mem == pop->output_tensors[0].mem ? 1 : 0;
+    const void *res = e == nullptr && add != nullptr ? in_ptr(const_cast<op_t *>(add), o) : nullptr;
     // every launch of the chain is still this one's to make
     auto left = [](const tensor_t *t, void (*hook)(void *), const void *ctx) {
         const hip_mem_t *m = as_hip(t->mem);
         return m->pending == hook && m->pending_ctx == ctx;
     };
-    if (!left(&p->ir_expand->output_tensors[0], conv_launch_plain, e) || !left(&p->ir_dw->output_tensors[0], conv_launch_plain, d)
+    if ((e != nullptr && !left(&p->ir_expand->output_tensors[0], conv_launch_plain, e)) || !left(&p->ir_dw->output_tensors[0], conv_launch_plain, d)
         || (p->ir_relu1 && !left(&p->ir_relu1->output_tensors[0], relu_launch_deferred, p->ir_relu1))
         || (p->ir_relu2 && !left(&p->ir_relu2->output_tensors[0], relu_launch_deferred, p->ir_relu2)))
         return false;
-    const void *x = in_ptr(p->ir_expand, 0);
+    const void *x = in_ptr(head, 0);
     if (x == y)
         return false;
+    if (e == nullptr) {
+        const ew_op_t *a = reinterpret_cast<const ew_op_t *>(add);
+        if ((add == nullptr ? hipq_depthwise_point_run(d->plan, p->plan, x, p->ir_relu2 != nullptr, nullptr, 0, 1.0f, 0, 1.0f, 0, 8, y, op_stream(pop))
+                            : hipq_depthwise_point_run(d->plan, p->plan, x, p->ir_relu2 != nullptr, res, o == 0, a->qi.alpha[o], a->qi.zp[o],
+                                                       a->qo.alpha[0], a->qo.zp[0], a->qo.bits[0], y, op_stream(pop)))
+            != 0)
+            return false;
+        g_fused_relus += p->ir_relu2 != nullptr;
+        g_fused_adds += add != nullptr;
+        ++g_fused_pairs;
+        return true;
+    }
     int first = 0, zp = 0, bits = 8;
     float alpha = 1.0f;
     if (add != nullptr) {
         const ew_op_t *a = reinterpret_cast<const ew_op_t *>(add);
         first = add->input_tensors[0]->mem == p->ir_expand->input_tensors[0]->mem;
         // the kernel reads the residual as the expanding layer reads it; either operator may have been prepared again since
-        const int o = first ? 0 : 1;
         if (a->qi.alpha[o] != e->desc.ialpha || a->qi.zp[o] != e->desc.izp)
             return false;
         alpha = a->qo.alpha[0], zp = a->qo.zp[0], bits = a->qo.bits[0];
@@ -1350,7 +1403,7 @@ void dequantize_prepare(op_t *op)
 long *const *hip_counters(void)
 {
     static long *const c[kHipCounters] = {&g_fused_adds,     &g_fused_relus,  &g_fused_pools, &g_chained_convs,
-                                          &g_fused_dequants, &g_fused_blocks, &g_fused_inverted, &g_fused_tails};
+                                          &g_fused_dequants, &g_fused_blocks, &g_fused_inverted, &g_fused_pairs, &g_fused_tails};
     return c;
 }
 
@@ -1426,6 +1479,7 @@ ART_PUBLIC long hip_module_chained_convs(void) { return g_chained_convs; }
 ART_PUBLIC long hip_module_fused_dequants(void) { return g_fused_dequants; }
 ART_PUBLIC long hip_module_fused_blocks(void) { return g_fused_blocks; }
 ART_PUBLIC long hip_module_fused_inverted(void) { return g_fused_inverted; }
+ART_PUBLIC long hip_module_fused_pairs(void) { return g_fused_pairs; }
 ART_PUBLIC long hip_module_fused_tails(void) { return g_fused_tails; }
 
 ART_PUBLIC void *hip_workspace_stream(workspace_t *w) { return reinterpret_cast<hip_workspace_t *>(w)->stream; }

@@ -71,6 +71,11 @@ _SIGS = {
     "hipq_inverted_residual_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_inverted_residual_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_float, C.c_int,
                                              C.c_int, C.c_void_p, C.c_void_p]),
+    "hipq_depthwise_point_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int, C.c_int]),
+    "hipq_depthwise_point_run": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float,
+                                           C.c_int, C.c_int, C.c_void_p, C.c_void_p]),
+    "hipq_depthwise_point_select": (C.c_int, [C.c_void_p, C.c_int]),
+    "hipq_depthwise_point_kernel": (C.c_char_p, [C.c_void_p, C.c_void_p]),
     "hipq_inverted_residual_select": (C.c_int, [C.c_void_p, C.c_int]),
     "hipq_inverted_residual_kernel": (C.c_char_p, [C.c_void_p, C.c_void_p, C.c_void_p]),
     "hipq_bottleneck_tail_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_float, C.c_int, C.c_int,
@@ -401,6 +406,31 @@ def inverted_residual_run(expand, depthwise, project, x, y, add=None, relus=0, o
     rf, oa, oz = add if add is not None else (False, 1.0, 0)
     check(lib().hipq_inverted_residual_run(expand.handle, depthwise.handle, project.handle, _ptr(x), relus,
                                            int(add is not None), int(bool(rf)), oa, oz, obits, _ptr(y), _stream()))
+    return y
+
+
+def depthwise_point_fusable(depthwise, point, add=None, obits=8):
+    """Can depthwise -> point [-> add] run as one kernel (include/hipq.h)?  add: None or (residual first?, the residual's scale, its
+    zero point, scale of the sum, its zero point)."""
+    rf, ra, rz, oa, oz = add if add is not None else (False, 1.0, 0, 1.0, 0)
+    return bool(lib().hipq_depthwise_point_fusable(depthwise.handle, point.handle, int(add is not None), int(bool(rf)), ra, rz, oa, oz, obits))
+
+
+def depthwise_point_select(point, shape=-1):
+    """Tuning hook: the division of the work of the kernel that `point` closes, by index, -1 by cost (include/hipq.h)."""
+    check(lib().hipq_depthwise_point_select(point.handle, int(shape)))
+
+
+def depthwise_point_kernel(depthwise, point):
+    """Name of the kernel that depthwise_point_run launches for these plans, "" where it does not."""
+    return lib().hipq_depthwise_point_kernel(depthwise.handle, point.handle).decode()
+
+
+def depthwise_point_run(depthwise, point, x, y, residual=None, add=None, relu=False, obits=8):
+    """y = point(depthwise(x)) [+ residual] in one launch (include/hipq.h: hipq_depthwise_point_run)."""
+    rf, ra, rz, oa, oz = add if add is not None else (False, 1.0, 0, 1.0, 0)
+    check(lib().hipq_depthwise_point_run(depthwise.handle, point.handle, _ptr(x), int(bool(relu)), _ptr(residual) if residual is not None else None,
+                                         int(bool(rf)), ra, rz, oa, oz, obits, _ptr(y), _stream()))
     return y
 
 

@@ -38,6 +38,7 @@ class HipqExecutor:
         self.pooled = {}     # conv output name -> the max-pooling node computed inside the convolution's kernel
         self.blocks = {}     # id(add node) -> (reduce, mid, widen conv nodes) of an identity bottleneck block run as one kernel
         self.invres = {}     # id(add or projecting conv node) -> (expand, depthwise, project conv nodes) run as one kernel
+        self.pairs = {}      # id(add or 1x1 conv node) -> (depthwise, 1x1 conv nodes) run as one kernel
         self.in_block = {}   # id(conv node) -> the add node of its block
         self.tails = {}      # id(add node) -> (mid, widen, next or None): the block from its 3x3 layer on as one kernel
         self.duals = {}      # id(add node) -> (widen, shortcut): both 1x1 convolutions and the add as one kernel
@@ -99,6 +100,20 @@ class HipqExecutor:
                 fn = (lambda ps=plans, i=self.buf[xin], o=out, add=add: hipq.inverted_residual_run(ps[0], ps[1], ps[2], i, o, add))
                 self.steps.append({"label": node.output, "kind": "inverted residual", "fn": fn, "ops": sum(p.ops for p in plans), "bytes": nb,
                                    "kernel": "conv_mfma_i8_inverted_residual" + ("+add" if add else "")})
+            elif id(node) in self.pairs:
+                convs = self.pairs[id(node)]
+                plans = [self._early.pop(id(c)) for c in convs]
+                self.plans += plans
+                xin = convs[0].inputs[0]
+                nb = int(np.prod(T[xin].shape)) + int(np.prod(y.shape)) + sum(case.weights[c.attrs["w"]].size + 4 * c.attrs["K"] for c in convs)
+                add = res = None
+                if node.kind == "add":
+                    other = [i for i in node.inputs if i != convs[1].output][0]
+                    add, res = (node.inputs[0] == other, T[other].alpha, T[other].zp, y.alpha, y.zp), self.buf[other]
+                    nb += int(np.prod(y.shape))
+                fn = (lambda ps=plans, i=self.buf[xin], o=out, res=res, add=add: hipq.depthwise_point_run(ps[0], ps[1], i, o, res, add))
+                self.steps.append({"label": node.output, "kind": "depthwise+point", "fn": fn, "ops": sum(p.ops for p in plans), "bytes": nb,
+                                   "kernel": "conv_mfma_i8_depthwise_point" + ("+add" if add else "")})
             elif node.kind == "add" and id(node) in self.blocks:
                 c1, c2, c3 = self.blocks[id(node)]
                 plans = [self._early.pop(id(c)) for c in (c1, c2, c3)]
@@ -333,6 +348,7 @@ class HipqExecutor:
                 return None
             return n
         self._find_inverted_residuals(conv_plan, prod, uses)
+        self._find_pairs(conv_plan, uses)
         for add in case.nodes:
             if add.kind != "add" or len(add.inputs) != 2 or add.inputs[0] == add.inputs[1]:
                 continue
@@ -355,7 +371,7 @@ class HipqExecutor:
                     break
                 for c, p in zip((c1, c2, c3), plans):
                     self._early.setdefault(id(c), p)  # keep the plans for the operators' own turns
-            if id(add) in self.blocks or id(add) in self.invres:
+            if id(add) in self.blocks or id(add) in self.invres or id(add) in self.pairs:
                 continue
             # a block with a projection shortcut: both inputs of the add are 1x1 convolutions read by nobody else
             pair = [prod.get(i) for i in add.inputs]
@@ -431,7 +447,7 @@ class HipqExecutor:
                 self._early[id(n)] = pl
             if self.share is not None:
                 # a part of a batch fuses exactly where the whole did: the tensors in between exist there or they do not
-                if self.share[0].buf.get(d.output) is not None:
+                if self.share[0].buf.get(d.output) is not None or self.share[0].buf.get(e.output) is not None:
                     continue
                 plans[2].special(2)
             st = T[add.output] if add is not None else None
@@ -443,6 +459,43 @@ class HipqExecutor:
                 self.in_block[id(n)] = last
             if add is None:
                 self.fused.pop(p.output, None)
+
+    def _find_pairs(self, conv_plan, uses):
+        """depthwise 3x3, 1x1 [and an add] that hipq_depthwise_point_run computes in one launch, where no larger block takes them."""
+        case = self.case
+        T = case.tensors
+
+        def only_use(name):
+            u = uses.get(name, [])
+            return u[0] if len(u) == 1 and name != case.output.name else None
+        for d in case.nodes:
+            if (d.kind != "conv" or d.attrs["k"] != 3 or d.attrs["pad"] != 1 or d.attrs["group"] != T[d.inputs[0]].shape[1]
+                    or d.attrs["group"] == 1 or id(d) in self.in_block or T[d.inputs[0]].dtype != "u8"):
+                continue
+            p = only_use(d.output)
+            if (p is None or p.kind != "conv" or p.attrs["k"] != 1 or p.attrs["pad"] != 0 or p.attrs["group"] != 1 or p.attrs["stride"] != 1
+                    or id(p) in self.in_block):
+                continue
+            add = self.fused.get(p.output)
+            plans = [conv_plan(n)[0] for n in (d, p)]
+            for n, pl in zip((d, p), plans):
+                self._early[id(n)] = pl
+            if self.share is not None:
+                # a part of a batch fuses exactly where the whole did
+                if self.share[0].buf.get(d.output) is not None:
+                    continue
+                plans[1].special(2)
+            how = None
+            if add is not None:
+                other = [i for i in add.inputs if i != p.output][0]
+                how = (add.inputs[0] == other, T[other].alpha, T[other].zp, T[add.output].alpha, T[add.output].zp)
+            if not hipq.depthwise_point_fusable(*plans, how):
+                continue
+            last = add if add is not None else p
+            self.pairs[id(last)] = (d, p)
+            for n in (d,) + ((p,) if add is not None else ()):
+                self.in_block[id(n)] = last
+            self.fused.pop(p.output, None)
 
     def _tensor(self, t):
         N, C, H, W = t.shape
@@ -462,7 +515,7 @@ class HipqExecutor:
     @property
     def elided(self):
         """Names of the tensors that are never materialised (absorbed into a fused kernel)."""
-        return set(self.fused) | {c.output for cs in self.invres.values() for c in cs[:2]} | set(self.pooled) | set(self.dequantized) | {c.output for cs in self.blocks.values() for c in cs} | {c.output for cs in self.tails.values() for c in cs[:2]} | {c.output for cs in self.duals.values() for c in cs}
+        return set(self.fused) | {c.output for cs in self.invres.values() for c in cs[:2]} | {cs[0].output for cs in self.pairs.values()} | {cs[1].output for k, cs in self.pairs.items() if k != id(cs[1])} | set(self.pooled) | set(self.dequantized) | {c.output for cs in self.blocks.values() for c in cs} | {c.output for cs in self.tails.values() for c in cs[:2]} | {c.output for cs in self.duals.values() for c in cs}
 
     def set_input(self, x):
         inp = self.case.input

@@ -467,6 +467,66 @@ def test_inverted_residual_block_with_changed_scales(own_rt):
     ws.delete()
 
 
+@pytest.mark.parametrize("residual", ["none", "tensor", "deferred"])
+@pytest.mark.parametrize("relus", [False, True], ids=["plain", "relus"])
+def test_depthwise_and_point_convolution_run_as_one_kernel(own_rt, relus, residual):
+    """Depthwise 3x3 [-> relu] -> conv_2d (24 -> 40, 1x1) [-> add with a tensor, or with a convolution whose launch is still due]: one
+    launch (hipq_depthwise_point_run).  A host that reads a tensor in between gets the operators one by one; every tensor can still
+    be read afterwards, pass after pass."""
+    import ctypes as C
+    from oracle import orc
+    pairs = own_rt.libs[1].hip_module_fused_pairs
+    pairs.restype = C.c_long
+    ws = own_rt.workspace("hip")
+    rng = np.random.default_rng(43)
+    x = rng.integers(0, 256, (2, 24, 15, 17), dtype=np.uint8)
+    r = rng.integers(0, 256, (2, 40, 15, 17), dtype=np.uint8)
+    wd, wp, wr = (rng.integers(1, 256, s, dtype=np.uint8) for s in ((24, 1, 3, 3), (40, 24, 1, 1), (40, 24, 1, 1)))
+    qd = dict(ialpha=0.06, izp=30, walpha=0.0026, wzp=128, oalpha=0.055, ozp=40)
+    qp = dict(ialpha=0.055, izp=40, walpha=0.0032, wzp=128, oalpha=0.07, ozp=121)
+    qr = dict(ialpha=0.06, izp=30, walpha=0.0030, wzp=128, oalpha=0.05, ozp=110)
+
+    def conv(t, w, q, pad, group):
+        return orc.conv2d_u8(t, w, None, pad, 1, group, q["ialpha"], q["izp"], q["walpha"], 128, q["oalpha"], q["ozp"])
+    wants = [conv(x, wd, qd, 1, 24)]
+    if relus:
+        wants.append(np.maximum(wants[-1], 40).astype(np.uint8))
+    wants.append(conv(wants[-1], wp, qp, 0, 1))
+    if residual == "deferred":
+        r = conv(x, wr, qr, 0, 1)
+    if residual != "none":
+        wants.append(orc.add_u8(r, wants[-1], 0.05, 110, 0.07, 121, 0.09, 10))
+    assert len(np.unique(wants[-1])) > 32
+    for peek in (None, 0, 1):
+        tx = ws.tensor(x)
+        ops = [ws.conv2d(tx, ws.tensor(wd), None, 1, 1, 24, qd).prepare()]
+        if relus:
+            ops.append(ws.relu(ops[-1].output(0), dict(ialpha=0.055, izp=40, oalpha=0.055, ozp=40)).prepare())
+        ops.append(ws.conv2d(ops[-1].output(0), ws.tensor(wp), None, 0, 1, 1, qp).prepare())
+        other = []
+        if residual != "none":
+            if residual == "deferred":
+                other = [ws.conv2d(tx, ws.tensor(wr), None, 0, 1, 1, qr).prepare()]
+            tr = other[0].output(0) if other else ws.tensor(r)
+            ops.append(ws.add(tr, ops[-1].output(0), dict(ialpha=[0.05, 0.07], izp=[110, 121], oalpha=0.09, ozp=10)).prepare())
+        for rep in range(2):
+            n0 = pairs()
+            for o in other:
+                o.run()
+            for j, o in enumerate(ops):
+                o.run()
+                if peek == j:
+                    assert same_bits(o.output(0).numpy(), wants[j]), (peek, rep)
+            assert same_bits(ops[-1].output(0).numpy(), wants[-1]), (peek, rep)
+            if residual != "deferred":  # there the add may take the other convolution's launch instead
+                assert pairs() == n0 + (1 if peek is None or peek == len(ops) - 1 else 0), (peek, rep, pairs() - n0)
+        for j, o in enumerate(ops):
+            assert same_bits(o.output(0).numpy(), wants[j]), (peek, j)
+        for o in ops[::-1] + other:
+            o.delete()
+    ws.delete()
+
+
 def test_whole_block_and_the_next_stage_first_layer_run_as_one_kernel(own_rt):
     """The same block followed by conv_2d (1024 -> 512, 1x1) that reads the sum: the add leaves its launch to that
     convolution, whose run() launches hipq_bottleneck_run_conv for all five operators; the sum is written as well.  A host
