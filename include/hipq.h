@@ -280,6 +280,9 @@ int hipq_conv2d_run_add2(const hipq_conv2d_plan *plan, const void *x, const hipq
  */
 int hipq_bottleneck_fusable(const hipq_conv2d_plan *reduce, const hipq_conv2d_plan *mid, const hipq_conv2d_plan *widen,
                             int residual_is_input0, float oalpha, int ozp, int obits);
+/* 1 where the block has pixels enough for one launch to be faster than three whose host time does not count (a pass that is
+ * replayed as a graph), or hipq_conv2d_plan_special(reduce, 2) asks for it */
+int hipq_bottleneck_pays(const hipq_conv2d_plan *reduce);
 int hipq_bottleneck_run(const hipq_conv2d_plan *reduce, const hipq_conv2d_plan *mid, const hipq_conv2d_plan *widen,
                         const void *x, int residual_is_input0, float oalpha, int ozp, int obits, void *y, void *stream);
 

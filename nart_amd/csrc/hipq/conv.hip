@@ -2303,6 +2303,11 @@ extern "C" int hipq_bottleneck_fusable(const hipq_conv2d_plan *p1, const hipq_co
     return p1->special == 2 || conv_block_preferred(a1) ? 1 : 0;
 }
 
+extern "C" int hipq_bottleneck_pays(const hipq_conv2d_plan *p1)
+{
+    return p1 && (p1->special == 2 || (long long)p1->args.P >= conv_block_pixels()) ? 1 : 0;
+}
+
 extern "C" int hipq_bottleneck_run(const hipq_conv2d_plan *p1, const hipq_conv2d_plan *p2, const hipq_conv2d_plan *p3, const void *x,
                                    int residual_is_input0, float oalpha, int ozp, int obits, void *y, void *stream)
 {

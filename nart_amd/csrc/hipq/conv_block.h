@@ -14,6 +14,8 @@ bool conv_block_applies(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &
 void launch_conv_block(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st);
 // true where the one kernel measured faster than the launches it replaces
 bool conv_block_preferred(const ConvArgs &a1);
+// The pixels from which on it is faster than three launches of a pass that is replayed as a graph
+long long conv_block_pixels();
 
 // The chain cut one layer later: a2 (3x3 / stride 1 / pad 1, reads a2.x), a3 (the widening 1x1 with the residual a3.res and
 // the add's parameters, sum to a3.y) and - an != nullptr - the 1x1 convolution that reads the sum (output to an->y).

@@ -581,6 +581,11 @@ void launch_conv_block_tail(const ConvArgs &a2, const ConvArgs &a3, const ConvAr
 // gaps; 128 channels (28x28) 40.6 against 49.0, where the tail form below does better still; 64 channels lose.
 bool conv_block_preferred(const ConvArgs &a1) { return a1.out_cs == 256; }
 
+// A work-group reads the block's 1.1 MB of weights for its 49 or so pixels, so the kernel takes 20 us however few there are, where
+// three launches that spread the weights over the chip take 10.5.  ResNet-50 at 224x224, its five blocks as one launch each -> as
+// three: 1 image 267 -> 214 us, 4 images 281 -> 246, 8 305 -> 279, 16 336 -> 321, 24 394 -> 415, 48 571 -> 602.
+long long conv_block_pixels() { return 20 * 196; }
+
 // Measured at batch 64: 128 middle channels (28x28 images) 32 us with the next layer, 27 without, against 14.0 + 28.6
 // and a launch gap; 64 channels (56x56) 43 to 48 with the next layer against 13.8 + 37.3 and the gap, but 58 without
 // (the sum's pixel tile is what that form saves); 256 channels belong to the whole-block kernel.

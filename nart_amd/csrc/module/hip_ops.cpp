@@ -272,6 +272,9 @@ bool conv_heads_block(op_t *op, const op_t *r)
         return false;
     const conv_op_t *c2 = reinterpret_cast<const conv_op_t *>(r), *c3 = reinterpret_cast<const conv_op_t *>(r2);
     const QSet &qi = add_inputs(a), &qo = add_output(a);
+    // operators that run one by one keep the one launch: one call of the host instead of three
+    if (reinterpret_cast<const hip_workspace_t *>(op->workspace)->passes && !hipq_bottleneck_pays(c1->plan))
+        return false;
     if (!c1->plan || !c2->plan || !c3->plan || qi.alpha[1 - i] != c1->desc.ialpha || qi.zp[1 - i] != c1->desc.izp
         || !hipq_bottleneck_fusable(c1->plan, c2->plan, c3->plan, i == 1, qo.alpha[0], qo.zp[0], qo.bits[0]))
         return false;

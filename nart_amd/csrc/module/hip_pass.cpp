@@ -218,6 +218,7 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
     hip_workspace_t *ws = reinterpret_cast<hip_workspace_t *>(ops[0]->workspace);
     if (off || !recordable(ws->stream))
         return false;
+    ws->passes = true;
     if (*state == nullptr)
         *state = new Pass;
     Pass &p = *static_cast<Pass *>(*state);

@@ -62,6 +62,7 @@ _SIGS = {
     "hipq_conv2d_add2_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_conv2d_run_add2": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int,
                                        C.c_void_p, C.c_void_p]),
+    "hipq_bottleneck_pays": (C.c_int, [C.c_void_p]),
     "hipq_bottleneck_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_bottleneck_conv_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int, C.c_void_p]),
     "hipq_bottleneck_run_conv": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int,
@@ -374,6 +375,11 @@ def run_add2(plan, x, shortcut, x_shortcut, shortcut_first, oalpha, ozp, y, obit
 def bottleneck_fusable(reduce, mid, widen, residual_first, oalpha, ozp, obits=8):
     """Can the identity bottleneck block reduce -> mid -> widen -> add(., x) run as one kernel (include/hipq.h)?"""
     return bool(lib().hipq_bottleneck_fusable(reduce.handle, mid.handle, widen.handle, int(bool(residual_first)), oalpha, ozp, obits))
+
+
+def bottleneck_pays(reduce):
+    """Is that kernel faster than three launches of a replayed graph (include/hipq.h)?"""
+    return bool(lib().hipq_bottleneck_pays(reduce.handle))
 
 
 def bottleneck_run(reduce, mid, widen, x, residual_first, oalpha, ozp, y, obits=8):

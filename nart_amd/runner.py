@@ -362,7 +362,9 @@ class HipqExecutor:
                     continue
                 plans = [conv_plan(c)[0] for c in (c1, c2, c3)]
                 st = T[add.output]
-                if hipq.bottleneck_fusable(plans[0], plans[1], plans[2], ci == 1, st.alpha, st.zp):
+                # a part of a batch fuses exactly where the whole did
+                pays = hipq.bottleneck_pays(plans[0]) if self.share is None else self.share[0].buf.get(c1.output) is None
+                if pays and hipq.bottleneck_fusable(plans[0], plans[1], plans[2], ci == 1, st.alpha, st.zp):
                     self.blocks[id(add)] = (c1, c2, c3)
                     for c, p in zip((c1, c2, c3), plans):
                         self.in_block[id(c)] = add

@@ -653,3 +653,13 @@ def test_inverted_residual_half_patch_per_wave(case, hw):
         want = orc.add_u8(t, x, a, z, 0.03, 77, 0.05, 20)
         y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (False, 0.05, 20))
         assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
+
+
+@pytest.mark.parametrize("n, pays", [(1, False), (16, False), (20, True), (64, True)])
+def test_whole_blocks_pay_from_some_pixels_on(n, pays):
+    """The executor leaves the three layers apart below 20 images of 14x14, where a block's weights take one work-group longer than
+    three launches; the kernel itself stays applicable, and asked for (special 2) it pays at any size."""
+    w = np.full((256, 1024, 1, 1), 129, np.uint8)
+    p = hipq.Conv2d((n, 1024, 14, 14), w, np.zeros(256, np.int32), 0, 1, 1, 0.05, 9, 0.001, 128, 0.06, 0)
+    assert hipq.bottleneck_pays(p) == pays
+    assert hipq.bottleneck_pays(p.special(2))
