@@ -112,19 +112,31 @@ __device__ static __forceinline__ uint32_t ashr_sat_u8x4_lanes(int32_t v0, int32
     return o;
 }
 
+// The fast form of the add with unsigned shifts, which issue in 2.4 clocks where arithmetic ones take 4: a term (x*m + c) >> s is
+// (x*m + (c + 2^31)) >>> s less 2^(31-s), and what the two terms are too large by is in the last constant.
+struct AddTerms {
+    uint32_t k0, k1;
+    int32_t add;
+    __device__ __forceinline__ AddTerms(const AddParams &p)
+        : k0((uint32_t)p.c0 ^ 0x80000000u), k1((uint32_t)p.c1 ^ 0x80000000u),
+          add((int32_t)((uint32_t)p.cadd - (0x80000000u >> p.s0) - (0x80000000u >> p.s1)))
+    {
+    }
+};
+
 template <bool FAST>
 __device__ static __forceinline__ uint32_t add_dword(uint32_t a, uint32_t b, const AddParams &p)
 {
     if (FAST) {
-        // operands fit 24 bits: v_mad_i32_i24 is a full-rate instruction.  The upper clamp moves in front of the last
+        // The upper clamp moves in front of the last
         // shift ((hi + 1) * 2^sh - 1 is the largest value that shifts to hi; sh <= 22), the lower one is the pack's.
         const int32_t phi = ((p.hi + 1) << p.sh) - 1;
+        const AddTerms k(p);
         int32_t v[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            const uint32_t x0 = (a >> (8 * e)) & 255, x1 = (b >> (8 * e)) & 255;
-            const int32_t t0 = __mul24((int)x0, (int)p.m0) + p.c0, t1 = __mul24((int)x1, (int)p.m1) + p.c1;
-            v[e] = min(((t0 >> p.s0) + (t1 >> p.s1)) + p.cadd, phi);
+            const uint32_t t0 = __umul24((a >> (8 * e)) & 255, p.m0) + k.k0, t1 = __umul24((b >> (8 * e)) & 255, p.m1) + k.k1;
+            v[e] = min((int32_t)((t0 >> p.s0) + (t1 >> p.s1) + (uint32_t)k.add), phi);
         }
         return ashr_sat_u8x4(v[0], v[1], v[2], v[3], p.sh);
     }

@@ -439,7 +439,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
                 load_chunk(cc + 1); // the next chunk's operands arrive during the arithmetic below
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const v4i o = requant_add16(a3, acc[t], rc[t]);
+                const v4i o = requant_add16<!(G == 2 && ST == 2 && NX == 0)>(a3, acc[t], rc[t]); // that one has no register to spare
                 if (!CHAIN && valid[t]) // 16 bytes of each of 32 pixels per instruction; the chained form stores whole rows below
                     *reinterpret_cast<v4i *>(a3.y + pix[t] * CW + ch + 16 * h) = o;
                 if (CHAIN) { // the sum tile: pixel row q, 16-byte piece c at piece c ^ (q & 15) of every 256 bytes

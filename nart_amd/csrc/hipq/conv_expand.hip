@@ -67,18 +67,13 @@ __device__ inline void plain_to_staging(const ConvArgs &a, const v16i (&acc)[TN]
 }
 
 // The same with the residual add applied in the accumulator layout, on a residual tile in LDS (16-byte piece c of
-// pixel row r at piece c ^ ((r >> 1) & 3) of its 64-byte row), which the result bytes overwrite: per element the
-// convolution's clamped result minus its zero point is clamp(q, lo - zp, hi - zp) with q = (mulhi(acc, mult) + 2^(t-1)) >> t;
-// the add's terms are (d * m + c) >> s; the sum is clamped and packed.  ADD_SAT: the add's clamp range is exactly [0, 255].
+// pixel row r at piece c ^ ((r >> 1) & 3) of its 64-byte row), which the result bytes overwrite; the sum is clamped and packed.
+// ADD_SAT: the add's clamp range is exactly [0, 255].
 template <bool ADD_SAT>
 __device__ inline void fused_in_place(const ConvArgs &a, const v16i (&acc)[2], uint8_t *rtile, int pl, int half)
 {
     const AddParams &q = a.addq;
-    const int mc = (int)(a.res_first ? q.m1 : q.m0), sc = a.res_first ? q.s1 : q.s0;
-    const int mr = (int)(a.res_first ? q.m0 : q.m1), sr = a.res_first ? q.s0 : q.s1, cr = a.res_first ? q.c0 : q.c1;
-    const int rc = 1 << (sc - 1);                    // rounding of the convolution's term (its zero point cancels)
-    const int qround = 1 << (a.qt - 1);
-    const int dlo = a.lo - a.q.zp, dhi = a.q.hi - a.q.zp; // clamp range of (conv byte - conv zero point)
+    const RequantAdd<> f(a);
     const int rsw = (pl >> 1) & 3;
 #pragma unroll
     for (int tn = 0; tn < 2; tn++)
@@ -89,13 +84,8 @@ __device__ inline void fused_in_place(const ConvArgs &a, const v16i (&acc)[2], u
             const uint32_t rv = *slot;
             int32_t y[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                int32_t d = (__mulhi(acc[tn][g * 4 + e], (int)a.q.mult) + qround) >> a.qt;
-                asm("v_med3_i32 %0, %1, %2, %3" : "=v"(d) : "v"(d), "s"(dlo), "v"(dhi));
-                const int32_t t0 = (__mul24(d, mc) + rc) >> sc;
-                const int32_t t1 = (__mul24((int)((rv >> (8 * e)) & 255), mr) + cr) >> sr;
-                y[e] = t0 + t1 + q.cadd;
-            }
+            for (int e = 0; e < 4; e++)
+                y[e] = f(acc[tn][g * 4 + e], rv, e);
             uint32_t packed;
             if (ADD_SAT) {
                 packed = ashr_sat_u8x4(y[0], y[1], y[2], y[3], q.sh); // the last shift, the clamp to [0, 255], the pack

@@ -34,32 +34,20 @@ __device__ static inline v4i requant16(const ConvArgs &a, const v16i &acc, uint3
     return o;
 }
 
-// The same followed by the residual add (op_quant_add_run on the requantised bytes and the residual's 16 bytes `res`),
-// in the 32-bit form: per element the convolution's clamped result minus its zero point is clamp(q, lo - zp, hi - zp)
-// with q = (mulhi(acc, mult) + 2^(t-1)) >> t; the add's terms are (d * m + c) >> s; the sum's last shift and its
-// saturation to [0, 255] are the shifting, saturating pack.
+// The same followed by the residual add (op_quant_add_run on the requantised bytes and the residual's 16 bytes `res`), in the
+// 32-bit form; the sum's last shift and its saturation to [0, 255] are the shifting, saturating pack.
+template <bool WIDE = true>
 __device__ static inline v4i requant_add16(const ConvArgs &a, const v16i &acc, const v4i res)
 {
-    const AddParams &q = a.addq;
-    const int mc = (int)(a.res_first ? q.m1 : q.m0), sc = a.res_first ? q.s1 : q.s0;
-    const int mr = (int)(a.res_first ? q.m0 : q.m1), sr = a.res_first ? q.s0 : q.s1, cr = a.res_first ? q.c0 : q.c1;
-    const int rc = 1 << (sc - 1); // rounding of the convolution's term (its zero point cancels)
-    const int qround = 1 << (a.qt - 1);
-    const int dlo = a.lo - a.q.zp, dhi = a.q.hi - a.q.zp;
+    const RequantAdd<WIDE> f(a);
     v4i o;
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-        const uint32_t rv = (uint32_t)res[g];
         int32_t y[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            int32_t d = (__mulhi(acc[g * 4 + e], (int)a.q.mult) + qround) >> a.qt;
-            asm("v_med3_i32 %0, %1, %2, %3" : "=v"(d) : "v"(d), "s"(dlo), "v"(dhi));
-            const int32_t t0 = (__mul24(d, mc) + rc) >> sc;
-            const int32_t t1 = (__mul24((int)((rv >> (8 * e)) & 255), mr) + cr) >> sr;
-            y[e] = t0 + t1 + q.cadd;
-        }
-        o[g] = (int)ashr_sat_u8x4(y[0], y[1], y[2], y[3], q.sh);
+        for (int e = 0; e < 4; e++)
+            y[e] = f(acc[g * 4 + e], (uint32_t)res[g], e);
+        o[g] = (int)ashr_sat_u8x4(y[0], y[1], y[2], y[3], a.addq.sh);
     }
     return o;
 }

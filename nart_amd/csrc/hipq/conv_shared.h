@@ -108,6 +108,46 @@ __device__ static inline uint32_t pack_low_bytes(int32_t r0, int32_t r1, int32_t
     return __builtin_amdgcn_perm((uint32_t)r1, (uint32_t)r0, 0x0c0c0400u) | __builtin_amdgcn_perm((uint32_t)r3, (uint32_t)r2, 0x04000c0cu);
 }
 
+// (acc * mult + add) >> 32: with a constant in add's high word one v_mad_i64_i32 (4.6 clocks) for a v_mul_hi_i32 (4) and an addition
+// (2.4).  add has to be hidden from the compiler as a whole, which would take the sum apart again.
+__device__ static __forceinline__ int32_t mulhi_add(int32_t acc, uint32_t mult, uint64_t add)
+{
+    return (int32_t)(((uint64_t)((int64_t)acc * (int)mult) + add) >> 32);
+}
+
+// The convolution's requantisation and the residual add in one (requant_add16 and the kernels that have their own loop): the convolution's
+// byte c is clamp(mulhi(acc, mult) + qadd) >> qt, never negative (a.lo >= 0), the two terms are those of AddTerms, the convolution's
+// zero point in its constant.  35 clocks a value by the instructions' rates, 42 with arithmetic shifts and a
+// multiplication and an addition for the convolution's product.
+// WIDE: the 64-bit multiply-add, which takes a register more.
+template <bool WIDE = true>
+struct RequantAdd {
+    uint64_t qadd;
+    uint32_t mult, mc, kc, mr, kr;
+    int qt, plo, phi, sc, sr, add;
+    __device__ __forceinline__ RequantAdd(const ConvArgs &a)
+    {
+        const AddParams &q = a.addq;
+        const AddTerms k(q);
+        mult = a.q.mult, qadd = (uint64_t)(uint32_t)a.qadd << 32, qt = a.qt, plo = a.lo << a.qt, phi = ((a.q.hi + 1) << a.qt) - 1;
+        mc = a.res_first ? q.m1 : q.m0, sc = a.res_first ? q.s1 : q.s0, kc = a.res_first ? k.k1 : k.k0;
+        mr = a.res_first ? q.m0 : q.m1, sr = a.res_first ? q.s0 : q.s1, kr = a.res_first ? k.k0 : k.k1;
+        add = k.add;
+        if (!WIDE)
+            return;
+        asm("" : "+s"(qadd));
+        asm("" : "+v"(mult)); // the addend in scalar registers: one vector register instead of two
+    }
+    // acc with byte e of res: the sum before its last shift
+    __device__ __forceinline__ int32_t operator()(int32_t acc, uint32_t res, int e) const
+    {
+        int32_t c = WIDE ? mulhi_add(acc, mult, qadd) : __mulhi(acc, (int)mult) + (int32_t)(qadd >> 32);
+        asm("v_med3_i32 %0, %1, %2, %3" : "=v"(c) : "v"(c), "s"(plo), "v"(phi));
+        const uint32_t t0 = (__umul24((uint32_t)c >> qt, mc) + kc) >> sc, t1 = (__umul24((res >> (8 * e)) & 255, mr) + kr) >> sr;
+        return (int32_t)(t0 + t1 + (uint32_t)add);
+    }
+};
+
 // One-multiply requantisation of four accumulators to the four bytes of a dword, for outputs whose clamp range lies in
 // [0, 255] (a.lo >= 0): mulhi and the rounding / zero-point constant as in conv_requant<true>, then the clamp IN FRONT of
 // the shift - lo << t and ((hi + 1) << t) - 1 are the smallest and largest values that shift to lo and hi - and the

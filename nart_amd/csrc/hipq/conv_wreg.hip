@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256, (4096 * (CPT + CPT2) <= 53248 ? 3 : 4096 * (CP
         reduce_all<CPT, 2, D>(acc, ringa, (int)a.xmask, ldw, ldb);
 #pragma unroll
         for (int t = 0; t < 2; t++) {
-            const v4i o = requant_add16(a, acc[t], res[t]);
+            const v4i o = requant_add16<CPT != 4 || S2 != 1>(a, acc[t], res[t]); // 4, 1: three work-groups a CU leave it no register
             if (valid[t])
                 *reinterpret_cast<v4i *>(a.y + pix[t] * a.out_cs + st0 + 16 * h) = o;
         }
