@@ -273,7 +273,10 @@ __global__ __launch_bounds__(256) void pool_u8_kernel(const PoolArgs p)
 // loads, one 128-bit store), 32-bit index arithmetic.  Maxima and sums are taken on the packed dwords (sums: bytes 0, 2 and
 // bytes 1, 3 as two 16-bit halves each; the host guarantees windows of at most 128 pixels).  Average pooling of 8 x 35 x 35 x 192,
 // 3x3 / stride 1: 6.75 us with four channels per thread -> 3.64.
-template <bool AVG>
+// K: windows of 2x2 or 3x3, whose loads are all under way before the first is used (a position outside the image reads a clamped
+// one and counts as zeros, which change neither a maximum of bytes nor a sum): maximum at stride 2 5.1 -> 3.2 us, average at stride 1
+// 4.8 -> 3.7 at that size; 0: any window, a load's latency after the other.
+template <bool AVG, int K>
 __global__ __launch_bounds__(256) void pool16_u8_kernel(const PoolArgs p, double inv_c16, double inv_ow, double inv_oh)
 {
     const int c16n = p.cs >> 4;
@@ -295,19 +298,35 @@ __global__ __launch_bounds__(256) void pool16_u8_kernel(const PoolArgs p, double
         const int hs = max(h0, 0), ws = max(w0, 0);
         const int he = min(h0 + p.kh, p.H), we = min(w0 + p.kw, p.W);
         u32x4 ev = {0, 0, 0, 0}, od = {0, 0, 0, 0}; // max: the maxima in ev; average: even bytes' and odd bytes' sums
-        for (int i = hs; i < he; i++)
-            for (int j = ws; j < we; j++) {
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(p.x + (size_t)((n * p.H + i) * p.W + j) * p.cs + c0);
+        auto take = [&](const u32x4 &v) {
 #pragma unroll
-                for (int d = 0; d < 4; d++) {
-                    if (AVG) {
-                        ev[d] += v[d] & 0x00ff00ffu;
-                        od[d] += (v[d] >> 8) & 0x00ff00ffu;
-                    } else {
-                        ev[d] = max_u8x4(ev[d], v[d]);
-                    }
+            for (int d = 0; d < 4; d++) {
+                if (AVG) {
+                    ev[d] += v[d] & 0x00ff00ffu;
+                    od[d] += (v[d] >> 8) & 0x00ff00ffu;
+                } else {
+                    ev[d] = max_u8x4(ev[d], v[d]);
                 }
             }
+        };
+        auto at = [&](int i, int j) { return *reinterpret_cast<const u32x4 *>(p.x + (size_t)((n * p.H + i) * p.W + j) * p.cs + c0); };
+        if constexpr (K > 0) {
+            u32x4 v[K * K];
+#pragma unroll
+            for (int i = 0; i < K; i++)
+#pragma unroll
+                for (int j = 0; j < K; j++)
+                    v[i * K + j] = at(min(max(h0 + i, 0), p.H - 1), min(max(w0 + j, 0), p.W - 1));
+#pragma unroll
+            for (int i = 0; i < K; i++)
+#pragma unroll
+                for (int j = 0; j < K; j++)
+                    take((unsigned)(h0 + i) < (unsigned)p.H && (unsigned)(w0 + j) < (unsigned)p.W ? v[i * K + j] : u32x4{0, 0, 0, 0});
+        } else {
+            for (int i = hs; i < he; i++)
+                for (int j = ws; j < we; j++)
+                    take(at(i, j));
+        }
         u32x4 o = ev;
         if (!same) { // else equal scales (a multiplier of exactly 2^shift), equal zero points, 8 bits: the maximum is the result
             uint32_t mult = p.mult;
@@ -344,7 +363,8 @@ __global__ __launch_bounds__(256) void pool16_u8_kernel(const PoolArgs p, double
 // NT / cpb thread groups; a thread sums its pixels on packed 16-bit lanes, unpacked every 256 of them, and the partial sums meet in
 // LDS in two steps.  What bounds it is one thread's list of pixels (a load latency per four), so the host takes the largest cpb
 // that still makes 1024 work-groups and 1024 threads where 256 would leave lists of more than four.  8 x 35 x 35 x 192:
-// 150 us with one thread per four channels and image -> 7.2 with 256 threads -> 4.1.
+// 150 us with one thread per four channels and image -> 7.2 with 256 threads -> 4.1.  The sums in LDS are loops of a fixed length, so
+// that their reads are under way together (ResNet-18 at batch 1, whose last kernels these are: 97.5 -> 96.1 us).
 template <int NT>
 __global__ __launch_bounds__(NT) void pool_gavg16_u8_kernel(const PoolArgs p, uint32_t mult, int shift, int cpb_log2)
 {
@@ -388,18 +408,27 @@ __global__ __launch_bounds__(NT) void pool_gavg16_u8_kernel(const PoolArgs p, ui
     for (int k = 0; k < PER; k++) {
         t[k] = 0;
         const int it = (tid & (items - 1)) + NT * k;
-        if (k * NT < items)
-            for (int g = tid / items; g < PG; g += parts)
-                t[k] += part[g * cpb + (it >> 4)][it & 15];
+        const int32_t *from = &part[(tid / items) * cpb + (it >> 4)][it & 15];
+        if (items <= NT) { // PG / parts = NT / cpb * items / NT
+#pragma unroll
+            for (int g = 0; g < 16; g++)
+                t[k] += k == 0 ? from[g * parts * cpb * 17] : 0;
+        } else if (k * NT < items) {
+            for (int g = 0; g < PG; g++)
+                t[k] += from[g * cpb * 17];
+        }
     }
     if (parts > 1) {
         __syncthreads();
         part[tid >> 4][tid & 15] = t[0];
         __syncthreads();
         t[0] = 0;
-        if (tid < items)
-            for (int g = 0; g < parts; g++)
-                t[0] += part[(g * items + tid) >> 4][tid & 15];
+        if (tid < items) { // parts: 2 (NT / 128, at the least) to 16
+            const int32_t *from = &part[tid >> 4][tid & 15];
+#pragma unroll
+            for (int g = 0; g < NT / 64; g++)
+                t[0] += g < parts ? from[g * cpb * 17] : 0;
+        }
     }
 #pragma unroll
     for (int k = 0; k < PER; k++) {
@@ -1122,6 +1151,18 @@ extern "C" int hipq_softmax_u8(const void *x, void *y, size_t npix, int C, int c
     return launch_status("softmax_u8_wide_kernel");
 }
 
+template <bool AVG>
+static void launch_pool16(const PoolArgs &p, unsigned grid, hipStream_t st)
+{
+    const double c16 = 1.0 / (p.cs / 16), ow = 1.0 / p.OW, oh = 1.0 / p.OH;
+    if (p.kh == 3 && p.kw == 3)
+        hipLaunchKernelGGL((pool16_u8_kernel<AVG, 3>), dim3(grid), dim3(256), 0, st, p, c16, ow, oh);
+    else if (p.kh == 2 && p.kw == 2)
+        hipLaunchKernelGGL((pool16_u8_kernel<AVG, 2>), dim3(grid), dim3(256), 0, st, p, c16, ow, oh);
+    else
+        hipLaunchKernelGGL((pool16_u8_kernel<AVG, 0>), dim3(grid), dim3(256), 0, st, p, c16, ow, oh);
+}
+
 extern "C" int hipq_pool_u8(const void *x, void *y, int N, int C, int H, int W, int OH, int OW, int cs, int kh, int kw,
                             int ph, int pw, int sh, int sw, int method, float ia, int iz, float oa, int oz, int obits,
                             void *stream)
@@ -1161,13 +1202,13 @@ extern "C" int hipq_pool_u8(const void *x, void *y, int N, int C, int H, int W, 
     if (vec16 && (long long)N * OH * OW * (cs / 16) < (1ll << 31) && (long long)N * H * W < (1ll << 31)) {
         const unsigned grid = (grid_for((size_t)N * OH * OW * (cs / 16)) + 7) / 8 * 8;
         if (!p.is_avg && p.shift <= 22) {
-            hipLaunchKernelGGL(pool16_u8_kernel<false>, dim3(grid), dim3(256), 0, st, p, 1.0 / (cs / 16), 1.0 / OW, 1.0 / OH);
+            launch_pool16<false>(p, grid, st);
             return launch_status("pool16_u8_kernel");
         }
         PoolArgs q = p; // average: the multiplier of a whole window; p.shift is that of the smallest one, a single pixel
         hipq_quant_scale(p.ia_over_oa / (float)(uint32_t)(kh * kw), 16, &q.mult, &q.shift);
         if (p.is_avg && (long long)kh * kw <= 128 && p.shift >= 1 && q.shift >= 1 && q.shift <= 22) {
-            hipLaunchKernelGGL(pool16_u8_kernel<true>, dim3(grid), dim3(256), 0, st, q, 1.0 / (cs / 16), 1.0 / OW, 1.0 / OH);
+            launch_pool16<true>(q, grid, st);
             return launch_status("pool16_u8_kernel");
         }
     }

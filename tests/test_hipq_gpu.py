@@ -1369,3 +1369,21 @@ def test_relu_word_and_wide_forms(ratio):
         xd = torch.from_numpy(x).cuda()
         got = hipq.relu_u8(xd, torch.zeros_like(xd), ratio * 0.02, iz, 0.02, oz, obits).cpu().numpy()
         assert np.array_equal(got, orc.relu_u8(x, ratio * 0.02, iz, 0.02, oz, obits)), (iz, oz, obits)
+
+
+@pytest.mark.parametrize("k", [2, 3, 4])
+@pytest.mark.parametrize("method", [0, 1])
+@pytest.mark.parametrize("shape,pad,st,ceil_mode", [((2, 48, 9, 7), 1, 1, False), ((3, 16, 10, 11), 1, 2, True), ((1, 80, 1, 2), 1, 1, False),
+                                                    ((2, 32, 7, 8), 0, 3, True)], ids=str)
+def test_pooling_windows_loaded_at_once(shape, pad, st, ceil_mode, k, method):
+    """2x2 and 3x3 windows against the general kernel's 4x4: clipped on every side, images smaller than a window, windows that hang
+    over the far edge in ceil mode."""
+    if shape[2] + 2 * pad < k or shape[3] + 2 * pad < k:
+        pytest.skip("the window is larger than the padded image")
+    rng = np.random.default_rng(sum(shape) + k)
+    x = rng.integers(0, 256, shape, dtype=np.uint8)
+    for q in ((0.02, 0, 0.02, 0), (0.03, 131, 0.05, 120)):
+        want = orc.pool_u8(x, (k, k), pad, st, method, ceil_mode, *q)
+        y = torch.zeros((shape[0], want.shape[2], want.shape[3], hipq.channel_stride(shape[1])), dtype=torch.uint8, device="cuda")
+        hipq.pool_u8(hipq.to_device_nhwc(x), y, shape[1], (k, k), pad, st, method, *q)
+        assert np.array_equal(hipq.from_device_nhwc(y, shape[1]), want)
