@@ -398,7 +398,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         const int q = 32 * t + p;
-        const v4i o = requant16(a2, acc2[t], a3.xmask);
+        const v4i o = requant16<!(G == 2 && PH == 4 && NX == 2)>(a2, acc2[t], a3.xmask);
         *reinterpret_cast<v4i *>(lds + M_OFF + row_off<CM>(q, (ct0 >> 4) + h)) = o;
     }
     __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
         reduce_all<4 * G, 2, DN>(accn, rr, (int)an.xmask, ldwn, ldbn);
 #pragma unroll
         for (int t = 0; t < 2; t++) {
-            const v4i o = requant16(an, accn[t], 0);
+            const v4i o = requant16<!(G == 2 && PH == 4 && NX == 2)>(an, accn[t], 0);
             if (valid[t])
                 *reinterpret_cast<v4i *>(an.y + pix[t] * (NX * CM) + cn + 16 * h) = o;
         }

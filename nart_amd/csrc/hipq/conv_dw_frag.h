@@ -49,15 +49,14 @@ struct DiagonalTap {
 };
 
 // 16 accumulators (16 consecutive channels of a position) -> their bytes, re-centred (XOR 0x80 = 128 less, as signed bytes).  The rounding
-// and the zero point ride along as the high word of a 64-bit multiply-add (v_mad_i64_i32 takes 4.4 clocks, v_mul_hi_i32 and the
-// addition 8 where few waves share a SIMD; the zero of the low word is hidden from the compiler, which would take the sum apart
-// again), and the last shift saturates to signed bytes, which have the 128 in the constants: 5 to 8 % of these kernels, which issue
-// vector instructions for three quarters of their time.
+// and the zero point ride along in the 64-bit multiply-add, and the last shift saturates to signed bytes, which have the 128 in
+// the constants: 5 to 8 % of these kernels, which issue vector instructions for three quarters of their time.
 __device__ static __forceinline__ v4i requant_centred(const ConvArgs &a, const v16i &s)
 {
-    uint32_t zero = 0;
-    asm("" : "+v"(zero));
-    const uint64_t add = (uint64_t)(uint32_t)(a.qadd - (128 << a.qt)) << 32 | zero;
+    uint64_t add = (uint64_t)(uint32_t)(a.qadd - (128 << a.qt)) << 32;
+    uint32_t mult = a.q.mult;
+    asm("" : "+s"(add));
+    asm("" : "+v"(mult));
     const int32_t plo = (a.lo - 128) * (1 << a.qt), phi = ((a.q.hi - 127) * (1 << a.qt)) - 1;
     v4i o;
 #pragma unroll
@@ -65,7 +64,7 @@ __device__ static __forceinline__ v4i requant_centred(const ConvArgs &a, const v
         int32_t r[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            r[k] = (int32_t)(((uint64_t)((int64_t)s[4 * g + k] * (int)a.q.mult) + add) >> 32);
+            r[k] = mulhi_add(s[4 * g + k], mult, add);
             asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r[k]) : "v"(r[k]), "s"(plo), "v"(phi));
         }
         uint32_t b;

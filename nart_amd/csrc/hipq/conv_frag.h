@@ -19,17 +19,18 @@ __device__ static inline int swz(int row)
 
 // 16 accumulators (16 consecutive channels of one pixel) -> 16 requantised bytes, each XORed with the low byte of flip.
 // For clamp ranges within [0, 255] (a.lo >= 0: the callers' hosts check it).
+template <bool WIDE = true>
 __device__ static inline v4i requant16(const ConvArgs &a, const v16i &acc, uint32_t flip)
 {
     v4i o;
     if (a.lo == 0 && a.q.hi == 255) {
 #pragma unroll
         for (int g = 0; g < 4; g++)
-            o[g] = (int)(conv_requant4<true>(a, acc[g * 4], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3]) ^ flip);
+            o[g] = (int)(conv_requant4<true, WIDE>(a, acc[g * 4], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3]) ^ flip);
     } else {
 #pragma unroll
         for (int g = 0; g < 4; g++)
-            o[g] = (int)(conv_requant4<false>(a, acc[g * 4], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3]) ^ flip);
+            o[g] = (int)(conv_requant4<false, WIDE>(a, acc[g * 4], acc[g * 4 + 1], acc[g * 4 + 2], acc[g * 4 + 3]) ^ flip);
     }
     return o;
 }

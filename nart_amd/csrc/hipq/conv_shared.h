@@ -152,14 +152,20 @@ struct RequantAdd {
 // [0, 255] (a.lo >= 0): mulhi and the rounding / zero-point constant as in conv_requant<true>, then the clamp IN FRONT of
 // the shift - lo << t and ((hi + 1) << t) - 1 are the smallest and largest values that shift to lo and hi - and the
 // shifting, saturating pack.  SAT: the range is exactly [0, 255], the pack's saturation is the clamp.
-template <bool SAT>
+template <bool SAT, bool WIDE = true>
 __device__ static __forceinline__ uint32_t conv_requant4(const ConvArgs &a, int32_t v0, int32_t v1, int32_t v2, int32_t v3)
 {
     int32_t r[4] = {v0, v1, v2, v3};
     const int32_t plo = a.lo << a.qt, phi = ((a.q.hi + 1) << a.qt) - 1;
+    uint64_t add = (uint64_t)(uint32_t)a.qadd << 32;
+    uint32_t mult = a.q.mult;
+    if (WIDE) {
+        asm("" : "+s"(add));
+        asm("" : "+v"(mult));
+    }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        r[e] = __mulhi(r[e], (int)a.q.mult) + a.qadd;
+        r[e] = WIDE ? mulhi_add(r[e], mult, add) : __mulhi(r[e], (int)a.q.mult) + a.qadd;
         if (!SAT)
             asm("v_med3_i32 %0, %1, %2, %3" : "=v"(r[e]) : "v"(r[e]), "s"(plo), "v"(phi));
     }
