@@ -29,8 +29,8 @@
 //     (more work-groups per CU, whose load, multiply and store phases overlap), three or four for long ones.
 //   * Epilogue.  mult = m * 2^7 with m < 2^24, and for 33 <= shift <= 52 (every realistic scale)
 //         floor((acc*mult + 2^(shift-1)) / 2^shift) + zp == (mulhi(acc, mult) + 2^(t-1) + zp*2^t) >> t,  t = shift-32
-//     because the low 32 bits of the product cannot carry across the floor.  That is one v_mul_hi_i32, one
-//     add, one shift and a saturating pack per output instead of a 64-bit multiply-add-shift.  Other shifts take
+//     because the low 32 bits of the product cannot carry across the floor.  That is one v_mad_i64_i32
+//     (the addend in the high word) and a shifting, saturating pack per output instead of 64-bit shifts.  Other shifts take
 //     the 64-bit path.  Each lane then holds 4 consecutive channels of one pixel per accumulator quad;
 //     the packed dwords are transposed through LDS so that every pixel's channels leave as 128-bit stores.
 //     A residual add can run here as well (hipq_conv2d_run_add): in the accumulator layout, against a residual
@@ -42,7 +42,10 @@
 //   * 1x1 / stride 1 layers with at most 64 input and 256 output channels run conv_mfma_pointwise_kernel: a wave per
 //     strip of 32 pixels, pixel fragments straight from global memory, no LDS staging of activations, no barriers.
 //   * Layers over few pixels or to few channels are streamed (conv_stream.hip); 3x3 layers on any image keep their pixels in LDS
-//     and their weights in registers (conv_hreg.hip); whole blocks are one kernel (conv_block.hip, conv_invres.hip).
+//     and their weights in registers (conv_hreg.hip); whole blocks are one kernel (conv_block.hip, conv_invres.hip), as are a depthwise layer and the 1x1 layer
+//     behind it (conv_dwpoint.hip).
+//   * Layers that have no kernel of their own - any window, data type and scale - run conv_resident_kernel where its fitted cost is
+//     below the tile kernels' (conv_resident.hip: pixels in LDS, weights in registers, no barrier in the loop).
 //   * Other shapes: C <= 4 inputs (the RGB stem) use a register-staged variant of the same tile computation,
 //     depthwise 3x3 a dot-product kernel, remaining depthwise / grouped shapes plain per-output kernels.
 #include <algorithm>
