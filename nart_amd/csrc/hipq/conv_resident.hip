@@ -188,6 +188,7 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(const ResidentGeom g
             *at ^= (int)geo.xmask;
         }
     }
+    wait_vmcnt<0>(); // this wave's loads have landed before the others may read them: a barrier alone says nothing of the load unit's writes
     __syncthreads();
 
     // ---- a slab's pixel operands
