@@ -438,7 +438,8 @@ class HipqExecutor:
                 continue
             e, p = prod.get(d.inputs[0]), only_use(d.output)
             if (not is_conv(e, 1) or only_use(e.output) is not d or not is_conv(p, 1) or T[e.inputs[0]].dtype != "u8"
-                    or any(n.attrs["group"] != 1 or n.attrs["stride"] != 1 for n in (e, p))):
+                    or any(n.attrs["group"] != 1 or n.attrs["stride"] != 1 for n in (e, p))
+                    or any(id(n) in self.in_block or id(n) in self.invres for n in (e, d, p))):  # of the block before, whose last layer is e
                 continue
             add = only_use(p.output)
             if (add is None or add.kind != "add" or sorted(add.inputs) != sorted([p.output, e.inputs[0]]) or p.attrs["relu"]

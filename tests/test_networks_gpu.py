@@ -57,6 +57,33 @@ def test_network_parity_with_fused_residual_adds(build):
     compare_all(case, ex, vals)
 
 
+def depthwise_chain(N=2, hw=28, widths=(64, 96, 96, 64, 128), strides=(1, 1, 2, 1), relu=True):
+    """Depthwise 3x3 and 1x1 layers in turn (separable convolutions): every 1x1 layer could end one fused block and begin the next."""
+    c = cases.Case("depthwise_chain_n%d" % N, 7)
+    t = c.input_u8((N, widths[0], hw, hw), 0.0186, 114)
+    for K, s in zip(widths[1:], strides):
+        t = c.conv(t, t.shape[1], 3, stride=s, group=t.shape[1], relu=relu, ozp=20)
+        t = c.conv(t, K, 1, relu=relu, ozp=20)
+    c.output = t
+    return c
+
+
+@pytest.mark.parametrize("relu", [False, True], ids=["plain", "relu"])
+@pytest.mark.parametrize("N,hw", [(2, 28), (24, 28), (1, 9)])
+def test_chain_of_separable_convolutions(N, hw, relu):
+    """A layer belongs to one fused launch only, whichever way the chain is divided."""
+    case = depthwise_chain(N, hw, relu=relu)
+    x = case_oracle.random_input(case, seed=8)
+    vals = case_oracle.run_case(case, x)
+    ex = HipqExecutor(case, fuse_add=True)
+    taken = [id(n) for group in list(ex.invres.values()) + list(ex.pairs.values()) for n in group]
+    assert len(taken) == len(set(taken)) and taken
+    ex.set_input(x)
+    ex.run()
+    torch.cuda.synchronize()
+    compare_all(case, ex, vals)
+
+
 def test_graph_replay_matches_eager():
     """A captured HIP graph of the whole pass must reproduce the eager result on every replay, with
     eager work and synchronisation in between (new inputs each time)."""
