@@ -6,7 +6,6 @@ is no host fallback — loading fails loudly if the library has not been built.
 """
 import ctypes as C
 import os
-import re
 
 import numpy as np
 
@@ -238,8 +237,6 @@ class Conv2d:
         self.handle = h
         self._address = h.value
         self.kernel = lib().hipq_conv2d_plan_kernel(h).decode()
-        m = re.match(r"conv_mfma_i8_(\d+x\d+)", self.kernel)
-        self._tile0 = TILE_INDEX.get(m.group(1), -1) if m else -1  # the built-in choice, for the tuner to return to
         self.ops = 2 * N * K * self.OH * self.OW * (Cc // group) * R * S
 
     @property

@@ -5,6 +5,7 @@ This is the Python-side counterpart of the reference's parade: a flat list of pr
 pass into a HIP graph so that a launch-bound step replays without per-kernel host overhead.
 All device tensors are channels-last with padded channel stride (see include/hipq.h).
 """
+import re
 import time
 
 import numpy as np
@@ -573,14 +574,13 @@ class HipqExecutor:
         chosen = {}
         for k, s in enumerate(self.steps):
             plan = s.get("plan")
-            if plan is None or not plan.kernel.startswith("conv_mfma") or "_c4" in plan.kernel or "_wzp" in plan.kernel:
+            # the tile kernels alone have tiles and stages to name, and only with aligned addressing; naming a tile would take any
+            # other kernel's layer away from it for good
+            tile0 = re.match(r"conv_mfma_i8_(\d+x\d+)(_signed|_halo|_k2|_perchannel|\+add)*$", s["kernel"])
+            if plan is None or not tile0:
                 continue
             if plan.desc.in_cs % 64 and not (plan.desc.R == 1 and plan.desc.S == 1):
                 continue  # the generic-addressing kernel has a single variant
-            if plan.kernel.endswith("pointwise") and s["kind"] != "conv+add":
-                continue  # the pointwise kernel has no tile or stages (the fused add runs a tile kernel)
-            if "expand" in s["kernel"] or "_stream_" in s["kernel"]:
-                continue  # neither have these two; naming a tile would take the layer away from them for good
             lo, hi = max(0, k - before), min(len(self.steps), k + 1 + after)
             base = self._time_window(lo, hi, reps)
             best, best_t = (-1, 0), base
@@ -593,7 +593,7 @@ class HipqExecutor:
             if best[0] >= 0:
                 plan.select(*best)
             else:  # back to the built-in choice
-                plan.select(plan._tile0, 0)
+                plan.select(hipq.TILE_INDEX[tile0.group(1)], 0)
             s["kernel"] = (plan.kernel_add or plan.kernel + "+add") if s["kind"] == "conv+add" else plan.kernel
             chosen[s["label"]] = (best, round(base, 2), round(best_t, 2))
             if verbose:

@@ -84,6 +84,29 @@ def test_chain_of_separable_convolutions(N, hw, relu):
     compare_all(case, ex, vals)
 
 
+def test_tuning_keeps_the_kernels_that_have_no_tiles():
+    """Naming a tile takes a layer away from the kernels that have none: the search leaves such layers alone, and a tile kernel for
+    which it finds nothing better runs in its own tile again."""
+    import re
+    case = cases.resnet18(N=1, hw=96)
+    ex = HipqExecutor(case, fuse_add=True)
+    runs = lambda s: s["plan"].kernel_add if s["kind"] == "conv+add" else s["plan"].kernel  # noqa: E731
+    steps = [s for s in ex.steps if s.get("plan") is not None and s["kind"] in ("conv", "conv+add")]
+    before = [runs(s) for s in steps]
+    chosen = ex.tune(reps=1)
+    for s, was in zip(steps, before):
+        if re.match(r"conv_mfma_i8_\d+x\d+", was) is None:
+            assert runs(s) == was, (was, runs(s))
+        elif s["label"] in chosen and chosen[s["label"]][0][0] < 0:
+            assert runs(s) == was, (was, runs(s))
+    assert any("resident" in b for b in before)
+    x = case_oracle.random_input(case, seed=9)
+    ex.set_input(x)
+    ex.run()
+    torch.cuda.synchronize()
+    compare_all(case, ex, case_oracle.run_case(case, x))
+
+
 def test_graph_replay_matches_eager():
     """A captured HIP graph of the whole pass must reproduce the eager result on every replay, with
     eager work and synchronisation in between (new inputs each time)."""
