@@ -1533,6 +1533,28 @@ static ConvArgs with_residual(const hipq_conv2d_plan *p)
     return a;
 }
 
+// The kernel that a launch of a plan with these arguments goes to: its name and its launch both come from here.  A shape that
+// the caller names is run.
+enum class Kernel { kResident, kStream, kHreg, kWreg, kRows, kExpand, kStem3, kTile };
+static Kernel kernel_for(const hipq_conv2d_plan *p, const ConvArgs &a, StreamShape *stream)
+{
+    if ((a.res != nullptr ? p->resident_add : p->resident).mb)
+        return Kernel::kResident;
+    if (p->stream.mb && stream_applies(p, stream))
+        return Kernel::kStream;
+    if (hreg_applies(p, a))
+        return Kernel::kHreg; // 3x3, any image size: the pixels in LDS once, weight operands straight into registers
+    if (wreg_applies(p, a))
+        return Kernel::kWreg; // few pixels: the pixel operand in LDS once, weight operands straight into registers
+    if (rows_applies(p, a))
+        return Kernel::kRows; // 3x3 with 64 channels: the input rows stay in LDS, the weights in registers
+    if (expand_applies(p, a))
+        return Kernel::kExpand; // a channel-widening 1x1 layer: pixel operands in registers, channel tiles in a loop
+    if (stem3_applies(p, a))
+        return Kernel::kStem3; // 3x3 / stride 2 on an RGB image: the input rows stay in LDS
+    return stream_applies(p, stream) ? Kernel::kStream : Kernel::kTile;
+}
+
 static void resident_name(const hipq_conv2d_plan *p, const ResidentShape &s, char *nm, size_t size, const char *behind)
 {
     // "stream": the layers that are a stream of weights, whichever of the two kernels they run
@@ -1549,26 +1571,22 @@ static void set_mfma_name(hipq_conv2d_plan *p, bool smallc)
         p->resident = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, p->args);
         p->resident_add = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, with_residual(p));
     }
-    if (p->resident.mb)
-        resident_name(p, p->resident, nm, sizeof nm, "");
-    else if (!smallc && hreg_applies(p, p->args))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_hreg3x3");
-    else if (!smallc && wreg_applies(p, p->args))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_wreg");
-    else if (!smallc && stream_applies(p, &ss))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_stream_%dx%d%s", 16 * ss.mb, 16 * ss.nb, p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else if (!smallc && rows_applies(p, p->args))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_rows3x3%s", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else if (!smallc && expand_applies(p, p->args))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_expand%s", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else if (pointwise_applies(p))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_pointwise%s", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else if (smallc && stem3_applies(p, p->args))
-        snprintf(nm, sizeof nm, "conv_mfma_i8_stem3x3");
-    else
-        snprintf(nm, sizeof nm, "conv_mfma_i8_%dx%d%s%s%s%s", kTiles[p->tile].bm, kTiles[p->tile].bn, smallc ? "_c4" : "",
-                 p->has_wzp ? "_wzp" : "", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "",
-                 halo_applies(p) ? "_halo" : (!smallc && k2_applies(p)) ? "_k2" : "");
+    const char *const sgn = p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "";
+    switch (kernel_for(p, p->args, &ss)) {
+    case Kernel::kResident: resident_name(p, p->resident, nm, sizeof nm, ""); break;
+    case Kernel::kStream: snprintf(nm, sizeof nm, "conv_mfma_i8_stream_%dx%d%s", 16 * ss.mb, 16 * ss.nb, sgn); break;
+    case Kernel::kHreg: snprintf(nm, sizeof nm, "conv_mfma_i8_hreg3x3"); break;
+    case Kernel::kWreg: snprintf(nm, sizeof nm, "conv_mfma_i8_wreg"); break;
+    case Kernel::kRows: snprintf(nm, sizeof nm, "conv_mfma_i8_rows3x3%s", sgn); break;
+    case Kernel::kExpand: snprintf(nm, sizeof nm, "conv_mfma_i8_expand%s", sgn); break;
+    case Kernel::kStem3: snprintf(nm, sizeof nm, "conv_mfma_i8_stem3x3"); break;
+    case Kernel::kTile:
+        if (pointwise_applies(p))
+            snprintf(nm, sizeof nm, "conv_mfma_i8_pointwise%s", sgn);
+        else
+            snprintf(nm, sizeof nm, "conv_mfma_i8_%dx%d%s%s%s%s", kTiles[p->tile].bm, kTiles[p->tile].bn, smallc ? "_c4" : "",
+                     p->has_wzp ? "_wzp" : "", sgn, halo_applies(p) ? "_halo" : (!smallc && k2_applies(p)) ? "_k2" : "");
+    }
     p->name = nm;
     if (p->d_q)
         p->name += "_perchannel";
@@ -1872,22 +1890,18 @@ extern "C" const char *hipq_conv2d_plan_kernel_add(const hipq_conv2d_plan *p)
     const ConvArgs a = with_residual(p);
     char buf[96];
     StreamShape ss;
-    if (p->resident_add.mb)
-        resident_name(p, p->resident_add, buf, sizeof buf, "+add");
-    else if (hreg_applies(p, a))
-        snprintf(buf, sizeof buf, "conv_mfma_i8_hreg3x3+add");
-    else if (wreg_applies(p, a))
-        snprintf(buf, sizeof buf, "conv_mfma_i8_wreg+add");
-    else if (stream_applies(p, &ss))
-        snprintf(buf, sizeof buf, "conv_mfma_i8_stream_%dx%d%s+add", 16 * ss.mb, 16 * ss.nb, p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else if (rows_applies(p, a))
-        snprintf(buf, sizeof buf, "conv_mfma_i8_rows3x3+add");
-    else if (expand_applies(p, a))
-        snprintf(buf, sizeof buf, "conv_mfma_i8_expand%s+add", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "");
-    else
+    const char *const sgn = p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "";
+    switch (kernel_for(p, a, &ss)) {
+    case Kernel::kResident: resident_name(p, p->resident_add, buf, sizeof buf, "+add"); break;
+    case Kernel::kStream: snprintf(buf, sizeof buf, "conv_mfma_i8_stream_%dx%d%s+add", 16 * ss.mb, 16 * ss.nb, sgn); break;
+    case Kernel::kHreg: snprintf(buf, sizeof buf, "conv_mfma_i8_hreg3x3+add"); break;
+    case Kernel::kWreg: snprintf(buf, sizeof buf, "conv_mfma_i8_wreg+add"); break;
+    case Kernel::kRows: snprintf(buf, sizeof buf, "conv_mfma_i8_rows3x3+add"); break;
+    case Kernel::kExpand: snprintf(buf, sizeof buf, "conv_mfma_i8_expand%s+add", sgn); break;
+    default: // the 3x3 stem kernel has no add
         snprintf(buf, sizeof buf, "conv_mfma_i8_%dx%d%s%s%s%s+add", kTiles[p->tile].bm, kTiles[p->tile].bn,
-                 p->variant == kMfmaSmallC ? "_c4" : "", p->has_wzp ? "_wzp" : "", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "",
-                 p->variant == kMfma && k2_applies(p) ? "_k2" : "");
+                 p->variant == kMfmaSmallC ? "_c4" : "", p->has_wzp ? "_wzp" : "", sgn, p->variant == kMfma && k2_applies(p) ? "_k2" : "");
+    }
     nm = buf;
     if (p->d_q)
         nm += "_perchannel";
@@ -2072,14 +2086,8 @@ static void launch_mfma(const hipq_conv2d_plan *p, const ConvArgs &a, hipStream_
 {
     const int nblk = a.nbm * a.nbn;
     const dim3 grid((nblk + 7) / 8 * 8), block(256);
-    StreamShape ss;
-    const bool streams = stream_applies(p, &ss); // the kernel the plan is named after wins over the halo kernel
-    if (p->variant == kMfma && !streams && launch_halo<BM, BN, WM, WN>(p, a, grid, st))
+    if (p->variant == kMfma && launch_halo<BM, BN, WM, WN>(p, a, grid, st))
         return;
-    if (streams) {
-        if (launch_conv_stream(a, ss, st))
-            return; // an unknown forced shape: the tile kernels below
-    }
     if (pointwise_applies(p) && a.acc_out == nullptr && a.res == nullptr) {
         // persistent work-groups (four waves, a strip of 32 pixels each per turn), five to a CU
         const int nstrips = (a.P + 31) / 32, want = (nstrips + 3) / 4;
@@ -2672,29 +2680,15 @@ static int run_conv(const hipq_conv2d_plan *p, ConvArgs &a, hipStream_t st)
     switch (p->variant) {
     case kMfma:
     case kMfmaSmallC:
-        if (const ResidentShape &r = a.res != nullptr ? p->resident_add : p->resident; r.mb) {
-            launch_conv_resident(a, r, st); // any layer whose pixels fit LDS, weight operands straight into registers
-            break;
-        }
-        if (hreg_applies(p, a)) {
-            launch_conv_hreg(a, st); // 3x3, any image size: the pixels in LDS once, weight operands straight into registers
-            break;
-        }
-        if (wreg_applies(p, a)) {
-            launch_conv_wreg(a, st); // few pixels: the pixel operand in LDS once, weight operands straight into registers
-            break;
-        }
-        if (rows_applies(p, a)) {
-            launch_conv_rows(a, st); // 3x3 with 64 channels: the input rows stay in LDS, the weights in registers
-            break;
-        }
-        if (expand_applies(p, a)) {
-            launch_conv_expand(a, st); // a channel-widening 1x1 layer: pixel operands in registers, channel tiles in a loop
-            break;
-        }
-        if (stem3_applies(p, a)) {
-            launch_conv_stem3x3(a, st); // 3x3 / stride 2 on an RGB image: the input rows stay in LDS
-            break;
+        switch (StreamShape ss; kernel_for(p, a, &ss)) {
+        case Kernel::kResident: launch_conv_resident(a, a.res != nullptr ? p->resident_add : p->resident, st); return launch_status(p->name.c_str());
+        case Kernel::kStream: launch_conv_stream(a, ss, st); return launch_status(p->name.c_str());
+        case Kernel::kHreg: launch_conv_hreg(a, st); return launch_status(p->name.c_str());
+        case Kernel::kWreg: launch_conv_wreg(a, st); return launch_status(p->name.c_str());
+        case Kernel::kRows: launch_conv_rows(a, st); return launch_status(p->name.c_str());
+        case Kernel::kExpand: launch_conv_expand(a, st); return launch_status(p->name.c_str());
+        case Kernel::kStem3: launch_conv_stem3x3(a, st); return launch_status(p->name.c_str());
+        case Kernel::kTile: break;
         }
         switch (p->tile) {
         case 0: launch_mfma<128, 128, 2, 2>(p, a, st); break;

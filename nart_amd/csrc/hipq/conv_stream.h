@@ -10,7 +10,6 @@ struct StreamShape {
     int mb, nb, nw;
 };
 
-// false: no instantiation for this shape, nothing launched
-bool launch_conv_stream(const ConvArgs &a, const StreamShape &s, hipStream_t st);
+void launch_conv_stream(const ConvArgs &a, const StreamShape &s, hipStream_t st);
 
 } // namespace hipq

@@ -267,17 +267,16 @@ static void launch_shape(const ConvArgs &a, hipStream_t st)
     }
 }
 
-bool launch_conv_stream(const ConvArgs &a, const StreamShape &s, hipStream_t st)
+void launch_conv_stream(const ConvArgs &a, const StreamShape &s, hipStream_t st)
 {
     switch (s.mb * 10 + s.nb) {
-    case 81: launch_shape<8, 1>(a, st); return true;
-    case 42: launch_shape<4, 2>(a, st); return true;
-    case 41: launch_shape<4, 1>(a, st); return true;
-    case 22: launch_shape<2, 2>(a, st); return true;
-    case 21: launch_shape<2, 1>(a, st); return true;
-    case 12: launch_shape<1, 2>(a, st); return true;
-    case 11: launch_shape<1, 1>(a, st); return true;
-    default: return false;
+    case 81: launch_shape<8, 1>(a, st); break;
+    case 42: launch_shape<4, 2>(a, st); break;
+    case 41: launch_shape<4, 1>(a, st); break;
+    case 22: launch_shape<2, 2>(a, st); break;
+    case 21: launch_shape<2, 1>(a, st); break;
+    case 12: launch_shape<1, 2>(a, st); break;
+    default: launch_shape<1, 1>(a, st); break;
     }
 }
 

@@ -139,6 +139,11 @@ int hipGraphLaunch(void *e, void *st)
     return kSuccess;
 }
 
+/* the device functions' names, by the host stubs that launch them */
+static struct { const void *f; const char *name; } g_kernels[4096];
+static size_t g_nkernels;
+const char *stub_last_kernel = "";
+
 /* a launch is __hipPushCallConfiguration, the kernel's host stub, __hipPopCallConfiguration and hipLaunchKernel */
 typedef struct { uint32_t x, y, z; } dim3;
 static dim3 g_grid, g_block;
@@ -148,7 +153,10 @@ int __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, void *st) { return g_
 int __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, void **st) { return *g = g_grid, *b = g_block, *lds = g_lds, *st = g_stream, kSuccess; }
 int hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t lds, void *st)
 {
-    (void)f, (void)g, (void)b, (void)args, (void)lds;
+    (void)g, (void)b, (void)args, (void)lds;
+    for (size_t i = 0; i < g_nkernels; i++)
+        if (g_kernels[i].f == f)
+            stub_last_kernel = g_kernels[i].name;
     enqueue(st, (action){0});
     stub_kernels++;
     return kSuccess;
@@ -161,5 +169,7 @@ void **__hipRegisterFatBinary(const void *d)
 void __hipUnregisterFatBinary(void **h) { (void)h; }
 void __hipRegisterFunction(void **h, const void *f, char *d, const char *n, unsigned t, void *a, void *b, void *c, void *e, int *w)
 {
-    (void)h, (void)f, (void)d, (void)n, (void)t, (void)a, (void)b, (void)c, (void)e, (void)w;
+    (void)h, (void)d, (void)t, (void)a, (void)b, (void)c, (void)e, (void)w;
+    if (g_nkernels < sizeof g_kernels / sizeof *g_kernels)
+        g_kernels[g_nkernels].f = f, g_kernels[g_nkernels++].name = n;
 }

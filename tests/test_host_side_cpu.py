@@ -56,6 +56,62 @@ def a_chained_add_names_its_kernels():
         assert kernels.value - before == (1 if one else 2), (N, HW, mode, name)
 
 
+def a_plan_launches_the_kernel_that_it_names():
+    """By the built-in rule, in every mode and with a named shape, without and with a residual: the name that a plan gives is that of the
+    kernel it launches, and a shape that the caller names is run."""
+    import random
+    import re
+    import numpy as np
+    from nart_amd import hipq
+    last = C.c_char_p.in_dll(STUB, "stub_last_kernel")
+    x = np.zeros(64, np.uint8).ctypes.data  # never touched
+    names = (("resident", "conv_resident_kernel"), ("stream", "conv_mfma_stream_kernel"), ("hreg3x3", "conv_hreg_kernel"), ("wreg", "conv_wreg_kernel"),
+             ("rows3x3", "conv3x3_c64_rows_kernel"), ("expand", "conv_mfma_expand_kernel"), ("stem3x3", "conv_stem3x3_kernel"),
+             ("pointwise", "conv_mfma_pointwise_kernel"), ("halo", "conv_mfma_halo_kernel"), ("k2", "conv_mfma_dma_k2_kernel"), ("c4", "conv_mfma_kernel"),
+             ("", "conv_mfma_dma_kernel"))
+
+    def check(plan, what):
+        for name, add in ((plan.kernel, False), (plan.kernel_add, True)):
+            if add:
+                rc = hipq.lib().hipq_conv2d_run_add(plan.handle, x, x, 0, 0.05, 3, 0.09, 10, 8, x, None)
+            else:
+                rc = hipq.lib().hipq_conv2d_run(plan.handle, x, x, None, None)
+            hipq.check(rc)
+            assert re.match(r"conv_mfma_i8_", name), name
+            want = [k for n, k in names if n in re.split(r"[_+]", name[len("conv_mfma_i8_"):]) or n == ""][0]
+            assert want in last.value.decode(), (what, name, last.value.decode())
+            seen.add(want)
+    rng, seen = random.Random(6), set()
+    layers = [(11, 256, 13, 256, 3, 1), (1, 128, 28, 128, 3, 1), (64, 256, 14, 256, 3, 2), (8, 64, 56, 64, 3, 1), (64, 64, 56, 256, 1, 1), (1, 64, 14, 96, 3, 1), (1, 64, 32, 256, 1, 1),
+              (2, 3, 64, 32, 3, 2), (2, 3, 64, 64, 7, 2), (16, 512, 14, 512, 1, 1), (1, 480, 14, 64, 1, 1), (64, 2048, 7, 512, 1, 1), (1, 32, 20, 48, 1, 1)]
+    while len(layers) < 120:
+        N, C_, H, K, R, s = rng.choice((1, 2, 6, 16)), rng.choice((3, 20, 64, 96, 128, 256, 480)), rng.randrange(3, 40), rng.choice((16, 64, 135, 256, 512)), rng.choice((1, 3, 5)), rng.choice((1, 1, 2))
+        layers.append((N, C_, H, K, R, s))
+    for N, C_, H, K, R, s in layers:
+        plan = hipq.Conv2d((N, C_, H, H), np.full((K, C_, R, R), 129, np.uint8), None, R // 2, s, 1, 0.05, 9, 0.002, rng.choice((128, 128, 128, 90)), 0.05, 9)
+        for mode in (1, 0, 2, 3):
+            plan.special(mode)
+            check(plan, (N, C_, H, K, R, s, mode))
+        plan.special(1)
+        for shape in ((64, 32, 4), (16, 16, 4)):
+            try:
+                plan.stream(*shape)
+            except hipq.HipqError:
+                continue
+            assert "stream_%dx%d" % shape[:2] in plan.kernel and "stream_%dx%d" % shape[:2] in plan.kernel_add, (plan.kernel, plan.kernel_add)
+            check(plan, (N, C_, H, K, R, s, shape))
+            plan.stream()
+        if C_ > 4:
+            plan.resident(32, 16, 1, 4)
+            assert "resident_32x16" in plan.kernel and "resident_32x16" in plan.kernel_add
+            check(plan, (N, C_, H, K, R, s, "resident"))
+            plan.resident()
+            plan.select(3, 0)
+            check(plan, (N, C_, H, K, R, s, "tile"))
+        plan.close()
+    assert len(seen) == len(names), seen
+
+
 def runtime():
     from nart_amd import art
     lib = os.path.join(ROOT, "nart_amd", "lib")
@@ -320,7 +376,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
