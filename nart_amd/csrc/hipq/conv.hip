@@ -1557,9 +1557,7 @@ static Kernel kernel_for(const hipq_conv2d_plan *p, const ConvArgs &a, StreamSha
 
 static void resident_name(const hipq_conv2d_plan *p, const ResidentShape &s, char *nm, size_t size, const char *behind)
 {
-    // "stream": the layers that are a stream of weights, whichever of the two kernels they run
-    StreamShape ss;
-    snprintf(nm, size, "conv_mfma_i8_%sresident_%dx%d%s%s%s", stream_applies(p, &ss) ? "stream_" : "", 16 * s.mb, 16 * s.nb * s.nwc,
+    snprintf(nm, size, "conv_mfma_i8_resident_%dx%d%s%s%s", 16 * s.mb, 16 * s.nb * s.nwc,
              p->has_wzp ? "_wzp" : "", p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "", behind);
 }
 

@@ -364,10 +364,13 @@ def test_ip_as_1x1():
     assert np.array_equal(yd.cpu().numpy().reshape(M, -1)[:, :No], want)
 
 
+STREAM_SHAPES = ((128, 16, 4), (64, 32, 4), (64, 16, 4), (32, 16, 4), (32, 32, 4), (16, 16, 4), (16, 32, 4))  # rows, channels, waves
+
+
 def test_fc_streaming_kernel():
-    """Fully-connected layers (op_quant_ip_u8xu8_run, ip.cpp:133-209) on the streaming kernel: BASELINE configs[1] at
-    its stated shape (M=128, K=4096, N=4096, full-range values, log-uniform scales) and the shapes around it, accumulators
-    and bytes against the oracle; every work-group shape the kernel is instantiated for gives the same bytes."""
+    """Fully-connected layers (op_quant_ip_u8xu8_run, ip.cpp:133-209): 128 x 4096 -> 4096 (full-range values, log-uniform scales)
+    and the shapes around it, accumulators and bytes against the oracle, on the kernel that the built-in rule takes and on the
+    streaming kernel in every work-group shape that it is instantiated for."""
     rng = np.random.default_rng(141)
     shapes = [(128, 4096, 4096, False), (1, 512, 1000, False), (64, 2048, 1000, True), (5, 128, 37, False),
               (17, 256, 16, True), (130, 384, 100, False), (256, 1024, 48, False), (33, 1280, 1000, False)]
@@ -385,7 +388,7 @@ def test_fc_streaming_kernel():
         if relu:
             want_y = np.maximum(want_y, q[5]).astype(np.uint8)
         plan = hipq.Conv2d((M, Kd, 1, 1), w.reshape(No, Kd, 1, 1), b, 0, 1, 1, *q, relu=relu)
-        assert "_stream_" in plan.kernel, plan.kernel
+        assert "_stream_" in plan.kernel or "_resident_" in plan.kernel, plan.kernel
         xd = hipq.to_device_nhwc(x.reshape(M, Kd, 1, 1))
         acc = torch.zeros((M, 1, 1, plan.desc.out_cs), dtype=torch.int32, device="cuda")
         yd = plan(xd, acc=acc)
@@ -395,11 +398,17 @@ def test_fc_streaming_kernel():
         first = yd.cpu().numpy().reshape(M, -1)
         assert np.array_equal(first[:, :No], want_y), (M, Kd, No, plan.kernel)
         assert len(np.unique(want_y)) > 8 or M < 8, "degenerate case: the scales saturate the outputs"
-        for rows, cols, waves in ((128, 16, 4), (64, 32, 4), (64, 16, 4), (32, 16, 4), (32, 32, 4), (16, 16, 4), (16, 32, 4)):
+        for rows, cols, waves in STREAM_SHAPES:
             plan.stream(rows, cols, waves)
             assert plan.kernel.endswith("_stream_%dx%d" % (rows, cols)), plan.kernel
             y2 = plan(xd).cpu().numpy().reshape(M, -1)
             assert np.array_equal(y2[:, :No], want_y), (M, Kd, No, rows, cols, waves)
+            plan(xd, acc=acc.zero_())
+            assert np.array_equal(acc.cpu().numpy().reshape(M, -1)[:, :No], want_acc), (M, Kd, No, rows, cols, waves, "accumulators")
+            yf = torch.full((M, No), 7.0, dtype=torch.float32, device="cuda")
+            plan.run_dequant(xd, yf)
+            want_f = np.ascontiguousarray(orc.dequantize_u8(want_y, q[4], q[5])).reshape(M, No)
+            assert np.array_equal(yf.cpu().numpy().view(np.uint32), want_f.view(np.uint32)), (M, Kd, No, rows, cols, waves, "floats")
         plan.stream()
         # the dequantize that reads the layer, in the layer's epilogue (hipq_conv2d_run_dequant): the float bit patterns of
         # op_dequantize_run_u8 on the layer's bytes; refused for another scale or zero point than the bytes are written with
@@ -411,7 +420,7 @@ def test_fc_streaming_kernel():
         assert np.array_equal(yf.cpu().numpy().view(np.uint32), np.ascontiguousarray(want_f).reshape(M, No).view(np.uint32)), (M, Kd, No)
         # the tile kernels serve the same plan when the streaming kernel is switched off, with the same bytes
         plan.special(0)
-        assert "_stream_" not in plan.kernel and not plan.dequant_fusable(q[4], q[5])
+        assert not any(k in plan.kernel for k in ("_stream_", "_resident_")) and not plan.dequant_fusable(q[4], q[5])
         y3 = plan(xd).cpu().numpy().reshape(M, -1)
         assert np.array_equal(y3[:, :No], want_y), (M, Kd, No, plan.kernel)
         plan.close()
@@ -422,9 +431,10 @@ def test_fc_streaming_kernel():
 
 
 def test_streaming_kernel_on_convolutions_over_few_pixels():
-    """conv_mfma_stream_kernel with the general pixel gather: any kernel size, stride and padding over at most 256 output
-    pixels (1024 for long reductions) whose channels are whole 128-byte lines (the late stages of a network at batch 1), accumulators and
-    bytes against the oracle; with the residual add fused, both operand orders; special(0) gives the same bytes."""
+    """conv_mfma_stream_kernel with the general pixel gather, in every work-group shape: any kernel size, stride and padding over at
+    most 1024 output pixels whose channels are whole 128-byte lines (the late stages of a network at batch 1), accumulators and
+    bytes against the oracle; with the residual add fused, both operand orders; the built-in rule's kernel and special(0) give the same
+    bytes."""
     rng = np.random.default_rng(91)
     cases = [  # N, C, H, W, K, R, pad, stride
         (1, 512, 7, 7, 512, 3, 1, 1), (1, 256, 14, 14, 512, 3, 1, 2), (1, 256, 14, 14, 256, 3, 1, 1), (2, 128, 9, 9, 64, 3, 1, 1),
@@ -438,22 +448,30 @@ def test_streaming_kernel_on_convolutions_over_few_pixels():
         ia, wa = rand_q(rng), rand_q(rng)
         q = (ia, int(rng.integers(0, 256)), wa, 128, float(np.float32(ia * wa * np.sqrt(C * R * R) * 40.0)), int(rng.integers(0, 256)))
         kern = check_conv(x, w, b, pad, st, 1, q, tag="stream conv %d" % i)
-        assert "_stream_" in kern, kern
+        assert "_stream_" in kern or "_resident_" in kern, kern
         plan = hipq.Conv2d(x.shape, w, b, pad, st, 1, *q)
-        conv = orc.conv2d_u8(x, w, b, pad, st, 1, *q)
+        conv, conv_acc = orc.conv2d_u8(x, w, b, pad, st, 1, *q, return_acc=True)
         xd = hipq.to_device_nhwc(x)
         res = rng.integers(0, 256, conv.shape, dtype=np.uint8)
         rd = hipq.to_device_nhwc(res)
         ra, rz = float(np.float32(q[4] * (1.0, 1.7, 300.0)[i % 3])), int(rng.integers(0, 256))
         sa, sz = float(np.float32(max(q[4], ra) * 1.3)), int(rng.integers(0, 256))
-        assert "_stream_" in plan.kernel_add and plan.kernel_add.endswith("+add"), plan.kernel_add
-        for res_first in (False, True):
-            want = orc.add_u8(res, conv, ra, rz, q[4], q[5], sa, sz) if res_first else orc.add_u8(conv, res, q[4], q[5], ra, rz, sa, sz)
-            y = plan.empty_output()
-            plan.run_add(xd, rd, res_first, ra, rz, sa, sz, y)
-            assert np.array_equal(hipq.from_device_nhwc(y, K), want), (i, res_first, plan.kernel_add)
+        sums = [orc.add_u8(res, conv, ra, rz, q[4], q[5], sa, sz) if first else orc.add_u8(conv, res, q[4], q[5], ra, rz, sa, sz)
+                for first in (False, True)]
+        for shape in (None,) + STREAM_SHAPES:
+            if shape is not None:
+                plan.stream(*shape)
+                assert "_stream_%dx%d" % shape[:2] in plan.kernel and "_stream_%dx%d" % shape[:2] in plan.kernel_add, (plan.kernel, plan.kernel_add)
+                acc = torch.zeros((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
+                assert np.array_equal(hipq.from_device_nhwc(plan(xd, acc=acc), K), conv), (i, shape)
+                assert np.array_equal(acc.cpu().numpy()[..., :K].transpose(0, 3, 1, 2), conv_acc), (i, shape, "accumulators")
+            assert plan.kernel_add.endswith("+add"), plan.kernel_add
+            for first in (False, True):
+                y = plan.run_add(xd, rd, first, ra, rz, sa, sz, plan.empty_output())
+                assert np.array_equal(hipq.from_device_nhwc(y, K), sums[first]), (i, first, plan.kernel_add)
+        plan.stream()
         plan.special(0)
-        assert "_stream_" not in plan.kernel
+        assert not any(k in plan.kernel for k in ("_stream_", "_resident_"))
         assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), conv), (i, plan.kernel)
 
 
@@ -476,14 +494,25 @@ def test_streaming_kernel_on_any_channel_count(wzp):
         ia, wa = rand_q(rng), rand_q(rng)
         q = (ia, int(rng.integers(0, 256)), wa, wzp, float(np.float32(ia * wa * np.sqrt(C * R * R) * 40.0)), int(rng.integers(0, 256)))
         kern = check_conv(x, w, b, pad, st, 1, q, tag="any channels %d" % i)
-        assert "_stream_" in kern, kern
-        seen.add(kern)
+        assert "_stream_" in kern or "_resident_" in kern, kern
+        want, want_acc = orc.conv2d_u8(x, w, b, pad, st, 1, *q, return_acc=True)
+        plan, xd = hipq.Conv2d(x.shape, w, b, pad, st, 1, *q), hipq.to_device_nhwc(x)
+        for shape in STREAM_SHAPES:
+            plan.stream(*shape)
+            seen.add(plan.kernel)
+            acc = torch.zeros((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
+            got = hipq.from_device_nhwc(plan(xd, acc=acc), K)
+            assert np.array_equal(acc.cpu().numpy()[..., :K].transpose(0, 3, 1, 2), want_acc) and np.array_equal(got, want), (i, plan.kernel)
+            assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), want), (i, plan.kernel)
         if wzp == 128:
             xs, ws = x.view(np.int8), w.view(np.int8)
             p8 = hipq.Conv2d(x.shape, ws, b, pad, st, 1, q[0], 0, q[2], 0, q[4], 0, obits=7, dtype=hipq.DTYPE_I8)
             want8 = orc.conv2d_i8(xs, ws, b, pad, st, 1, q[0], q[2], q[4], 7)
-            assert np.array_equal(hipq.from_device_nhwc(p8(hipq.to_device_nhwc(xs)), K).view(np.int8), want8), i
-    assert len(seen) >= 3, seen
+            for shape in (None,) + STREAM_SHAPES:
+                if shape is not None:
+                    p8.stream(*shape)
+                assert np.array_equal(hipq.from_device_nhwc(p8(hipq.to_device_nhwc(xs)), K).view(np.int8), want8), (i, p8.kernel)
+    assert len(seen) == len(STREAM_SHAPES), seen
 
 
 def test_output_stride_wider_than_the_channels():
@@ -1253,21 +1282,12 @@ def test_two_group_kernel_matches_the_oracle():
         plan = hipq.Conv2d(x.shape, w, b, pad, stride, 1, *q)
         nslab = (R * R * plan.desc.in_cs + 63) // 64
         eligible = nslab % 2 == 0 and nslab >= 8
-        # few pixels of whole 128-byte lines go to the streaming kernel unless a tile is named
-        npix = N * plan.OH * plan.OW
-        stream = plan.desc.in_cs % 128 == 0 and (npix <= 256 or (npix <= 1024 and R * R * plan.desc.in_cs >= 512))
-        assert ("_stream_" in plan.kernel) == stream
-        assert plan.kernel.endswith("_k2") == (eligible and not stream), (plan.kernel, nslab)  # every case has at most 256 tiles of the rule's own tile
         xd = hipq.to_device_nhwc(x)
-        assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), want), (x.shape, K, plan.kernel)
-        if not stream:  # the fused residual add takes the same kernel where it applies, in both operand orders
-            assert plan.kernel_add.endswith("_k2+add") == eligible, plan.kernel_add
-            res = rng.integers(0, 256, want.shape, dtype=np.uint8)
-            ra, rz, sa, sz = rand_q(rng, 1e-2, 1e-1), int(rng.integers(0, 256)), rand_q(rng, 3e-2, 3e-1), int(rng.integers(0, 256))
-            for first in (False, True):
-                yd = plan.run_add(xd, hipq.to_device_nhwc(res), first, ra, rz, sa, sz, plan.empty_output())
-                want_add = orc.add_u8(res, want, ra, rz, q[4], q[5], sa, sz) if first else orc.add_u8(want, res, q[4], q[5], ra, rz, sa, sz)
-                assert np.array_equal(hipq.from_device_nhwc(yd, K), want_add), (x.shape, K, first, plan.kernel_add)
+        assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), want), (x.shape, K, plan.kernel)  # whatever the built-in rule takes
+        res = rng.integers(0, 256, want.shape, dtype=np.uint8)
+        ra, rz, sa, sz = rand_q(rng, 1e-2, 1e-1), int(rng.integers(0, 256)), rand_q(rng, 3e-2, 3e-1), int(rng.integers(0, 256))
+        sums = [orc.add_u8(res, want, ra, rz, q[4], q[5], sa, sz) if first else orc.add_u8(want, res, q[4], q[5], ra, rz, sa, sz)
+                for first in (False, True)]
         plan.special(2)
         for tile in (0, 2, 3, 4):
             plan.select(tile, 0)
@@ -1278,6 +1298,17 @@ def test_two_group_kernel_matches_the_oracle():
             acc = torch.empty((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
             plan(xd, acc=acc)
             assert np.array_equal(acc.cpu().numpy()[..., :K].transpose(0, 3, 1, 2), want_acc), (x.shape, tile)
+            # the fused residual add takes the same kernel where it applies, in both operand orders
+            assert plan.kernel_add.endswith("_k2+add") == eligible, plan.kernel_add
+            for first in (False, True):
+                yd = plan.run_add(xd, hipq.to_device_nhwc(res), first, ra, rz, sa, sz, plan.empty_output())
+                assert np.array_equal(hipq.from_device_nhwc(yd, K), sums[first]), (x.shape, K, first, plan.kernel_add)
+        plan.special(1)
+        plan.select(3, 0)  # by the built-in rule: up to a tile per CU (every case but the last; the long reductions up to 400)
+        assert plan.kernel.endswith("_k2") == (eligible and plan.kernel_add.endswith("_k2+add")), plan.kernel
+        assert plan.kernel.endswith("_k2") == (eligible and (-(-N * plan.OH * plan.OW // 64)) * (-(-plan.desc.out_cs // 128)) <= (400 if nslab >= 32 else 256))
+        assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), want), (x.shape, K, plan.kernel)
+        plan.special(2)
         plan.select(1, 0)  # the 256-pixel tile has no two-group variant
         assert not plan.kernel.endswith("_k2")
         plan.select(3, 3)  # an explicit stage count means the four-wave kernel
@@ -1289,7 +1320,9 @@ def test_two_group_kernel_matches_the_oracle():
         xs, ws = x.view(np.int8), w.view(np.int8)
         want8 = orc.conv2d_i8(xs, ws, b, pad, stride, 1, q[0], q[2], q[4], 7)
         p8 = hipq.Conv2d(x.shape, ws, b, pad, stride, 1, q[0], 0, q[2], 0, q[4], 0, obits=7, dtype=hipq.DTYPE_I8)
-        assert p8.kernel.endswith("_k2") == (eligible and not stream), p8.kernel
+        assert np.array_equal(hipq.from_device_nhwc(p8(hipq.to_device_nhwc(xs)), K).view(np.int8), want8), (x.shape, K, p8.kernel)
+        p8.special(2).select(4, 0)
+        assert p8.kernel.endswith("_k2") == eligible, p8.kernel
         assert np.array_equal(hipq.from_device_nhwc(p8(hipq.to_device_nhwc(xs)), K).view(np.int8), want8), (x.shape, K)
     # asymmetric weights keep the generic kernel
     x = rng.integers(0, 256, (1, 256, 8, 8), dtype=np.uint8)

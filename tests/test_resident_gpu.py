@@ -63,7 +63,7 @@ def test_resident_kernel_matches_the_oracle_in_every_shape(case):
             assert C >= 1024  # the region of a fully-connected layer's rows does not fit LDS
             continue
         print("resident", case, (mb, nb, nwc, ks), plan.kernel, flush=True)
-        assert "resident_%dx%d" % (16 * mb, 16 * nb * nwc) in plan.kernel
+        assert plan.kernel.startswith("conv_mfma_i8_resident_%dx%d" % (16 * mb, 16 * nb * nwc)), plan.kernel
         got = hipq.from_device_nhwc(plan(xd, torch.full_like(plan.empty_output(), 99)), K)
         assert np.array_equal(got, want), (mb, nb, nwc, ks, int((got != want).sum()), np.argwhere(got != want)[:6].tolist())
         acc = torch.zeros((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
