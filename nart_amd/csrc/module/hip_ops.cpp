@@ -383,6 +383,9 @@ bool conv_heads_depthwise_point(op_t *op)
     }
     if (r == nullptr || r->entry->tp != &op_conv_2d_tp || reinterpret_cast<conv_op_t *>(r)->plan == nullptr)
         return false;
+    // a 1x1 layer that begins a whole block is that block's: the executor looks for blocks first and for pairs among what is left, too
+    if (conv_heads_inverted_residual(r))
+        return false;
     conv_op_t *p = reinterpret_cast<conv_op_t *>(r);
     int i = 0;
     const op_t *a = add_reading(r, &i), *next = only_reader(r);

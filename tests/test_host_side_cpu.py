@@ -170,6 +170,40 @@ def small_parade(rt, ws, hw=64):
     return p, one
 
 
+def a_chain_of_separable_layers_is_divided_blocks_first():
+    """Depthwise and 1x1 layers in turn: a 1x1 layer that begins a whole inverted residual block belongs to that block, not to the
+    depthwise layer in front of it - the division that the executor makes as well."""
+    import numpy as np
+    from nart_amd import hipq
+    rt = runtime()
+    ws = rt.workspace("hip")
+    count = {n: getattr(rt.libs[1], "hip_module_fused_" + n) for n in ("inverted", "pairs")}
+    for f in count.values():
+        f.restype = C.c_long
+    kernels = C.c_long.in_dll(STUB, "stub_kernels")
+    for N, HW, widths in ((1, 14, (32, 96, 32)), (1, 14, (32, 96, 32, 64)), (1, 28, (16, 64, 24))):
+        # depthwise, 1x1 to widths[1], depthwise, 1x1 to widths[2], ...
+        ops, cur = [], ws.tensor(np.zeros((N, widths[0], HW, HW), np.uint8))
+        plans, c = [], widths[0]
+        for K in widths[1:]:
+            for k, cols, g, out in ((3, 1, c, c), (1, c, 1, K)):
+                w = np.full((out, cols, k, k), 130, np.uint8)
+                ops.append(ws.conv2d(cur, ws.tensor(w), None, k // 2, 1, g, dict(ialpha=0.05, izp=9, walpha=0.002, wzp=128, oalpha=0.05, ozp=9)).prepare())
+                plans.append(hipq.Conv2d((N, c, HW, HW), w, None, k // 2, 1, g, 0.05, 9, 0.002, 128, 0.05, 9))
+                cur = ops[-1].output(0)
+            c = K
+        assert hipq.depthwise_point_fusable(*plans[:2]) and hipq.inverted_residual_fusable(*plans[1:4]), widths
+        last_pair = len(widths) > 3 and hipq.depthwise_point_fusable(*plans[4:6])
+        for again in range(2):  # the first run brings the input into the device's layout as well
+            before, launches = {n: f() for n, f in count.items()}, kernels.value
+            for o in ops:
+                o.run()
+            assert {n: f() - before[n] for n, f in count.items()} == {"inverted": 1, "pairs": int(last_pair)}, widths
+            assert not again or kernels.value - launches == 2 + (0 if len(widths) == 3 else 1 if last_pair else 2), widths
+        for o in ops:
+            o.delete()
+
+
 def a_pass_that_cannot_be_recorded_runs_its_operators():
     """On the null stream, which cannot be captured, and where the runtime refuses the graph: every pass runs operator by
     operator, and no error stays behind for the next launch to find."""
@@ -377,6 +411,7 @@ def operators_of_two_workspaces_wait_for_each_other():
 
 
 CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+         a_chain_of_separable_layers_is_divided_blocks_first,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
