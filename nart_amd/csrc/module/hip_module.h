@@ -62,7 +62,7 @@ struct hip_workspace_t {
     int dev_id;
     hipStream_t stream; // every kernel of this workspace is launched here
     bool own_stream;
-    bool passes;    // operators run as passes that are replayed (hip_pass.cpp): launches cost the host nothing
+    bool passes;    // from the first pass that may be recorded on (hip_pass.cpp): launches are taken to cost the host nothing
     uint64_t epoch; // counts prepare and destroy calls of this workspace's operators (a recorded pass is good for one value)
 };
 

@@ -144,6 +144,7 @@ struct conv_op_t {
     const void *w_seen;    // identity of the weights the plan was packed from
     uint64_t pc_seen;      // checksum of the per-channel weight scales the plan was built with (0: per tensor)
     int defer;             // 0 undecided, 1 leave the launch to the add / relu that reads the output, -1 launch at run()
+    bool defer_in_passes;  // what hip_workspace_t::passes was when that was decided
     // A convolution that heads a bottleneck block (1x1, then 3x3, then 1x1 and the add with the block's input) which
     // hipq_bottleneck_run computes in one launch: the block's 3x3 convolution and its add (else null).
     const op_t *blk_next, *blk_add;
@@ -258,6 +259,16 @@ const op_t *add_reading(const op_t *r, int *idx)
     return a;
 }
 
+// Which operators leave their launches to others depends on whether the workspace runs passes (conv_heads_block): what was decided
+// before its first one is decided anew.
+void decide_again_in_passes(const op_t *op, int *defer, bool *in_passes)
+{
+    const bool passes = reinterpret_cast<const hip_workspace_t *>(op->workspace)->passes;
+    if (*in_passes != passes)
+        *defer = 0;
+    *in_passes = passes;
+}
+
 // op: a 1x1 convolution, r (its only reader): a 3x3 convolution, then a 1x1 convolution, then the add with op's input
 bool conv_heads_block(op_t *op, const op_t *r)
 {
@@ -272,7 +283,7 @@ bool conv_heads_block(op_t *op, const op_t *r)
         return false;
     const conv_op_t *c2 = reinterpret_cast<const conv_op_t *>(r), *c3 = reinterpret_cast<const conv_op_t *>(r2);
     const QSet &qi = add_inputs(a), &qo = add_output(a);
-    // operators that run one by one keep the one launch: one call of the host instead of three
+    // where launches cost the host nothing, few pixels are faster as three launches; operators that run one by one keep the one call
     if (reinterpret_cast<const hip_workspace_t *>(op->workspace)->passes && !hipq_bottleneck_pays(c1->plan))
         return false;
     if (!c1->plan || !c2->plan || !c3->plan || qi.alpha[1 - i] != c1->desc.ialpha || qi.zp[1 - i] != c1->desc.izp
@@ -440,6 +451,7 @@ void conv_run(op_t *op)
         c->computed_ahead = false;
         return;
     }
+    decide_again_in_passes(op, &c->defer, &c->defer_in_passes);
     if (c->defer == 0)
         c->defer = (c->ir_project != op && conv_heads_inverted_residual(op)) || (c->ir_project != nullptr && c->ir_project != op)
                 || conv_heads_depthwise_point(op) || sole_reader_fuses(op)
@@ -585,6 +597,7 @@ struct ew_op_t {
     size_t bytes; // device bytes to process (pad channels included)
     int defer;    // 0 undecided, 1 leave the (fused) launch to a reader of the output (relu: a max pooling; add: a 1x1
                   // convolution), -1 launch at run()
+    bool defer_in_passes; // what hip_workspace_t::passes was when that was decided
 };
 
 const QSet &add_inputs(const op_t *add_op) { return reinterpret_cast<const ew_op_t *>(add_op)->qi; }
@@ -767,7 +780,7 @@ static bool whole_block_chains(op_t *op, op_t *mid, const conv_op_t *c, int o, c
                                         e->qo.bits[0], rc->plan);
 }
 
-// Does the add leave its launch to a reader?  Decided once per prepare: a convolution was deferred into this add, and a
+// Does the add leave its launch to a reader?  Decided once per prepare, and again when the workspace begins to run passes: a convolution was deferred into this add, and a
 // 1x1 convolution of this workspace reads the sum and can run as the tail of the same kernel.
 bool add_defers(op_t *op)
 {
@@ -775,6 +788,7 @@ bool add_defers(op_t *op)
     const int i = deferred_conv_input(op);
     if (i < 0)
         return false;
+    decide_again_in_passes(op, &e->defer, &e->defer_in_passes);
     if (e->defer == 0) {
         static const bool off = getenv("NART_HIP_NO_FUSION") != nullptr;
         e->defer = -1;

@@ -204,6 +204,41 @@ def a_chain_of_separable_layers_is_divided_blocks_first():
             o.delete()
 
 
+def blocks_are_decided_again_for_recorded_passes():
+    """A bottleneck block of few pixels is one launch where its operators run one by one, three where a pass is recorded: also when the
+    operators have run before the workspace's first pass, and again when they are prepared anew."""
+    import numpy as np
+    from nart_amd import hipq
+    rt = runtime()
+    ws = rt.workspace("hip")
+    blocks = rt.libs[1].hip_module_fused_blocks
+    blocks.restype = C.c_long
+    kernels = C.c_long.in_dll(STUB, "stub_kernels")
+    x = ws.tensor(np.zeros((2, 1024, 14, 14), np.uint8))
+    ops, cur = [], x
+    for K, c, k, q in ((256, 1024, 1, dict(ialpha=0.05, izp=9, walpha=0.0011, wzp=128, oalpha=0.06, ozp=0)),
+                       (256, 256, 3, dict(ialpha=0.06, izp=0, walpha=0.0016, wzp=128, oalpha=0.055, ozp=0)),
+                       (1024, 256, 1, dict(ialpha=0.055, izp=0, walpha=0.0035, wzp=128, oalpha=0.07, ozp=121))):
+        ops.append(ws.conv2d(cur, ws.tensor(np.full((K, c, k, k), 130, np.uint8)), None, k // 2, 1, 1, q).prepare())
+        cur = ops[-1].output(0)
+    ops.append(ws.add(cur, x, dict(ialpha=[0.07, 0.05], izp=[121, 9], oalpha=0.09, ozp=0)).prepare())
+
+    def one():
+        before, launches = blocks(), kernels.value
+        for o in ops:
+            o.run()
+        return blocks() - before, kernels.value - launches
+    assert one()[0] == 1  # the first run brings the input into the device's layout as well
+    assert [one() for _ in range(3)] == [(1, 1)] * 3
+    p, pass_of = small_parade(rt, ws)
+    assert pass_of() == "eager"
+    assert [one() for _ in range(3)] == [(0, 3)] * 3, "decided before the workspace ran passes"
+    for o in ops:
+        o.prepare()
+    assert [one() for _ in range(2)] == [(0, 3)] * 2
+    p.delete()
+
+
 def a_pass_that_cannot_be_recorded_runs_its_operators():
     """On the null stream, which cannot be captured, and where the runtime refuses the graph: every pass runs operator by
     operator, and no error stays behind for the next launch to find."""
@@ -411,7 +446,7 @@ def operators_of_two_workspaces_wait_for_each_other():
 
 
 CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
-         a_chain_of_separable_layers_is_divided_blocks_first,
+         a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
