@@ -1412,7 +1412,7 @@ def test_pooling_windows_loaded_at_once(shape, pad, st, ceil_mode, k, method):
     """2x2 and 3x3 windows against the general kernel's 4x4: clipped on every side, images smaller than a window, windows that hang
     over the far edge in ceil mode."""
     if shape[2] + 2 * pad < k or shape[3] + 2 * pad < k:
-        pytest.skip("the window is larger than the padded image")
+        pad = k // 2  # the window would be larger than the padded image
     rng = np.random.default_rng(sum(shape) + k)
     x = rng.integers(0, 256, shape, dtype=np.uint8)
     for q in ((0.02, 0, 0.02, 0), (0.03, 131, 0.05, 120)):

@@ -88,3 +88,73 @@ def test_resident_kernel_matches_the_oracle_in_every_shape(case):
         plan.resident(48, 16, 1, 8)
     plan.resident()
     assert np.array_equal(hipq.from_device_nhwc(plan(xd), K), want), plan.kernel
+
+
+RECTANGULAR = [  # N, C, H, W, K, (R, S), (pad_h, pad_w), (stride_h, stride_w), data type, weight zero point
+    (2, 64, 13, 9, 72, (1, 7), (0, 3), (1, 1), "u8", 128),    # a slab is a whole tap
+    (3, 128, 11, 16, 40, (7, 1), (3, 0), (1, 2), "u8", 128),
+    (2, 64, 9, 14, 130, (3, 5), (0, 2), (2, 1), "u8", 128),
+    (4, 256, 7, 10, 24, (1, 1), (0, 0), (1, 3), "u8", 128),   # 1x1 with a stride in one direction
+    (5, 48, 8, 5, 33, (5, 3), (2, 1), (1, 3), "u8", 128),     # pieces of a slab in different taps
+    (2, 16, 12, 30, 20, (1, 29), (0, 14), (1, 1), "u8", 128),  # as many taps as the masks hold, in one row
+    (1, 32, 31, 6, 20, (29, 1), (14, 0), (2, 1), "u8", 128),  # in one column
+    (2, 80, 10, 7, 50, (4, 2), (1, 0), (3, 1), "i8", 0),      # windows of an even height
+    (2, 20, 9, 12, 17, (2, 5), (0, 1), (2, 3), "u8", 90),     # the weight zero point's sums
+]
+
+
+@pytest.mark.parametrize("case", RECTANGULAR, ids=lambda c: "-".join(map(str, c)).replace(" ", ""))
+def test_windows_pads_and_strides_that_differ_by_direction(case):
+    N, C, H, W, K, (R, S), pad, st, dtype, wzp = case
+    rng = np.random.default_rng(N * 1000 + C + R)
+    x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = rng.integers(*((0, 256) if wzp in (0, 128) else (wzp - 90, wzp + 91)), (K, C, R, S), dtype=np.uint8)
+    b = rng.integers(-30000, 30000, K).astype(np.int32)
+    oa = float(np.float32(0.02 * 0.004 * np.sqrt(C * R * S) * 40.0))
+    if dtype == "i8":
+        xs, ws = x.view(np.int8), w.view(np.int8)
+        want, want_acc = orc.conv2d_i8(xs, ws, b, pad, st, 1, 0.02, 0.004, oa, 7, return_acc=True)
+        want = want.view(np.uint8)
+        plan = hipq.Conv2d(x.shape, ws, b, pad, st, 1, 0.02, 0, 0.004, 0, oa, 0, obits=7, dtype=hipq.DTYPE_I8)
+    else:
+        want, want_acc = orc.conv2d_u8(x, w, b, pad, st, 1, 0.02, 77, 0.004, wzp, oa, 120, return_acc=True)
+        plan = hipq.Conv2d(x.shape, w, b, pad, st, 1, 0.02, 77, 0.004, wzp, oa, 120)
+    assert len(np.unique(want)) > 8
+    xd = hipq.to_device_nhwc(x)
+    for mb, nb, nwc, ks in SHAPES:
+        plan.resident(16 * mb, 16 * nb, nwc, ks)
+        print("resident", case, (mb, nb, nwc, ks), plan.kernel, flush=True)
+        got = hipq.from_device_nhwc(plan(xd, torch.full_like(plan.empty_output(), 99)), K)
+        assert np.array_equal(got, want), (mb, nb, nwc, ks, int((got != want).sum()), np.argwhere(got != want)[:6].tolist())
+        acc = torch.zeros((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
+        plan(xd, acc=acc)
+        assert np.array_equal(acc.cpu().numpy()[..., :K].transpose(0, 3, 1, 2), want_acc), (mb, nb, nwc, ks, "acc")
+
+
+@pytest.mark.parametrize("case", [(1, 64, 56, 56, 128, 3, 1, 2, 128), (1, 256, 14, 14, 256, 3, 1, 1, 128), (11, 2048, 7, 7, 512, 1, 0, 1, 128),
+                                  (2, 242, 27, 31, 130, 5, 2, 2, 128), (4, 100, 40, 40, 120, 3, 1, 1, 101)], ids=lambda c: "-".join(map(str, c)))
+def test_the_built_in_rule_takes_the_kernel(case):
+    N, C, H, W, K, R, pad, st, wzp = case
+    rng = np.random.default_rng(C)
+    x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = rng.integers(wzp - 90, wzp + 91, (K, C, R, R), dtype=np.uint8)
+    b = rng.integers(-30000, 30000, K).astype(np.int32)
+    q = (0.02, 77, 0.004, wzp, float(np.float32(0.02 * 0.004 * np.sqrt(C * R * R) * 40.0)), 120)
+    plan = hipq.Conv2d(x.shape, w, b, pad, st, 1, *q)
+    assert plan.kernel.startswith("conv_mfma_i8_resident_"), plan.kernel
+    want = orc.conv2d_u8(x, w, b, pad, st, 1, *q)
+    assert np.array_equal(hipq.from_device_nhwc(plan(hipq.to_device_nhwc(x)), K), want)
+
+
+def test_layers_outside_the_kernels_range_stay_where_they_were():
+    """More taps than a mask holds, pads of half the window and more: refused by name, and computed by another kernel."""
+    rng = np.random.default_rng(5)
+    for R, S, pad, st in ((7, 7, 3, 1), (5, 6, 0, 1), (3, 3, 2, 1), (2, 2, 1, 1), (1, 1, 1, 1)):
+        x = rng.integers(0, 256, (2, 32, 12, 13), dtype=np.uint8)
+        w = rng.integers(0, 256, (24, 32, R, S), dtype=np.uint8)
+        q = (0.02, 77, 0.004, 128, float(np.float32(0.02 * 0.004 * np.sqrt(32 * R * S) * 40.0)), 120)
+        plan = hipq.Conv2d(x.shape, w, None, pad, st, 1, *q)
+        assert "_resident_" not in plan.kernel
+        with pytest.raises(hipq.HipqError):
+            plan.resident(32, 16, 1, 4)
+        assert np.array_equal(hipq.from_device_nhwc(plan(hipq.to_device_nhwc(x)), 24), orc.conv2d_u8(x, w, None, pad, st, 1, *q)), (R, S, pad)
