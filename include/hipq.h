@@ -180,8 +180,10 @@ int hipq_conv2d_plan_stream(hipq_conv2d_plan *plan, int rows, int cols, int wave
 
 /*
  * Tuning: the shape of the kernel that keeps a layer's pixels in LDS and loads its weights straight into registers
- * (conv_resident.hip).  pixels and channels: a wave's share, 16 x 16 to 128 x 32; channel_waves: waves of a work-group side by side
- * over the output channels; reduction_waves: waves that share every reduction.  0, 0, 0, 0 returns to the built-in rule, which
+ * (conv_resident.hip).  pixels and channels: a wave's share, one of 16 x 16, 32 x 16, 32 x 32, 64 x 16, 64 x 32, 64 x 64, 128 x 32;
+ * channel_waves: waves of a work-group side by side over the output channels; reduction_waves: waves that share every reduction.  The
+ * kernel takes windows of up to 29 taps with less than half of the window as padding, and reductions of up to 131 072 bytes
+ * (window x channel stride).  0, 0, 0, 0 returns to the built-in rule, which
  * takes the kernel where a fitted cost says that it is faster than the tile and streaming kernels.  hipq_conv2d_plan_special
  * (any mode but 1), naming a tile and naming a shape of the streaming kernel leave it to the caller's choice as well.
  * Identical results for every choice.  Shapes that are not built, or whose pixels do not fit LDS, return an error.
@@ -329,7 +331,7 @@ const char *hipq_inverted_residual_kernel(const hipq_conv2d_plan *expand, const 
  * A depthwise 3x3 layer and the 1x1 / stride 1 layer that reads it in one launch, with the add behind them where `residual` is not
  * null: bit-identical to hipq_conv2d_run (hipq_conv2d_run_relu where `relu` is set, for the depthwise layer) twice and hipq_add_u8
  * (src/op/conv_2d_uint8_impl.c:39-165, src/op/add.c:83-148); the tensor in between never travels to memory.  The requirements
- * on the layers are those of hipq_inverted_residual_run, for any number of channels; the residual (scale ralpha, zero point rzp)
+ * on the layers are those of hipq_inverted_residual_run, for up to 2048 channels on either side of the 1x1 layer; the residual (scale ralpha, zero point rzp)
  * has the output's shape.  y must not be x; it may be the residual.
  * hipq_depthwise_point_fusable answers (1 / 0) whether the plans run this way (by rule where it is faster;
  * hipq_conv2d_plan_special(point, 2): wherever it can); hipq_depthwise_point_run fails with an error otherwise.

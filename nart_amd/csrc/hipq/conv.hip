@@ -1388,9 +1388,11 @@ static bool stream_applies(const hipq_conv2d_plan *p, StreamShape *shape = nullp
         return false;
     // Two classes keep the kernels they had: 3x3 layers on 64 channels (resident rows, halo tiles) and 1x1 layers on an image whose
     // last slab is partial (the two-group kernel).  Both sides measured: the rows kernel is level (3.3 and 3.4 us either
-    // way at 49 and 196 pixels, 3.8 against 3.9 at 3136); the halo kernel takes 5.0 where streaming takes 3.4 to 4.4, the
-    // two-group kernel 3.9 to 7.8 where streaming takes 2.6 to 4.6, until some 6000 pixels x 256 channels (5.9 against 20, 5.2
-    // against 12).  What draws the line is the kernel that these layers are pinned to in the tests, not speed.
+    // way at 49 and 196 pixels, 3.8 against 3.9 at 3136); the halo kernel takes 5.0 to 5.3 where streaming takes 3.4 to 4.4 and
+    // conv_resident_kernel 3.3 to 3.9, the two-group kernel 3.9 to 7.8 where streaming takes 2.6 to 4.6 (conv_resident_kernel 3.3 to
+    // 3.7 on 64 to 320 pixels, 4.8 against 4.6 on 13 254), until some 6000 pixels x 256 channels (5.9 against 20, 5.2
+    // against 12).  So for few pixels neither line lies where speed would put it: a plan's name is public, and these layers have kept
+    // theirs so far.
     const ConvArgs &a = p->args;
     const bool point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
     if (!p->has_wzp && !fc
@@ -1454,8 +1456,8 @@ static bool wreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
 // Over more than 512 pixels it is ahead of the register-fed kernel's patches (256 -> 256 at 14x14, batch 64: 12.7 -> 11.2 us)
 // and, by the fitted costs, of the tile and streaming kernels (13x13, batch 11: 9.2 -> 5.3 us).  64-channel layers keep their
 // resident rows but for 32 000 to 90 000 pixels (56x56, batch 12, with the add: 7.4 -> 6.6 us; level at 100 000, 24 against
-// 15 us at 200 000, where the halo of a tile outweighs its nine steps), and up to 4 096 pixels the halo kernel, which they are
-// pinned to in the tests (5.2 us against 3.3 on 2400 pixels of 135 output channels).
+// 15 us at 200 000, where the halo of a tile outweighs its nine steps), and up to 4 096 pixels the halo kernel, as above
+// (5.2 us against 3.3 on 2400 pixels of 135 output channels).
 static bool hreg_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
 {
     double us = 0;
@@ -1475,8 +1477,10 @@ static bool stem3_applies(const hipq_conv2d_plan *p, const ConvArgs &a)
     return p->variant == kMfmaSmallC && p->special >= 1 && !p->tile_selected && !p->has_wzp && conv_stem3x3_applies(a, a.rowb);
 }
 
-// conv_resident_kernel (conv_resident.hip): any layer whose pixels fit LDS.  Against what the tile and the streaming kernels take,
-// fitted to 820 layers of the range that its own cost is fitted to (nine in ten within 15 %).
+// conv_resident_kernel (conv_resident.hip): layers whose pixels fit LDS (conv_resident_applies).  Against what the tile and the streaming
+// kernels take, fitted to 820 layers of the range that its own cost is fitted to (nine in ten within 15 %): also large layers, weight
+// zero points and scales per channel, which tile_cost and stream_cost above, the choice between those two on few pixels, have not
+// seen.
 static double tile_us(const hipq_conv2d_plan *p)
 {
     const ConvArgs &a = p->args;
@@ -1498,10 +1502,10 @@ static double stream_us(const hipq_conv2d_plan *p, const StreamShape &s)
     return 2.56 + (double)((wgs + kCUs - 1) / kCUs) * ((point ? 0.0147 : 0.0233) * (s.mb + s.nb) * a.nslab + 0.193 * s.mb * s.nb + (point ? 0 : 0.34) + (p->d_q ? 0.32 : 0));
 }
 
-// Which shape, if any, the built-in rule takes it in.  The margins are what keeps layers from getting slower where both fits are a few
-// per cent off: with them 3 of 250 layers that changed kernel got more than 4 % slower (and the 250 a quarter faster), 9 with a twentieth
-// throughout.  Layers that have a kernel of their own keep it, and so do those that stream_applies keeps out for the
-// tests' sake.
+// Which shape, if any, the built-in rule takes it in.  The margins, set by hand, are what keeps layers from getting slower where both fits
+// are a few per cent off: of 220 layers that the fits have not seen 69 change kernel and take 0.76 of the time on average, one of them
+// 8 % more (7.1 -> 7.6 us); with a margin of a twentieth throughout three times as many layers of the fit got slower.  Layers that have a
+// kernel of their own keep it, without a comparison, and so do the two classes that stream_applies keeps out.
 static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a)
 {
     ResidentShape s = {0, 0, 0, 0};
@@ -1511,11 +1515,12 @@ static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &
         return {0, 0, 0, 0};
     StreamShape ss;
     const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
-    // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.5 us streamed, 7.7 with resident rows; 128
-    // rows 10.5 against 9.1
+    // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.2 us streamed, 7.6 with resident rows; 128
+    // rows 9.9 against 9.1
     if (streams && fc && ss.mb < 4)
         return {0, 0, 0, 0};
-    // a 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 8.5 against 10.5 us
+    // a 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 7.5 against 8.2 us in its best
+    // shape
     if (!streams && (halo_applies(p) || (point && (a.P > 8192 || a.stride_h > 1 || a.stride_w > 1 || (k2_applies(p) && (a.in_cs % 64 != 0 || a.P > 2048))))))
         return {0, 0, 0, 0};
     const double now = streams ? stream_us(p, ss) : tile_us(p);

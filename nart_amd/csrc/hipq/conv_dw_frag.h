@@ -50,7 +50,7 @@ struct DiagonalTap {
 
 // 16 accumulators (16 consecutive channels of a position) -> their bytes, re-centred (XOR 0x80 = 128 less, as signed bytes).  The rounding
 // and the zero point ride along in the 64-bit multiply-add, and the last shift saturates to signed bytes, which have the 128 in
-// the constants: 5 to 8 % of these kernels, which issue vector instructions for three quarters of their time.
+// the constants: 5 to 8 % of these kernels' time.
 __device__ static __forceinline__ v4i requant_centred(const ConvArgs &a, const v16i &s)
 {
     uint64_t add = (uint64_t)(uint32_t)(a.qadd - (128 << a.qt)) << 32;

@@ -13,11 +13,12 @@
 // The waves of a work-group split the channels of one patch and add their partial sums up in LDS, or, where there are many patches and
 // one slice, every wave has patches of its own.  Output channel tiles are divided into groups: each group computes the depthwise
 // layer again, which costs less than idle CUs, and spreads a 7x7 image over more CUs.
-// What bounds it: many patches of few channels - memory and vector issue (the requantisations); few pixels of many channels - the chain
-// launch, region, slices, sum, in which a CU's vector units and matrix cores take turns.
-// Measured, the two launches -> this one (back to back and warm): 32 -> 16 channels at 112x112, 64 images: 25.0 -> 15.1 us (38 MB of
-// input and output), 1 image: 5.4 -> 3.1; 64 -> 128 at 56x56, stride 2, 1 image: 6.4 -> 4.1; 192 -> 64 at 28x28, stride 2, 6 images:
-// 5.5 -> 4.4; 960 -> 160 at 7x7, 64 images: 9.6 -> 8.4, 1 image: 5.7 -> 6.0 (there the two launches stay).
+// What bounds it: many patches of few channels - memory and vector issue (the requantisations: 44 % of a CU's busy time at 4 clocks an
+// instruction, matrix cores 14 %); few pixels of many channels - the chain launch, region, slices, sum, in which a CU's vector units (29
+// to 35 %) and matrix cores (4 to 7 %) take turns and mostly wait.
+// Measured, the two launches -> this one (back to back and warm): 32 -> 16 channels at 112x112, 64 images: 24.8 -> 14.7 us (38 MB of
+// input and output), 1 image: 5.2 -> 3.0; 64 -> 128 at 56x56, stride 2, 1 image: 6.1 -> 4.1; 192 -> 64 at 28x28, stride 2, 6 images:
+// 5.5 -> 4.3; 960 -> 160 at 7x7, 64 images: 9.9 -> 8.8, 1 image: 5.7 -> 6.1 (there the two launches stay).
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply requantisations.
 #include "conv_dwpoint.h"
 
@@ -492,8 +493,9 @@ double conv_dwpoint_us(const ConvArgs &d, const ConvArgs &p)
 }
 
 // The two launches: their latencies, the bytes of the first one's input and output, the products of the second and its output; fitted to
-// the same pairs (nine in ten within 19 %).  Chosen by this they take 0.80 of the two launches on average, 2 % more than the best choice
-// would, and one in twenty 14 % more.
+// the same pairs (nine in ten within 19 %).  Of 150 pairs that the fits have not seen this fuses 113, which take 0.73 of the two
+// launches on average, two of them longer (8.7 -> 10.2 us, 11.6 -> 12.2); of the other 37 it would have been faster for four (8.0 ->
+// 5.7 us at most).
 double conv_dwpoint_apart_us(const ConvArgs &d, const ConvArgs &p)
 {
     const double in = (double)d.N * d.H * d.W * d.in_cs * 1e-6, mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6;

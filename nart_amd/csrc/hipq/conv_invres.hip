@@ -12,8 +12,8 @@
 //     LDS: the 16 accumulators of a lane are 16 consecutive channels of one position, requantised to 16 bytes of its row in LDS;
 //   * depthwise, also on the matrix cores: for each of the nine taps a diagonal matrix of the slice's 32 weights, made from a dword by
 //     a byte permutation and four ANDs, times the rows at that tap.  31 of 32 products are with zeros, and still nine matrix
-//     instructions and 45 others replace the 130 dot products, byte alignments and LDS reads of 32 outputs of 32 channels: vector issue
-//     is what these kernels wait for, the matrix cores idle;
+//     instructions and 45 others replace the 130 dot products, byte alignments and LDS reads of 32 outputs of 32 channels: the
+//     matrix cores idle, and vector instructions are the largest part of a wave's chain;
 //   * project: the requantised sums are, as they lie in the lanes, one k-step of every output channel tile's reduction, whose
 //     accumulators a wave keeps over its slices.
 // Patches of 2x4 outputs do not fill a multiply's 32 columns.  Theirs keeps the expanded pixels as rows (a lane has four runs of four
@@ -24,16 +24,18 @@
 // Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch and add their partial sums up
 // in LDS.  Many patches and few slices: every wave has a patch of its own and takes all slices through it, so that no barrier
 // and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
-// 55 us at 56x56, batch 64, against 26.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
+// 57 us at 56x56, batch 64, against 26.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
 // instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice; but a wave of 8x8 outputs
-// with a patch of its own holds 100 registers where one of 4x8 holds 60: 28.4 us against 26.2 for that block, 13.3 against 11.2 for
+// with a patch of its own holds 100 registers where one of 4x8 holds 60: 30.6 us against 26.1 for that block, 13.7 against 11.5 for
 // 32 -> 192 -> 32 at 28x28).
-// What bounds it: vector issue - with a patch per wave three quarters of a CU's busy time at batch 64, the requantisations first;
-// with a shared patch the chain launch - region - slices - sum as well.
-// Measured, the three launches -> the depthwise layer as dot products -> this one (batch 64, back to back and warm): 16 -> 96 -> 24 at
-// 112x112, stride 2: 60 -> 33 -> 27.6 us; 24 -> 144 -> 24 at 56x56: 39 -> 33 -> 26.2; 24 -> 144 -> 32, stride 2: 27 -> 20 -> 15.6;
-// 32 -> 192 -> 32 at 28x28: 19.5 -> 14.6 -> 11.2; 64 -> 384 -> 64 at 14x14: 14.9 -> 12 -> 10.3; 96 -> 576 -> 96: 18.3 -> 17.3 -> 14.4;
-// batch 1 (2x4): 8.3 .. 9.6 -> 4.1 .. 6.0.
+// What bounds it, at batch 64: with a patch per wave vector issue first (the requantisations; 54 % of a CU's busy time at 4 clocks an
+// instruction, matrix cores 9 to 10 %).  With a shared patch neither (vector issue 29 to 31 %, matrix cores 3 to 8 %): 1.5 waves
+// per SIMD, each of which goes region - expand - LDS - depthwise - project - sum with a slice after the other and waits in between.
+// Measured, the three launches -> the depthwise layer as dot products -> this one (batch 64, 40 launches back to back, tensors of random
+// bytes, warm): 16 -> 96 -> 24 at 112x112, stride 2: 45 -> 33.6 -> 27.0 us; 24 -> 144 -> 24 at 56x56: 39 -> 31.3 -> 26.1; 24 -> 144 -> 32,
+// stride 2: 25 -> 18.7 -> 14.5; 32 -> 192 -> 32 at 28x28: 16.9 -> 15.0 -> 11.6; 64 -> 384 -> 64 at 14x14: 12.9 -> 11.5 -> 10.6;
+// 96 -> 576 -> 96: 17.1 -> 16.4 -> 15.2; batch 1, 24 -> 144 -> 24: 9.4 -> 5.0 -> 4.8, 96 -> 576 -> 96: 8.9 -> 7.8 -> 7.6.  With a network's own
+// bytes and clamps the blocks with an add take up to 9 % longer (28.6, 12.5, 11.1, 15.7 us at batch 64).
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
 // requantisations, at most 160 input and output channels; with the add stride 1 and as many output as input channels.
 #include "conv_invres.h"

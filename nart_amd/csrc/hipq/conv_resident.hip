@@ -1,5 +1,6 @@
-// Convolutions whose input pixels stay in LDS while the weights go straight into registers: any kernel size, stride, channel count
-// and data type, for the layers that have no kernel of their own.  gfx950 only.
+// Convolutions whose input pixels stay in LDS while the weights go straight into registers: any stride, channel count and data type, and
+// windows of up to 29 taps with less than half of the window as padding (conv_resident_applies), for the layers that have no kernel of
+// their own.  gfx950 only.
 //
 // Reproduces op_conv_2d_u8xu8_run (art/modules/quant/src/op/conv_2d_uint8_impl.c:39-165), op_quant_ip_u8xu8_run (ip.cpp:133-209),
 // their int8 variants and, with a residual, op_quant_add_run (add.c:83-148) bit for bit, like the tile kernels of conv.hip.
@@ -495,7 +496,8 @@ double shape_cost(const ConvArgs &a, const ResidentShape &s)
 
 bool conv_resident_applies(const ConvArgs &a)
 {
-    // the first tap of a pixel is never behind that of the pixel before, and a tap mask has 32 bits
+    // the first tap of a pixel is never behind that of the pixel before (pads below half of the window); a tap mask has 32 bits, and the
+    // loads behind the last slab may enter two taps more; tap numbers by multiplication (m_cpr) hold for 2048 slabs
     return a.group == 1 && a.in_cs % 16 == 0 && a.rowb == a.in_cs && 2 * a.pad_h < a.R && 2 * a.pad_w < a.S && a.R * a.S <= 29 && a.nslab <= 2048;
 }
 

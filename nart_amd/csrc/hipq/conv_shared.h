@@ -49,14 +49,15 @@ struct ConvArgs {
     double inv_ohw, inv_ow; // 1 / (OH*OW), 1 / OW (depthwise 3x3: 1 / work items per row, 1 / channel quads)
     double inv_oh;          // 1 / OH
     // per-output-channel requantisation (a weight scale per channel): multipliers and shifts, padded like bias2;
-    // nullptr = the per-tensor pair in q.  Such plans requantise with the 64-bit form, channel by channel.
+    // nullptr = the per-tensor pair in q.  Channel by channel: with one multiplication where a kernel has that form and fastch allows
+    // it (conv_resident.hip), otherwise with the 64-bit form.
     const uint32_t *qmult;
     const int32_t *qshift;
     int fastch; // 1: the one-multiply requantisation is valid for every channel's shift
     const uint8_t *res; // fused residual add: the other operand (same layout as y), or nullptr
     int res_first;      // 1: the residual is input 0 of the add, the convolution's output input 1
     AddParams addq;
-    // fused dequantize (streaming kernel only): the float value of every output byte, (byte - zero point) * deq_alpha, goes
+    // fused dequantize (streaming and resident kernels): the float value of every output byte, (byte - zero point) * deq_alpha, goes
     // to deq_out[pixel][K] and the bytes themselves are not written; nullptr = off
     float *deq_out;
     float deq_alpha;

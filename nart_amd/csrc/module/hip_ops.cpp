@@ -780,8 +780,9 @@ static bool whole_block_chains(op_t *op, op_t *mid, const conv_op_t *c, int o, c
                                         e->qo.bits[0], rc->plan);
 }
 
-// Does the add leave its launch to a reader?  Decided once per prepare, and again when the workspace begins to run passes: a convolution was deferred into this add, and a
-// 1x1 convolution of this workspace reads the sum and can run as the tail of the same kernel.
+// Does the add leave its launch to a reader?  Decided once per prepare, and again when the workspace begins to run passes: a
+// convolution was deferred into this add, and a 1x1 convolution of this workspace reads the sum and can run as the tail of the same
+// kernel.
 bool add_defers(op_t *op)
 {
     ew_op_t *e = reinterpret_cast<ew_op_t *>(op);
