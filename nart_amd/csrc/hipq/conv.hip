@@ -1504,8 +1504,8 @@ static double stream_us(const hipq_conv2d_plan *p, const StreamShape &s)
 
 // Which shape, if any, the built-in rule takes it in.  The margins, set by hand, are what keeps layers from getting slower where both fits
 // are a few per cent off: of 220 layers that the fits have not seen 69 change kernel and take 0.76 of the time on average, one of them
-// 8 % more (7.1 -> 7.6 us); with a margin of a twentieth throughout three times as many layers of the fit got slower.  Layers that have a
-// kernel of their own keep it, without a comparison, and so do the two classes that stream_applies keeps out.
+// 8 % more (7.1 -> 7.6 us).  Layers that have a kernel of their own keep it, without a comparison, and so do the two classes that
+// stream_applies keeps out.
 static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a)
 {
     ResidentShape s = {0, 0, 0, 0};

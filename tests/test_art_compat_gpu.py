@@ -95,7 +95,19 @@ def test_float_network_ends_and_missing_modules(tmp_path):
     assert ctx2.loaded_workspaces == ["hip"]
 
 
-@pytest.mark.parametrize("build", [lambda: cases.resnet18(N=2, hw=96), lambda: cases.mobilenet_v2(N=1, hw=70), lambda: cases.resnet50(N=2, hw=64)])
+def bottleneck_chain(N, blocks=3):
+    """Identity bottleneck blocks of 256 middle channels on 14x14 images: one launch each, or three in a recorded pass on few images."""
+    c = cases.Case("bottleneck_chain_n%d" % N, 12)
+    t = c.input_u8((N, 1024, 14, 14), 0.0186, 114)
+    for _ in range(blocks):
+        b = c.conv(c.conv(t, 256, 1, ozp=0), 256, 3, ozp=0)
+        t = c.add(c.conv(b, 1024, 1), t)
+    c.output = t
+    return c
+
+
+@pytest.mark.parametrize("build", [lambda: cases.resnet18(N=2, hw=96), lambda: cases.mobilenet_v2(N=1, hw=70), lambda: cases.resnet50(N=2, hw=64),
+                                   lambda: bottleneck_chain(2)])
 def test_recorded_passes_follow_their_inputs(tmp_path, build):
     """The first pass runs operator by operator, the second is recorded, later ones replay the record: every one on new
     inputs, with other GPU work and synchronisations between, with and without a new input, before and after a reshape."""

@@ -237,6 +237,27 @@ def blocks_are_decided_again_for_recorded_passes():
         o.prepare()
     assert [one() for _ in range(2)] == [(0, 3)] * 2
     p.delete()
+    # the passes themselves: operator by operator, recorded and replayed, below and above the pixels from which one launch pays
+    from nart_amd import cases, engine
+    did = {n: C.c_long.in_dll(STUB, "stub_" + n) for n in ("captures", "graph_launches")}
+    for N, want in ((2, 0), (20, 3)):
+        c = cases.Case("chain", 12)
+        t = c.input_u8((N, 1024, 14, 14), 0.0186, 114)
+        for _ in range(3):
+            b = c.conv(c.conv(t, 256, 1, ozp=0), 256, 3, ozp=0)
+            t = c.add(c.conv(b, 1024, 1), t)
+        for _ in range(6):  # long enough to be recorded where the blocks are one launch each
+            t = c.conv(t, 64, 1)
+        c.output = t
+        p = engine.Parade(rt, engine.write_engine(c), [ws])
+        before = {n: v.value for n, v in did.items()}
+        for k in range(4):
+            p.inputs()[0].write(np.zeros((N, 1024, 14, 14), np.uint8))
+            n = blocks()
+            p.run()
+            assert blocks() - n == want, (N, k)
+        assert [v.value - before[n] for n, v in did.items()] == [1, 3], N
+        p.delete()
 
 
 def a_pass_that_cannot_be_recorded_runs_its_operators():
