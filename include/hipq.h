@@ -273,8 +273,8 @@ int hipq_conv2d_run_add2(const hipq_conv2d_plan *plan, const void *x, const hipq
  * op_conv_2d_u8xu8_run (src/op/conv_2d_uint8_impl.c:39-165) three times, then op_quant_add_run (src/op/add.c:83-148) -
  * but t1, t2 and the widening layer's own output never travel to memory.  `reduce`: a 1x1 / stride 1 convolution from
  * CW = 256, 512 or 1024 channels to CM = CW / 4; `mid`: 3x3 / stride 1 / pad 1, CM -> CM; `widen`: 1x1, CM -> CW; all on
- * images whose height and width are multiples of 7, uint8 tensors with dense channel strides, weight zero points 128,
- * per-tensor weight scales, each layer reading its input with the scale and zero point the previous one writes.  The
+ * images whose height and width are multiples of 7 (at CM = 256: any from 7 on), uint8 tensors with dense channel strides, weight
+ * zero points 128, per-tensor weight scales, each layer reading its input with the scale and zero point the previous one writes.  The
  * residual is x itself, read with `reduce`'s input scale and zero point; the add's inputs are (widen(...), x), or
  * (x, widen(...)) when residual_is_input0 != 0; oalpha / ozp / obits (8) describe the sum.  y must not be x.
  * hipq_bottleneck_fusable answers (1 / 0) whether three plans and an add can run this way; hipq_bottleneck_run fails
@@ -353,9 +353,9 @@ const char *hipq_depthwise_point_kernel(const hipq_conv2d_plan *depthwise, const
  * residual, ...) and hipq_conv2d_run(next, y, y_next): op_conv_2d_u8xu8_run (src/op/conv_2d_uint8_impl.c:39-165), then
  * op_quant_add_run (src/op/add.c:83-148), then op_conv_2d_u8xu8_run again; t never travels to memory and y is written
  * but not read back.  `mid`: 3x3 / stride 1 / pad 1, CM -> CM with CM = 64, 128 or 256; `widen`: 1x1, CM -> 4 CM;
- * `next`: 1x1 / stride 1, 4 CM -> CM (the first layer of the next block); images of 8 x 8, 4 x 14 or 7 x 7 pixel patches
- * (height and width multiples of 8 and 8, of 4 and 14, or of 7 and 7); uint8 tensors with dense channel strides, weight
- * zero points 128, per-tensor weight scales, each layer reading its input with the scale and zero point it is written
+ * `next`: 1x1 / stride 1, 4 CM -> CM (the first layer of the next block); images that hold an 8 x 8, a 4 x 14 or a 7 x 7 pixel
+ * patch (where the patches that are used do not divide the image some overlap: y must not be the residual then); uint8 tensors
+ * with dense channel strides, weight zero points 128, per-tensor weight scales, each layer reading its input with the scale and zero point it is written
  * with.  The residual (any tensor of y's shape, e.g. a projection shortcut) and the add are described as in
  * hipq_conv2d_run_add; next_relu as in hipq_conv2d_run_add_conv.  hipq_bottleneck_tail_fusable answers (1 / 0);
  * hipq_bottleneck_tail_run fails with an error otherwise (run the operators separately).

@@ -2588,6 +2588,8 @@ extern "C" int hipq_bottleneck_tail_run(const hipq_conv2d_plan *p2, const hipq_c
                  "hipq_bottleneck_tail_run: these plans (%s, %s%s%s) and this add do not run as one kernel: run hipq_conv2d_run, "
                  "hipq_conv2d_run_add and hipq_conv2d_run", p2->name.c_str(), p3->name.c_str(), next ? ", " : "",
                  next ? next->name.c_str() : "");
+    HIPQ_REQUIRE(y != residual || conv_block_tail_disjoint(a2),
+                 "hipq_bottleneck_tail_run: on a %dx%d image patches overlap, so the sum cannot overwrite the residual", a2.OH, a2.OW);
     a2.x = static_cast<const uint8_t *>(x);
     a2.y = nullptr;
     a2.acc_out = a3.acc_out = nullptr;

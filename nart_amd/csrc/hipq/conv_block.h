@@ -21,6 +21,8 @@ long long conv_block_pixels();
 // the add's parameters, sum to a3.y) and - an != nullptr - the 1x1 convolution that reads the sum (output to an->y).
 bool conv_block_tail_applies(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an);
 void launch_conv_block_tail(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st);
+// no two patches share a pixel
+bool conv_block_tail_disjoint(const ConvArgs &a2);
 bool conv_block_tail_preferred(const ConvArgs &a2, bool chained);
 
 } // namespace hipq

@@ -30,7 +30,7 @@
 // accumulators are 16 consecutive channels of one pixel: one 128-bit LDS or global store, no transpose.
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
 // requantisation in all three layers, 32-bit form of the add to 8 bits, CM of 64, 128 or 256, image height and width
-// multiples of 7.
+// multiples of 7 - or, with CM = 256, any from 7 on: the last patch then overlaps its neighbour and both compute the same bytes.
 #include "conv_block.h"
 #include "conv_frag.h"
 
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(128 * G, 2) void conv_bottleneck_kernel(const ConvA
         return;
     const int ppi = geo.PY * geo.PX;
     const int n = gid / ppi, pr = gid - n * ppi, pi = pr / geo.PX, pj = pr - pi * geo.PX;
-    const int y0 = pi * kPatch, x0 = pj * kPatch;
+    const int y0 = min(pi * kPatch, geo.H - kPatch), x0 = min(pj * kPatch, geo.W - kPatch); // the last ones end where the image does
     const int ry0 = max(y0 - 1, 0), rx0 = max(x0 - 1, 0);
     const int RW = min(x0 + kPatch, geo.W - 1) - rx0 + 1, RH = min(y0 + kPatch, geo.H - 1) - ry0 + 1;
     const int M1 = RW * RH;          // pixels of the region: at most 81 (64 when MT1 == 2: the host checks)
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
         return;
     const int ppi = geo.PY * geo.PX;
     const int n = gid / ppi, pr = gid - n * ppi, pi = pr / geo.PX, pj = pr - pi * geo.PX;
-    const int y0 = pi * PH, x0 = pj * PW;
+    const int y0 = min(pi * PH, geo.H - PH), x0 = min(pj * PW, geo.W - PW); // the last ones end where the image does
 
     // ---- the 3x3 layer's input patch with its border -> LDS, re-centred; out-of-image positions read the pad source ----
     {
@@ -496,18 +496,27 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
     }
 }
 
-// the patch shape of the tail kernel for an H x W image: 8x8 fills every pixel slot, 4x14 seven in eight, 7x7 three in four
+// The patch shape of the tail kernel for an H x W image: the one that covers it with the fewest patches, so that the ones an image is
+// a multiple of come first (8x8 fills every pixel slot, 4x14 seven in eight, 7x7 three in four).  Where a side is no multiple, the last
+// patch ends where the image does and computes the pixels that it shares with its neighbour again: the same bytes, written twice.
 static bool tail_patch(int H, int W, int *ph, int *pw)
 {
-    if (H % 8 == 0 && W % 8 == 0)
-        *ph = 8, *pw = 8;
-    else if (H % 4 == 0 && W % 14 == 0)
-        *ph = 4, *pw = 14;
-    else if (H % 7 == 0 && W % 7 == 0)
-        *ph = 7, *pw = 7;
-    else
-        return false;
-    return true;
+    static const int shapes[][2] = {{8, 8}, {4, 14}, {7, 7}};
+    int best = 0;
+    for (const auto &s : shapes) {
+        if (H < s[0] || W < s[1])
+            continue;
+        const int n = ((H + s[0] - 1) / s[0]) * ((W + s[1] - 1) / s[1]);
+        if (best == 0 || n < best)
+            best = n, *ph = s[0], *pw = s[1];
+    }
+    return best > 0;
+}
+
+bool conv_block_tail_disjoint(const ConvArgs &a2)
+{
+    int ph = 0, pw = 0;
+    return tail_patch(a2.OH, a2.OW, &ph, &pw) && a2.OH % ph == 0 && a2.OW % pw == 0;
 }
 
 bool conv_block_tail_applies(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an)
@@ -541,7 +550,7 @@ template <int G, int PH, int PW, int ST>
 static void launch_tail_gp(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
 {
     BlockGeom geo;
-    geo.H = a2.OH, geo.W = a2.OW, geo.PY = a2.OH / PH, geo.PX = a2.OW / PW;
+    geo.H = a2.OH, geo.W = a2.OW, geo.PY = (a2.OH + PH - 1) / PH, geo.PX = (a2.OW + PW - 1) / PW;
     geo.IH = a2.H, geo.IW = a2.W;
     geo.npatch = a2.N * geo.PY * geo.PX;
     const dim3 grid((unsigned)((geo.npatch + 7) / 8 * 8)), block(128 * G);
@@ -579,7 +588,20 @@ void launch_conv_block_tail(const ConvArgs &a2, const ConvArgs &a3, const ConvAr
 
 // Measured at batch 64: blocks of 256 middle channels (14x14 images) 25.6 us against 8.0 + 13.2 + 14.5 and two launch
 // gaps; 128 channels (28x28) 40.6 against 49.0, where the tail form below does better still; 64 channels lose.
-bool conv_block_preferred(const ConvArgs &a1) { return a1.out_cs == 256; }
+// Images that are no multiple of 7 either way need as many patches as the next larger one, so the line is drawn by what both
+// sides were measured to take (256 middle channels, 9x9 to 18x18, 8 to 64 images): 20 + 0.032 for every patch a generation of
+// one work-group per CU, 12 + 0.00194 a pixel for the three launches.  13x13: 16 images 21.1 against 17.9, 32 23.3 against 23.0,
+// 64 28.1 against 34.3; 12x12, 64 images 27.7 against 32.1; 10x10 26.4 against 24.0; 16x16 71 against 42.
+bool conv_block_preferred(const ConvArgs &a1)
+{
+    if (a1.out_cs != 256)
+        return false;
+    if (a1.H % kPatch == 0 && a1.W % kPatch == 0)
+        return true;
+    const double patches = (double)a1.N * ((a1.H + kPatch - 1) / kPatch) * ((a1.W + kPatch - 1) / kPatch);
+    const double gens = (double)(((long long)patches + 255) / 256);
+    return gens * 20 + 0.032 * patches < 12 + 0.00194 * a1.P;
+}
 
 // A work-group reads the block's 1.1 MB of weights for its 49 or so pixels, so the kernel takes 20 us however few there are, where
 // three launches that spread the weights over the chip take 10.5.  ResNet-50 at 224x224, its five blocks as one launch each -> as
@@ -589,7 +611,14 @@ long long conv_block_pixels() { return 20 * 196; }
 // Measured at batch 64: 128 middle channels (28x28 images) 32 us with the next layer, 27 without, against 14.0 + 28.6
 // and a launch gap; 64 channels (56x56) 43 to 48 with the next layer against 13.8 + 37.3 and the gap, but 58 without
 // (the sum's pixel tile is what that form saves); 256 channels belong to the whole-block kernel.
-bool conv_block_tail_preferred(const ConvArgs &a2, bool chained) { return a2.in_cs == 128 || (a2.in_cs == 64 && chained); }
+// Images that no patch divides, with the next layer: 64 channels at 50x50, 1 / 11 / 64 images 10.0 / 17.5 / 40.6 us as two or three launches,
+// 8.3 / 13.6 / 37.2 as one; at 25x25 10.0 / 12.1 / 20.0 and 7.7 / 8.1 / 15.2; 128 channels at 25x25 11.1 / 14.2 / 36.3 and 9.4 / 10.8 / 28.8, at 13x13
+// 10.0 / 11.0 / 16.8 and 10.0 / 10.3 / 11.4.  With twice the channels in the next layer 128 channels lose up to 1.2 us below some 600
+// pixels (20x20, 1 image 10.4 against 11.4; 25x25 10.9 against 10.8).
+bool conv_block_tail_preferred(const ConvArgs &a2, bool chained)
+{
+    return (a2.in_cs == 128 && (conv_block_tail_disjoint(a2) || a2.P >= 600)) || (a2.in_cs == 64 && chained);
+}
 
 bool conv_block_applies(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an)
 {
@@ -611,14 +640,14 @@ bool conv_block_applies(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &
         && same_image(a2)
         && one(a3) && a3.C == cm && a3.in_cs == cm && a3.K == cw && a3.out_cs == cw && a3.nslab == cm / 64 && a3.kout_pad >= cw
         && same_image(a3) && a3.res != nullptr && a3.addq.fast && a3.addq.hi == 255
-        && a1.H % kPatch == 0 && a1.W % kPatch == 0 && (long long)a1.N * a1.H * a1.W * cw < (1ll << 31);
+        && a1.H >= kPatch && a1.W >= kPatch && (cm == 256 || (a1.H % kPatch == 0 && a1.W % kPatch == 0)) && (long long)a1.N * a1.H * a1.W * cw < (1ll << 31);
 }
 
 template <int G>
 static void launch_block_g(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
 {
     BlockGeom geo;
-    geo.H = a1.H, geo.W = a1.W, geo.PY = a1.H / kPatch, geo.PX = a1.W / kPatch;
+    geo.H = a1.H, geo.W = a1.W, geo.PY = (a1.H + kPatch - 1) / kPatch, geo.PX = (a1.W + kPatch - 1) / kPatch;
     geo.npatch = a1.N * geo.PY * geo.PX;
     const dim3 grid((unsigned)((geo.npatch + 7) / 8 * 8)), block(128 * G);
     const bool small = geo.PY <= 2 && geo.PX <= 2; // every region is at most 8 x 8 pixels

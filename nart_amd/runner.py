@@ -364,7 +364,12 @@ class HipqExecutor:
                 plans = [conv_plan(c)[0] for c in (c1, c2, c3)]
                 st = T[add.output]
                 # a part of a batch fuses exactly where the whole did
-                pays = hipq.bottleneck_pays(plans[0]) if self.share is None else self.share[0].buf.get(c1.output) is None
+                if self.share is None:
+                    pays = hipq.bottleneck_pays(plans[0])
+                else:
+                    pays = self.share[0].buf.get(c1.output) is None
+                    if pays:
+                        plans[0].special(2)
                 if pays and hipq.bottleneck_fusable(plans[0], plans[1], plans[2], ci == 1, st.alpha, st.zp):
                     self.blocks[id(add)] = (c1, c2, c3)
                     for c, p in zip((c1, c2, c3), plans):
@@ -401,6 +406,12 @@ class HipqExecutor:
                 if c2 is None or any(id(c) in self.in_block for c in (c2, c3)) or c3.attrs["pad"] != 0 or c2.attrs["pad"] != 1:
                     continue
                 p2, p3 = conv_plan(c2)[0], conv_plan(c3)[0]
+                if self.share is not None:  # as above
+                    if self.share[0].buf.get(c2.output) is not None:
+                        self._early.setdefault(id(c2), p2)
+                        self._early.setdefault(id(c3), p3)
+                        continue
+                    p2.special(2)
                 st, ot = T[add.output], T[add.inputs[1 - ci]]
                 nxt, pn = None, None
                 for nd in uses.get(add.output, []):

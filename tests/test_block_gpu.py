@@ -663,3 +663,58 @@ def test_whole_blocks_pay_from_some_pixels_on(n, pays):
     p = hipq.Conv2d((n, 1024, 14, 14), w, np.zeros(256, np.int32), 0, 1, 1, 0.05, 9, 0.001, 128, 0.06, 0)
     assert hipq.bottleneck_pays(p) == pays
     assert hipq.bottleneck_pays(p.special(2))
+
+
+RAGGED_TAILS = [  # N, CW, H, W: the last patch of a row or column overlaps its neighbour by all but one, by one, or not at all
+    (2, 256, 9, 15), (1, 256, 25, 25), (1, 512, 13, 29), (3, 512, 5, 15), (2, 512, 25, 25), (1, 1024, 9, 8), (1, 256, 7, 8), (1, 512, 15, 8),
+]
+
+
+@pytest.mark.parametrize("case", RAGGED_TAILS, ids=lambda c: "x".join(map(str, c)))
+def test_bottleneck_tail_on_ragged_images(case):
+    """Images that no patch divides: the pixels that two patches share are computed by both and lie where one of them would put them."""
+    test_bottleneck_tail(case)
+
+
+@pytest.mark.parametrize("case", [(2, 512, 13, 13, 25, 26), (1, 512, 9, 17, 18, 33), (1, 512, 25, 25, 50, 49)], ids=lambda c: "x".join(map(str, c)))
+def test_strided_bottleneck_tail_on_ragged_images(case):
+    test_bottleneck_tail_with_a_strided_3x3_layer(case)
+
+
+@pytest.mark.parametrize("case", [(2, 1024, 13, 13), (1, 1024, 8, 8), (1, 1024, 7, 9), (1, 1024, 16, 10)], ids=lambda c: "x".join(map(str, c)))
+def test_bottleneck_block_on_ragged_images(case):
+    test_bottleneck_block(case)
+
+
+def test_overlapping_patches_do_not_overwrite_their_residual():
+    """A patch reads its residual before it writes the sum, its neighbour's shared pixels perhaps after: y must be another tensor there
+    (and may be the residual where patches are disjoint)."""
+    rng = np.random.default_rng(11)
+    for H, W, ok in ((16, 16, True), (16, 17, False)):
+        t1, res, layers, rq, sq, nx = make_tail(rng, 1, 256, H, W, False)
+        plans = plans_of(t1, layers)
+        xd, rd, want = hipq.to_device_nhwc(t1), hipq.to_device_nhwc(res), torch.zeros_like(hipq.to_device_nhwc(res))
+        hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], want)
+        if ok:
+            hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], rd)
+            torch.cuda.synchronize()
+            assert torch.equal(rd, want)
+        else:
+            with pytest.raises(hipq.HipqError, match="cannot overwrite the residual"):
+                hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], rd)
+
+
+@pytest.mark.parametrize("n, hw, block, tail", [(11, 13, False, True), (64, 13, True, True), (64, 10, False, True), (1, 20, False, False), (2, 20, False, True)])
+def test_rules_on_ragged_images(n, hw, block, tail):
+    """Where the one-launch forms are chosen on images that their patches do not divide: whole blocks by the two fitted costs, tails of 128
+    channels with a wider next layer from 600 pixels on."""
+    rng = np.random.default_rng(n)
+    x, xq, layers, sq = make_block(rng, 1, 1024, 7, 7)
+    shapes = ((n, 1024, hw, hw), (n, 256, hw, hw), (n, 256, hw, hw))
+    plans = [hipq.Conv2d(s, L["w"], L["b"], L["pad"], 1, 1, *L["q"]) for s, L in zip(shapes, layers)]
+    assert hipq.bottleneck_fusable(*plans, False, sq[0], sq[1]) == block
+    t1, res, tl, rq, sq2, nx = make_tail(rng, 1, 512, 7, 7, False, True)
+    p2 = hipq.Conv2d((n, 128, hw, hw), tl[0]["w"], tl[0]["b"], 1, 1, 1, *tl[0]["q"])
+    p3 = hipq.Conv2d((n, 128, hw, hw), tl[1]["w"], tl[1]["b"], 0, 1, 1, *tl[1]["q"])
+    pn = hipq.Conv2d((n, 512, hw, hw), nx["w"], nx["b"], 0, 1, 1, *nx["q"])
+    assert hipq.bottleneck_tail_fusable(p2, p3, False, rq[0], rq[1], sq2[0], sq2[1], pn) == tail
