@@ -268,6 +268,18 @@ int hipq_conv2d_run_add2(const hipq_conv2d_plan *plan, const void *x, const hipq
                          int shortcut_is_input0, float oalpha, int ozp, int obits, void *y, void *stream);
 
 /*
+ * Two convolutions that do not depend on each other - the first layer of a residual block and its projection shortcut - in one
+ * launch, bit-identical to hipq_conv2d_run (hipq_conv2d_run_relu where relu / relu_other is set) on each: op_conv_2d_u8xu8_run
+ * (src/op/conv_2d_uint8_impl.c:39-165) twice.  Both from a multiple of 64 channels with a window that conv_resident_kernel
+ * takes, uint8 tensors, weight zero points 128, per-tensor weight scales.  Neither may write what the other reads or writes.
+ * hipq_conv2d_pair_fusable answers (1 / 0): where one launch is faster by rule, or, after hipq_conv2d_plan_special(plan, 2),
+ * wherever it is possible; hipq_conv2d_run_pair fails with an error where it is not.
+ */
+int hipq_conv2d_pair_fusable(const hipq_conv2d_plan *plan, const hipq_conv2d_plan *other);
+int hipq_conv2d_run_pair(const hipq_conv2d_plan *plan, const void *x, int relu, void *y, const hipq_conv2d_plan *other,
+                         const void *x_other, int relu_other, void *y_other, void *stream);
+
+/*
  * An identity bottleneck block of a residual network in one launch: y = add(widen(mid(reduce(x))), x), bit-identical to
  * hipq_conv2d_run(reduce, x, t1), hipq_conv2d_run(mid, t1, t2) and hipq_conv2d_run_add(widen, t2, residual = x, ...) -
  * op_conv_2d_u8xu8_run (src/op/conv_2d_uint8_impl.c:39-165) three times, then op_quant_add_run (src/op/add.c:83-148) -

@@ -2546,6 +2546,59 @@ extern "C" int hipq_conv2d_run_add2(const hipq_conv2d_plan *p, const void *x, co
     return launch_status("conv_wreg_dual_kernel");
 }
 
+// Two layers that do not depend on each other - a block's first layer and its projection shortcut - in one launch of
+// conv_resident_kernel's tiles
+static bool pair_shapes(const hipq_conv2d_plan *p, const hipq_conv2d_plan *q, ResidentShape *sp, ResidentShape *sq, double *us)
+{
+    for (const hipq_conv2d_plan *l : {p, q})
+        if (!l || l->variant != kMfma || !l->special || l->tile_selected || l->stream.mb || l->resident_named || l->has_wzp)
+            return false;
+    return conv_resident_choose_pair(p->args, q->args, sp, sq, us);
+}
+
+extern "C" int hipq_conv2d_pair_fusable(const hipq_conv2d_plan *p, const hipq_conv2d_plan *q)
+{
+    ResidentShape sp, sq;
+    double us;
+    if (!pair_shapes(p, q, &sp, &sq, &us))
+        return 0;
+    if (p->special == 2)
+        return 1;
+    // built-in rule: few pixels, where each of the two is little more than a launch; with more work the kernels that they have on their
+    // own are ahead of conv_resident_kernel's tiles.  Measured on 3x3 / stride 2 layers and their 1x1 shortcuts as two launches and as one:
+    // 64 -> 128 channels at 56x56, 1 / 8 / 16 / 32 images 6.8 / 8.1 / 9.0 / 11.3 and 5.1 / 6.6 / 8.2 / 12.4 us; 128 -> 256 at 28x28
+    // 6.9 / 8.2 / 8.5 / 9.8 and 4.7 / 6.3 / 7.9 / 10.3; 256 -> 512 at 14x14 7.1 / 9.0 / 11.1 / 13.1 and 4.9 / 6.1 / 8.1 / 10.6.  16 images are 16 million
+    // of outputs x slabs (of which the shortcut has a tenth)
+    double work = 0;
+    for (const hipq_conv2d_plan *l : {p, q})
+        work += (double)l->args.P * l->args.K * l->args.nslab;
+    return work <= 20e6 ? 1 : 0;
+}
+
+extern "C" int hipq_conv2d_run_pair(const hipq_conv2d_plan *p, const void *x, int relu, void *y, const hipq_conv2d_plan *q, const void *xq,
+                                    int relu_q, void *yq, void *stream)
+{
+    clear_error();
+    HIPQ_REQUIRE(p && q && x && y && xq && yq, "hipq_conv2d_run_pair: null argument");
+    HIPQ_REQUIRE(y != yq && yq != x && y != xq, "hipq_conv2d_run_pair: neither layer may write what the other reads or writes");
+    HIPQ_REQUIRE(!(relu && p->d.dtype != HIPQ_DTYPE_U8) && !(relu_q && q->d.dtype != HIPQ_DTYPE_U8),
+                 "hipq_conv2d_run_pair: relu for uint8 plans only (op_quant_relu_run is a uint8 operator)");
+    ResidentShape sp, sq;
+    double us;
+    HIPQ_REQUIRE(pair_shapes(p, q, &sp, &sq, &us), "hipq_conv2d_run_pair: these two plans (%s, %s) do not run in one launch: run hipq_conv2d_run "
+                 "twice", p->name.c_str(), q->name.c_str());
+    ConvArgs a = p->args, b = q->args;
+    a.x = static_cast<const uint8_t *>(x), a.y = static_cast<uint8_t *>(y);
+    b.x = static_cast<const uint8_t *>(xq), b.y = static_cast<uint8_t *>(yq);
+    a.acc_out = b.acc_out = nullptr;
+    if (relu)
+        a.lo = std::min(p->d.ozp, a.q.hi); // the ReLU clamp, as in hipq_conv2d_run_relu
+    if (relu_q)
+        b.lo = std::min(q->d.ozp, b.q.hi);
+    launch_conv_resident_pair(a, sp, b, sq, static_cast<hipStream_t>(stream));
+    return launch_status("conv_resident_pair_kernel");
+}
+
 // hipq_bottleneck_tail_*: the launch arguments of the three layers; false if the chain does not run as one kernel
 static bool tail_args(const hipq_conv2d_plan *p2, const hipq_conv2d_plan *p3, int residual_is_input0, float res_alpha, int res_zp,
                       float oalpha, int ozp, int obits, const hipq_conv2d_plan *next, ConvArgs *a2, ConvArgs *a3, ConvArgs *an)

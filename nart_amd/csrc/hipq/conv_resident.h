@@ -16,6 +16,9 @@ bool conv_resident_applies(const ConvArgs &a);
 bool conv_resident_cost(const ConvArgs &a, const ResidentShape &s, double *us);
 // the cheapest shape; false: none
 bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us);
+// two layers that do not depend on each other in one launch: shapes for both; false: they do not run that way
+bool conv_resident_choose_pair(const ConvArgs &a, const ConvArgs &b, ResidentShape *sa, ResidentShape *sb, double *us);
+void launch_conv_resident_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, const ResidentShape &t, hipStream_t st);
 void launch_conv_resident(const ConvArgs &a, const ResidentShape &s, hipStream_t st);
 
 } // namespace hipq

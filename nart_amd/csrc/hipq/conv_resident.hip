@@ -74,23 +74,20 @@ enum Finish { kTensor, kChannels, kAny };
 
 } // namespace
 
-// SPLIT: several waves share a reduction
+// The tile gid of a layer.  SPLIT: several waves share a reduction
 template <int MB, int NB, bool SPLIT, int GATHER, int FINISH>
-__global__ __launch_bounds__(512) void conv_resident_kernel(const ResidentGeom geo, const ConvArgs a)
+__device__ static __forceinline__ void resident_tile(const ResidentGeom &geo, const ConvArgs &a, const int gid, uint8_t *const lds)
 {
     constexpr int D = NB == 1 ? (MB == 1 ? 9 : 8) : NB == 2 && MB < 8 ? 6 : FINISH == kTensor || MB < 8 ? 4 : 2; // slabs of weights ahead
     constexpr int XD = MB == 1 ? 3 : 2; // slabs of pixel operands, the present one among them
     constexpr bool CENTRE = GATHER != kPoint && !SPLIT; // re-centre the region in LDS, not every operand
     static_assert(D % XD == 0, "ring positions");
-    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
     // all of geo at once: the compiler would load it piece by piece as it is used, a round trip each
     asm volatile("" ::"s"(geo.x), "s"(geo.wpack), "s"(geo.bias2), "s"(geo.wslab), "s"(geo.xmask), "s"(geo.h), "s"(geo.sh_w), "s"(geo.last), "s"(geo.total), "s"(geo.nload), "s"(geo.rb),
                  "s"(geo.m_ks), "s"(geo.m_ohw), "s"(geo.per), "s"(geo.oh), "s"(geo.taprows));
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = geo.nwaves;
     const int r = lane & 15, q = lane >> 4;
-    // work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of the list
-    const int gid = (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8);
     if (gid >= geo.total)
         return;
     const int outer = (int)quot(gid, geo.m_tile), inner = gid - outer * (geo.mt_inner ? geo.mtiles : geo.ntiles);
@@ -374,6 +371,37 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(const ResidentGeom g
     }
 }
 
+// work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of a layer's list
+template <int MB, int NB, bool SPLIT, int GATHER, int FINISH>
+__global__ __launch_bounds__(512) void conv_resident_kernel(const ResidentGeom geo, const ConvArgs a)
+{
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    resident_tile<MB, NB, SPLIT, GATHER, FINISH>(geo, a, (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8), lds);
+}
+
+namespace {
+
+struct PairArgs {
+    ResidentGeom geo;
+    ConvArgs a;
+};
+
+} // namespace
+
+// Two layers that do not depend on each other in one launch: the first work-groups of every XCD take the first layer's tiles.  What it is
+// for is a block's 3x3 / stride 2 layer and its 1x1 shortcut on few images, each a launch's latency and little else: 64 -> 128 channels at
+// 56x56, one image, 6.8 us as two launches, 5.1 as one; 256 -> 512 at 14x14 7.1 and 4.9; ResNet-18 at batch 1, three such pairs, 97.3 ->
+// 88.4 us.  Bound by the larger layer's chain of pixels, weights and sums.
+template <int MB, int NB, bool SPLIT>
+__global__ __launch_bounds__(512) void conv_resident_pair_kernel(const PairArgs first, const PairArgs second)
+{
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    const int xcd = (int)(blockIdx.x % 8), i = (int)(blockIdx.x / 8);
+    const bool behind = i >= first.geo.per_xcd;
+    const PairArgs &k = ((const PairArgs *)__builtin_amdgcn_kernarg_segment_ptr())[behind ? 1 : 0]; // by address: no select per argument
+    resident_tile<MB, NB, SPLIT, kWhole, kTensor>(k.geo, k.a, xcd * k.geo.per_xcd + i - (behind ? first.geo.per_xcd : 0), lds);
+}
+
 namespace {
 
 uint32_t magic(int d) { return (uint32_t)(((1ull << 31) + d - 1) / d); }
@@ -406,10 +434,9 @@ long long tiles(const ConvArgs &a, const ResidentShape &s)
     return m * n * std::max(m, n);
 }
 
-template <int MB, int NB, bool SPLIT>
-void launch_shape(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
+ResidentGeom geometry(const ConvArgs &a, const ResidentShape &s)
 {
-    const int nw = s.nwc * s.ks, lds = lds_bytes(a, s);
+    const int MB = s.mb, NB = s.nb, nw = s.nwc * s.ks;
     ResidentGeom g;
     g.x = a.x, g.wpack = a.wpack, g.bias2 = a.bias2;
     g.wslab = (uint32_t)a.kout_pad * 64, g.kout_pad = (uint32_t)a.kout_pad, g.padword = a.padword, g.xmask = a.xmask;
@@ -429,6 +456,14 @@ void launch_shape(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
     g.taprows = 0;
     for (int i = 0; i < a.R; i++)
         g.taprows |= 1u << (i * a.S);
+    return g;
+}
+
+template <int MB, int NB, bool SPLIT>
+void launch_shape(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
+{
+    const int nw = s.nwc * s.ks, lds = lds_bytes(a, s);
+    const ResidentGeom g = geometry(a, s);
     const dim3 grid((unsigned)(g.per_xcd * 8)), block(64 * nw);
     if (a.bwz != 0 || a.acc_out != nullptr || a.deq_out != nullptr || !(a.qmult != nullptr ? a.fastch : a.fastq))
         hipLaunchKernelGGL((conv_resident_kernel<MB, NB, SPLIT, kPieces, kAny>), grid, block, lds, st, g, a);
@@ -538,6 +573,59 @@ void launch_conv_resident(const ConvArgs &a, const ResidentShape &s, hipStream_t
     case 42: launch_tile<4, 2>(a, s, st); break;
     case 44: launch_tile<4, 4>(a, s, st); break;
     default: launch_tile<8, 2>(a, s, st); break;
+    }
+}
+
+namespace {
+
+// both layers as their tiles of whole 64-byte slabs, requantised with one scale
+bool pair_applies(const ConvArgs &a)
+{
+    return conv_resident_applies(a) && a.in_cs % 64 == 0 && a.bwz == 0 && a.acc_out == nullptr && a.deq_out == nullptr && a.qmult == nullptr && a.fastq && a.lo >= 0;
+}
+
+template <int MB, int NB>
+void launch_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, const ResidentShape &t, hipStream_t st)
+{
+    const PairArgs first = {geometry(a, s), a}, second = {geometry(b, t), b};
+    const dim3 grid((unsigned)((first.geo.per_xcd + second.geo.per_xcd) * 8)), block(64 * s.nwc * s.ks);
+    const int lds = std::max(lds_bytes(a, s), lds_bytes(b, t));
+    if (s.ks > 1 || t.ks > 1)
+        hipLaunchKernelGGL((conv_resident_pair_kernel<MB, NB, true>), grid, block, lds, st, first, second);
+    else
+        hipLaunchKernelGGL((conv_resident_pair_kernel<MB, NB, false>), grid, block, lds, st, first, second);
+}
+
+} // namespace
+
+bool conv_resident_choose_pair(const ConvArgs &a, const ConvArgs &b, ResidentShape *sa, ResidentShape *sb, double *us)
+{
+    if (!pair_applies(a) || !pair_applies(b))
+        return false;
+    double best = 1e30;
+    for (const ResidentShape &s : kShapes)
+        for (const ResidentShape &t : kShapes) {
+            double ta, tb;
+            if (s.mb != t.mb || s.nb != t.nb || s.nwc * s.ks != t.nwc * t.ks || s.mb * s.nb > 8 || !conv_resident_cost(a, s, &ta) || !conv_resident_cost(b, t, &tb)
+                || (s.mb > 1 && (8 * s.mb >= (a.P + 15) / 16 * 16 || 8 * s.mb >= (b.P + 15) / 16 * 16)))
+                continue;
+            // the larger one's time, and half of what the smaller one takes beside its launch: its tiles share CUs
+            const double c = std::max(ta, tb) + 0.5 * (std::min(ta, tb) - 2.2);
+            if (c < best)
+                best = c, *sa = s, *sb = t;
+        }
+    *us = best;
+    return best < 1e30;
+}
+
+void launch_conv_resident_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, const ResidentShape &t, hipStream_t st)
+{
+    switch (s.mb * 10 + s.nb) {
+    case 11: launch_pair<1, 1>(a, s, b, t, st); break;
+    case 21: launch_pair<2, 1>(a, s, b, t, st); break;
+    case 22: launch_pair<2, 2>(a, s, b, t, st); break;
+    case 41: launch_pair<4, 1>(a, s, b, t, st); break;
+    default: launch_pair<4, 2>(a, s, b, t, st); break;
     }
 }
 

@@ -61,6 +61,8 @@ _SIGS = {
     "hipq_conv2d_add2_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_conv2d_run_add2": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int,
                                        C.c_void_p, C.c_void_p]),
+    "hipq_conv2d_pair_fusable": (C.c_int, [C.c_void_p, C.c_void_p]),
+    "hipq_conv2d_run_pair": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
     "hipq_bottleneck_pays": (C.c_int, [C.c_void_p]),
     "hipq_bottleneck_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int]),
     "hipq_bottleneck_conv_fusable": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_float, C.c_int, C.c_int, C.c_void_p]),
@@ -367,6 +369,18 @@ def run_add2(plan, x, shortcut, x_shortcut, shortcut_first, oalpha, ozp, y, obit
     check(lib().hipq_conv2d_run_add2(plan.handle, _ptr(x), shortcut.handle, _ptr(x_shortcut), int(bool(shortcut_first)), oalpha, ozp,
                                      obits, _ptr(y), _stream()))
     return y
+
+
+def pair_fusable(plan, other):
+    """Do two convolutions that do not depend on each other run as one launch (include/hipq.h: hipq_conv2d_pair_fusable)?"""
+    return bool(lib().hipq_conv2d_pair_fusable(plan.handle, other.handle))
+
+
+def run_pair(plan, x, y, other, x_other, y_other, relu=False, relu_other=False):
+    """y = plan(x) and y_other = other(x_other) in one launch (include/hipq.h: hipq_conv2d_run_pair)."""
+    check(lib().hipq_conv2d_run_pair(plan.handle, _ptr(x), int(bool(relu)), _ptr(y), other.handle, _ptr(x_other), int(bool(relu_other)),
+                                     _ptr(y_other), _stream()))
+    return y, y_other
 
 
 def bottleneck_fusable(reduce, mid, widen, residual_first, oalpha, ozp, obits=8):

@@ -213,6 +213,19 @@ class HipqExecutor:
                 self.fused.pop(node.output, None)
                 if out is None:
                     raise RuntimeError("shared executor: %s is fused away in the parent but not here" % y.name)
+                other = self._pair_of(node, plan, conv_plan, done) if fuse_add else None
+                if other is not None:
+                    # a block's first layer and its projection shortcut, which read the same tensor, in one launch
+                    nd, p2, nb2 = other
+                    y2 = self.buf[nd.output] = self._tensor(T[nd.output])
+                    if y2 is None:
+                        raise RuntimeError("shared executor: %s is fused away in the parent but not here" % nd.output)
+                    self.plans.append(p2)
+                    done.add(id(nd))
+                    fn = (lambda p=plan, i=ins[0], o=out, p2=p2, y2=y2: hipq.run_pair(p, i, o, p2, i, y2))
+                    self.steps.append({"label": node.output, "kind": "conv, conv", "kernel": "conv_mfma_i8_resident_pair", "fn": fn,
+                                       "ops": plan.ops + p2.ops, "bytes": nbytes + nb2 - int(np.prod(x.shape)), "plan": plan})
+                    continue
                 fn = (lambda p=plan, i=ins[0], o=out: p(i, o))
                 self._add(node, plan.kernel, fn, plan.ops, nbytes)
                 self.steps[-1]["plan"] = plan
@@ -330,6 +343,19 @@ class HipqExecutor:
                 self._add(node, "add_u8_kernel", fn, 0, 3 * int(np.prod(y.shape)))
             else:
                 raise ValueError("unknown node kind " + node.kind)
+
+    def _pair_of(self, node, plan, conv_plan, done):
+        """A later convolution that reads what this one reads and that one launch computes with it (hipq.pair_fusable), with its plan
+        and bytes; None: there is none."""
+        for nd in self.case.nodes[self.case.nodes.index(node) + 1:]:
+            if (nd.kind != "conv" or nd.inputs[0] != node.inputs[0] or nd.attrs["group"] != 1 or id(nd) in done or id(nd) in self.in_block
+                    or id(nd) in self.invres or id(nd) in self.pairs or nd.output in self.fused):
+                continue
+            p2, nb2 = conv_plan(nd)
+            if hipq.pair_fusable(plan, p2):
+                return nd, p2, nb2
+            self._early[id(nd)] = p2
+        return None
 
     def _find_blocks(self, conv_plan):
         """Identity bottleneck blocks - 1x1, 3x3, 1x1 and the add of the last one's output with the first one's input,

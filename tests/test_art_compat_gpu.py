@@ -165,3 +165,25 @@ def test_arrays_of_every_size_reach_the_device(shape):
             want = orc.dequantize_u8(q, alpha, zp)
             assert np.array_equal(outputs[c.output.name].view(np.uint32), want.reshape(outputs[c.output.name].shape).view(np.uint32)), (kind, k)
             assert np.array_equal(parade._inputs[c.input.name].numpy().view(np.uint8), np.array(x).view(np.uint8))
+
+
+@pytest.mark.parametrize("n", [1, 3])
+def test_first_layer_and_shortcut_run_as_one_launch_in_recorded_passes(n, tmp_path):
+    """ResNet-18's three strided stages begin with two convolutions of one tensor: from the second pass on one launch computes both, in the
+    pass that is recorded and in every replay, and new inputs give the oracle's bytes each time."""
+    import ctypes
+    case = cases.resnet18(N=n, hw=64, seed=3)
+    fp = _write(str(tmp_path), case)
+    parade = art.load_parade(fp, art.create_context_from_json(fp + ".json"))
+    inputs, outputs = art.get_empty_io(parade)
+    chained = ctypes.CDLL(os.path.join(os.path.dirname(art.__file__), "lib", "libart_module_hip.so")).hip_module_chained_convs
+    chained.restype = ctypes.c_long
+    rng = np.random.default_rng(n)
+    for k in range(5):
+        x = rng.integers(0, 256, case.input.shape, dtype=np.uint8)
+        inputs[case.input.name][:] = x
+        before = chained()
+        parade.run(inputs, outputs)
+        assert chained() - before == (3 if k else 0), k
+        want = casecpu.run_case(case, x)[case.output.name].reshape(n, -1)
+        assert np.array_equal(outputs[case.output.name], want), k

@@ -158,3 +158,57 @@ def test_layers_outside_the_kernels_range_stay_where_they_were():
         with pytest.raises(hipq.HipqError):
             plan.resident(32, 16, 1, 4)
         assert np.array_equal(hipq.from_device_nhwc(plan(hipq.to_device_nhwc(x)), 24), orc.conv2d_u8(x, w, None, pad, st, 1, *q)), (R, S, pad)
+
+
+PAIRS = [  # N, (C, H, W, K, R, stride) of both layers: a block's first layer and its shortcut, and layers of other inputs
+    (1, (64, 56, 56, 128, 3, 2), (64, 56, 56, 128, 1, 2)),
+    (2, (512, 7, 7, 512, 3, 1), (256, 14, 14, 512, 1, 2)),
+    (3, (128, 13, 11, 72, 3, 2), (128, 13, 11, 40, 1, 2)),   # ragged in pixels and channels
+    (16, (64, 40, 40, 128, 3, 2), (64, 40, 40, 128, 1, 2)),  # many tiles of both
+    (1, (64, 5, 5, 16, 1, 1), (1024, 3, 3, 264, 3, 1)),      # one tile beside many slabs, the smaller layer first
+    (5, (64, 9, 7, 200, 5, 1), (192, 1, 1, 33, 1, 1)),       # 25 taps; fully connected
+]
+
+
+@pytest.mark.parametrize("case", PAIRS, ids=lambda c: "-".join("x".join(map(str, v)) if isinstance(v, tuple) else str(v) for v in c))
+def test_two_layers_in_one_launch_match_the_oracle(case):
+    N, *layers = case
+    rng = np.random.default_rng(77 + N + layers[0][0])
+    plans, xs, wants = [], [], []
+    for C, H, W, K, R, st in layers:
+        x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+        w = rng.integers(0, 256, (K, C, R, R), dtype=np.uint8)
+        b = rng.integers(-30000, 30000, K).astype(np.int32)
+        q = (0.02, int(rng.integers(0, 256)), 0.004, 128, float(np.float32(0.02 * 0.004 * np.sqrt(C * R * R) * 150.0)), int(rng.integers(60, 160)))
+        plans.append(hipq.Conv2d(x.shape, w, b, R // 2, st, 1, *q))
+        xs.append(hipq.to_device_nhwc(x))
+        wants.append((orc.conv2d_u8(x, w, b, R // 2, st, 1, *q), q[5]))
+    plans[0].special(2)
+    for relus in ((False, False), (True, False), (False, True)):
+        assert hipq.pair_fusable(*plans)
+        ys = [p.empty_output().fill_(7) for p in plans]
+        hipq.run_pair(plans[0], xs[0], ys[0], plans[1], xs[1], ys[1], *relus)
+        torch.cuda.synchronize()
+        for y, (want, ozp), relu, layer in zip(ys, wants, relus, layers):
+            want = np.maximum(want, ozp).astype(np.uint8) if relu else want
+            bad = hipq.from_device_nhwc(y, layer[3]) != want
+            assert not bad.any(), (layer, relu, int(bad.sum()), np.argwhere(bad)[:8].tolist())
+            assert len(np.unique(want)) > 8
+
+
+def test_what_does_not_run_as_a_pair():
+    """int8 tensors, weight zero points, scales per channel, channels that are no multiple of 64, more work than the rule allows, and a layer
+    that writes what the other reads."""
+    def layer(N=1, C=64, H=14, K=64, dtype=hipq.DTYPE_U8, wzp=128, wa=0.004):
+        i8 = dtype == hipq.DTYPE_I8
+        w = np.ones((K, C, 3, 3), np.int8 if i8 else np.uint8)
+        return hipq.Conv2d((N, C, H, H), w, None, 1, 1, 1, 0.02, 0 if i8 else 120, wa, 0 if i8 else wzp, 0.1, 0 if i8 else 120, obits=7 if i8 else 8, dtype=dtype)
+    good = layer()
+    assert hipq.pair_fusable(good, layer()) and not hipq.pair_fusable(layer(64, 256, 28, 256), good)
+    for other in (layer(dtype=hipq.DTYPE_I8), layer(wzp=101), layer(wa=np.full(64, 0.004, np.float32)), layer(C=48)):
+        assert not hipq.pair_fusable(good, other) and not hipq.pair_fusable(other, good)
+    x, y = torch.zeros((1, 14, 14, 64), dtype=torch.uint8, device="cuda"), good.empty_output()
+    with pytest.raises(hipq.HipqError, match="do not run in one launch"):
+        hipq.run_pair(good, x, y, layer(wzp=101), x, torch.zeros_like(y))
+    with pytest.raises(hipq.HipqError, match="neither layer"):
+        hipq.run_pair(good, x, y, layer(), y, torch.zeros_like(y))
