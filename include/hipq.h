@@ -181,11 +181,13 @@ int hipq_conv2d_plan_stream(hipq_conv2d_plan *plan, int rows, int cols, int wave
 /*
  * Tuning: the shape of the kernel that keeps a layer's pixels in LDS and loads its weights straight into registers
  * (conv_resident.hip).  pixels and channels: a wave's share, one of 16 x 16, 32 x 16, 32 x 32, 64 x 16, 64 x 32, 64 x 64, 128 x 32;
- * channel_waves: waves of a work-group side by side over the output channels; reduction_waves: waves that share every reduction.  The
- * kernel takes windows of up to 29 taps with less than half of the window as padding, and reductions of up to 131 072 bytes
- * (window x channel stride).  0, 0, 0, 0 returns to the built-in rule, which
- * takes the kernel where a fitted cost says that it is faster than the tile and streaming kernels.  hipq_conv2d_plan_special
- * (any mode but 1), naming a tile and naming a shape of the streaming kernel leave it to the caller's choice as well.
+ * channel_waves: waves of a work-group side by side over the output channels; reduction_waves: waves that share every reduction.
+ * reduction_waves 0 names the form with 32 x 32 tiles, a share of 128 or 64 pixels by 64 or 32 channels and 1 to 8 channel_waves;
+ * launches with what that form does not compute (weight zero points other than 128, accumulators or floats to write, a residual beside
+ * a scale per channel) run another kernel.  The kernel takes windows of up to 29 taps with less than half of the window as padding, and
+ * reductions of up to 131 072 bytes (window x channel stride).  0, 0, 0, 0 returns to the built-in rule, which takes the kernel where a
+ * fitted cost says that it is faster than the tile and streaming kernels.  hipq_conv2d_plan_special (any mode but 1), naming a tile and
+ * naming a shape of the streaming kernel leave it to the caller's choice as well.
  * Identical results for every choice.  Shapes that are not built, or whose pixels do not fit LDS, return an error.
  */
 int hipq_conv2d_plan_resident(hipq_conv2d_plan *plan, int pixels, int channels, int channel_waves, int reduction_waves);

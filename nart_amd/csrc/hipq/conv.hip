@@ -1314,7 +1314,9 @@ struct hipq_conv2d_plan {
     bool tile_selected = false;     // hipq_conv2d_plan_select named a tile: the tile kernels, not the streaming kernel
     int dwpoint_shape = -1; // the same of the depthwise layer and this plan as one kernel (hipq_depthwise_point_select)
     int invres_shape = -1; // patch shape of the inverted residual block this plan projects (hipq_inverted_residual_select); -1: by cost
-    ResidentShape resident = {0, 0, 0, 0}, resident_add = {0, 0, 0, 0}; // of conv_resident_kernel, without and with a residual; mb = 0: another kernel
+    // of conv_resident_kernel, without [0] and with a residual [1]; mb = 0: another kernel.  narrow: for launches that a shape with 32 x 32
+    // tiles cannot take
+    ResidentShape resident[2] = {}, narrow[2] = {};
     bool resident_named = false;           // by the caller (hipq_conv2d_plan_resident)
     StreamShape stream = {0, 0, 0}; // explicit shape of the streaming kernel (hipq_conv2d_plan_stream); mb = 0: built-in rule
     bool has_wzp;
@@ -1506,26 +1508,37 @@ static double stream_us(const hipq_conv2d_plan *p, const StreamShape &s)
 // are a few per cent off: of 220 layers that the fits have not seen 69 change kernel and take 0.76 of the time on average, one of them
 // 8 % more (7.1 -> 7.6 us).  Layers that have a kernel of their own keep it, without a comparison, and so do the two classes that
 // stream_applies keeps out.
-static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a)
+static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a, ResidentShape *narrow)
 {
-    ResidentShape s = {0, 0, 0, 0};
-    double us;
+    ResidentShape s = {0, 0, 0, 0}, wide = {0, 0, 0, 0};
+    *narrow = s;
+    double us = 1e30, wide_us = 1e30;
     if (!(p->variant == kMfma && p->special == 1 && !p->tile_selected && !p->stream.mb && conv_resident_applies(a)) || hreg_applies(p, a) || wreg_applies(p, a)
-        || rows_applies(p, a) || expand_applies(p, a) || pointwise_applies(p) || !conv_resident_choose(a, &s, &us))
+        || rows_applies(p, a) || expand_applies(p, a) || pointwise_applies(p))
         return {0, 0, 0, 0};
     StreamShape ss;
-    const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1;
+    const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1, halo = !streams && halo_applies(p);
+    const double now = streams ? stream_us(p, ss) : tile_us(p), margin = streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
     // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.2 us streamed, 7.6 with resident rows; 128
-    // rows 9.9 against 9.1
-    if (streams && fc && ss.mb < 4)
-        return {0, 0, 0, 0};
-    // a 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 7.5 against 8.2 us in its best
-    // shape
-    if (!streams && (halo_applies(p) || (point && (a.P > 8192 || a.stride_h > 1 || a.stride_w > 1 || (k2_applies(p) && (a.in_cs % 64 != 0 || a.P > 2048))))))
-        return {0, 0, 0, 0};
-    const double now = streams ? stream_us(p, ss) : tile_us(p);
-    const double margin = streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
-    return us < margin * now ? s : ResidentShape{0, 0, 0, 0};
+    // rows 9.9 against 9.1.  A 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 7.5
+    // against 8.2 us in its best shape
+    const bool small = streams ? fc && ss.mb < 4 : halo || (point && (a.P > 8192 || a.stride_h > 1 || a.stride_w > 1 || (k2_applies(p) && (a.in_cs % 64 != 0 || a.P > 2048))));
+    if (small || !conv_resident_choose(a, &s, &us) || us >= margin * now)
+        s = {0, 0, 0, 0}, us = now;
+    *narrow = s;
+    // With 32 x 32 tiles, for layers with work for every SIMD, against whichever of the others it would be.  The halo kernel keeps its layers of
+    // few pixels, as above; a 1x1 layer with a stride would fill LDS with pixels that nobody reads, and one with one scale has no
+    // requantisation to gain by (136 -> 135 channels, 15 images of 94x81, 15.8 us in tiles and 19.1 here; 641 -> 443, 7 of 32x33, 8.4
+    // and 9.0).  The margins leave out what the fits cannot tell apart: of 900 layers 44 change kernel, from 0.96 to 1.42 times as fast,
+    // 1.17 on average.  Scales per channel and signed ranges, which the other kernels requantise in twice the instructions, gain 1.05 to 1.75
+    // times down to the line; what the fit gives the 16 x 16 tiles for those is a sixth below what they measure (96 -> 200 channels
+    // on 25 125 pixels: 10.8 us estimated, 14.2 measured, 12.4 here), so that their line lies as much higher.
+    const bool few = halo && a.P <= 8192, channels = a.qmult != nullptr || a.lo < 0;
+    const double line = !channels ? 0.88 : s.mb && s.ks == 1 ? 1.08 : 0.97;
+    if (!few && !(streams && fc && ss.mb < 4) && !(point && (!channels || a.stride_h > 1 || a.stride_w > 1)) && conv_resident_choose_wide(a, &wide, &wide_us)
+        && wide_us < line * us)
+        return wide;
+    return s;
 }
 
 // the arguments of a launch with a residual that ordinary scale ratios and 8 bits allow: which kernel it goes to hangs on these
@@ -1538,12 +1551,19 @@ static ConvArgs with_residual(const hipq_conv2d_plan *p)
     return a;
 }
 
+// the shape of conv_resident_kernel for a launch; mb = 0: another kernel's
+static ResidentShape resident_for(const hipq_conv2d_plan *p, const ConvArgs &a)
+{
+    const ResidentShape s = p->resident[a.res != nullptr];
+    return s.mb && s.ks == 0 && !conv_resident_wide_applies(a) ? p->narrow[a.res != nullptr] : s;
+}
+
 // The kernel that a launch of a plan with these arguments goes to: its name and its launch both come from here.  A shape that
 // the caller names is run.
 enum class Kernel { kResident, kStream, kHreg, kWreg, kRows, kExpand, kStem3, kTile };
 static Kernel kernel_for(const hipq_conv2d_plan *p, const ConvArgs &a, StreamShape *stream)
 {
-    if ((a.res != nullptr ? p->resident_add : p->resident).mb)
+    if (resident_for(p, a).mb)
         return Kernel::kResident;
     if (p->stream.mb && stream_applies(p, stream))
         return Kernel::kStream;
@@ -1570,13 +1590,15 @@ static void set_mfma_name(hipq_conv2d_plan *p, bool smallc)
 {
     char nm[96];
     StreamShape ss;
-    if (!p->resident_named) {
-        p->resident = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, p->args);
-        p->resident_add = smallc ? ResidentShape{0, 0, 0, 0} : choose_resident(p, with_residual(p));
-    }
+    if (!p->resident_named)
+        for (int add = 0; add < 2; add++) {
+            p->resident[add] = p->narrow[add] = {0, 0, 0, 0};
+            if (!smallc)
+                p->resident[add] = choose_resident(p, add ? with_residual(p) : p->args, &p->narrow[add]);
+        }
     const char *const sgn = p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "";
     switch (kernel_for(p, p->args, &ss)) {
-    case Kernel::kResident: resident_name(p, p->resident, nm, sizeof nm, ""); break;
+    case Kernel::kResident: resident_name(p, resident_for(p, p->args), nm, sizeof nm, ""); break;
     case Kernel::kStream: snprintf(nm, sizeof nm, "conv_mfma_i8_stream_%dx%d%s", 16 * ss.mb, 16 * ss.nb, sgn); break;
     case Kernel::kHreg: snprintf(nm, sizeof nm, "conv_mfma_i8_hreg3x3"); break;
     case Kernel::kWreg: snprintf(nm, sizeof nm, "conv_mfma_i8_wreg"); break;
@@ -1895,7 +1917,7 @@ extern "C" const char *hipq_conv2d_plan_kernel_add(const hipq_conv2d_plan *p)
     StreamShape ss;
     const char *const sgn = p->d.dtype == HIPQ_DTYPE_I8 ? "_signed" : "";
     switch (kernel_for(p, a, &ss)) {
-    case Kernel::kResident: resident_name(p, p->resident_add, buf, sizeof buf, "+add"); break;
+    case Kernel::kResident: resident_name(p, resident_for(p, with_residual(p)), buf, sizeof buf, "+add"); break;
     case Kernel::kStream: snprintf(buf, sizeof buf, "conv_mfma_i8_stream_%dx%d%s+add", 16 * ss.mb, 16 * ss.nb, sgn); break;
     case Kernel::kHreg: snprintf(buf, sizeof buf, "conv_mfma_i8_hreg3x3+add"); break;
     case Kernel::kWreg: snprintf(buf, sizeof buf, "conv_mfma_i8_wreg+add"); break;
@@ -1977,7 +1999,8 @@ extern "C" int hipq_conv2d_plan_resident(hipq_conv2d_plan *p, int pixels, int ch
                  reduction_waves, p->name.c_str());
     HIPQ_REQUIRE(p->variant == kMfma, "hipq_conv2d_plan_resident: only the MFMA kernels have variants (this plan runs %s)", p->name.c_str());
     p->resident_named = named;
-    p->resident = p->resident_add = s;
+    for (int add = 0; add < 2; add++)
+        p->resident[add] = s, p->narrow[add] = {0, 0, 0, 0};
     set_mfma_name(p, false);
     return 0;
 }
@@ -2739,7 +2762,7 @@ static int run_conv(const hipq_conv2d_plan *p, ConvArgs &a, hipStream_t st)
     case kMfma:
     case kMfmaSmallC:
         switch (StreamShape ss; kernel_for(p, a, &ss)) {
-        case Kernel::kResident: launch_conv_resident(a, a.res != nullptr ? p->resident_add : p->resident, st); return launch_status(p->name.c_str());
+        case Kernel::kResident: launch_conv_resident(a, resident_for(p, a), st); return launch_status(p->name.c_str());
         case Kernel::kStream: launch_conv_stream(a, ss, st); return launch_status(p->name.c_str());
         case Kernel::kHreg: launch_conv_hreg(a, st); return launch_status(p->name.c_str());
         case Kernel::kWreg: launch_conv_wreg(a, st); return launch_status(p->name.c_str());

@@ -5,7 +5,8 @@
 
 namespace hipq {
 
-// a work-group's share: 16 mb pixels by 16 nb nwc output channels; ks waves share every reduction, so it has nwc ks of them
+// a work-group's share: 16 mb pixels by 16 nb nwc output channels; ks waves share every reduction, so it has nwc ks of them.  ks = 0: the
+// form with 32 x 32 tiles (mb and nb even), nwc waves
 struct ResidentShape {
     int mb, nb, nwc, ks;
 };
@@ -16,6 +17,9 @@ bool conv_resident_applies(const ConvArgs &a);
 bool conv_resident_cost(const ConvArgs &a, const ResidentShape &s, double *us);
 // the cheapest shape; false: none
 bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us);
+// the same among the shapes with 32 x 32 tiles, which not every launch of a plan can take: conv_resident_wide_applies
+bool conv_resident_wide_applies(const ConvArgs &a);
+bool conv_resident_choose_wide(const ConvArgs &a, ResidentShape *shape, double *us);
 // two layers that do not depend on each other in one launch: shapes for both; false: they do not run that way
 bool conv_resident_choose_pair(const ConvArgs &a, const ConvArgs &b, ResidentShape *sa, ResidentShape *sb, double *us);
 void launch_conv_resident_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, const ResidentShape &t, hipStream_t st);

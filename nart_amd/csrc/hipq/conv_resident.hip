@@ -22,10 +22,15 @@
 // kernel); 128 -> 128, 3x3, at 28x28 4.6 -> 4.1; 256 -> 256 at 14x14 4.6 -> 3.9; 512 -> 512 at 7x7 6.5 -> 4.9 (streaming kernel);
 // 2048 -> 512, 1x1, 11 images of 7x7 8.8 -> 7.0; int8 with a scale per channel, 96 -> 200, 3x3, five images of 75x67 18.2 -> 12.3;
 // 242 -> 394, 5x5 / stride 2, six images of 47x54 35 -> 20.
+//
+// Layers with work for every SIMD go through the same LDS rows in 32 x 32 tiles (conv_resident_wide_kernel), a launch of several
+// layers in one list of work-groups (conv_resident_pair_kernel).
 #include "conv_resident.h"
 
 #include <algorithm>
 #include <cmath>
+
+#include "conv_frag.h"
 
 namespace hipq {
 
@@ -379,6 +384,251 @@ __global__ __launch_bounds__(512) void conv_resident_kernel(const ResidentGeom g
     resident_tile<MB, NB, SPLIT, GATHER, FINISH>(geo, a, (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8), lds);
 }
 
+// The same with 32 x 32 tiles, for layers with work for every SIMD: a wave owns 32 MT pixels by 32 NT channels and the whole reduction.
+// Both tile sizes multiply at the same rate, but the larger needs half of the operand bytes for it: MT pixel operands of LDS and NT
+// weight operands per MT NT multiplies.  In the loop the matrix pipe bounds it (on operands of random bytes a SIMD gives one such multiply
+// per 49 clocks); the rest is the fill of LDS before it and the requantisation behind it, which another
+// work-group of the CU fills where LDS holds two.  Signed and per-channel results leave through
+// the saturating pack of two pixels of a channel.  Measured on rotating tensors, before (the 16 x 16 form or the tile kernel) -> after:
+// 46 -> 83, 3x3, 26 images of 101x103 39 -> 24.7 us; 16 -> 16, 3x3, 62 images of 134x182 60 -> 26; int8 with a scale per channel, 96 -> 200,
+// 3x3, five images of 75x67 14.2 -> 12.4; 1x1 with a scale per channel 28 -> 16.
+template <int MT, int NT, int GATHER, int FINISH>
+__global__ __launch_bounds__(512, 2) void conv_resident_wide_kernel(const ResidentGeom geo, const ConvArgs a)
+{
+    constexpr int D = MT * NT == 8 ? 6 : 8; // steps of weights ahead, two a slab
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+    asm volatile("" ::"s"(geo.x), "s"(geo.wpack), "s"(geo.bias2), "s"(geo.wslab), "s"(geo.xmask), "s"(geo.h), "s"(geo.sh_w), "s"(geo.last), "s"(geo.total), "s"(geo.nload), "s"(geo.rb),
+                 "s"(geo.m_ohw), "s"(geo.oh), "s"(geo.taprows));
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = geo.nwaves;
+    const int p = lane & 31, h = lane >> 5;
+    const int gid = (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8);
+    if (gid >= geo.total)
+        return;
+    const int outer = (int)quot(gid, geo.m_tile), inner = gid - outer * (geo.mt_inner ? geo.mtiles : geo.ntiles);
+    const int mt = geo.mt_inner ? inner : outer, nt = geo.mt_inner ? outer : inner;
+    const int m0 = mt * (32 * MT), n0 = (nt * nwaves + wave) * (32 * NT);
+
+    // ---- the region -> LDS, as above
+    const int img0 = (int)quot_any((uint32_t)m0, geo.m_ohw, geo.s_ohw);
+    const int rem0 = m0 - img0 * geo.ohw;
+    const int oh0 = (int)quot_any((uint32_t)rem0, geo.m_ow1, geo.s_ow1), ow0 = rem0 - oh0 * geo.ow;
+    const int q0 = img0 * geo.h * geo.w + oh0 * geo.sh_w + ow0 * geo.stride_w - geo.pads;
+    {
+        const int pad = (int)(geo.padword ^ geo.xmask);
+        for (int c = tid; c < geo.cpr; c += 64 * nwaves)
+            *reinterpret_cast<v4i *>(lds + c * 16) = v4i{pad, pad, pad, pad};
+    }
+    uint8_t *const own = lds + geo.rb + wave * 1024;
+    for (int k = 0; k < geo.nload; k++) {
+        const int id = (k * nwaves + wave) * 64 + lane, row = (int)quot(id, geo.m_lpr), c = min(id - row * geo.lpr, geo.cpr - 1);
+        const uint32_t off = (uint32_t)min(max((q0 + row) * geo.cpr + c, 0), geo.last) * 16;
+        __builtin_amdgcn_global_load_lds((gptr_t)(geo.x + off), (lptr_t)(own + k * nwaves * 1024), 16, 0, 0);
+    }
+
+    // ---- weights: row i of a channel tile computes channel 16 ((i >> 2) & 1) + 4 (i >> 3) + (i & 3), so that a lane's accumulators are 16
+    // consecutive channels of one pixel
+    uint32_t woff[NT][2];
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        const int ch = min(n0 + 32 * n + 16 * ((p >> 2) & 1) + 4 * (p >> 3) + (p & 3), (int)geo.kout_pad - 1);
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++)
+            woff[n][kk] = (uint32_t)(ch * 64 + (((2 * kk + h) ^ ((ch >> 2) & 3)) << 4));
+    }
+    v4i w[D][NT];
+    uint64_t wnext = (uint64_t)geo.wpack;
+    auto load_w = [&](v4i(&to)[NT], int kk) {
+        asm("" : "+s"(wnext));
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+            to[n] = *reinterpret_cast<gv4i_t>(reinterpret_cast<gbytes_t>(wnext) + woff[n][kk]);
+        wnext += kk ? geo.wslab : 0;
+    };
+    const int steps = geo.per;
+    v16i acc[NT][MT];
+    int clane[NT]; // this lane's channels, where it has any
+#pragma unroll
+    for (int n = 0; n < NT; n++) {
+        clane[n] = min(n0 + 32 * n + 16 * h, (int)geo.kout_pad - 16);
+        frag::init_acc(acc[n][0], geo.bias2 + clane[n], false);
+#pragma unroll
+        for (int t = 1; t < MT; t++)
+            acc[n][t] = acc[n][0];
+    }
+#pragma unroll
+    for (int i = 0; i < D; i++)
+        if (i < steps)
+            load_w(w[i], i & 1);
+    // a channel's scale each: here, where they are, not behind the reduction, a round trip later
+    constexpr bool EARLY = FINISH == kChannels && NT == 1;
+    v4i qm_[EARLY ? 4 : 1], qt_[EARLY ? 4 : 1];
+    if (EARLY && a.qmult != nullptr)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            qm_[g] = *reinterpret_cast<const v4i *>(a.qmult + clane[0] + 4 * g);
+            qt_[g] = *reinterpret_cast<const v4i *>(a.qshift + clane[0] + 4 * g);
+        }
+    asm volatile("" ::"s"(a.y), "s"(a.out_cs), "s"(a.q.mult), "s"(a.lo), "s"(a.qadd), "s"(a.qmult), "s"(a.res), "s"(a.addq.m0), "s"(a.addq.c0));
+
+    // ---- this lane's pixels m0 + 32 t + p, as above
+    uint32_t base[MT], mask[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+        const int m = min(m0 + 32 * t + p, geo.P - 1) - m0;
+        const int xq = ow0 + m, dy = (int)quot(xq, geo.m_ow), ow = xq - dy * geo.ow;
+        const int yq = oh0 + dy, dn = (int)quot(yq, geo.m_oh), oh = yq - dn * geo.oh;
+        const int ih = oh * geo.stride_h - geo.pad_h, iw = ow * geo.stride_w - geo.pad_w;
+        base[t] = (uint32_t)((((img0 + dn) * geo.h + ih) * geo.w + iw - q0 + 1) * geo.rb) + (GATHER == kWhole ? 16 * h : 0);
+        const uint32_t cols = (1u << min(geo.S, geo.w - iw)) - (1u << max(0, -iw));
+        const uint32_t rows = geo.taprows & ((1u << (min(geo.R, geo.h - ih) * geo.S)) - (1u << (max(0, -ih) * geo.S)));
+        mask[t] = cols * rows;
+    }
+    wait_vmcnt<0>(); // this wave's loads have landed
+    if (geo.xmask != 0)
+        for (int k = 0; k < geo.nload; k++) {
+            v4i *at = reinterpret_cast<v4i *>(own + k * nwaves * 1024 + lane * 16);
+            *at ^= (int)geo.xmask;
+        }
+    __syncthreads();
+
+    // ---- a step's pixel operands: 32 bytes of the reduction.  kWhole: channel strides that are multiples of 32, where a step lies in one
+    // tap; kPieces: each half of it has a tap of its own
+    int tap = 0, cu = 0; // kPieces: cu is the step
+    uint32_t at[MT];
+    auto enter_tap = [&]() {
+        const int step = ((int)quot((uint32_t)tap, geo.m_s) * (geo.w - geo.S) + tap) * geo.rb;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+            at[t] = (int)(mask[t] << (31 - tap)) < 0 ? base[t] + step : (uint32_t)(16 * h);
+    };
+    if (GATHER == kWhole)
+        enter_tap();
+    v4i x[2][MT];
+    auto load_x = [&](v4i(&to)[MT]) { // the next step's; behind the last one whatever its address names
+        if (GATHER == kWhole) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                to[t] = *reinterpret_cast<const v4i *>(lds + (at[t] + cu));
+            cu += 32;
+            if (cu == geo.cpr * 16) {
+                cu = 0, tap++;
+                enter_tap();
+            }
+            return;
+        }
+        const int kp = 2 * cu + h, tp = (int)quot((uint32_t)kp, geo.m_cpr);
+        const int step = (int)quot((uint32_t)tp, geo.m_s) * (geo.w - geo.S) + tp;
+        const uint32_t off = (uint32_t)(step * geo.rb + 16 * (kp - tp * geo.cpr));
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+            to[t] = *reinterpret_cast<const v4i *>(lds + ((int)(mask[t] << (31 - tp)) < 0 ? base[t] + off : 0u));
+        cu = min(cu + 1, steps - 1);
+    };
+    auto multiply = [&](const v4i(&wf)[NT], const v4i(&xf)[MT]) {
+#pragma unroll
+        for (int n = 0; n < NT; n++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                acc[n][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wf[n], xf[t], acc[n][t], 0, 0, 0);
+    };
+    load_x(x[0]);
+    int i0 = 0;
+    for (; i0 + 2 * D <= steps; i0 += D)
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+            load_x(x[(j + 1) & 1]);
+            multiply(w[j], x[j & 1]);
+            load_w(w[j], j & 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    for (; i0 < steps; i0 += D)
+#pragma unroll
+        for (int j = 0; j < D; j++) {
+            if (i0 + j < steps) {
+                load_x(x[(j + 1) & 1]);
+                multiply(w[j], x[j & 1]);
+                if (i0 + j + D < steps)
+                    load_w(w[j], j & 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+    // ---- bytes: 16 consecutive channels of a pixel
+    auto store = [&](int t, int c0, const v4i &o) {
+        const int m = m0 + 32 * t + p;
+        if (m < geo.P && c0 < a.out_cs)
+            *reinterpret_cast<v4i *>(a.y + (size_t)m * a.out_cs + c0) = o;
+    };
+    if constexpr (FINISH == kTensor) {
+#pragma unroll
+        for (int n = 0; n < NT; n++) {
+            const int c0 = n0 + 32 * n + 16 * h;
+            if (a.res == nullptr) {
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    store(t, c0, frag::requant16(a, acc[n][t], 0));
+            } else { // the 32-bit form of the add to 8 bits (wide_applies)
+                v4i res[MT];
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    res[t] = ldg128(a.res + (size_t)min(m0 + 32 * t + p, geo.P - 1) * a.out_cs + min(c0, a.out_cs - 16));
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    store(t, c0, frag::requant_add16(a, acc[n][t], res[t]));
+            }
+        }
+    } else {
+        // The clamp from below in front of the shift, then the shifting, saturating pack on two pixels of ONE channel, whose shift is the same:
+        // a multiply-add, a maximum and three quarters of a byte permutation a value beside half a pack
+        auto channels = [&](auto sgn) {
+#pragma unroll
+            for (int n = 0; n < NT; n++) {
+                v4i out[MT];
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    v4i qm, qt;
+                    if (a.qmult != nullptr) {
+                        qm = EARLY ? qm_[EARLY ? g : 0] : *reinterpret_cast<const v4i *>(a.qmult + clane[n] + 4 * g);
+                        qt = (EARLY ? qt_[EARLY ? g : 0] : *reinterpret_cast<const v4i *>(a.qshift + clane[n] + 4 * g)) - 32;
+                    } else {
+                        qm = v4i{(int)a.q.mult, (int)a.q.mult, (int)a.q.mult, (int)a.q.mult}, qt = v4i{a.qt, a.qt, a.qt, a.qt};
+                    }
+                    uint32_t two[4][MT / 2]; // bytes 0 and 1 of a channel's two pixels
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        uint64_t add = (uint64_t)(uint32_t)((2 * a.q.zp + 1) << (qt[e] - 1)) << 32; // rounding and zero point
+                        asm("" : "+v"(add));
+                        const int32_t plo = a.lo << qt[e];
+#pragma unroll
+                        for (int t = 0; t < MT / 2; t++) {
+                            int32_t v[2];
+#pragma unroll
+                            for (int u = 0; u < 2; u++)
+                                v[u] = max(mulhi_add(acc[n][2 * t + u][4 * g + e], (uint32_t)qm[e], add), plo);
+                            if (decltype(sgn)::value)
+                                asm("v_ashr_pk_i8_i32 %0, %1, %2, %3" : "=v"(two[e][t]) : "v"(v[0]), "v"(v[1]), "v"(qt[e]));
+                            else
+                                asm("v_ashr_pk_u8_i32 %0, %1, %2, %3" : "=v"(two[e][t]) : "v"(v[0]), "v"(v[1]), "v"(qt[e]));
+                        }
+                    }
+#pragma unroll
+                    for (int t = 0; t < MT / 2; t++) {
+                        out[2 * t][g] = (int)(__builtin_amdgcn_perm(two[1][t], two[0][t], 0x0c0c0400u) | __builtin_amdgcn_perm(two[3][t], two[2][t], 0x04000c0cu));
+                        out[2 * t + 1][g] = (int)(__builtin_amdgcn_perm(two[1][t], two[0][t], 0x0c0c0501u) | __builtin_amdgcn_perm(two[3][t], two[2][t], 0x05010c0cu));
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    store(t, n0 + 32 * n + 16 * h, out[t]);
+            }
+        };
+        if (a.lo < 0)
+            channels(std::true_type{});
+        else
+            channels(std::false_type{});
+    }
+}
+
 namespace {
 
 struct PairArgs {
@@ -420,9 +670,11 @@ int region_rows(const ConvArgs &a, int mb)
 // bytes of a pixel's LDS row: an odd number of 16-byte pieces
 int lds_row(const ConvArgs &a) { return 16 * (a.in_cs / 16 | 1); }
 
+int waves_of(const ResidentShape &s) { return s.nwc * std::max(s.ks, 1); }
+
 int lds_bytes(const ConvArgs &a, const ResidentShape &s)
 {
-    const int chunk = s.nwc * s.ks * 1024;
+    const int chunk = waves_of(s) * 1024;
     const long long row = lds_row(a), region = row + (region_rows(a, s.mb) * row + chunk - 1) / chunk * chunk;
     const long long red = s.ks > 1 ? (long long)chunk * s.mb * s.nb : 0;
     return (int)std::min<long long>(std::max(region, red), 1 << 30);
@@ -436,7 +688,7 @@ long long tiles(const ConvArgs &a, const ResidentShape &s)
 
 ResidentGeom geometry(const ConvArgs &a, const ResidentShape &s)
 {
-    const int MB = s.mb, NB = s.nb, nw = s.nwc * s.ks;
+    const int MB = s.mb, NB = s.nb, nw = waves_of(s);
     ResidentGeom g;
     g.x = a.x, g.wpack = a.wpack, g.bias2 = a.bias2;
     g.wslab = (uint32_t)a.kout_pad * 64, g.kout_pad = (uint32_t)a.kout_pad, g.padword = a.padword, g.xmask = a.xmask;
@@ -447,11 +699,11 @@ ResidentGeom geometry(const ConvArgs &a, const ResidentShape &s)
     g.mt_inner = (long long)a.nslab * 64 * a.out_cs > (long long)a.N * a.H * a.W * a.in_cs;
     g.m_tile = magic(g.mt_inner ? g.mtiles : g.ntiles);
     g.nload = (region_rows(a, MB) * g.rb + nw * 1024 - 1) / (nw * 1024);
-    g.m_cpr = magic(g.cpr), g.m_lpr = magic(g.lpr), g.m_s = magic(a.S), g.m_ks = magic(s.ks);
+    g.m_cpr = magic(g.cpr), g.m_lpr = magic(g.lpr), g.m_s = magic(a.S), g.m_ks = magic(std::max(s.ks, 1));
     hipq_div_magic((uint32_t)(a.OH * a.OW), &g.m_ohw, &g.s_ohw);
     hipq_div_magic((uint32_t)a.OW, &g.m_ow1, &g.s_ow1);
     g.m_ow = magic(a.OW), g.m_oh = magic(a.OH);
-    g.ks = s.ks, g.nwaves = nw, g.nwc = s.nwc, g.per = (a.nslab + s.ks - 1) / s.ks, g.nslab = a.nslab;
+    g.ks = s.ks, g.nwaves = nw, g.nwc = s.nwc, g.per = s.ks ? (a.nslab + s.ks - 1) / s.ks : (a.Ktot + 31) / 32, g.nslab = a.nslab;
     g.oh = a.OH, g.pad_h = a.pad_h, g.pad_w = a.pad_w, g.stride_h = a.stride_h, g.P = a.P, g.R = a.R, g.S = a.S;
     g.taprows = 0;
     for (int i = 0; i < a.R; i++)
@@ -477,6 +729,26 @@ void launch_shape(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
         hipLaunchKernelGGL((conv_resident_kernel<MB, NB, SPLIT, kPieces, kTensor>), grid, block, lds, st, g, a);
 }
 
+template <int MT, int NT, int GATHER>
+void launch_wide_gather(const ConvArgs &a, const ResidentGeom &g, const dim3 grid, const dim3 block, int lds, hipStream_t st)
+{
+    if (a.qmult != nullptr || a.lo < 0)
+        hipLaunchKernelGGL((conv_resident_wide_kernel<MT, NT, GATHER, kChannels>), grid, block, lds, st, g, a);
+    else
+        hipLaunchKernelGGL((conv_resident_wide_kernel<MT, NT, GATHER, kTensor>), grid, block, lds, st, g, a);
+}
+
+template <int MT, int NT>
+void launch_wide(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
+{
+    const ResidentGeom g = geometry(a, s);
+    const dim3 grid((unsigned)(g.per_xcd * 8)), block(64 * s.nwc);
+    if (a.in_cs % 32 == 0)
+        launch_wide_gather<MT, NT, kWhole>(a, g, grid, block, lds_bytes(a, s), st);
+    else
+        launch_wide_gather<MT, NT, kPieces>(a, g, grid, block, lds_bytes(a, s), st);
+}
+
 template <int MB, int NB>
 void launch_tile(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
 {
@@ -497,12 +769,47 @@ constexpr ResidentShape kShapes[] = {{1, 1, 1, 8}, {1, 1, 1, 4}, {2, 1, 1, 8}, {
 
 bool point(const ConvArgs &a) { return a.R == 1 && a.S == 1 && a.stride_h == 1 && a.stride_w == 1 && a.in_cs % 64 == 0; }
 
+// the 32 x 32 form: no sums to share, weight zero point 128, one-multiply requantisation, whole 16-byte runs of channels to store
+bool wide_applies(const ConvArgs &a)
+{
+    const bool channels = a.qmult != nullptr || a.lo < 0; // the saturating pack is their upper clamp
+    return a.bwz == 0 && a.acc_out == nullptr && a.deq_out == nullptr && (a.qmult != nullptr ? a.fastch : a.fastq) && a.out_cs % 16 == 0
+        && (!channels || (a.lo < 0 ? a.lo >= -128 && a.q.hi == 127 : a.q.hi == 255))
+        && (a.res == nullptr || (!channels && a.addq.fast && a.addq.hi == 255));
+}
+
+// Microseconds of a launch of the 32 x 32 form, fitted to 4900 launches: 400 layers of 300 000 to 24 million outputs in the shapes that
+// fit LDS (nine in ten within 20 % of the fit).  A launch; for every generation of resident work-groups its start and end, and per step and per
+// tile of a wave its chain; per CU the multiplies, those of them that are of channels the layer has, the pixels' KB, the weights'
+// KB and the tiles; the tensors' MB.
+double wide_cost(const ConvArgs &a, const ResidentShape &s)
+{
+    static const double kCost[2][2][11] = {
+        {{2.684, 1.019, 0.0112, 0.0036, 0.0133, 0.0203, 0.0325, 0.0271, 0.0332, 0.1241, 0.0001},  // a step lies in one tap: one scale,
+         {2.603, 1.107, 0.0121, 0.0056, 0.0073, 0.0099, 0.0276, 0.0590, 0.0564, 0.1477, 0.0019}}, // channels' scales or signed
+        {{2.888, 0.662, 0.0096, 0.0086, 0.0053, 0.0244, 0.0675, 0.0426, 0.0265, 0.1094, 0.0000},  // it does not
+         {3.216, 0.311, 0.0077, 0.0000, 0.0125, 0.0128, 0.0613, 0.0918, 0.0454, 0.1694, 0.0038}}};
+    const bool channels = a.qmult != nullptr || a.lo < 0;
+    const double *const k = kCost[a.in_cs % 32 != 0][channels];
+    const int mt = s.mb / 2, nt = s.nb / 2, nw = s.nwc, steps = (a.Ktot + 31) / 32, ct = (a.out_cs + 31) / 32;
+    const int groups = (a.out_cs + 16 * s.nb * nw - 1) / (16 * s.nb * nw);
+    const double wgs = (double)((a.P + 16 * s.mb - 1) / (16 * s.mb)) * groups;
+    const int waves = mt * nt == 8 || (mt * nt == 4 && (nt == 2 || channels)) ? 2 : mt * nt == 4 || channels ? 3 : 4; // of a SIMD, by their registers
+    const int held = std::max(1, std::min(160 * 1024 / lds_bytes(a, s), 4 * waves / nw));
+    const double gens = std::ceil(wgs / (256.0 * held)), cu = std::max(1.0, wgs / 256), most = std::ceil(wgs / 256), used = (double)std::min(nw * nt * groups, ct) / groups;
+    const double region = 1e-3 * region_rows(a, s.mb) * lds_row(a), mb = 1e-6 * ((double)a.P * a.out_cs + (double)a.N * a.H * a.W * a.in_cs);
+    return k[0] + gens * (k[1] + steps * (k[2] * mt * nt + k[6]) + k[9] * mt * nt) + most * (0.25 * steps * mt * (k[3] * nt * nw + k[4] * used) + k[8] * nw * mt * nt)
+           + cu * (k[5] * region + k[10] * steps * nt * nw) + k[7] * mb;
+}
+
 // Microseconds of a launch in one shape, fitted to 12 000 launches: 490 layers of 1 to 200 000 pixels and 16 to 8192 channels in every
 // shape that fits LDS (half of them within 8 % of the fit, nine in ten within 18).  A launch; for every generation of
 // resident work-groups its start and end; for every slab that a wave takes its chain, alone and per pixel tile; per CU the weight and
 // the pixel bytes that it pulls, the output tiles, the partial sums, the pixels that its waves locate.
 double shape_cost(const ConvArgs &a, const ResidentShape &s)
 {
+    if (s.ks == 0)
+        return wide_cost(a, s);
     // launch, generation, slab, slab x pixel tile, KB of weights, KB of pixels, output tile, partial tile, pixel tile of a SIMD
     static const double kCost[2][5][9] = {
         {{2.505, 0.101, 0.0027, 0.0142, 0.0086, 0.0295, 0.0156, 0, 0},        // whole reductions: 1x1,
@@ -538,11 +845,11 @@ bool conv_resident_applies(const ConvArgs &a)
 
 bool conv_resident_cost(const ConvArgs &a, const ResidentShape &s, double *us)
 {
-    bool built = false;
+    bool built = s.ks == 0 && wide_applies(a) && s.nwc >= 1 && s.nwc <= 8 && (s.mb == 8 || s.mb == 4) && (s.nb == 4 || s.nb == 2);
     for (const ResidentShape &k : kShapes)
         built = built || (k.mb == s.mb && k.nb == s.nb && k.nwc == s.nwc && k.ks == s.ks);
     // LDS, and the ranges of the quotients by multiplication
-    if (!built || lds_bytes(a, s) > 160 * 1024 || (a.in_cs / 16 + 1) * (long long)(region_rows(a, s.mb) + 1) + 64 * s.nwc * s.ks >= 65536 || tiles(a, s) >= (1ll << 30)
+    if (!built || lds_bytes(a, s) > 160 * 1024 || (a.in_cs / 16 + 1) * (long long)(region_rows(a, s.mb) + 1) + 64 * waves_of(s) >= 65536 || tiles(a, s) >= (1ll << 30)
         || (long long)(a.OW + 16 * s.mb) * a.OW >= (1ll << 30) || (long long)(a.OH + 16 * s.mb + 1) * a.OH >= (1ll << 30))
         return false;
     *us = shape_cost(a, s);
@@ -563,8 +870,36 @@ bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us)
     return best < 1e30;
 }
 
+bool conv_resident_wide_applies(const ConvArgs &a) { return wide_applies(a); }
+
+bool conv_resident_choose_wide(const ConvArgs &a, ResidentShape *shape, double *us)
+{
+    double best = 1e30;
+    for (int mb : {8, 4})
+        for (int nb : {4, 2})
+            for (int nw = 1; nw <= 8; nw++) {
+                const int tiles = (a.out_cs + 16 * nb - 1) / (16 * nb);
+                if (nw > tiles || (nw > 1 && (tiles + nw - 2) / (nw - 1) == (tiles + nw - 1) / nw))
+                    continue; // the same groups of channels with fewer waves
+                const ResidentShape s = {mb, nb, nw, 0};
+                double t;
+                if (conv_resident_cost(a, s, &t) && t < best)
+                    best = t, *shape = s;
+            }
+    *us = best;
+    return best < 1e30;
+}
+
 void launch_conv_resident(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
 {
+    if (s.ks == 0) {
+        switch (s.mb * 10 + s.nb) {
+        case 84: return launch_wide<4, 2>(a, s, st);
+        case 82: return launch_wide<4, 1>(a, s, st);
+        case 44: return launch_wide<2, 2>(a, s, st);
+        default: return launch_wide<2, 1>(a, s, st);
+        }
+    }
     switch (s.mb * 10 + s.nb) {
     case 11: launch_tile<1, 1>(a, s, st); break;
     case 21: launch_tile<2, 1>(a, s, st); break;

@@ -160,6 +160,99 @@ def test_layers_outside_the_kernels_range_stay_where_they_were():
         assert np.array_equal(hipq.from_device_nhwc(plan(hipq.to_device_nhwc(x)), 24), orc.conv2d_u8(x, w, None, pad, st, 1, *q)), (R, S, pad)
 
 
+WIDE = [c for c in CASES if c[10] in (0, 128)] + [
+    (3, 96, 13, 21, 200, 3, 1, 1, "i8", True, 0),    # a step lies in one tap, a slab does not
+    (2, 32, 40, 37, 40, 3, 1, 2, "u8", False, 128),   # a step is a whole tap
+    (1, 272, 9, 9, 260, 3, 0, 1, "u8", True, 128),    # an odd number of pieces a tap, an odd number of steps
+    (2, 48, 17, 15, 112, 5, 2, 1, "i8", False, 0),
+]
+
+
+@pytest.mark.parametrize("case", WIDE, ids=lambda c: "-".join(map(str, c)))
+def test_resident_kernel_with_32x32_tiles_matches_the_oracle(case):
+    """Every tile of a wave and several numbers of waves; what the form does not compute - accumulators, an add outside the 32-bit form, an
+    add with scales per channel - another kernel does."""
+    N, C, H, W, K, R, pad, st, dtype, per_channel, wzp = case
+    rng = np.random.default_rng(C + K)
+    x = rng.integers(0, 256, (N, C, H, W), dtype=np.uint8)
+    w = rng.integers(0, 256, (K, C, R, R), dtype=np.uint8)
+    b = rng.integers(-30000, 30000, K).astype(np.int32)
+    ia, izp, ozp = 0.02, 77, 120
+    wa = (0.004 * rng.uniform(0.5, 1.5, K)).astype(np.float32) if per_channel else 0.004
+    oa = float(np.float32(ia * 0.004 * np.sqrt(C * R * R) * 40.0))  # some values saturate on either side
+    if dtype == "i8":
+        xs, ws = x.view(np.int8), w.view(np.int8)
+        want, want_acc = orc.conv2d_i8(xs, ws, b, pad, st, 1, ia, 0.004, oa, 7, return_acc=True)
+        if per_channel:
+            want = orc.requant_per_channel_i8(want_acc, ia, wa, oa, 7)
+        plan = hipq.Conv2d(x.shape, ws, b, pad, st, 1, ia, 0, wa, 0, oa, 0, obits=7, dtype=hipq.DTYPE_I8)
+        want = want.view(np.uint8)
+    else:
+        want, want_acc = orc.conv2d_u8(x, w, b, pad, st, 1, ia, izp, 0.004, wzp, oa, ozp, return_acc=True)
+        if per_channel:
+            want = orc.conv2d_u8_per_channel(x, w, b, pad, st, 1, ia, izp, wa, wzp, oa, ozp)
+        plan = hipq.Conv2d(x.shape, w, b, pad, st, 1, ia, izp, wa, wzp, oa, ozp)
+    xd = hipq.to_device_nhwc(x)
+    res = rng.integers(0, 256, want.shape, dtype=np.uint8)
+    rd = hipq.to_device_nhwc(res)
+    ran = 0
+    for mb, nb in ((8, 4), (8, 2), (4, 4), (4, 2)):
+        for waves in (1, 3, 8):
+            try:
+                plan.resident(16 * mb, 16 * nb, waves, 0)
+            except hipq.HipqError:
+                assert C >= 512  # the region does not fit LDS
+                continue
+            print("wide", case, (mb, nb, waves), plan.kernel, flush=True)
+            assert plan.kernel.startswith("conv_mfma_i8_resident_%dx%d" % (16 * mb, 16 * nb * waves)), plan.kernel
+            got = hipq.from_device_nhwc(plan(xd, torch.full_like(plan.empty_output(), 99)), K)
+            assert np.array_equal(got, want), (mb, nb, waves, int((got != want).sum()), np.argwhere(got != want)[:6].tolist())
+            if dtype == "u8":
+                assert np.array_equal(hipq.from_device_nhwc(plan.run_relu(xd), K), np.maximum(want, ozp)), (mb, nb, waves, "relu")
+                ra = float(np.float32(oa * (300.0 if ran % 3 == 2 else 1.4)))  # the general form of the add too
+                sa = float(np.float32(max(oa, ra) * 1.3))
+                first = bool(ran & 1)
+                y = plan.run_add(xd, rd, first, ra, 9, sa, 20, plan.empty_output())
+                added = orc.add_u8(res, want, ra, 9, oa, ozp, sa, 20) if first else orc.add_u8(want, res, oa, ozp, ra, 9, sa, 20)
+                assert np.array_equal(hipq.from_device_nhwc(y, K), added), (mb, nb, waves, "add", first)
+            ran += 1
+    if ran:
+        acc = torch.zeros((N, plan.OH, plan.OW, plan.desc.out_cs), dtype=torch.int32, device="cuda")
+        got = hipq.from_device_nhwc(plan(xd, acc=acc), K)
+        assert np.array_equal(acc.cpu().numpy()[..., :K].transpose(0, 3, 1, 2), want_acc) and np.array_equal(got, want), "acc"
+    assert ran or C >= 512
+
+
+def test_32x32_tiles_keep_out_of_what_they_do_not_compute():
+    """A weight zero point, eight signed bits (whose low byte wraps), channels that are no multiple of 16 to store, an odd tile."""
+    rng = np.random.default_rng(9)
+    x = rng.integers(0, 256, (2, 64, 20, 20), dtype=np.uint8)
+    w = rng.integers(0, 256, (64, 64, 3, 3), dtype=np.uint8)
+
+    def refused(plan, *shape):
+        with pytest.raises(hipq.HipqError):
+            plan.resident(*(shape or (64, 32, 2, 0)))
+    refused(hipq.Conv2d(x.shape, w, None, 1, 1, 1, 0.02, 77, 0.004, 101, 0.5, 120))
+    refused(hipq.Conv2d(x.shape, w.view(np.int8), None, 1, 1, 1, 0.02, 0, 0.004, 0, 0.5, 0, obits=8, dtype=hipq.DTYPE_I8))
+    refused(hipq.Conv2d(x.shape, w[:3], None, 1, 1, 1, 0.02, 77, 0.004, 128, 0.5, 120))
+    for shape in ((96, 32, 2, 0), (64, 48, 2, 0), (64, 32, 9, 0), (32, 32, 2, 0)):
+        refused(hipq.Conv2d(x.shape, w, None, 1, 1, 1, 0.02, 77, 0.004, 128, 0.5, 120), *shape)
+
+
+@pytest.mark.parametrize("case, wide", [((5, 96, 75, 67, 200, 3, "i8"), True), ((26, 46, 101, 103, 83, 3, "u8"), True), ((1, 64, 14, 14, 128, 5, "u8"), False)],
+                         ids=["ragged_i8", "large", "small"])
+def test_the_rule_takes_32x32_tiles_where_there_is_work(case, wide):
+    N, C, H, W, K, R, dtype = case
+    i8 = dtype == "i8"
+    plan = hipq.Conv2d((N, C, H, W), np.ones((K, C, R, R), np.int8 if i8 else np.uint8), None, R // 2, 1, 1, 0.02, 0 if i8 else 128,
+                       np.full(K, 0.005, np.float32) if i8 else 0.005, 0 if i8 else 128, 0.1, 0 if i8 else 120, obits=7 if i8 else 8,
+                       dtype=hipq.DTYPE_I8 if i8 else hipq.DTYPE_U8)
+    pixels, channels = (int(v) for v in plan.kernel.split("_resident_")[1].split("_")[0].split("x")) if "_resident_" in plan.kernel else (0, 0)
+    print(plan.kernel)
+    built = {(16 * mb, 16 * nb * nwc) for mb, nb, nwc, ks in SHAPES}
+    assert (pixels in (64, 128) and (pixels, channels) not in built) == wide, plan.kernel
+
+
 PAIRS = [  # N, (C, H, W, K, R, stride) of both layers: a block's first layer and its shortcut, and layers of other inputs
     (1, (64, 56, 56, 128, 3, 2), (64, 56, 56, 128, 1, 2)),
     (2, (512, 7, 7, 512, 3, 1), (256, 14, 14, 512, 1, 2)),
