@@ -332,9 +332,10 @@ int hipq_inverted_residual_run(const hipq_conv2d_plan *expand, const hipq_conv2d
                                void *stream);
 /*
  * Tuning hook (no counterpart in the reference): the patch of output pixels that a work-group of that kernel takes - 0 2x4, 1 4x8,
- * 2 8x8 (stride 1, at most 96 output channels), 3 a patch per wave (at most 64 input and output channels), 4 the same with
- * half the patch (stride 1), -1 by cost, which also replaces a shape that is not built for the channels.  Identical results for every choice.
- * hipq_inverted_residual_kernel names what runs, conv_invres_s<stride>_<2x4 | 4x8 | 8x8 | own | own4x8>_k<k-steps>_n<channel tiles>
+ * 2 8x8 (stride 1, at most 96 output and 1440 hidden channels), 3 a patch per wave (at most 64 input and output channels), 4 the same with
+ * half the patch (stride 1), 5 7x7 (as 2), -1 by cost, which also replaces a shape that is not built for the channels.  Identical results
+ * for every choice.
+ * hipq_inverted_residual_kernel names what runs, conv_invres_s<stride>_<2x4 | 4x8 | 8x8 | own | own4x8 | 7x7>_k<k-steps>_n<channel tiles>
  * ("" where the plans do not run this way); the string is valid until the calling thread's next call.
  */
 int hipq_inverted_residual_select(hipq_conv2d_plan *project, int shape);

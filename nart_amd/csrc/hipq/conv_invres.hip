@@ -14,28 +14,34 @@
 //     a byte permutation and four ANDs, times the rows at that tap.  31 of 32 products are with zeros, and still nine matrix
 //     instructions and 45 others replace the 130 dot products, byte alignments and LDS reads of 32 outputs of 32 channels: the
 //     matrix cores idle, and vector instructions are the largest part of a wave's chain;
-//   * project: the requantised sums are, as they lie in the lanes, one k-step of every output channel tile's reduction, whose
-//     accumulators a wave keeps over its slices.
+//   * the requantised sums are, as they lie in the lanes, one k-step of the last layer's pixel operand.  Where the waves split one patch
+//     they put them into LDS, and after the only barrier the last layer's output tiles go to the waves instead of the slices (its
+//     first weights wait in LDS by then); where a wave has a patch it multiplies them at once.
 // Patches of 2x4 outputs do not fill a multiply's 32 columns.  Theirs keeps the expanded pixels as rows (a lane has four runs of four
 // consecutive pixels of ONE channel), takes dot products of such a run with {w0, w1, w2, 0} and {0, w0, w1, w2} (two neighbouring
-// outputs; one at stride 2), and passes the result to the last layer through LDS.
+// outputs; one at stride 2), and puts the result into LDS byte by byte.
 // Positions outside the image hold the depthwise layer's pad byte; the border of a patch is expanded again by its neighbours,
 // which costs vector instructions (the requantisation), not memory.
-// Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch and add their partial sums up
-// in LDS.  Many patches and few slices: every wave has a patch of its own and takes all slices through it, so that no barrier
-// and no sum ties it to others - with shared patches each wave of a 24 -> 144 -> 24 block had one slice between two barriers,
-// 57 us at 56x56, batch 64, against 26.  Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
-// instructions is then a third as long as for 4x8), 4x8 or 8x8 otherwise (fewer positions expanded twice; but a wave of 8x8 outputs
-// with a patch of its own holds 100 registers where one of 4x8 holds 60: 30.6 us against 26.1 for that block, 13.7 against 11.5 for
-// 32 -> 192 -> 32 at 28x28).
+// Two divisions of the work.  Few patches: the waves of a work-group split the slices of one patch, then its output tiles.  (Partial sums
+// of every output in every wave, added up in LDS, took the registers of eight waves instead of twelve or sixteen and 64 atomic
+// additions a wave: 64 -> 384 -> 64 at 14x14, batch 64, 11.8 us, this way 9.4; 64 -> 384 -> 96 12.6 and 9.5; 96 -> 576 -> 96 16.1 and
+// 12.8; 32 -> 192 -> 64 from 28x28, stride 2, 12.3 and 9.0; 64 -> 384 -> 64 on one image 6.5 and 5.9.)  Many patches and few slices: every
+// wave has a patch of its own and takes all slices through it, so that no barrier ties it to others - with shared patches each wave of
+// a 24 -> 144 -> 24 block has one slice between two barriers, 46 us at 56x56, batch 64, against 27.
+// Patches are 2x4 outputs where even so the chip is nearly empty (a slice's chain of
+// instructions is then a third as long as for 4x8), 4x8, 8x8 or 7x7 otherwise: fewer positions expanded twice, and 7x7 fills three of a
+// multiply's tiles with its region where 8x8 fills three and an eighth, and divides images of 14x14 and 28x28 (64 -> 384 -> 64
+// 10.4 and 9.4 us).  But a wave of 8x8 outputs
+// with a patch of its own holds 168 registers where one of 4x8 holds 110: 29.2 us against 26.8 for 24 -> 144 -> 24, 14.2 against 12.2 for
+// 32 -> 192 -> 32 at 28x28.
+// A work-group's first instructions count: its pixels, its waves' weights and biases of all layers are under way before the first wait,
+// with quotients from the host (0.6 us of each block; until then the weights followed the pixels).
 // What bounds it, at batch 64: with a patch per wave vector issue first (the requantisations; 54 % of a CU's busy time at 4 clocks an
-// instruction, matrix cores 9 to 10 %).  With a shared patch neither (vector issue 29 to 31 %, matrix cores 3 to 8 %): 1.5 waves
-// per SIMD, each of which goes region - expand - LDS - depthwise - project - sum with a slice after the other and waits in between.
-// Measured, the three launches -> the depthwise layer as dot products -> this one (batch 64, 40 launches back to back, tensors of random
-// bytes, warm): 16 -> 96 -> 24 at 112x112, stride 2: 45 -> 33.6 -> 27.0 us; 24 -> 144 -> 24 at 56x56: 39 -> 31.3 -> 26.1; 24 -> 144 -> 32,
-// stride 2: 25 -> 18.7 -> 14.5; 32 -> 192 -> 32 at 28x28: 16.9 -> 15.0 -> 11.6; 64 -> 384 -> 64 at 14x14: 12.9 -> 11.5 -> 10.6;
-// 96 -> 576 -> 96: 17.1 -> 16.4 -> 15.2; batch 1, 24 -> 144 -> 24: 9.4 -> 5.0 -> 4.8, 96 -> 576 -> 96: 8.9 -> 7.8 -> 7.6.  With a network's own
-// bytes and clamps the blocks with an add take up to 9 % longer (28.6, 12.5, 11.1, 15.7 us at batch 64).
+// instruction, matrix cores 9 to 10 %).  With a shared patch the chain of a wave, region - expand - LDS - depthwise - LDS -
+// project, a slice after the other, with three waves a SIMD.
+// Measured, the three launches -> this one (batch 64, launches back to back, random bytes): 24 -> 144 -> 24 at 56x56: 39.5 -> 26.8 us;
+// 32 -> 192 -> 32 at 28x28: 18.4 -> 12.2; 64 -> 384 -> 64 at 14x14: 14.7 -> 9.4; 96 -> 576 -> 96: 18.1 -> 12.8; 160 -> 960 -> 160 at 7x7: 15.1 -> 14.0;
+// batch 1, 24 -> 144 -> 24: 10.4 -> 5.8.
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply
 // requantisations, at most 160 input and output channels; with the add stride 1 and as many output as input channels.
 #include "conv_invres.h"
@@ -51,16 +57,29 @@ using namespace frag;
 
 namespace {
 
-// waves of a work-group: three per SIMD leave each 168 registers, where that is enough for a shape's accumulators
-constexpr int max_waves(int TILES, int PT, int NK, int CT) { return PT > 1 || CT > 4 || (TILES > 1 && CT > 2 && (TILES > 4 || NK > 2)) ? 8 : 12; }
+constexpr int kStaged = 6; // k-steps of the last layer's weights that wait in LDS, at most
+
+// waves of a work-group: four per SIMD leave each 128 registers, three 168
+constexpr int max_waves(bool MATRIX, int TILES, int NK) { return NK <= (MATRIX ? 1 : 2) && TILES <= (MATRIX ? 4 : 1) ? 16 : 12; }
 
 struct InvresGeom {
-    int PY, PX; // patches per image
+    int ppi, PX, patches, per_xcd; // patches of an image, of a row of it, all; work-groups of an XCD
+    uint32_t m_ppi, m_px;          // x / ppi and x / PX (hipq_div_magic)
+    int s_ppi, s_px;
+    int nw;               // waves
+    int pieces, m_pieces; // 16-byte pieces of an input pixel; id / pieces == (id * m_pieces) >> 16, id < 4096
     int nT;     // slices of 32 hidden channels
     int nk, ct; // k-steps of the expanding layer, channel tiles of the projecting one
     int xrow;   // bytes of a pixel row of the input region in LDS
     int region; // bytes of an input region with its masks in LDS
     int wave_bytes; // bytes of a wave's own buffers
+    int hidden;     // bytes of the patch's depthwise results in LDS
+    int ks, per;    // waves that share a tile of the last layer, k-steps of one
+    int slab;       // bytes of two k-steps of all its channel tiles
+    int weights;    // where the first weights of the last layer lie in LDS
+    int depth;      // k-steps of them, for each wave
+    int bias;       // where the last layer's biases lie
+    int m_tiles;    // i / tiles == (i * m_tiles) >> 16, i below 16
 };
 
 // S: stride, PH x PW: output pixels of a patch.  Rows and columns of the input region; tiles of 32 positions; pixel tiles of 32
@@ -73,7 +92,7 @@ struct Patch {
     static constexpr bool MATRIX = PH * PW >= 32;
     static constexpr int QW = (S * (PW - 1) + 3 + 3) / 4, RH = S * (PH - 1) + 3, RW = MATRIX ? S * (PW - 1) + 3 : 4 * QW, NP = RH * RW;
     static constexpr int TILES = (NP + 31) / 32, PT = (PH * PW + 31) / 32;
-    static constexpr int E_BYTES = TILES * 1024, D_BYTES = MATRIX ? 0 : PT * 1024, MASK_BYTES = MATRIX ? 0 : TILES * 32;
+    static constexpr int E_BYTES = TILES * 1024, MASK_BYTES = MATRIX ? 0 : TILES * 32;
 };
 
 __device__ static __forceinline__ int32_t dot4(uint32_t a, int b, int32_t c)
@@ -89,13 +108,16 @@ __device__ static __forceinline__ int32_t dot4_from(uint32_t a, int32_t b, int32
     return d;
 }
 
+// x / d for any x below 2^31 (hipq_div_magic)
+__device__ static __forceinline__ int quot(int x, uint32_t m, int s) { return m ? (int)(__umulhi((uint32_t)x, m) >> s) : x; }
+
 } // namespace
 
-// NK: k-steps of 32 input channels; CT: tiles of 32 output channels (both may be more than the layer has: the weights are zeros
-// there).  OWN: every wave has a patch of its own and takes all slices through it; otherwise the waves
-// of a work-group split the slices of one patch.
+// NK: k-steps of 32 input channels (may be more than the layer has: the weights are zeros there).  OWN: every wave has a patch of its
+// own and takes all slices through it, over the accumulators of CT tiles of 32 output channels; otherwise the waves of a work-group split
+// the slices of one patch and then the output tiles.
 template <int S, int PH, int PW, int NK, int CT, bool OWN>
-__global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES, Patch<S, PH, PW>::PT, NK, CT)) void conv_invres_kernel(const ConvArgs e, const ConvArgs d, const ConvArgs pr,
+__global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::MATRIX, Patch<S, PH, PW>::TILES, NK)) void conv_invres_kernel(const ConvArgs e, const ConvArgs d, const ConvArgs pr,
                                                                                 const InvresGeom geo)
 {
     using G = Patch<S, PH, PW>;
@@ -103,26 +125,25 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
     constexpr bool MATRIX = G::MATRIX;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = geo.nw;
     const int p = lane & 31, h = lane >> 5;
     const int ch = slice_channel(p); // the channel of a slice that this lane's column stands for
     // work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of the patches
-    const int ppi = geo.PY * geo.PX;
-    int gid = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+    int gid = (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8);
     if (OWN)
         gid = gid * nw + wave;
-    if (gid >= ppi * d.N)
+    if (gid >= geo.patches)
         return;
-    const int n = gid / ppi, pi = gid - n * ppi, py = pi / geo.PX;
+    const int n = quot(gid, geo.m_ppi, geo.s_ppi), pi = gid - n * geo.ppi, py = quot(pi, geo.m_px, geo.s_px);
     const int oy0 = py * PH, ox0 = (pi - py * geo.PX) * PW;
     const int iy0 = S * oy0 - 1, ix0 = S * ox0 - 1; // the region's first row and column
     const bool inside = iy0 >= 0 && ix0 >= 0 && iy0 + RH <= e.H && ix0 + RW <= e.W; // no position to replace
-    uint8_t *const xbuf = lds + (OWN ? wave * (geo.region + geo.wave_bytes) : 0);
+    uint8_t *const xbuf = lds + (OWN ? wave * (geo.region + geo.wave_bytes) : geo.hidden);
     uint32_t *const masks = reinterpret_cast<uint32_t *>(xbuf + geo.region - G::MASK_BYTES); // dot products: which bytes of a run lie inside the image
     uint8_t *const ebuf = xbuf + geo.region + (OWN ? 0 : wave * geo.wave_bytes);
 
     // ---- a slice's weights and constants, each loaded as soon as the slice before has used its own
-    v4i we[NK], wp[CT];
+    v4i we[NK], wp[OWN ? CT : 1];
     // MATRIX: the folded biases of the lane's 16 consecutive channels, and the depthwise weights of the channel that its row of a multiply
     // stands for, a kernel row each; otherwise biases and weights of the channel that its column stands for, the weights in both
     // alignments
@@ -155,27 +176,60 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
     };
     auto load_p = [&](int T) {
 #pragma unroll
-        for (int ct = 0; ct < CT; ct++)
+        for (int ct = 0; OWN && ct < CT; ct++)
             wp[ct] = ct == 0 || ct < geo.ct ? ldg128(pr.wfrag1 + ((size_t)((T >> 1) * (pr.kout_pad >> 5) + ct) * 2 + (T & 1)) * 1024 + lane * 16)
                                             : v4i{0, 0, 0, 0};
     };
-    int T = OWN ? 0 : wave;
-    const int dT = OWN ? 1 : nw; // never more waves than slices
 
-    // ---- the input region -> LDS, re-centred; positions outside the image are never used (the mask below)
-    {
-        const int tid = OWN ? lane : (int)threadIdx.x, nthr = OWN ? 64 : (int)blockDim.x;
-        const int pieces = e.in_cs >> 4, inv = 65536 / pieces + 1; // id / pieces == (id * inv) >> 16: id < 4096, pieces <= 10
-        for (int id = tid; id < NP * pieces; id += nthr) {
-            const int px = (id * inv) >> 16, c = id - px * pieces, ry = px / RW, rx = px - ry * RW;
-            const int iy = iy0 + ry, ix = ix0 + rx;
-            if ((unsigned)iy < (unsigned)e.H && (unsigned)ix < (unsigned)e.W)
-                *reinterpret_cast<v4i *>(xbuf + px * geo.xrow + c * 16)
-                    = ldg128(e.x + (uint32_t)(((n * e.H + iy) * e.W + ix) * e.in_cs + c * 16)) ^ (int)0x80808080;
+    // ---- the input region -> LDS, re-centred.  Positions outside the image are never used (the mask below) and hold the bytes of one inside.
+    // A thread's first pieces are under way before the weights
+    constexpr int AHEAD = OWN ? (NP <= 64 ? 2 : 4) : PT;
+    const int tid = OWN ? lane : (int)threadIdx.x, nthr = OWN ? 64 : nw * 64, total = NP * geo.pieces;
+    v4i piece[AHEAD];
+    auto load_pieces = [&](int id0) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            const int id = min(id0 + j * nthr, total - 1), px = (id * geo.m_pieces) >> 16, ry = px / RW;
+            const int iy = min(max(iy0 + ry, 0), e.H - 1), ix = min(max(ix0 + px - ry * RW, 0), e.W - 1);
+            piece[j] = ldg128(e.x + (uint32_t)(((n * e.H + iy) * e.W + ix) * e.in_cs + (id - px * geo.pieces) * 16));
         }
+    };
+    auto store_pieces = [&](int id0) {
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) {
+            const int id = min(id0 + j * nthr, total - 1), px = (id * geo.m_pieces) >> 16;
+            *reinterpret_cast<v4i *>(xbuf + px * geo.xrow + (id - px * geo.pieces) * 16) = piece[j] ^ (int)0x80808080;
+        }
+    };
+    load_pieces(tid);
+    load_e(OWN ? 0 : wave); // never more waves than slices
+    load_d(OWN ? 0 : wave);
+    load_p(0);
+    // otherwise: a wave's tile of the last layer, 32 channels by 32 pixels, or its share of the tile's k-steps with ks waves a tile.  The
+    // first steps' weights wait in LDS while the slices are computed, and so do the folded biases
+    const int tiles = geo.ct * PT, items = tiles * geo.ks;
+    uint8_t *const wbuf = lds + geo.weights + wave * geo.depth * 1024;
+    auto step = [&](int ct, int k) { // the lane's weights; k-steps lie in pairs, a pair of every channel tile after the other
+        k = min(k, geo.nT - 1);
+        return pr.wfrag1 + ((uint32_t)((k >> 1) * geo.slab + (2 * ct + (k & 1)) * 1024) + lane * 16);
+    };
+    if constexpr (!OWN) {
+        const int share = wave * geo.m_tiles >> 16, ct = (wave - share * tiles) / PT;
+        const int k0 = share * geo.per;
+#pragma unroll
+        for (int j = 0; j < kStaged; j++)
+            if (j < geo.depth && wave < items)
+                __builtin_amdgcn_global_load_lds((gptr_t)step(ct, k0 + j), (lptr_t)(wbuf + j * 1024), 16, 0, 0);
+        for (int c = wave; 2 * c < geo.ct; c += nw)
+            __builtin_amdgcn_global_load_lds((gptr_t)(pr.bias2 + min(64 * c + lane, 32 * geo.ct - 1)), (lptr_t)(lds + geo.bias + 256 * c), 4, 0, 0);
+    }
+    store_pieces(tid);
+    for (int id = tid + AHEAD * nthr; id < total; id += AHEAD * nthr) {
+        load_pieces(id);
+        store_pieces(id);
     }
     if (!MATRIX && !inside)
-        for (int q = (OWN ? lane : (int)threadIdx.x); q < TILES * 8; q += OWN ? 64 : (int)blockDim.x) {
+        for (int q = (OWN ? lane : (int)threadIdx.x); q < TILES * 8; q += nthr) {
             const int ry = q / QW, rx = (q - ry * QW) * 4, iy = iy0 + ry;
             uint32_t m = 0;
             if (q < RH * QW && (unsigned)iy < (unsigned)e.H)
@@ -188,7 +242,7 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
 #pragma unroll
         for (int t = 0; t < TILES; t++) {
             const int pos = 32 * t + p, ry = pos / RW;
-            outside |= (unsigned)(iy0 + ry) < (unsigned)e.H && (unsigned)(ix0 + pos - ry * RW) < (unsigned)e.W ? 0u : 1u << t;
+            outside |= (int)((unsigned)(iy0 + ry) >= (unsigned)e.H) | (int)((unsigned)(ix0 + pos - ry * RW) >= (unsigned)e.W) ? 1u << t : 0u;
         }
     int first[PT]; // the lane's outputs 32 t + p: their first tap in the expanded region
 #pragma unroll
@@ -196,25 +250,22 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
         const int m = min(32 * t + p, PH * PW - 1);
         first[t] = (S * (m / PW) * RW + S * (m % PW)) * 32 + 16 * h;
     }
-    load_e(T);
-    load_d(T);
-    load_p(T);
-    v16i acc[CT][PT];
+    v16i acc[OWN ? CT : 1][PT]; // from the folded bias of the lane's 16 consecutive channels
+    if constexpr (OWN)
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++)
+        for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-        for (int t = 0; t < PT; t++) {
-            // OWN: the accumulators start at the folded bias of the lane's 16 consecutive channels
-            init_acc(acc[ct][t], pr.bias2 + 32 * (ct < geo.ct ? ct : 0) + 16 * h, !OWN);
-        }
+            for (int t = 0; t < PT; t++)
+                init_acc(acc[ct][t], pr.bias2 + 32 * (ct < geo.ct ? ct : 0) + 16 * h, false);
     const int epad = (int)(d.padword ^ 0x80808080u);
     if (OWN)
         lds_order();
-    else
-        __syncthreads(); // the region and the masks are in LDS
+    else {
+        wait_vmcnt<0>();
+        __syncthreads(); // the region, the masks and the last layer's first weights are in LDS
+    }
 
-    for (; T < geo.nT; T += dT) {
-        const int Tn = min(T + dT, geo.nT - 1); // past the end: harmless loads
+    auto slice = [&](int T, int Tn) { // Tn: the wave's next one, past the end a harmless load
         v4i b[PT]; // the depthwise layer's bytes, as the last layer's pixel operand
         if constexpr (MATRIX) {
             // ---- expand: a lane's 16 channels of a position are 16 bytes of the position's row
@@ -290,7 +341,6 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
             lds_order();
             // ---- depthwise: half h of the wave takes PH / 2 output rows of this lane's channel
             constexpr int HR = PH / 2, IR = S * (HR - 1) + 3;
-            uint8_t *const dbuf = ebuf + G::E_BYTES;
             int32_t o[HR][PW];
 #pragma unroll
             for (int ir = 0; ir < IR; ir++) {
@@ -317,68 +367,120 @@ __global__ __launch_bounds__(OWN ? 256 : 64 * max_waves(Patch<S, PH, PW>::TILES,
                 }
             }
             load_d(Tn);
-            // this lane's channel of its outputs, as bytes of the pixel rows that the last layer multiplies
+            // this lane's channel of its outputs, as bytes of the operand that the last layer multiplies
 #pragma unroll
             for (int r = 0; r < HR; r++)
 #pragma unroll
                 for (int x4 = 0; x4 < PW; x4 += 4) {
                     const uint32_t v = conv_requant4<false>(d, o[r][x4], o[r][x4 + 1], o[r][x4 + 2], o[r][x4 + 3]) ^ 0x80808080u;
-                    uint8_t *to = dbuf + (((HR * h + r) * PW + x4) * 32) + ch;
-                    to[0] = (uint8_t)v, to[32] = (uint8_t)(v >> 8), to[64] = (uint8_t)(v >> 16), to[96] = (uint8_t)(v >> 24);
+                    uint8_t *to = lds + T * 1024 + ((ch >> 4) * 32 + (HR * h + r) * PW + x4) * 16 + (ch & 15);
+                    to[0] = (uint8_t)v, to[16] = (uint8_t)(v >> 8), to[32] = (uint8_t)(v >> 16), to[48] = (uint8_t)(v >> 24);
                 }
-            lds_order();
-#pragma unroll
-            for (int t = 0; t < PT; t++)
-                b[t] = *reinterpret_cast<const v4i *>(dbuf + (32 * t + p) * 32 + 16 * h);
         }
         // ---- project: one k-step of every channel tile (rows past the patch, where it has fewer than 32 pixels, are never stored)
+        if constexpr (OWN) {
 #pragma unroll
-        for (int ct = 0; ct < CT; ct++)
+            for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+                for (int t = 0; t < PT; t++)
+                    acc[ct][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wp[ct], b[t], acc[ct][t], 0, 0, 0);
+            load_p(Tn);
+        } else if constexpr (MATRIX) {
 #pragma unroll
             for (int t = 0; t < PT; t++)
-                acc[ct][t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(wp[ct], b[t], acc[ct][t], 0, 0, 0);
-        load_p(Tn);
+                *reinterpret_cast<v4i *>(lds + (T * PT + t) * 1024 + lane * 16) = b[t];
+        }
         lds_order();
-    }
-
-    auto store = [&](int ct, int t, const v16i &s) {
-        const int m = 32 * t + p, oy = oy0 + m / PW, ox = ox0 + m % PW, c0 = 32 * ct + 16 * h;
-        if (m >= PH * PW || oy >= pr.OH || ox >= pr.OW || c0 >= pr.out_cs)
-            return;
-        const size_t at = (size_t)((n * pr.OH + oy) * pr.OW + ox) * pr.out_cs + c0;
-        const v4i v = pr.res != nullptr ? requant_add16(pr, s, ldg128(pr.res + at)) : requant16(pr, s, 0);
-        *reinterpret_cast<v4i *>(pr.y + at) = v;
     };
-    if (OWN) {
+
+    auto place = [&](int ct, int t, uint32_t *at) { // of the lane's 16 channels of its pixel
+        const int m = 32 * t + p, oy = oy0 + m / PW, ox = ox0 + m % PW, c0 = 32 * ct + 16 * h;
+        *at = (uint32_t)(((n * pr.OH + oy) * pr.OW + ox) * pr.out_cs + c0); // below 2^31
+        return (m < PH * PW) & (oy < pr.OH) & (ox < pr.OW) & (c0 < pr.out_cs);
+    };
+    if constexpr (OWN) {
+        for (int T = 0; T < geo.nT; T++)
+            slice(T, min(T + 1, geo.nT - 1));
 #pragma unroll
         for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-            for (int t = 0; t < PT; t++)
-                store(ct, t, acc[ct][t]);
-        return;
-    }
-    // ---- the waves' partial sums meet in LDS (where the region was), over the folded bias
-    __syncthreads();
-    int32_t *const red = reinterpret_cast<int32_t *>(lds);
-    for (int i = threadIdx.x; i < CT * PT * 1024; i += blockDim.x) {
-        const int l = i & 63, r = (i >> 6) & 15, ct = (i >> 10) / PT;
-        red[i] = pr.bias2[32 * min(ct, geo.ct - 1) + 16 * (l >> 5) + r];
-    }
-    __syncthreads();
+            for (int t = 0; t < PT; t++) {
+                uint32_t at;
+                if (place(ct, t, &at))
+                    *reinterpret_cast<v4i *>(pr.y + at) = pr.res != nullptr ? requant_add16(pr, acc[ct][t], ldg128(pr.res + at)) : requant16(pr, acc[ct][t], 0);
+            }
+    } else {
+        for (int T = wave; T < geo.nT; T += nw)
+            slice(T, min(T + nw, geo.nT - 1));
+        // ---- project, from the whole patch's depthwise results
+        constexpr int D = 4; // k-steps of weights ahead
+        for (int i = wave; i == wave || i < items; i += nw) {
+            asm("" : "+s"(i)); // what hangs on it is computed here, not kept in registers from the front
+            const bool work = i < items;
+            const int share = work ? i * geo.m_tiles >> 16 : 0, tile = work ? i - share * tiles : 0, ct = tile / PT, t = tile - ct * PT;
+            const int k0 = min(share * geo.per, geo.nT), k1 = work ? min(k0 + geo.per, geo.nT) : k0;
+            uint32_t at;
+            const bool store = place(ct, t, &at) && work && share == 0;
+            const v4i *const bias = reinterpret_cast<const v4i *>(lds + geo.bias + 128 * ct + 64 * h);
+            v4i res = {0, 0, 0, 0};
+            if (S == 1 && store && pr.res != nullptr) { // the residual is the block's input
+                const int m = 32 * t + p;
+                res = *reinterpret_cast<const v4i *>(xbuf + ((m / PW + 1) * RW + m % PW + 1) * geo.xrow + 32 * ct + 16 * h) ^ (int)0x80808080;
+            }
+            v16i sum;
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++)
+            for (int j = 0; j < 4; j++) {
+                const v4i q = share > 0 ? v4i{0, 0, 0, 0} : bias[j];
+                sum[4 * j] = q[0], sum[4 * j + 1] = q[1], sum[4 * j + 2] = q[2], sum[4 * j + 3] = q[3];
+            }
+            const int kr = i == wave ? min(k0 + geo.depth, k1) : k0;
+            v4i w[D];
+            if (kr < k1)
 #pragma unroll
-        for (int t = 0; t < PT; t++)
+                for (int j = 0; j < D; j++)
+                    w[j] = ldg128(step(ct, kr + j));
+            if (i == wave)
+                __syncthreads(); // the slices are there
+            constexpr int GROUP = MATRIX && NK == 1 ? 3 : kStaged; // as many as the registers hold
+            for (int k = k0; k < kr; k += GROUP) {
+                v4i ws[GROUP], xs[GROUP];
 #pragma unroll
-            for (int r = 0; r < 16; r++)
-                atomicAdd(&red[((ct * PT + t) * 16 + r) * 64 + lane], acc[ct][t][r]);
-    __syncthreads();
-    for (int i = wave; i < CT * PT; i += nw) {
-        v16i s;
+                for (int j = 0; j < GROUP; j++) {
+                    const int kj = min(k + j, kr - 1);
+                    ws[j] = *reinterpret_cast<const v4i *>(wbuf + (kj - k0) * 1024 + lane * 16);
+                    xs[j] = *reinterpret_cast<const v4i *>(lds + (kj * PT + t) * 1024 + lane * 16);
+                }
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-            s[r] = red[(i * 16 + r) * 64 + lane];
-        store(i / PT, i % PT, s);
+                for (int j = 0; j < GROUP; j++)
+                    if (k + j < kr)
+                        sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(ws[j], xs[j], sum, 0, 0, 0);
+            }
+            for (int k = kr; k < k1; k += D)
+#pragma unroll
+                for (int j = 0; j < D; j++) {
+                    if (k + j < k1)
+                        sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[j], *reinterpret_cast<const v4i *>(lds + ((k + j) * PT + t) * 1024 + lane * 16), sum, 0, 0, 0);
+                    if (k + D < k1)
+                        w[j] = ldg128(step(ct, k + j + D));
+                }
+            if (geo.ks > 1) { // the shares meet where the region was (no wave has two items then)
+                v4i *const red = reinterpret_cast<v4i *>(xbuf) + tile * 256 + lane;
+                if (share > 0)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        red[(share - 1) * tiles * 256 + j * 64] = v4i{sum[4 * j], sum[4 * j + 1], sum[4 * j + 2], sum[4 * j + 3]};
+                __syncthreads();
+                if (work && share == 0)
+                    for (int s = 0; s + 1 < geo.ks; s++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            const v4i q = red[s * tiles * 256 + j * 64];
+                            sum[4 * j] += q[0], sum[4 * j + 1] += q[1], sum[4 * j + 2] += q[2], sum[4 * j + 3] += q[3];
+                        }
+            }
+            if (store)
+                *reinterpret_cast<v4i *>(pr.y + at) = pr.res != nullptr ? requant_add16(pr, sum, res) : requant16(pr, sum, 0);
+        }
     }
 }
 
@@ -402,12 +504,17 @@ Channels channels_of(const ConvArgs &e, const ConvArgs &p)
     return {5, 5};
 }
 
-enum Shape { k2x4, k4x8, k8x8, kOwn, kOwn4, kShapes }; // kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2; kOwn4: 4x8 at stride 1
+// kOwn: a patch per wave, 8x8 outputs at stride 1, 4x8 at stride 2; kOwn4: 4x8 at stride 1
+enum Shape { k2x4, k4x8, k8x8, kOwn, kOwn4, k7x7, kShapes };
+
+bool own(int shape) { return shape == kOwn || shape == kOwn4; }
 
 // how a launch divides the work
 struct Division {
-    int PY, PX, nT, xrow, region, wave_bytes;
+    int PY, PX, nT, xrow, region, wave_bytes, hidden, ks, weights, depth, bias;
     int nw, rounds; // waves of a work-group; slices that one of them takes one after the other
+    int waves;      // of a SIMD that the registers allow
+    int tiles;      // of the last layer
     unsigned lds;
     long long wgs;
 };
@@ -415,7 +522,8 @@ struct Division {
 Division divide(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
     const Channels c = channels_of(e, p);
-    const int S = d.stride_h, ph = shape == k2x4 ? 2 : shape == k8x8 || (shape == kOwn && S == 1) ? 8 : 4, pw = shape == k2x4 ? 4 : 8;
+    const int S = d.stride_h, ph = shape == k2x4 ? 2 : shape == k7x7 ? 7 : shape == k8x8 || (shape == kOwn && S == 1) ? 8 : 4;
+    const int pw = shape == k2x4 ? 4 : shape == k7x7 ? 7 : 8;
     const bool matrix = ph * pw >= 32; // these as in Patch
     const int tiles = ((S * (ph - 1) + 3) * (matrix ? S * (pw - 1) + 3 : (S * (pw - 1) + 6) / 4 * 4) + 31) / 32, pt = (ph * pw + 31) / 32;
     Division v;
@@ -425,19 +533,24 @@ Division divide(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int sha
     // ones 16 bytes apart
     v.xrow = e.in_cs == 16 ? 16 : c.nk == 1 ? 32 : 32 * c.nk + 16;
     v.region = (tiles * 32 * v.xrow + 16 + (matrix ? 0 : tiles * 32) + 15) / 16 * 16;
-    v.wave_bytes = tiles * 1024 + (matrix ? 0 : pt * 1024);
+    v.wave_bytes = tiles * 1024;
     const long long patches = (long long)d.N * v.PY * v.PX;
-    if (shape >= kOwn) {
+    if (own(shape)) {
         v.nw = 4, v.rounds = v.nT, v.wgs = (patches + 3) / 4;
-        v.lds = (unsigned)(4 * (v.region + v.wave_bytes));
+        v.lds = (unsigned)(4 * (v.region + v.wave_bytes)), v.hidden = v.weights = v.depth = v.bias = 0, v.ks = 1, v.tiles = c.ct * pt;
+        v.waves = shape == kOwn4 || S == 2 ? (c.ct == 1 ? 4 : 3) : c.ct == 1 ? 3 : 2;
     } else {
-        v.nw = std::min(v.nT, max_waves(tiles, pt, c.nk, c.ct));
-        while (v.region + v.nw * v.wave_bytes > 160 * 1024)
-            v.nw--; // one wave needs at most 14 KB beside 63 KB of pixels
-        v.rounds = (v.nT + v.nw - 1) / v.nw;
+        const int out = v.tiles = (p.out_cs + 31) / 32 * pt;
+        v.nw = std::min(v.nT, max_waves(matrix, tiles, c.nk)), v.rounds = (v.nT + v.nw - 1) / v.nw;
         v.nw = (v.nT + v.rounds - 1) / v.rounds; // the same rounds with fewer waves
+        v.ks = std::max(1, std::min(v.nw / out, v.nT / 6)); // shares of six k-steps: a shorter one takes longer to add up than to multiply
+        const int rest = std::max(v.region + v.nw * v.wave_bytes, (v.ks - 1) * out * 4096), holders = std::min(v.nw, out * v.ks);
+        v.hidden = v.nT * pt * 1024, v.bias = v.hidden + rest, v.weights = v.bias + (p.out_cs + 63) / 64 * 256;
+        v.depth = std::min((v.nT + v.ks - 1) / v.ks, kStaged);
+        while (v.depth > 0 && v.weights + holders * v.depth * 1024 > 160 * 1024)
+            v.depth--;
         v.wgs = patches;
-        v.lds = (unsigned)std::max(v.region + v.nw * v.wave_bytes, c.ct * pt * 4096);
+        v.lds = (unsigned)(v.weights + holders * v.depth * 1024), v.waves = max_waves(matrix, tiles, c.nk) / 4;
     }
     return v;
 }
@@ -448,37 +561,44 @@ void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
     using G = Patch<S, PH, PW>;
     const Division v = divide(e, d, p, shape);
     InvresGeom geo;
-    geo.PY = v.PY, geo.PX = v.PX, geo.nT = v.nT, geo.xrow = v.xrow, geo.region = v.region, geo.wave_bytes = v.wave_bytes;
     geo.nk = (e.in_cs + 31) / 32, geo.ct = (p.out_cs + 31) / 32;
+    geo.ppi = v.PY * v.PX, geo.PX = v.PX, geo.patches = d.N * geo.ppi, geo.per_xcd = (int)((v.wgs + 7) / 8), geo.nw = v.nw;
+    hipq_div_magic((uint32_t)geo.ppi, &geo.m_ppi, &geo.s_ppi);
+    hipq_div_magic((uint32_t)geo.PX, &geo.m_px, &geo.s_px);
+    geo.pieces = e.in_cs / 16, geo.m_pieces = 65536 / geo.pieces + 1, geo.slab = p.kout_pad / 32 * 2048;
+    geo.nT = v.nT, geo.xrow = v.xrow, geo.region = v.region, geo.wave_bytes = v.wave_bytes, geo.hidden = v.hidden;
+    geo.ks = v.ks, geo.per = (v.nT + v.ks - 1) / v.ks, geo.m_tiles = 65536 / (geo.ct * G::PT) + 1;
+    geo.weights = v.weights, geo.depth = v.depth, geo.bias = v.bias;
     static_assert(G::E_BYTES == G::TILES * 1024, "divide()");
     hipLaunchKernelGGL((conv_invres_kernel<S, PH, PW, NK, CT, OWN>), dim3((unsigned)((v.wgs + 7) / 8 * 8)), dim3(64 * v.nw), v.lds, st, e, d, p, geo);
 }
 
 // ---- the shapes, and what each takes
 
-// Time by shape, in us, fitted to 460 blocks (1 to 128 images of 3x3 to 130x130, the channel counts of mobile networks; nine in ten
+// Time by shape, in us, fitted to 626 blocks (1 to 128 images of 3x3 to 128x128, 16 to 160 channels widened 1 to 6 times; nine in ten
 // within 20 % of the fit).  A launch; for every generation of resident work-groups its start and end; for every
-// slice that a wave then takes its chain, alone, per channel tile and per k-step; and per SIMD of the chip the slices and the patches,
-// which share the vector units.
+// slice that a wave then takes its chain, alone and per k-step; the k-steps of the last layer that a wave takes, or a slice's channel tiles
+// where each wave has a patch; and per SIMD of the chip the slices and the patches, which share the vector units.  Chosen by this the
+// blocks take 0.6 % more than the best shape would on average, one in twenty more than 5 %.
 double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    // launch, slice, slice x channel tiles, slice x k-steps, slices per SIMD, generation, patches per SIMD
+    // launch, slice, k-steps of the last layer, slice x k-steps, slices per SIMD, generation, patches per SIMD
     static const double kCost[2][kShapes][7] = {
-        {{2.909, 0, 0.325, 0, 0.461, 1.071, 0}, {1.845, 0, 0.445, 0, 0.479, 2.666, 0}, {2.087, 0.323, 0.783, 0.128, 0.253, 2.985, 0},
-         {1.250, 1.240, 0.226, 0.058, 0.298, 2.046, 0.956}, {1.197, 0.605, 0.123, 0.129, 0.279, 1.566, 0.504}},
-        {{2.287, 0, 0.368, 0.016, 0.382, 1.932, 0}, {2.669, 0, 0.465, 0.148, 0.832, 2.360, 0}, {}, {2.845, 1.062, 0.146, 0.186, 0.096, 0.266, 1.780}, {}}};
+        {{3.871, 0, 0.105, 0.136, 0.567, 0.251, 0}, {3.926, 0.224, 0.165, 0.313, 0.722, 0, 0}, {4.572, 0.823, 0.229, 0.189, 1.044, 0, 0.084},
+         {4.108, 1.191, 0, 0.278, 0.418, 0, 0.956}, {3.607, 0.525, 0.070, 0.172, 0.303, 0, 0.607}, {4.523, 0.535, 0.214, 0.205, 0.965, 0.022, 0}},
+        {{3.673, 0.126, 0.117, 0.255, 0.559, 0, 0}, {3.956, 0.395, 0.209, 0.488, 0.827, 0, 0}, {}, {1.583, 1.003, 0.154, 0.139, 0.477, 2.009, 0.251}, {}, {}}};
     const int s = d.stride_h;
     const Channels c = channels_of(e, p);
-    if ((shape >= kOwn && (c.nk > 2 || c.ct > 2)) || (shape == kOwn4 && s == 2) || (shape == k8x8 && (s == 2 || c.ct > 3)))
+    if ((own(shape) && (c.nk > 2 || c.ct > 2)) || (shape == kOwn4 && s == 2) || ((shape == k8x8 || shape == k7x7) && (s == 2 || c.ct > 3)))
         return 1e30; // not built: the accumulators or the region would be too much for a wave
     const Division v = divide(e, d, p, shape);
-    // waves per SIMD that the registers allow
-    const int waves = shape == kOwn4 || (shape == kOwn && s == 2) ? (c.ct == 1 ? 4 : 3)
-        : shape == kOwn ? (c.ct == 1 ? 3 : 2) : max_waves(shape == k2x4 ? s : s == 1 ? 2 : 5, shape == k8x8 ? 2 : 1, c.nk, c.ct) / 4;
-    const int held = std::max(1, std::min((int)(160 * 1024 / v.lds), 4 * waves / v.nw)); // work-groups of a CU
+    if (v.lds > 160 * 1024) // 8x8 and 7x7 patches of 1450 hidden channels and more; the smaller patches hold the 2048 that a layer can have here
+        return 1e30;
+    const int held = std::max(1, std::min((int)(160 * 1024 / v.lds), v.waves / ((v.nw + 3) / 4))); // work-groups of a CU, the first wave of each on the first SIMD
     const double gens = (double)((v.wgs + 256 * held - 1) / (256 * held)), steps = gens * v.rounds;
     const double patches = (double)d.N * v.PY * v.PX;
-    const double f[7] = {1, steps, steps * c.ct, steps * c.nk, patches * v.nT / 1024, gens, patches / 1024};
+    const double last = own(shape) ? steps * c.ct : gens * ((v.tiles * v.ks + v.nw - 1) / v.nw) * ((v.nT + v.ks - 1) / v.ks);
+    const double f[7] = {1, steps, last, steps * c.nk, patches * v.nT / 1024, gens, patches / 1024};
     double t = 0;
     for (int i = 0; i < 7; i++)
         t += kCost[s - 1][shape][i] * f[i];
@@ -510,12 +630,15 @@ void launch_tiles(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
             if (shape == kOwn4)
                 return launch_shape<1, 4, 8, NK, CT, true>(e, d, p, shape, st);
     }
-    if constexpr (S == 1 && CT <= 3)
+    if constexpr (S == 1 && CT <= 3) {
         if (shape == k8x8)
-            return launch_shape<S, 8, 8, NK, CT, false>(e, d, p, shape, st);
+            return launch_shape<S, 8, 8, NK, 0, false>(e, d, p, shape, st);
+        if (shape == k7x7)
+            return launch_shape<S, 7, 7, NK, 0, false>(e, d, p, shape, st);
+    }
     if (shape == k4x8)
-        return launch_shape<S, 4, 8, NK, CT, false>(e, d, p, shape, st);
-    launch_shape<S, 2, 4, NK, CT, false>(e, d, p, k2x4, st);
+        return launch_shape<S, 4, 8, NK, 0, false>(e, d, p, shape, st);
+    launch_shape<S, 2, 4, NK, 0, false>(e, d, p, k2x4, st);
 }
 
 template <int S>
@@ -554,9 +677,9 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
         && e.N == d.N && e.OH == d.H && e.OW == d.W && (long long)e.P * e.in_cs < (1ll << 31);
 }
 
-// The three launches: their latencies, the hidden tensor's bytes at the output's resolution, the products of both 1x1 layers (fitted to
-// the same blocks, nine in ten within 10 %).  Chosen by this the 460 blocks take 1.4 % more than the best choice would on average, one
-// in twenty more than 9 %, one in a hundred 23 %.
+// The three launches: their latencies, the hidden tensor's bytes at the output's resolution, the products of both 1x1 layers (nine in ten
+// within 10 %).  Of the 626 blocks 618 go the one launch's way by this, 2 of them more than 15 % slower than apart, none that stay apart
+// is more than 16 % slower.
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
@@ -571,7 +694,7 @@ bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs 
 
 const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted)
 {
-    static const char *const kPatch[kShapes] = {"2x4", "4x8", "8x8", "own", "own4x8"};
+    static const char *const kPatch[kShapes] = {"2x4", "4x8", "8x8", "own", "own4x8", "7x7"};
     static thread_local char nm[48];
     double us;
     const int shape = choose_shape(e, d, p, wanted, &us);

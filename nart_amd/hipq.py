@@ -409,7 +409,7 @@ def inverted_residual_fusable(expand, depthwise, project, add=None, obits=8):
 
 
 def inverted_residual_select(project, shape=-1):
-    """Tuning hook: the patch shape of the block that `project` closes, 0..4, -1 by cost (include/hipq.h)."""
+    """Tuning hook: the patch shape of the block that `project` closes, 0..5, -1 by cost (include/hipq.h)."""
     check(lib().hipq_inverted_residual_select(project.handle, int(shape)))
 
 

@@ -655,6 +655,43 @@ def test_inverted_residual_half_patch_per_wave(case, hw):
         assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
 
 
+# channels, hidden channels, image, shape: 7x7 patches that overhang on both sides, fit exactly, are larger than the image; the most hidden
+# channels that a shape takes, most of them without room in LDS for the last layer's weights; more output tiles than waves
+INVRES_SPLITS = [(ci, 80, co, hw, 5) for ci, co in ((24, 24), (24, 40), (40, 60), (64, 72), (96, 96)) for hw in ((13, 11), (7, 14), (3, 2))]
+INVRES_SPLITS += [(16, 1152, 16, (9, 5), 2), (96, 1152, 96, (5, 4), 5), (96, 32, 96, (9, 5), 2), (160, 2048, 160, (3, 9), 1), (160, 2000, 24, (3, 5), 0)]
+
+
+@pytest.mark.parametrize("case", INVRES_SPLITS, ids=lambda c: "%d_%d_%d_%s_%d" % (c[:3] + ("%dx%d" % c[3],) + c[4:]))
+def test_inverted_residual_splits_of_the_hidden_channels(case):
+    ci, ch, co, hw, sh = case
+    rng = np.random.default_rng(ci + ch + co + hw[0])
+    x = rng.integers(0, 256, (2, ci, *hw), dtype=np.uint8)
+    t, a, z, plans = x, 0.03, 77, []
+    for k, (C, K, R, group) in enumerate(((ci, ch, 1, 1), (ch, ch, 3, ch), (ch, co, 1, 1))):
+        w = rng.integers(1, 256, (K, C // group, R, R), dtype=np.uint8)
+        sigma = 74.0 * 74.0 * math.sqrt(w[0].size) * (0.7 if k else 1.0)
+        b = rng.integers(-int(sigma), int(sigma) + 1, K).astype(np.int32)
+        oa = float(np.float32(0.03 * rng.uniform(0.75, 1.35)))
+        q = (a, z, float(np.float32(oa * 45.0 / (a * sigma))), 128, oa, 30 if k < 2 else 120)
+        plans.append(hipq.Conv2d(t.shape, w, b, R // 2, 1, group, *q, relu=k < 2))
+        t = orc.conv2d_u8(t, w, b, R // 2, 1, group, *q)
+        if k < 2:
+            t = np.maximum(t, q[5]).astype(np.uint8)
+        a, z = q[4], q[5]
+    plans[2].special(2)
+    hipq.inverted_residual_select(plans[2], sh)
+    name = hipq.inverted_residual_kernel(*plans)
+    assert name.startswith("conv_invres_s1_%s_k" % ("2x4", "4x8", "8x8", "own", "own4x8", "7x7")[sh]), name
+    print(name, case, flush=True)
+    xd = hipq.to_device_nhwc(x)
+    got = hipq.from_device_nhwc(hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99)), co)
+    assert np.array_equal(got, t), (name, int((got != t).sum()))
+    if ci == co:
+        want = orc.add_u8(t, x, a, z, 0.03, 77, 0.05, 20)
+        y = hipq.inverted_residual_run(*plans, xd, torch.full_like(plans[2].empty_output(), 99), (False, 0.05, 20))
+        assert np.array_equal(hipq.from_device_nhwc(y, co), want), (name, "add")
+
+
 @pytest.mark.parametrize("n, pays", [(1, False), (16, False), (20, True), (64, True)])
 def test_whole_blocks_pay_from_some_pixels_on(n, pays):
     """The executor leaves the three layers apart below 20 images of 14x14, where a block's weights take one work-group longer than
