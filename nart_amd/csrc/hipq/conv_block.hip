@@ -66,7 +66,7 @@ struct BlockGeom {
 // most 2 x 2 patches; 3: up to 9 x 9 = 81).
 // NX: 0, or 2 - the 1x1 convolution that reads the sum (CW -> 2 CM channels, the first layer of the next stage) is computed
 // as well: the sum tile takes the x tile's place in LDS, row = output index m, and is that layer's pixel operand.
-template <int G, int MT1, int NX>
+template <int G, int MT1, int NX, bool EXACT>
 __global__ __launch_bounds__(128 * G, 2) void conv_bottleneck_kernel(const ConvArgs a1, const ConvArgs a2, const ConvArgs a3,
                                                                     const ConvArgs an, const BlockGeom geo)
 {
@@ -218,6 +218,7 @@ __global__ __launch_bounds__(128 * G, 2) void conv_bottleneck_kernel(const ConvA
             pixo[t] = (n * geo.H + y0 + py) * geo.W + x0 + px;
             yoff[t] = (size_t)pixo[t] * CW;
         }
+        const RequantAdd<EXACT> f(a3); // EXACT: a3.addq is in its exact form
         for (int cc = 0; cc < 4; cc++) {
             const int ch = 128 * wave + 32 * cc; // first of the chunk's 32 channels
             v16i acc[2];
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(128 * G, 2) void conv_bottleneck_kernel(const ConvA
                 res[t] = *reinterpret_cast<const v4i *>(lds + jres[t] * CW + (c16 & ~15) * 16 + (((c16 & 15) ^ (jres[t] & 15)) << 4));
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const v4i o = requant_add16(a3, acc[t], res[t]);
+                const v4i o = requant_add16(f, acc[t], res[t]);
                 if (valid[t])
                     *reinterpret_cast<v4i *>(a3.y + yoff[t] + ch + 16 * h) = o;
                 if (NX) {
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(128 * G, 2) void conv_bottleneck_kernel(const ConvA
 //   * layer 3 + add as above, the sum stored and - CHAIN - kept in LDS, 64 pixel rows of CW bytes;
 //   * CHAIN: the next layer (CW -> CM, or CW -> 2 CM where the next stage begins) reads that tile as its pixel operand.
 // ST: the 3x3 layer's stride (1, or 2 - the first block of a stage: the grid then holds (2 PH + 1) x (2 PW + 1) input pixels).
-template <int G, int PH, int PW, int NX, int ST>
+template <int G, int PH, int PW, int NX, int ST, bool EXACT>
 __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && ST == 1 && (NX == 1 || PH == 4) ? 4 : 3) : 2)) void conv_bottleneck_tail_kernel(const ConvArgs a2, const ConvArgs a3, const ConvArgs an,
                                                                          const BlockGeom geo)
 {
@@ -418,6 +419,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
             __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
             __builtin_amdgcn_s_barrier();
         }
+        const RequantAdd<EXACT, EXACT || !(G == 2 && ST == 2 && NX == 0)> f(a3); // that one has no register to spare
         for (int cc = 0; cc < 4; cc++) {
             const int ch = 128 * wave + 32 * cc;
             v16i acc[2];
@@ -439,7 +441,7 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
                 load_chunk(cc + 1); // the next chunk's operands arrive during the arithmetic below
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                const v4i o = requant_add16<!(G == 2 && ST == 2 && NX == 0)>(a3, acc[t], rc[t]); // that one has no register to spare
+                const v4i o = requant_add16(f, acc[t], rc[t]);
                 if (!CHAIN && valid[t]) // 16 bytes of each of 32 pixels per instruction; the chained form stores whole rows below
                     *reinterpret_cast<v4i *>(a3.y + pix[t] * CW + ch + 16 * h) = o;
                 if (CHAIN) { // the sum tile: pixel row q, 16-byte piece c at piece c ^ (q & 15) of every 256 bytes
@@ -546,20 +548,33 @@ bool conv_block_tail_applies(const ConvArgs &a2, const ConvArgs &a3, const ConvA
         && an->nslab == cw / 64 && an->kout_pad >= an->K && an->res == nullptr && same_image(*an);
 }
 
-template <int G, int PH, int PW, int ST>
-static void launch_tail_gp(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
+template <int G, int PH, int PW, int ST, bool EXACT>
+static void launch_tail_form(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
 {
+    // The chained form of 128 channels has no register for the exact form's two (28x28, batch 64: 33.8 us with it, 32.2 without).  The
+    // others, exact against not: 64 channels chained, 56x56, 39.4 us against 43.0, 128 channels after a stride 36.0 against 37.8
+    constexpr bool CHAINED = EXACT && !(G == 2 && ST == 1);
     BlockGeom geo;
     geo.H = a2.OH, geo.W = a2.OW, geo.PY = (a2.OH + PH - 1) / PH, geo.PX = (a2.OW + PW - 1) / PW;
     geo.IH = a2.H, geo.IW = a2.W;
     geo.npatch = a2.N * geo.PY * geo.PX;
     const dim3 grid((unsigned)((geo.npatch + 7) / 8 * 8)), block(128 * G);
     if (an && an->K == 2 * a2.in_cs)
-        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 2, ST>), grid, block, 0, st, a2, a3, *an, geo);
+        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 2, ST, CHAINED>), grid, block, 0, st, a2, a3, *an, geo);
     else if (an)
-        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 1, ST>), grid, block, 0, st, a2, a3, *an, geo);
+        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 1, ST, CHAINED>), grid, block, 0, st, a2, a3, *an, geo);
     else
-        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 0, ST>), grid, block, 0, st, a2, a3, a3, geo);
+        hipLaunchKernelGGL((conv_bottleneck_tail_kernel<G, PH, PW, 0, ST, EXACT>), grid, block, 0, st, a2, a3, a3, geo);
+}
+
+template <int G, int PH, int PW, int ST>
+static void launch_tail_gp(const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
+{
+    ConvArgs exact = a3;
+    if (!(G == 2 && ST == 1 && an) && make_add_exact(&exact.addq))
+        launch_tail_form<G, PH, PW, ST, true>(a2, exact, an, st);
+    else
+        launch_tail_form<G, PH, PW, ST, false>(a2, a3, an, st);
 }
 
 template <int G, int ST>
@@ -643,8 +658,8 @@ bool conv_block_applies(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &
         && a1.H >= kPatch && a1.W >= kPatch && (cm == 256 || (a1.H % kPatch == 0 && a1.W % kPatch == 0)) && (long long)a1.N * a1.H * a1.W * cw < (1ll << 31);
 }
 
-template <int G>
-static void launch_block_g(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
+template <int G, bool EXACT>
+static void launch_block_form(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
 {
     BlockGeom geo;
     geo.H = a1.H, geo.W = a1.W, geo.PY = (a1.H + kPatch - 1) / kPatch, geo.PX = (a1.W + kPatch - 1) / kPatch;
@@ -652,13 +667,23 @@ static void launch_block_g(const ConvArgs &a1, const ConvArgs &a2, const ConvArg
     const dim3 grid((unsigned)((geo.npatch + 7) / 8 * 8)), block(128 * G);
     const bool small = geo.PY <= 2 && geo.PX <= 2; // every region is at most 8 x 8 pixels
     if (small && an)
-        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 2, 2>), grid, block, 0, st, a1, a2, a3, *an, geo);
+        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 2, 2, EXACT>), grid, block, 0, st, a1, a2, a3, *an, geo);
     else if (small)
-        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 2, 0>), grid, block, 0, st, a1, a2, a3, a3, geo);
+        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 2, 0, EXACT>), grid, block, 0, st, a1, a2, a3, a3, geo);
     else if (an)
-        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 3, 2>), grid, block, 0, st, a1, a2, a3, *an, geo);
+        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 3, 2, EXACT>), grid, block, 0, st, a1, a2, a3, *an, geo);
     else
-        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 3, 0>), grid, block, 0, st, a1, a2, a3, a3, geo);
+        hipLaunchKernelGGL((conv_bottleneck_kernel<G, 3, 0, EXACT>), grid, block, 0, st, a1, a2, a3, a3, geo);
+}
+
+template <int G>
+static void launch_block_g(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)
+{
+    ConvArgs exact = a3; // 256 channels, 14x14, batch 64: 28.1 us against 29.2
+    if (make_add_exact(&exact.addq))
+        launch_block_form<G, true>(a1, a2, exact, an, st);
+    else
+        launch_block_form<G, false>(a1, a2, a3, an, st);
 }
 
 void launch_conv_block(const ConvArgs &a1, const ConvArgs &a2, const ConvArgs &a3, const ConvArgs *an, hipStream_t st)

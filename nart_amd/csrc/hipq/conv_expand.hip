@@ -73,7 +73,7 @@ template <bool ADD_SAT>
 __device__ inline void fused_in_place(const ConvArgs &a, const v16i (&acc)[2], uint8_t *rtile, int pl, int half)
 {
     const AddParams &q = a.addq;
-    const RequantAdd<> f(a);
+    const RequantAdd<false> f(a);
     const int rsw = (pl >> 1) & 3;
 #pragma unroll
     for (int tn = 0; tn < 2; tn++)

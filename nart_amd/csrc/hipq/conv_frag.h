@@ -35,12 +35,11 @@ __device__ static inline v4i requant16(const ConvArgs &a, const v16i &acc, uint3
     return o;
 }
 
-// The same followed by the residual add (op_quant_add_run on the requantised bytes and the residual's 16 bytes `res`), in the
-// 32-bit form; the sum's last shift and its saturation to [0, 255] are the shifting, saturating pack.
-template <bool WIDE = true>
-__device__ static inline v4i requant_add16(const ConvArgs &a, const v16i &acc, const v4i res)
+// The same followed by the residual add (op_quant_add_run on the requantised bytes and the residual's 16 bytes `res`), in the form f
+// (RequantAdd); the sum's last shift and its saturation to [0, 255] are the shifting, saturating pack.
+template <class F>
+__device__ static __forceinline__ v4i requant_add16(const F &f, const v16i &acc, const v4i res)
 {
-    const RequantAdd<WIDE> f(a);
     v4i o;
 #pragma unroll
     for (int g = 0; g < 4; g++) {
@@ -48,9 +47,16 @@ __device__ static inline v4i requant_add16(const ConvArgs &a, const v16i &acc, c
 #pragma unroll
         for (int e = 0; e < 4; e++)
             y[e] = f(acc[g * 4 + e], (uint32_t)res[g], e);
-        o[g] = (int)ashr_sat_u8x4(y[0], y[1], y[2], y[3], a.addq.sh);
+        o[g] = (int)ashr_sat_u8x4(y[0], y[1], y[2], y[3], f.sh);
     }
     return o;
+}
+
+// the 32-bit form, which every pair of scales of the fast add has
+template <bool WIDE = true>
+__device__ static __forceinline__ v4i requant_add16(const ConvArgs &a, const v16i &acc, const v4i res)
+{
+    return requant_add16(RequantAdd<false, WIDE>(a), acc, res);
 }
 
 // accumulators of a lane <- the folded bias of its 16 consecutive channels (or zero for the wave that does not carry it)

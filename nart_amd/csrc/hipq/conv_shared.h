@@ -120,32 +120,44 @@ __device__ static __forceinline__ int32_t mulhi_add(int32_t acc, uint32_t mult, 
 // byte c is clamp(mulhi(acc, mult) + qadd) >> qt, never negative (a.lo >= 0), the two terms are those of AddTerms, the convolution's
 // zero point in its constant.  35 clocks a value by the instructions' rates, 42 with arithmetic shifts and a
 // multiplication and an addition for the convolution's product.
-// WIDE: the 64-bit multiply-add, which takes a register more.
-template <bool WIDE = true>
+// EXACT: a.addq is in its exact form (make_add_exact), the terms are added up in 64 bits, two multiply-adds in place of two, two shifts and
+// the sum: 27 clocks.  WIDE: 64-bit multiply-adds, which take a register more.
+template <bool EXACT, bool WIDE = true>
 struct RequantAdd {
-    uint64_t qadd;
+    uint64_t qadd, k;
     uint32_t mult, mc, kc, mr, kr;
-    int qt, plo, phi, sc, sr, add;
+    int qt, plo, phi, sc, sr, add, sh;
     __device__ __forceinline__ RequantAdd(const ConvArgs &a)
     {
         const AddParams &q = a.addq;
-        const AddTerms k(q);
         mult = a.q.mult, qadd = (uint64_t)(uint32_t)a.qadd << 32, qt = a.qt, plo = a.lo << a.qt, phi = ((a.q.hi + 1) << a.qt) - 1;
-        mc = a.res_first ? q.m1 : q.m0, sc = a.res_first ? q.s1 : q.s0, kc = a.res_first ? k.k1 : k.k0;
-        mr = a.res_first ? q.m0 : q.m1, sr = a.res_first ? q.s0 : q.s1, kr = a.res_first ? k.k0 : k.k1;
-        add = k.add;
-        if (!WIDE)
-            return;
-        asm("" : "+s"(qadd));
-        asm("" : "+v"(mult)); // the addend in scalar registers: one vector register instead of two
+        mc = a.res_first ? q.m1 : q.m0, mr = a.res_first ? q.m0 : q.m1, sh = q.sh;
+        if (EXACT) {
+            k = (uint64_t)(uint32_t)q.c1 << 32 | (uint32_t)q.c0;
+        } else {
+            const AddTerms t(q);
+            sc = a.res_first ? q.s1 : q.s0, kc = a.res_first ? t.k1 : t.k0;
+            sr = a.res_first ? q.s0 : q.s1, kr = a.res_first ? t.k0 : t.k1;
+            add = t.add;
+        }
+        if (WIDE) {
+            asm("" : "+s"(qadd));
+            asm("" : "+v"(mult)); // the addend in scalar registers: one vector register instead of two
+        }
+        if (EXACT) {
+            asm("" : "+s"(k));
+            asm("" : "+v"(mc));
+        }
     }
-    // acc with byte e of res: the sum before its last shift
+    // acc with byte e of res: the sum before its last shift, by sh
     __device__ __forceinline__ int32_t operator()(int32_t acc, uint32_t res, int e) const
     {
         int32_t c = WIDE ? mulhi_add(acc, mult, qadd) : __mulhi(acc, (int)mult) + (int32_t)(qadd >> 32);
         asm("v_med3_i32 %0, %1, %2, %3" : "=v"(c) : "v"(c), "s"(plo), "v"(phi));
-        const uint32_t t0 = (__umul24((uint32_t)c >> qt, mc) + kc) >> sc, t1 = (__umul24((res >> (8 * e)) & 255, mr) + kr) >> sr;
-        return (int32_t)(t0 + t1 + (uint32_t)add);
+        const uint32_t x = (res >> (8 * e)) & 255;
+        if (EXACT)
+            return (int32_t)((x * (uint64_t)mr + ((uint64_t)((uint32_t)c >> qt) * mc + k)) >> 32);
+        return (int32_t)(((__umul24((uint32_t)c >> qt, mc) + kc) >> sc) + ((__umul24(x, mr) + kr) >> sr) + (uint32_t)add);
     }
 };
 

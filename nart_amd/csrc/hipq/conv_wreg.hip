@@ -157,7 +157,8 @@ __global__ __launch_bounds__(256, 2) void conv_wreg_kernel(const ConvArgs a, con
 // and never travel to memory (a launch, and a write and a read of the widest tensor of the block, disappear).  Both pixel
 // operands go to LDS at the start; b is reduced first and its 16 bytes per lane and pixel tile wait in registers while a is
 // reduced into the same accumulators.
-template <int CPT, int CPT2, int S2>
+// EXACT: a.addq is in its exact form.
+template <int CPT, int CPT2, int S2, bool EXACT>
 __global__ __launch_bounds__(256, (4096 * (CPT + CPT2) <= 53248 ? 3 : 4096 * (CPT + CPT2) <= 81920 ? 2 : 1)) void conv_wreg_dual_kernel(const ConvArgs a, const ConvArgs b, const WregGeom geo)
 {
     constexpr int RB = 64 * CPT, RB2 = 64 * CPT2, X_BYTES = 64 * RB, X2_BYTES = 64 * RB2;
@@ -243,9 +244,10 @@ __global__ __launch_bounds__(256, (4096 * (CPT + CPT2) <= 53248 ? 3 : 4096 * (CP
             ring_fill1<CPT2, D>(ring, ldw2);
         }
         reduce_all<CPT, 2, D>(acc, ringa, (int)a.xmask, ldw, ldb);
+        const RequantAdd<EXACT, EXACT || CPT != 4 || S2 != 1> f(a); // 4, 1: three work-groups a CU leave it no register
 #pragma unroll
         for (int t = 0; t < 2; t++) {
-            const v4i o = requant_add16<CPT != 4 || S2 != 1>(a, acc[t], res[t]); // 4, 1: three work-groups a CU leave it no register
+            const v4i o = requant_add16(f, acc[t], res[t]);
             if (valid[t])
                 *reinterpret_cast<v4i *>(a.y + pix[t] * a.out_cs + st0 + 16 * h) = o;
         }
@@ -282,14 +284,22 @@ void launch_conv_wreg_dual(const ConvArgs &a, const ConvArgs &b, hipStream_t st)
     geo.nnb = nblk / geo.nbpw;
     const dim3 grid((unsigned)((geo.npg * geo.nnb + 7) / 8 * 8)), block(256);
     const int c1 = a.in_cs / 64;
+    ConvArgs ex = a; // 256 channels and 512 after a stride, 14x14, batch 64: 23.5 us in the exact form, 24.8 without; no register for it at stride 1
+    const bool exact = !(c1 == 4 && b.stride_h == 1) && make_add_exact(&ex.addq);
     if (c1 == 4 && b.stride_h == 1)
-        hipLaunchKernelGGL((conv_wreg_dual_kernel<4, 8, 1>), grid, block, 0, st, a, b, geo);
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<4, 8, 1, false>), grid, block, 0, st, a, b, geo);
+    else if (c1 == 4 && exact)
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<4, 8, 2, true>), grid, block, 0, st, ex, b, geo);
     else if (c1 == 4)
-        hipLaunchKernelGGL((conv_wreg_dual_kernel<4, 8, 2>), grid, block, 0, st, a, b, geo);
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<4, 8, 2, false>), grid, block, 0, st, a, b, geo);
+    else if (b.stride_h == 1 && exact)
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 1, true>), grid, block, 0, st, ex, b, geo);
     else if (b.stride_h == 1)
-        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 1>), grid, block, 0, st, a, b, geo);
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 1, false>), grid, block, 0, st, a, b, geo);
+    else if (exact)
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 2, true>), grid, block, 0, st, ex, b, geo);
     else
-        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 2>), grid, block, 0, st, a, b, geo);
+        hipLaunchKernelGGL((conv_wreg_dual_kernel<8, 16, 2, false>), grid, block, 0, st, a, b, geo);
 }
 
 bool conv_wreg_applies(const ConvArgs &a)

@@ -50,6 +50,70 @@ extern "C" void hipq_quant_scale(float x, int bits, uint32_t *mult, int *shift)
     *shift = s + bits - 1;
 }
 
+// The exact form's constants: with u = max(s0, s1) the sum of the terms is (x0 m0 2^(u-s0) + x1 m1 2^(u-s1) + const) / 2^u, scaled by a 2^k
+// that puts as much of the result as fits 32-bit multipliers into the high word.  For each x0 the x1 whose sum lies less than the lost
+// fractions, at most 3 * 2^(u-1), above a multiple of 2^(sh+u) are found in the sorted residues of the second term.
+static bool exact_form(hipq::AddParams *p)
+{
+    const int u = std::max(p->s0, p->s1), d0 = u - p->s0, d1 = u - p->s1;
+    int k = 32 - u - p->sh;
+    while (k >= 0 && (((uint64_t)p->m0 << (d0 + k)) >> 32 || ((uint64_t)p->m1 << (d1 + k)) >> 32))
+        k--;
+    if (k < 0 || u + p->sh + k - 32 < 0 || u + p->sh > 40)
+        return false;
+    const int64_t mod = (int64_t)1 << (u + p->sh), rest = ((int64_t)p->cadd) << u;
+    struct Term {
+        int64_t at, lost;
+    } t1[256];
+    for (int x = 0; x < 256; x++) {
+        const int64_t v = (int64_t)x * p->m1 + p->c1;
+        t1[x] = {(v << d1) & (mod - 1), (v & (((int64_t)1 << p->s1) - 1)) << d1};
+    }
+    std::sort(t1, t1 + 256, [](const Term &a, const Term &b) { return a.at < b.at; });
+    const int64_t most = (int64_t)3 << (u - 1);
+    for (int x = 0; x < 256; x++) {
+        const int64_t v = (int64_t)x * p->m0 + p->c0, at = ((v << d0) + rest) & (mod - 1), lost = (v & (((int64_t)1 << p->s0) - 1)) << d0;
+        const int64_t from = (mod - at) & (mod - 1); // the residue that makes a multiple
+        int i = (int)(std::lower_bound(t1, t1 + 256, from, [](const Term &a, int64_t b) { return a.at < b; }) - t1);
+        for (int n = 0; n < 256; n++, i++) {
+            const Term &t = t1[i & 255];
+            const int64_t above = (t.at - from) & (mod - 1);
+            if (above >= most)
+                break;
+            if (above < lost + t.lost)
+                return false;
+        }
+    }
+    const uint64_t at_zero = (((uint64_t)(int64_t)p->c0 << d0) + ((uint64_t)(int64_t)p->c1 << d1) + (uint64_t)rest) << k;
+    p->m0 <<= d0 + k, p->m1 <<= d1 + k, p->sh += u + k - 32;
+    p->c0 = (int32_t)(uint32_t)at_zero, p->c1 = (int32_t)(uint32_t)(at_zero >> 32);
+    return true;
+}
+
+// The search takes some 10 us, and a launch asks for its add's constants each time: every thread remembers the last forms by the constants
+// that they follow from.
+bool hipq::make_add_exact(AddParams *p)
+{
+    struct Seen {
+        AddParams from, to;
+        bool known, exact;
+    };
+    static thread_local Seen seen[64];
+    if (!p->fast)
+        return false;
+    const uint32_t h = (p->m0 * 0x9e3779b1u ^ p->m1 * 0x85ebca6bu ^ (uint32_t)p->c0 * 0xc2b2ae35u ^ (uint32_t)p->c1 * 0x27d4eb2fu ^ (uint32_t)p->cadd) * 0x9e3779b1u;
+    Seen &e = seen[h >> 26];
+    const AddParams &f = e.from;
+    if (!(e.known && f.m0 == p->m0 && f.m1 == p->m1 && f.s0 == p->s0 && f.s1 == p->s1 && f.sh == p->sh && f.c0 == p->c0 && f.c1 == p->c1 && f.cadd == p->cadd)) {
+        e.from = e.to = *p;
+        e.exact = exact_form(&e.to);
+        e.known = true;
+    }
+    if (e.exact)
+        p->m0 = e.to.m0, p->m1 = e.to.m1, p->sh = e.to.sh, p->c0 = e.to.c0, p->c1 = e.to.c1;
+    return e.exact;
+}
+
 bool hipq::make_add_params(float ia0, int iz0, float ia1, int iz1, float oa, int oz, int obits, AddParams *p)
 {
     int s0, s1;

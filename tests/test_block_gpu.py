@@ -219,6 +219,38 @@ def test_bottleneck_tail_with_a_strided_3x3_layer(case):
     assert not hipq.bottleneck_tail_fusable(plans[0], plans[1], False, rq[0], rq[1], sq[0], sq[1])
 
 
+# the sum's scale over the root of the operands' squares, the residual's over the convolution's: sums in 64 bits, sums in 32 (one ratio of 1 or
+# more, of which the exact form has no multiplier), scales far apart, equal ones
+ADD_SCALES = [(1.1, 0.83), (1.1, 1.57), (0.66, 0.9), (0.5, 1.0), (1.0, 1.0), (2.0, 1.0), (1.3, 1 / 90), (1.3, 60.0), (3.7, 0.4)]
+
+
+@pytest.mark.parametrize("scales", ADD_SCALES, ids=lambda s: "%.2f-%.2f" % s)
+@pytest.mark.parametrize("case", [(1, 256, 16, 16, 1), (1, 512, 14, 28, 1), (1, 512, 7, 14, 2), (1, 1024, 7, 7, 1)], ids=lambda c: "x".join(map(str, c)))
+def test_sums_of_any_pair_of_scales(case, scales):
+    N, CW, H, W, st = case
+    rng = np.random.default_rng(CW + H + int(scales[0] * 100))
+    t1, res, layers, rq, sq, nx = make_tail(rng, N, CW, H, W, False, False, (2 * H, 2 * W) if st == 2 else None)
+    q3 = layers[1]["q"]
+    ra = float(np.float32(q3[4] * scales[1]))
+    sa, sz = float(np.float32(math.hypot(q3[4], ra) * scales[0])), sq[1]
+    plans = plans_of(t1, layers, stride=st)
+    pn = hipq.Conv2d((N, CW, H, W), nx["w"], nx["b"], 0, 1, 1, sa, sz, *nx["q"][2:])
+    t = orc.conv2d_u8(t1, layers[0]["w"], layers[0]["b"], 1, st, 1, *layers[0]["q"])
+    c = orc.conv2d_u8(t, layers[1]["w"], layers[1]["b"], 0, 1, 1, *q3)
+    xd, rd = hipq.to_device_nhwc(t1), hipq.to_device_nhwc(res)
+    for res_first, chain in ((False, False), (True, True)):
+        print("scales", case, scales, res_first, chain, flush=True)
+        if not hipq.bottleneck_tail_fusable(plans[0], plans[1], res_first, ra, rq[1], sa, sz, pn if chain else None):
+            assert max(ra, q3[4]) < sa / 8 or max(ra, q3[4]) > 30 * min(ra, q3[4])  # shifts beyond the fast form's
+            continue
+        want = orc.add_u8(res, c, ra, rq[1], q3[4], q3[5], sa, sz) if res_first else orc.add_u8(c, res, q3[4], q3[5], ra, rq[1], sa, sz)
+        y = torch.zeros_like(rd)
+        yn = torch.zeros((N, H, W, nx["w"].shape[0]), dtype=torch.uint8, device="cuda") if chain else None
+        hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, res_first, ra, rq[1], sa, sz, y, pn if chain else None, yn)
+        got = hipq.from_device_nhwc(y, CW)
+        assert np.array_equal(got, want), (case, scales, res_first, chain, int((got != want).sum()))
+
+
 def test_bottleneck_refusals():
     """What the one-launch forms do not serve is refused by the predicates and fails loudly in the run entry points."""
     rng = np.random.default_rng(7)
