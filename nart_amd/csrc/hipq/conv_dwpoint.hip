@@ -49,7 +49,15 @@ struct PairGeom {
     int nT;     // slices of 32 channels
     int ct;     // tiles of 32 output channels
     int groups; // of output channel tiles, a work-group each
+    int nw;     // waves
+    int red;    // where a shared patch's sums lie in LDS
+    int ppi, items, per_xcd;         // patches of an image, work-groups, those of an XCD
+    uint32_t m_groups, m_ppi, m_px;  // x / groups, x / ppi and x / PX (hipq_div_magic)
+    int s_groups, s_ppi, s_px;
 };
+
+// x / d for any x below 2^31 (hipq_div_magic)
+__device__ static __forceinline__ int quot(int x, uint32_t m, int s) { return m ? (int)(__umulhi((uint32_t)x, m) >> s) : x; }
 
 } // namespace
 
@@ -60,18 +68,17 @@ __global__ __launch_bounds__(64 * max_waves(PH / 4, CT)) void conv_dwpoint_kerne
     constexpr int PW = G::PW, RW = G::RW, NP = G::NP, PT = G::PT, NR = G::NR;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = geo.nw;
     const int p = lane & 31, h = lane >> 5;
     const int ch = slice_channel(p);
     // work-groups go to the 8 XCDs in turn: XCD x takes the x-th contiguous eighth of the work, the groups of a patch side by side.
     // (Eighths of the patches with all their groups left XCDs idle where patches are few: 18 patches in 13 groups took 7.0 us, two
     // rounds of work-groups on six XCDs, against 4.5.)
-    const int ppi = geo.PY * geo.PX;
-    const int item = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
-    const int gid = item / geo.groups;
-    if (gid >= ppi * d.N)
+    const int item = (int)(blockIdx.x % 8) * geo.per_xcd + (int)(blockIdx.x / 8);
+    if (item >= geo.items)
         return;
-    const int n = gid / ppi, pi = gid - n * ppi, py = pi / geo.PX;
+    const int gid = quot(item, geo.m_groups, geo.s_groups);
+    const int n = quot(gid, geo.m_ppi, geo.s_ppi), pi = gid - n * geo.ppi, py = quot(pi, geo.m_px, geo.s_px);
     const int oy0 = py * PH, ox0 = (pi - py * geo.PX) * PW;
     const int iy0 = S * oy0 - 1, ix0 = S * ox0 - 1; // the region's first row and column
     const int ct0 = (item - gid * geo.groups) * CT;
@@ -84,11 +91,9 @@ __global__ __launch_bounds__(64 * max_waves(PH / 4, CT)) void conv_dwpoint_kerne
 #pragma unroll
     for (int i = 0; i < NR; i++) {
         const int pos = min((lane + 64 * i) >> 1, NP - 1), ry = pos / RW, iy = iy0 + ry, ix = ix0 + pos - ry * RW;
-        const bool in = (unsigned)iy < (unsigned)d.H && (unsigned)ix < (unsigned)d.W;
+        const bool in = ((unsigned)iy < (unsigned)d.H) & ((unsigned)ix < (unsigned)d.W);
         valid |= in ? 1u << i : 0u;
         from[i] = (uint32_t)(((n * d.H + min(max(iy, 0), d.H - 1)) * d.W + min(max(ix, 0), d.W - 1)) * d.in_cs);
-        if (!in) // the same byte in every slice
-            *reinterpret_cast<v4i *>(buf + (lane + 64 * i) * 16) = v4i{epad, epad, epad, epad};
     }
 
     // ---- a slice's pixels, weights and constants, each loaded as soon as the slice before has used its own
@@ -117,17 +122,31 @@ __global__ __launch_bounds__(64 * max_waves(PH / 4, CT)) void conv_dwpoint_kerne
     load_x(T);
     load_d(T);
     load_p(T);
+    // the sums, from the folded bias of the lane's 16 consecutive channels in the first wave; what is here does not wait for the loads
+    v16i acc[CT][PT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int t = 0; t < PT; t++) {
+            if (wave == 0)
+                init_acc(acc[ct][t], pr.bias2 + 32 * min(ct0 + ct, geo.ct - 1) + 16 * h, false);
+            else
+                acc[ct][t] = v16i{};
+        }
+    int32_t *const red = reinterpret_cast<int32_t *>(lds + geo.red);
+    for (int i = threadIdx.x; i < CT * PT * 256; i += 64 * nw)
+        reinterpret_cast<v4i *>(red)[i] = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < NR; i++)
+        if (!(valid >> i & 1)) // the same byte in every slice
+            *reinterpret_cast<v4i *>(buf + (lane + 64 * i) * 16) = v4i{epad, epad, epad, epad};
     const DiagonalTap taps(lane);
     int first[PT]; // the lane's outputs 32 t + p: their first tap in the region
 #pragma unroll
     for (int t = 0; t < PT; t++)
         first[t] = (S * (4 * t + (p >> 3)) * RW + S * (p & 7)) * 32 + 16 * h;
-    v16i acc[CT][PT];
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++)
-#pragma unroll
-        for (int t = 0; t < PT; t++)
-            acc[ct][t] = v16i{};
+    __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();       // the sums are zero
 
     while (true) {
         const bool more = T + nw < geo.nT;
@@ -167,22 +186,17 @@ __global__ __launch_bounds__(64 * max_waves(PH / 4, CT)) void conv_dwpoint_kerne
         lds_order();
     }
 
-    auto store = [&](int ct, int t, const v16i &s) {
-        const int oy = oy0 + 4 * t + (p >> 3), ox = ox0 + (p & 7), c0 = 32 * (ct0 + ct) + 16 * h;
-        if (oy >= pr.OH || ox >= pr.OW || c0 >= pr.out_cs)
-            return;
-        const size_t at = (size_t)((n * pr.OH + oy) * pr.OW + ox) * pr.out_cs + c0;
-        const v4i v = pr.res != nullptr ? requant_add16(pr, s, ldg128(pr.res + at)) : requant16(pr, s, 0);
-        *reinterpret_cast<v4i *>(pr.y + at) = v;
+    // ---- the waves' partial sums meet in LDS; a wave's output tile, i, is the one it takes first: its residual is under way meanwhile
+    auto place = [&](int i, uint32_t *at) { // of the lane's 16 channels of its pixel
+        const int ct = i / PT, oy = oy0 + 4 * (i - ct * PT) + (p >> 3), ox = ox0 + (p & 7), c0 = 32 * (ct0 + ct) + 16 * h;
+        *at = (uint32_t)(((n * pr.OH + oy) * pr.OW + ox) * pr.out_cs + c0); // below 2^31
+        return (i < CT * PT) & (oy < pr.OH) & (ox < pr.OW) & (c0 < pr.out_cs);
     };
-    // ---- the waves' partial sums meet in LDS (where the regions were), over the folded bias
-    __syncthreads();
-    int32_t *const red = reinterpret_cast<int32_t *>(lds);
-    for (int i = threadIdx.x; i < CT * PT * 1024; i += blockDim.x) {
-        const int l = i & 63, r = (i >> 6) & 15, ct = (i >> 10) / PT;
-        red[i] = pr.bias2[32 * min(ct0 + ct, geo.ct - 1) + 16 * (l >> 5) + r];
-    }
-    __syncthreads();
+    uint32_t at;
+    bool in = place(wave, &at);
+    v4i res = {0, 0, 0, 0};
+    if (in && pr.res != nullptr)
+        res = ldg128(pr.res + at);
 #pragma unroll
     for (int ct = 0; ct < CT; ct++)
 #pragma unroll
@@ -192,11 +206,17 @@ __global__ __launch_bounds__(64 * max_waves(PH / 4, CT)) void conv_dwpoint_kerne
                 atomicAdd(&red[((ct * PT + t) * 16 + r) * 64 + lane], acc[ct][t][r]);
     __syncthreads();
     for (int i = wave; i < CT * PT; i += nw) {
+        if (i != wave) {
+            in = place(i, &at);
+            if (in && pr.res != nullptr)
+                res = ldg128(pr.res + at);
+        }
         v16i s;
 #pragma unroll
         for (int r = 0; r < 16; r++)
             s[r] = red[(i * 16 + r) * 64 + lane];
-        store(i / PT, i % PT, s);
+        if (in)
+            *reinterpret_cast<v4i *>(pr.y + at) = pr.res != nullptr ? requant_add16(pr, s, res) : requant16(pr, s, 0);
     }
 }
 
@@ -378,6 +398,10 @@ PairDivision divide(const ConvArgs &d, const ConvArgs &p, const PairShape &s)
     v.geo.PY = (p.OH + s.ph - 1) / s.ph, v.geo.PX = (p.OW + 7) / 8, v.geo.nT = (d.in_cs + 31) / 32, v.geo.ct = (p.out_cs + 31) / 32;
     v.groups = v.geo.groups = (v.geo.ct + s.ct - 1) / s.ct;
     v.patches = (long long)d.N * v.geo.PY * v.geo.PX;
+    v.geo.red = 0, v.geo.ppi = v.geo.PY * v.geo.PX, v.geo.items = (int)v.patches * v.groups, v.geo.per_xcd = (v.geo.items + 7) / 8;
+    hipq_div_magic((uint32_t)v.groups, &v.geo.m_groups, &v.geo.s_groups);
+    hipq_div_magic((uint32_t)v.geo.ppi, &v.geo.m_ppi, &v.geo.s_ppi);
+    hipq_div_magic((uint32_t)v.geo.PX, &v.geo.m_px, &v.geo.s_px);
     if (s.narrow) {
         const bool three = s.ph == 8 ? s.ct == 1 && p.out_cs == 16 : st == 1 || s.ct == 1; // waves per SIMD that the registers allow, or two
         v.held = three ? 3 : 2;
@@ -389,8 +413,9 @@ PairDivision divide(const ConvArgs &d, const ConvArgs &p, const PairShape &s)
         v.rounds = (v.geo.nT + v.nw - 1) / v.nw;
         v.nw = (v.geo.nT + v.rounds - 1) / v.rounds; // the same rounds with fewer waves
         v.wgs = v.patches;
-        v.lds = (unsigned)std::max(v.nw * bytes, s.ct * (s.ph / 4) * 4096);
+        v.geo.red = v.nw * bytes, v.lds = (unsigned)(v.geo.red + s.ct * (s.ph / 4) * 4096);
     }
+    v.geo.nw = v.nw;
     return v;
 }
 
