@@ -18,7 +18,9 @@
 // to 35 %) and matrix cores (4 to 7 %) take turns and mostly wait.
 // Measured, the two launches -> this one (back to back and warm): 32 -> 16 channels at 112x112, 64 images: 24.8 -> 14.7 us (38 MB of
 // input and output), 1 image: 5.2 -> 3.0; 64 -> 128 at 56x56, stride 2, 1 image: 6.1 -> 4.1; 192 -> 64 at 28x28, stride 2, 6 images:
-// 5.5 -> 4.3; 960 -> 160 at 7x7, 64 images: 9.9 -> 8.8, 1 image: 5.7 -> 6.1 (there the two launches stay).
+// 5.5 -> 4.3; 960 -> 160 at 7x7, 64 images: 10.6 -> 9.1, 1 image: 6.6 -> 6.8 (there the two launches stay).  A shared patch's biases,
+// residual and the place where its sums meet are ready before them: 1.1 to 1.4 times as fast as with the three in the chain (960 ->
+// 320, 64 images, 11.2 -> 9.2).
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply requantisations.
 #include "conv_dwpoint.h"
 
@@ -432,16 +434,16 @@ void launch_shape(const ConvArgs &d, const ConvArgs &p, const PairShape &s, hipS
         hipLaunchKernelGGL((conv_dwpoint_narrow_kernel<S, PH, CT, false>), grid, block, v.lds, st, d, p, v.geo);
 }
 
-// Time by shape, in us, fitted to 900 pairs of layers (1 to 128 images of 3x3 to 130x130, 16 to 1024 channels to 12 to 400; nine in
-// ten within 20 % of the fit).  Shared patches: a launch; per generation of resident work-groups its start, the waves' sums that meet in
+// Time by shape, in us, fitted to 420 pairs of layers (1 to 128 images of 3x3 to 128x128, 16 to 1024 channels to 12 to 400; nine in
+// ten within 18 % of the fit; the shape it picks takes 1.3 % more than the best one on average), narrow ones to 900.  Shared patches: a launch; per generation of resident work-groups its start, the waves' sums that meet in
 // LDS, and the tiles that a wave finishes; per slice that a wave takes its chain, alone and per wave on its SIMD; the slices per SIMD of the
 // chip.  Narrow ones: a launch; per patch that a wave takes its chain, alone and per wave on its SIMD; the patches, and their channel
 // tiles, per SIMD of the chip; generations.
 double shape_cost(const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    static const double kShared[3][7] = {{1.721, 0, 0.908, 0.022, 0.881, 0.077, 1.528}, // 4x8, stride 1
-                                         {1.825, 0.067, 1.284, 0.042, 0.903, 0.158, 1.618}, // 8x8
-                                         {1.090, 0.668, 1.178, 0, 1.078, 0.183, 1.510}}; // 4x8, stride 2
+    static const double kShared[3][7] = {{2.473, 0.319, 0.738, 0.198, 0.805, 0.105, 0.304}, // 4x8, stride 1
+                                         {2.207, 1.202, 0.522, 0.501, 0.606, 0.143, 0.300}, // 8x8
+                                         {2.232, 0.727, 0.888, 0.240, 0.762, 0.207, 0.285}}; // 4x8, stride 2
     static const double kNarrow[3][6] = {{2.370, 0, 0.132, 0, 0.435, 0.557}, {2.379, 0.569, 0, 0, 0.794, 0.660}, {3.016, 0, 0.103, 0, 0.695, 0.155}};
     const PairShape &s = kShapes[shape];
     if ((d.stride_h == 2 && s.ph == 8) || (s.narrow && d.in_cs > 32))
@@ -517,14 +519,14 @@ double conv_dwpoint_us(const ConvArgs &d, const ConvArgs &p)
     return us;
 }
 
-// The two launches: their latencies, the bytes of the first one's input and output, the products of the second and its output; fitted to
-// the same pairs (nine in ten within 19 %).  Of 150 pairs that the fits have not seen this fuses 113, which take 0.73 of the two
-// launches on average, two of them longer (8.7 -> 10.2 us, 11.6 -> 12.2); of the other 37 it would have been faster for four (8.0 ->
-// 5.7 us at most).
+// The two launches: their latencies, the bytes of the tensor between them, the products of the second and its output, its weights, less 0.07 (a tie stays apart); fitted to
+// the same pairs (nine in ten within 12 %).  Of the 420 this fuses 320, which take 0.75 of the two launches on average, 14 of them longer
+// (10.7 -> 13.2 us at most); of the other 100 it would have been faster for 14, by a tenth at most.
 double conv_dwpoint_apart_us(const ConvArgs &d, const ConvArgs &p)
 {
-    const double in = (double)d.N * d.H * d.W * d.in_cs * 1e-6, mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6;
-    return d.stride_h == 1 ? 5.54 + 0.683 * in + 0.00243 * mid * p.out_cs + 0.182 * out : 5.93 + 0.959 * mid + 0.00471 * mid * p.out_cs + 0.036 * out;
+    const double mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6, in = d.in_cs * 1e-3, weights = (double)d.in_cs * p.out_cs * 1e-6;
+    return d.stride_h == 1 ? 6.10 + 0.580 * mid + 0.00154 * mid * p.out_cs + 0.216 * out + 0.254 * in + 2.171 * weights
+                           : 6.43 + 1.056 * mid + 0.00187 * mid * p.out_cs + 0.055 * out + 0.729 * weights;
 }
 
 const char *conv_dwpoint_name(const ConvArgs &d, const ConvArgs &p, int wanted)
