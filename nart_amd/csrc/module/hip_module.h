@@ -63,6 +63,9 @@ struct hip_workspace_t {
     hipStream_t stream; // every kernel of this workspace is launched here
     bool own_stream;
     bool passes;    // from the first pass that may be recorded on (hip_pass.cpp): launches are taken to cost the host nothing
+    // while hip_pass_run runs the operators of a pass: all of them, in their order, and whose turn it is; otherwise null
+    op_t *const *pass_ops;
+    size_t pass_n, pass_at;
     uint64_t epoch; // counts prepare and destroy calls of this workspace's operators (a recorded pass is good for one value)
 };
 

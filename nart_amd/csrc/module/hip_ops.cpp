@@ -59,8 +59,6 @@ void same_shape_and_geometry(const op_t *op, const tensor_t *t)
 // an operator of this workspace was prepared or is going away: a recorded pass that names it is no longer good
 void touch(op_t *op) { ++reinterpret_cast<hip_workspace_t *>(op->workspace)->epoch; }
 
-void remember_writer(op_t *op);
-
 void alloc_and_tag(op_t *op)
 {
     touch(op);
@@ -71,7 +69,6 @@ void alloc_and_tag(op_t *op)
         tensor_alloc(&op->output_tensors[i]);
         hip_mem_tag(&op->output_tensors[i]);
     }
-    remember_writer(op);
 }
 
 bool forget_reader(op_t *op); // false: the workspace is gone already
@@ -105,26 +102,7 @@ long g_fused_adds = 0, g_fused_relus = 0, g_fused_pools = 0, g_chained_convs = 0
 // (g_chained_convs: convolutions launched by another operator's call, which on few pixels is two kernels)
 long g_fused_blocks = 0, g_fused_inverted = 0, g_fused_pairs = 0, g_fused_tails = 0; // whole bottleneck / inverted residual blocks, blocks from their 3x3 layer on, as one launch
 
-// and which operator writes which memory
-std::map<const workspace_t *, std::map<const mem_t *, op_t *>> g_writers;
-
 reader_map &readers_of(op_t *op) { return g_readers[op->workspace]; }
-
-void remember_writer(op_t *op)
-{
-    for (size_t i = 0; i < op->output_size; ++i)
-        g_writers[op->workspace][op->output_tensors[i].mem] = op;
-}
-
-// the operator of op's workspace that writes a memory; null: none
-op_t *writer_of(const op_t *op, const mem_t *m)
-{
-    const auto wit = g_writers.find(op->workspace);
-    if (wit == g_writers.end())
-        return nullptr;
-    const auto it = wit->second.find(m);
-    return it == wit->second.end() ? nullptr : it->second;
-}
 
 bool forget_reader(op_t *op)
 {
@@ -133,9 +111,6 @@ bool forget_reader(op_t *op)
         return false;
     for (auto &kv : it->second)
         kv.second.erase(op);
-    auto &writers = g_writers[op->workspace];
-    for (auto w = writers.begin(); w != writers.end();)
-        w = w->second == op ? writers.erase(w) : std::next(w);
     return true;
 }
 
@@ -182,7 +157,6 @@ struct conv_op_t {
     // this pass's output has already been written, by the kernel of the pooling operator whose output this convolution
     // reads (hipq_conv2d_run_maxpool_conv) or with another convolution (conv_run_pair): run() has nothing left to do
     bool computed_ahead;
-    unsigned long turns; // how often run() has been called
 };
 
 void conv_config(op_t *op)
@@ -470,13 +444,25 @@ bool sole_reader_fuses(op_t *op)
         && r->input_tensors[0]->mem != r->input_tensors[1]->mem && strncmp(hipq_conv2d_plan_kernel(c->plan), "conv_mfma", 9) == 0;
 }
 
-// The convolution o left its launch to an add whose other input is a convolution that leaves its launch to the same add: that one will be
-// fused, and o launched by itself all the same.
-bool launches_anyway(op_t *o)
+bool writes(const op_t *op, const mem_t *m)
+{
+    for (size_t i = 0; i < op->output_size; ++i)
+        if (op->output_tensors[i].mem == m)
+            return true;
+    return false;
+}
+
+// The convolution o of the pass left its launch to an add whose other input is a convolution that leaves its launch to the same add: that
+// one will be fused, and o launched by itself all the same.
+bool launches_anyway(const hip_workspace_t *ws, const op_t *o)
 {
     int i = 0;
-    const op_t *a = add_reading(o, &i);
-    const op_t *w = a != nullptr ? writer_of(o, a->input_tensors[1 - i]->mem) : nullptr;
+    const op_t *a = add_reading(o, &i), *w = nullptr;
+    if (a == nullptr)
+        return false;
+    for (size_t k = 0; k < ws->pass_n && ws->pass_ops[k] != a; ++k)
+        if (writes(ws->pass_ops[k], a->input_tensors[1 - i]->mem))
+            w = ws->pass_ops[k];
     if (w == nullptr || w == o || w->entry->tp != &op_conv_2d_tp || only_reader(w) != a)
         return false;
     const conv_op_t *c = reinterpret_cast<const conv_op_t *>(w);
@@ -484,26 +470,26 @@ bool launches_anyway(op_t *o)
 }
 
 // A residual block's first layer and its projection shortcut, which read the same tensor, in one launch (hipq_conv2d_run_pair): op's
-// turn launches both, and the other one's finds its work done.  Only where whole passes run, and only with a convolution whose turn in
-// this pass is still to come: one that has had exactly one less.
+// turn launches both, and the other one's finds its work done.  Only inside a pass that the module runs, and with a convolution
+// whose turn in it is still to come.
 bool conv_run_pair(op_t *op)
 {
     static const bool off = getenv("NART_HIP_NO_FUSION") != nullptr;
     conv_op_t *c = reinterpret_cast<conv_op_t *>(op);
-    if (off || !reinterpret_cast<const hip_workspace_t *>(op->workspace)->passes || op->entry->tp != &op_conv_2d_tp || c->desc.dtype != HIPQ_DTYPE_U8)
+    const hip_workspace_t *ws = reinterpret_cast<const hip_workspace_t *>(op->workspace);
+    if (off || ws->pass_ops == nullptr || ws->pass_ops[ws->pass_at] != op || op->entry->tp != &op_conv_2d_tp || c->desc.dtype != HIPQ_DTYPE_U8)
         return false;
-    const reader_map &rm = readers_of(op);
-    const auto it = rm.find(op->input_tensors[0]->mem);
-    if (it == rm.end())
-        return false;
-    for (const op_t *r : it->second) {
-        conv_op_t *o = reinterpret_cast<conv_op_t *>(const_cast<op_t *>(r));
-        // one that is launched by itself, and not with another operator
-        if (r == op || r->workspace != op->workspace || r->entry->tp != &op_conv_2d_tp || r->input_tensors[0]->mem != op->input_tensors[0]->mem
-            || o->plan == nullptr || !o->defer_in_passes || o->computed_ahead || o->turns + 1 != c->turns || o->ir_project != nullptr
-            || !(o->defer == -1 || (o->defer == 1 && launches_anyway(&o->o))) || !hipq_conv2d_pair_fusable(c->plan, o->plan))
+    const mem_t *x = op->input_tensors[0]->mem;
+    for (size_t k = ws->pass_at + 1; k < ws->pass_n; ++k) {
+        op_t *r = ws->pass_ops[k];
+        if (r->entry->tp != &op_conv_2d_tp || r->input_tensors[0]->mem != x)
             continue;
-        if (hipq_conv2d_run_pair(c->plan, in_ptr(op, 0), 0, out_ptr(op), o->plan, in_ptr(op, 0), 0, out_ptr(&o->o), op_stream(op)) != 0)
+        conv_op_t *o = reinterpret_cast<conv_op_t *>(r);
+        // one that is launched by itself, and not with another operator
+        if (o->plan == nullptr || !o->defer_in_passes || o->computed_ahead || o->ir_project != nullptr
+            || !(o->defer == -1 || (o->defer == 1 && launches_anyway(ws, r))) || !hipq_conv2d_pair_fusable(c->plan, o->plan))
+            continue;
+        if (hipq_conv2d_run_pair(c->plan, in_ptr(op, 0), 0, out_ptr(op), o->plan, in_ptr(op, 0), 0, out_ptr(r), op_stream(op)) != 0)
             continue;
         o->computed_ahead = true;
         ++g_chained_convs;
@@ -515,7 +501,6 @@ bool conv_run_pair(op_t *op)
 void conv_run(op_t *op)
 {
     conv_op_t *c = reinterpret_cast<conv_op_t *>(op);
-    ++c->turns;
     if (c->computed_ahead) {
         c->computed_ahead = false;
         return;
@@ -1523,7 +1508,6 @@ void ws_delete(workspace_t *w)
         hip_stream_forget(ws->stream);
     }
     g_readers.erase(w);
-    g_writers.erase(w);
     free(ws);
 }
 

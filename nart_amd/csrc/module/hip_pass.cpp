@@ -149,6 +149,16 @@ void collect_outputs(Pass &p, op_t *const *ops, size_t n)
         }
 }
 
+// Operator by operator.  What an operator may compute ahead of another's turn (conv_run_pair) it reads off the list.
+void run_operators(op_t *const *ops, size_t n)
+{
+    hip_workspace_t *ws = reinterpret_cast<hip_workspace_t *>(ops[0]->workspace);
+    ws->pass_ops = ops, ws->pass_n = n;
+    for (ws->pass_at = 0; ws->pass_at < n; ++ws->pass_at)
+        op_run(ops[ws->pass_at]);
+    ws->pass_ops = nullptr;
+}
+
 bool record(Pass &p, op_t *const *ops, size_t n)
 {
     if (!collect_inputs(p, ops, n))
@@ -161,8 +171,7 @@ bool record(Pass &p, op_t *const *ops, size_t n)
         before[c] = *hip_counters()[c];
     if (!worked(hipStreamBeginCapture(p.st, hipStreamCaptureModeThreadLocal)))
         return false;
-    for (size_t i = 0; i < n; ++i)
-        op_run(ops[i]);
+    run_operators(ops, n);
     collect_outputs(p, ops, n);
     hipGraph_t g = nullptr;
     size_t nodes = 0;
@@ -237,11 +246,14 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
             p.forget(false, true); // the next record copies back what has been read by then
     }
     if (p.exec == nullptr) {
-        if (p.runs++ < p.wait)
-            return false;
+        if (p.runs++ < p.wait) {
+            run_operators(ops, n);
+            return true;
+        }
         if (!record(p, ops, n)) {
             p.forget(true);
-            return false;
+            run_operators(ops, n);
+            return true;
         }
     } else {
         ++p.served;

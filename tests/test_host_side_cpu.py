@@ -260,6 +260,71 @@ def blocks_are_decided_again_for_recorded_passes():
         p.delete()
 
 
+def launched(o):
+    """How many kernels an operator's run() launches."""
+    kernels = C.c_long.in_dll(STUB, "stub_kernels")
+    before = kernels.value
+    o.run()
+    return kernels.value - before
+
+
+def operators_run_one_by_one_launch_themselves():
+    """Two convolutions of one tensor run as one launch inside a pass only: on a workspace that has run passes, whatever is run between
+    them and however often each has run, each run() launches its own kernel and reads what the tensor holds then."""
+    import numpy as np
+    rt = runtime()
+    ws = rt.workspace("hip")
+    p, pass_of = small_parade(rt, ws)
+    assert pass_of() == "eager"
+    x = ws.tensor(np.zeros((1, 64, 14, 14), np.uint8))
+    q = dict(ialpha=0.05, izp=9, walpha=0.002, wzp=128, oalpha=0.05, ozp=9)
+    a, b = (ws.conv2d(x, ws.tensor(np.full((128, 64, r, r), 130, np.uint8)), None, r // 2, 2, 1, q).prepare() for r in (3, 1))
+    for o in (a, b, a, b, a, a, b, b, a, b, a, b):
+        x.write(np.ones((1, 64, 14, 14), np.uint8))  # one kernel brings it in
+        assert launched(o) == 2 and launched(o) == 1
+        if o is b:
+            pass_of()
+
+
+def two_parades_of_one_input_launch_their_own_layers():
+    """Two parades of a workspace whose input is one memory, each with a convolution of it that could run with the other's: a pass computes
+    the layers of its own parade, recorded or not, in whatever order the passes come."""
+    import numpy as np
+    from nart_amd import cases, engine
+    rt = runtime()
+    ws = rt.workspace("hip")
+    parades = []
+    for r in (3, 1):
+        c = cases.Case("chain", 3)
+        t = c.conv(c.input_u8((1, 64, 14, 14), 0.05, 9), 128, r, stride=2)
+        for _ in range(9):
+            t = c.conv(t, 64, 1)
+        c.output = t
+        parades.append(engine.Parade(rt, engine.write_engine(c), [ws], prepare=False))
+    inputs = [p.inputs()[0] for p in parades]
+    rt.core.tensor_share.argtypes = [C.c_void_p, C.c_void_p]
+    rt.core.tensor_share(inputs[0].ptr, inputs[1].ptr)
+    for p in parades:
+        rt.core.parade_prepare(p.ptr)
+    kernels, replays = (C.c_long.in_dll(STUB, "stub_" + n) for n in ("kernels", "graph_launches"))
+    x = np.zeros((1, 64, 14, 14), np.uint8)
+    eager = []
+    for p in parades:
+        before = kernels.value
+        p.run()
+        eager.append(kernels.value - before)
+    assert eager == [11, 10]  # the first one's pass brings the input in
+    for k, order in enumerate(((0, 0, 1), (1, 0, 1), (0, 1, 0))):
+        for i in order:
+            inputs[0].write(x)
+            before, n = kernels.value, replays.value
+            parades[i].run()
+            assert replays.value == n + 1
+            launches = kernels.value - before
+            assert launches in (0, 1, 10, 11), (k, i, launches)  # replayed, replayed behind an upload, recorded
+    assert rt.libs[1].hip_module_chained_convs() == 0
+
+
 def a_pass_that_cannot_be_recorded_runs_its_operators():
     """On the null stream, which cannot be captured, and where the runtime refuses the graph: every pass runs operator by
     operator, and no error stays behind for the next launch to find."""
@@ -468,6 +533,7 @@ def operators_of_two_workspaces_wait_for_each_other():
 
 CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
+         operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,

@@ -77,6 +77,34 @@ def test_passes_on_the_streams_of_a_workspace(own_rt, stream):
     ws.delete()
 
 
+def test_convolutions_of_one_tensor_one_by_one_between_passes(own_rt):
+    """Two convolutions that a pass would run as one launch, each run by itself on a workspace that has run passes, with a new input
+    before each run and the other one left out now and then: every output is that of the input as it was."""
+    from oracle import orc
+    ws = own_rt.workspace("hip")
+    case = cases.resnet18(N=1, hw=64)
+    p = engine.Parade(own_rt, engine.write_engine(case), [ws])
+    rng = np.random.default_rng(4)
+    q = dict(ialpha=0.05, izp=9, walpha=0.002, wzp=128, oalpha=0.5, ozp=120)
+    x = ws.tensor(np.zeros((1, 64, 14, 14), np.uint8))
+    layers = []
+    for r in (3, 1):
+        w, b = rng.integers(0, 256, (128, 64, r, r), dtype=np.uint8), rng.integers(-9000, 9000, 128).astype(np.int32)
+        layers.append((ws.conv2d(x, ws.tensor(w), ws.tensor(b), r // 2, 2, 1, q).prepare(), w, b, r))
+    for step, i in enumerate((0, 1, 0, 1, 0, 0, 1, 1, 0, 1)):
+        if step % 3 == 0:
+            xin = casecpu.random_input(case, step)
+            assert same_bits(p.forward(xin).reshape(case.output.shape), casecpu.run_case(case, xin)[case.output.name]), step
+        op, w, b, r = layers[i]
+        xv = rng.integers(0, 256, (1, 64, 14, 14), dtype=np.uint8)
+        x.write(xv)
+        op.run()
+        want = orc.conv2d_u8(xv, w, b, r // 2, 2, 1, *(q[k] for k in ("ialpha", "izp", "walpha", "wzp", "oalpha", "ozp")))
+        assert np.array_equal(op.output(0).numpy(), want), (step, i)
+    p.delete()
+    ws.delete()
+
+
 def test_version2_engine_file(own_rt):
     """Version-2 engine files (an optional pre-processing block after every input declaration) load on the repo's core
     and run on the hip workspace; the block is handed back unchanged."""
