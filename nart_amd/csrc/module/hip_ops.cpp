@@ -452,6 +452,14 @@ bool writes(const op_t *op, const mem_t *m)
     return false;
 }
 
+bool reads(const op_t *op, const mem_t *m)
+{
+    for (size_t i = 0; i < op->input_size; ++i)
+        if (op->input_tensors[i]->mem == m)
+            return true;
+    return false;
+}
+
 // The convolution o of the pass left its launch to an add whose other input is a convolution that leaves its launch to the same add: that
 // one will be fused, and o launched by itself all the same.
 bool launches_anyway(const hip_workspace_t *ws, const op_t *o)
@@ -470,8 +478,8 @@ bool launches_anyway(const hip_workspace_t *ws, const op_t *o)
 }
 
 // A residual block's first layer and its projection shortcut, which read the same tensor, in one launch (hipq_conv2d_run_pair): op's
-// turn launches both, and the other one's finds its work done.  Only inside a pass that the module runs, and with a convolution
-// whose turn in it is still to come.
+// turn launches both, and the other one's finds its work done.  Only inside a pass that the module runs, whose list says what comes
+// between the two: nothing that writes the tensor they read, and nothing ahead of the other one that has to do with the memory it writes.
 bool conv_run_pair(op_t *op)
 {
     static const bool off = getenv("NART_HIP_NO_FUSION") != nullptr;
@@ -480,7 +488,7 @@ bool conv_run_pair(op_t *op)
     if (off || ws->pass_ops == nullptr || ws->pass_ops[ws->pass_at] != op || op->entry->tp != &op_conv_2d_tp || c->desc.dtype != HIPQ_DTYPE_U8)
         return false;
     const mem_t *x = op->input_tensors[0]->mem;
-    for (size_t k = ws->pass_at + 1; k < ws->pass_n; ++k) {
+    for (size_t k = ws->pass_at + 1; k < ws->pass_n && !writes(ws->pass_ops[k - 1], x); ++k) {
         op_t *r = ws->pass_ops[k];
         if (r->entry->tp != &op_conv_2d_tp || r->input_tensors[0]->mem != x)
             continue;
@@ -489,7 +497,11 @@ bool conv_run_pair(op_t *op)
         if (o->plan == nullptr || !o->defer_in_passes || o->computed_ahead || o->ir_project != nullptr
             || !(o->defer == -1 || (o->defer == 1 && launches_anyway(ws, r))) || !hipq_conv2d_pair_fusable(c->plan, o->plan))
             continue;
-        if (hipq_conv2d_run_pair(c->plan, in_ptr(op, 0), 0, out_ptr(op), o->plan, in_ptr(op, 0), 0, out_ptr(r), op_stream(op)) != 0)
+        const mem_t *y = r->output_tensors[0].mem;
+        bool free = true;
+        for (size_t i = 0; i < k; ++i)
+            free = free && !reads(ws->pass_ops[i], y) && !writes(ws->pass_ops[i], y);
+        if (!free || hipq_conv2d_run_pair(c->plan, in_ptr(op, 0), 0, out_ptr(op), o->plan, in_ptr(op, 0), 0, out_ptr(r), op_stream(op)) != 0)
             continue;
         o->computed_ahead = true;
         ++g_chained_convs;

@@ -286,6 +286,12 @@ def operators_run_one_by_one_launch_themselves():
             pass_of()
 
 
+def shared(data, pairs):
+    """The engine file `data` with tensors that share one memory, (from, to) by their indices."""
+    import struct
+    return data[:-4] + struct.pack("<i", len(pairs)) + b"".join(struct.pack("<ii", *p) for p in pairs)
+
+
 def two_parades_of_one_input_launch_their_own_layers():
     """Two parades of a workspace whose input is one memory, each with a convolution of it that could run with the other's: a pass computes
     the layers of its own parade, recorded or not, in whatever order the passes come."""
@@ -323,6 +329,49 @@ def two_parades_of_one_input_launch_their_own_layers():
             launches = kernels.value - before
             assert launches in (0, 1, 10, 11), (k, i, launches)  # replayed, replayed behind an upload, recorded
     assert rt.libs[1].hip_module_chained_convs() == 0
+
+
+def layers_run_together_only_where_their_memories_allow():
+    """A convolution runs with a later one of the same tensor - unless an operator between the two writes that tensor's memory, or one
+    ahead of the second has to do with the memory that it writes (tensors of an engine file may share memories)."""
+    import numpy as np
+    from nart_amd import cases, engine
+    rt = runtime()
+    ws = rt.workspace("hip")
+    for share, pairs in ((None, 1), ("written between", 0), ("read between", 0), ("read before", 0)):
+        c = cases.Case("chain", 3)
+        x0 = c.input_u8((1, 16, 14, 14), 0.05, 9)
+        x, v, t = c.conv(x0, 64, 3), c.conv(x0, 64, 1), c.conv(x0, 128, 3, stride=2)
+        if share == "read before":
+            z = c.conv(t, 128, 1)
+        a = c.conv(x, 128, 3, stride=2)
+        u = c.add(x, v) if share == "written between" else x
+        if share == "read between":
+            z = c.conv(t, 128, 1)
+        b = c.conv(u, 128, 1, stride=2)
+        if share in (None, "written between"):
+            z = c.conv(t, 128, 1)
+        y = c.add(c.add(c.conv(a, 128, 1), b), z)
+        for _ in range(6):
+            y = c.conv(y, 64, 1)
+        c.output = y
+        names = [c.input.name] + [n.attrs[k] for n in c.nodes if n.kind == "conv" for k in ("w", "b")]
+        index = {}
+        for n in c.nodes:
+            index[n.output] = len(names)
+            names.append(n.output)
+        data = engine.write_engine(c)
+        if share == "written between":
+            data = shared(data, [(index[x.name], index[u.name])])
+        elif share:
+            data = shared(data, [(index[t.name], index[b.name])])
+        p = engine.Parade(rt, data, [ws])
+        for k in range(4):
+            p.inputs()[0].write(np.zeros(x0.shape, np.uint8))
+            before = rt.libs[1].hip_module_chained_convs()
+            p.run()
+            assert rt.libs[1].hip_module_chained_convs() - before == (pairs if k else 0), (share, k)
+        p.delete()
 
 
 def a_pass_that_cannot_be_recorded_runs_its_operators():
@@ -534,6 +583,7 @@ def operators_of_two_workspaces_wait_for_each_other():
 CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
+         layers_run_together_only_where_their_memories_allow,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
