@@ -224,6 +224,7 @@ static void *hm_cpu_data(const mem_t *mm)
     finish_upload(m);
     m->host_valid = true;
     m->dev_valid = m->q_valid = false;
+    ++m->fills;
     return m->host;
 }
 
@@ -260,6 +261,7 @@ void *hip_mem_dev_out(mem_t *mm, hipStream_t st)
     grow_dev(&m->dev, &m->dev_cap, dev_bytes(m));
     m->dev_valid = true;
     m->host_valid = m->down_issued = m->q_valid = false;
+    ++m->fills;
     return m->dev;
 }
 
@@ -273,6 +275,7 @@ static void *hm_data(const mem_t *mm)
     HIPM_HIP(hipDeviceSynchronize());
     as_hip(m)->up_pending = false;
     as_hip(m)->host_valid = as_hip(m)->down_issued = as_hip(m)->q_valid = false;
+    ++as_hip(m)->fills;
     return const_cast<void *>(p);
 }
 
@@ -470,6 +473,7 @@ extern "C" __attribute__((visibility("default"))) bool hip_mem_write(mem_t *mm, 
         return false;
     hip_mem_t *m = as_hip(mm);
     m->pending = nullptr; // about to be overwritten, all of it
+    ++m->fills;
     if (m->down_issued) { // the device is still writing the mirror
         wait_stream(m->prod_stream);
         m->down_issued = false;

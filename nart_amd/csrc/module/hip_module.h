@@ -98,6 +98,7 @@ struct hip_mem_t {
     // wants it waits for that stream.  host_read: the host has asked for device-written contents since a pass was last recorded.
     bool down_issued, host_read;
     bool q_valid; // see q_op
+    unsigned fills; // counts whatever may have changed the contents
 
     size_t size;        // logical size in bytes (dense NCHW), as requested through mem_alloc
     size_t host_cap;

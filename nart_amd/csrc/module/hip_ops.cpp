@@ -154,10 +154,18 @@ struct conv_op_t {
     op_t *ir_project;                             // the chain's last convolution (in all three; else null)
     op_t *ir_expand, *ir_dw;                      // in the last one; no ir_expand: the depthwise convolution is the first
     const op_t *ir_relu1, *ir_relu2, *ir_add;     // in the last one; null: none
-    // this pass's output has already been written, by the kernel of the pooling operator whose output this convolution
-    // reads (hipq_conv2d_run_maxpool_conv) or with another convolution (conv_run_pair): run() has nothing left to do
+    // the output has already been written, by the kernel of the pooling operator whose output this convolution reads
+    // (hipq_conv2d_run_maxpool_conv) or with another convolution (conv_run_pair): run() has nothing left to do, where input and output
+    // are what they were then (hip_mem_t::fills)
     bool computed_ahead;
+    unsigned ahead_in, ahead_out;
 };
+
+void set_computed_ahead(conv_op_t *c)
+{
+    c->computed_ahead = true;
+    c->ahead_in = as_hip(c->o.input_tensors[0]->mem)->fills, c->ahead_out = as_hip(c->o.output_tensors[0].mem)->fills;
+}
 
 void conv_config(op_t *op)
 {
@@ -503,7 +511,7 @@ bool conv_run_pair(op_t *op)
             free = free && !reads(ws->pass_ops[i], y) && !writes(ws->pass_ops[i], y);
         if (!free || hipq_conv2d_run_pair(c->plan, in_ptr(op, 0), 0, out_ptr(op), o->plan, in_ptr(op, 0), 0, out_ptr(r), op_stream(op)) != 0)
             continue;
-        o->computed_ahead = true;
+        set_computed_ahead(o);
         ++g_chained_convs;
         return true;
     }
@@ -515,7 +523,8 @@ void conv_run(op_t *op)
     conv_op_t *c = reinterpret_cast<conv_op_t *>(op);
     if (c->computed_ahead) {
         c->computed_ahead = false;
-        return;
+        if (as_hip(op->input_tensors[0]->mem)->fills == c->ahead_in && as_hip(op->output_tensors[0].mem)->fills == c->ahead_out)
+            return;
     }
     decide_again_in_passes(op, &c->defer, &c->defer_in_passes);
     if (c->defer == 0)
@@ -555,6 +564,7 @@ void build_plan(op_t *op, const hipq_conv2d_desc &d, const uint8_t *w, const voi
     conv_op_t *c = reinterpret_cast<conv_op_t *>(op);
     c->defer = 0; // decided at the next run, when every operator of the pass has been prepared
     c->ir_project = nullptr;
+    c->computed_ahead = false;
     const float *wa_pc = per_channel_walpha(c);
     uint64_t pc_id = 0;
     if (wa_pc) {
@@ -1310,9 +1320,9 @@ bool pool_run_fused(op_t *op)
             void *y0 = out_ptr(&nx[0]->o), *y1 = nx[1] ? out_ptr(&nx[1]->o) : nullptr;
             if (hipq_conv2d_run_maxpool_conv(c->plan, xin, out_ptr(op), y->H, y->W, relu, nx[0]->plan, 0, y0,
                                              nx[1] ? nx[1]->plan : nullptr, 0, y1, op_stream(op)) == 0) {
-                nx[0]->computed_ahead = true;
+                set_computed_ahead(nx[0]);
                 if (nx[1])
-                    nx[1]->computed_ahead = true;
+                    set_computed_ahead(nx[1]);
                 ++g_fused_pools;
                 g_chained_convs += n;
                 return true;

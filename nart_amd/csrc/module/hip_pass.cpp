@@ -271,6 +271,7 @@ bool hip_pass_run(void **state, op_t *const *ops, size_t n)
     for (const PassOutput &o : p.out) {
         o.m->dev_valid = o.dev_valid, o.m->host_valid = o.host_valid, o.m->down_issued = o.down_issued, o.m->q_valid = false;
         o.m->pending = o.pending, o.m->pending_ctx = o.pending_ctx;
+        ++o.m->fills;
     }
     return true;
 }

@@ -374,6 +374,36 @@ def layers_run_together_only_where_their_memories_allow():
         p.delete()
 
 
+def layers_computed_ahead_follow_their_tensors():
+    """The kernel of a stem and its pooling computes the convolution that reads the pooled tensor as well, whose run() then has nothing to
+    do - unless the pooled tensor, its own output or its scales have changed since."""
+    import numpy as np
+    rt = runtime()
+    ws = rt.workspace("hip")
+    x = ws.tensor(np.zeros((2, 3, 64, 96), np.uint8))
+    conv = ws.conv2d(x, ws.tensor(np.full((64, 3, 7, 7), 130, np.uint8)), None, 3, 2, 1,
+                     dict(ialpha=0.031, izp=77, walpha=0.0042, wzp=128, oalpha=0.09, ozp=0)).prepare()
+    pool = ws.pool(conv.output(0), 3, 1, 2, 0, False, dict(ialpha=0.09, izp=0, oalpha=0.09, ozp=0)).prepare()
+    q = dict(ialpha=0.09, izp=0, walpha=0.004, wzp=128, oalpha=0.07, ozp=0)
+    layer = ws.conv2d(pool.output(0), ws.tensor(np.full((64, 64, 1, 1), 130, np.uint8)), None, 0, 1, 1, q).prepare()
+
+    def ahead():
+        before = rt.libs[1].hip_module_chained_convs()
+        conv.run()
+        pool.run()
+        return rt.libs[1].hip_module_chained_convs() - before
+    for change, kernels in ((None, 0), ("input", 2), ("output", 1), ("scales", 1), (None, 0)):
+        assert ahead() == 1
+        if change == "input":
+            pool.output(0).write(np.ones((2, 64, 16, 24), np.uint8))  # one kernel brings it in
+        elif change == "output":
+            layer.output(0).write(np.ones((2, 64, 16, 24), np.uint8))
+        elif change == "scales":
+            layer.set_quant(**dict(q, oalpha=0.08)).config().prepare()
+        assert launched(layer) == kernels, change
+        assert launched(layer) == 1, change
+
+
 def a_pass_that_cannot_be_recorded_runs_its_operators():
     """On the null stream, which cannot be captured, and where the runtime refuses the graph: every pass runs operator by
     operator, and no error stays behind for the next launch to find."""
@@ -583,7 +613,7 @@ def operators_of_two_workspaces_wait_for_each_other():
 CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
-         layers_run_together_only_where_their_memories_allow,
+         layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
          a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
