@@ -369,7 +369,7 @@ const char *hipq_depthwise_point_kernel(const hipq_conv2d_plan *depthwise, const
  * op_quant_add_run (src/op/add.c:83-148), then op_conv_2d_u8xu8_run again; t never travels to memory and y is written
  * but not read back.  `mid`: 3x3 / stride 1 / pad 1, CM -> CM with CM = 64, 128 or 256; `widen`: 1x1, CM -> 4 CM;
  * `next`: 1x1 / stride 1, 4 CM -> CM (the first layer of the next block); images that hold an 8 x 8, a 4 x 14 or a 7 x 7 pixel
- * patch (where the patches that are used do not divide the image some overlap: y must not be the residual then); uint8 tensors
+ * patch (where none of them divides the image some overlap: y must not be the residual then); uint8 tensors
  * with dense channel strides, weight zero points 128, per-tensor weight scales, each layer reading its input with the scale and zero point it is written
  * with.  The residual (any tensor of y's shape, e.g. a projection shortcut) and the add are described as in
  * hipq_conv2d_run_add; next_relu as in hipq_conv2d_run_add_conv.  hipq_bottleneck_tail_fusable answers (1 / 0);

@@ -506,14 +506,19 @@ __global__ __launch_bounds__(128 * G, (G == 1 ? (NX ? 4 : 3) : G == 2 ? (NX && S
     }
 }
 
-// The patch shape of the tail kernel for an H x W image: the one that covers it with the fewest patches, so that the ones an image is
-// a multiple of come first (8x8 fills every pixel slot, 4x14 seven in eight, 7x7 three in four).  Where a side is no multiple, the last
-// patch ends where the image does and computes the pixels that it shares with its neighbour again: the same bytes, written twice.
+// The patch shape of the tail kernel for an H x W image: the first of 8x8, 4x14 and 7x7 that divides it (8x8 fills every pixel slot, 4x14
+// seven in eight, 7x7 three in four), also where another needs as many patches or fewer (14x14, 42x42): the sum may then overwrite the
+// residual.  Where none does, the one that covers the image with the fewest patches: the last ones end where the image does and compute
+// the pixels that they share with their neighbours again, the same bytes, written twice.
 static bool tail_patch(int H, int W, int *ph, int *pw)
 {
     static const int shapes[][2] = {{8, 8}, {4, 14}, {7, 7}};
     int best = 0;
     for (const auto &s : shapes) {
+        if (H % s[0] == 0 && W % s[1] == 0) {
+            *ph = s[0], *pw = s[1];
+            return true;
+        }
         if (H < s[0] || W < s[1])
             continue;
         const int n = ((H + s[0] - 1) / s[0]) * ((W + s[1] - 1) / s[1]);

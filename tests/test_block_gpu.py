@@ -759,11 +759,15 @@ def test_overlapping_patches_do_not_overwrite_their_residual():
     """A patch reads its residual before it writes the sum, its neighbour's shared pixels perhaps after: y must be another tensor there
     (and may be the residual where patches are disjoint)."""
     rng = np.random.default_rng(11)
-    for H, W, ok in ((16, 16, True), (16, 17, False)):
-        t1, res, layers, rq, sq, nx = make_tail(rng, 1, 256, H, W, False)
+    for CW, H, W, ok in ((256, 16, 16, True), (256, 16, 17, False), (512, 14, 14, True), (512, 21, 21, True), (256, 14, 21, True),
+                         (512, 7, 14, True), (1024, 14, 14, True), (256, 42, 42, True), (512, 13, 13, False)):
+        t1, res, layers, rq, sq, nx = make_tail(rng, 1, CW, H, W, False)
         plans = plans_of(t1, layers)
         xd, rd, want = hipq.to_device_nhwc(t1), hipq.to_device_nhwc(res), torch.zeros_like(hipq.to_device_nhwc(res))
         hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], want)
+        t = orc.conv2d_u8(t1, layers[0]["w"], layers[0]["b"], 1, 1, 1, *layers[0]["q"])
+        c = orc.conv2d_u8(t, layers[1]["w"], layers[1]["b"], 0, 1, 1, *layers[1]["q"])
+        assert np.array_equal(hipq.from_device_nhwc(want, CW), orc.add_u8(c, res, *layers[1]["q"][4:6], *rq, *sq)), (CW, H, W)
         if ok:
             hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], rd)
             torch.cuda.synchronize()
@@ -773,7 +777,8 @@ def test_overlapping_patches_do_not_overwrite_their_residual():
                 hipq.bottleneck_tail_run(plans[0], plans[1], xd, rd, False, rq[0], rq[1], sq[0], sq[1], rd)
 
 
-@pytest.mark.parametrize("n, hw, block, tail", [(11, 13, False, True), (64, 13, True, True), (64, 10, False, True), (1, 20, False, False), (2, 20, False, True)])
+@pytest.mark.parametrize("n, hw, block, tail", [(11, 13, False, True), (64, 13, True, True), (64, 10, False, True), (1, 20, False, False), (2, 20, False, True),
+                                                (1, 14, True, True), (1, 21, True, True)])
 def test_rules_on_ragged_images(n, hw, block, tail):
     """Where the one-launch forms are chosen on images that their patches do not divide: whole blocks by the two fitted costs, tails of 128
     channels with a wider next layer from 600 pixels on."""

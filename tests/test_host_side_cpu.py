@@ -112,6 +112,32 @@ def a_plan_launches_the_kernel_that_it_names():
     assert len(seen) == len(names), seen
 
 
+def block_tails_keep_to_patches_that_divide_an_image():
+    """hipq_bottleneck_tail_run may write the sum over the residual wherever some patch shape divides the image, also where another would
+    need as many overlapping patches or fewer, and takes 128 channels by rule on such images however few their pixels; where none
+    divides it, patches overlap: another tensor, and 600 pixels."""
+    import numpy as np
+    from nart_amd import hipq
+    x, y, z = 4096, 8192, 12288  # never touched
+    grids = {"conv_bottleneck_tail_kernelILi2ELi%dELi%dE" % (h, w): (h, w) for h, w in ((8, 8), (4, 14), (7, 7))}
+    last = C.c_char_p.in_dll(STUB, "stub_last_kernel")
+    for H, W, patch, divides in ((14, 14, (7, 7), True), (21, 21, (7, 7), True), (35, 35, (7, 7), True), (49, 49, (7, 7), True), (14, 21, (7, 7), True),
+                                 (14, 28, (7, 7), True), (7, 14, (7, 7), True), (42, 42, (7, 7), True), (63, 63, (7, 7), True), (28, 28, (4, 14), True),
+                                 (56, 56, (8, 8), True), (8, 14, (4, 14), True), (16, 17, (8, 8), False), (13, 13, (8, 8), False), (9, 29, (8, 8), False),
+                                 (25, 25, (4, 14), False), (7, 9, (7, 7), False)):
+        mid = hipq.Conv2d((1, 128, H, W), np.full((128, 128, 3, 3), 129, np.uint8), None, 1, 1, 1, 0.05, 9, 0.002, 128, 0.05, 9)
+        widen = hipq.Conv2d((1, 128, H, W), np.full((512, 128, 1, 1), 129, np.uint8), None, 0, 1, 1, 0.05, 9, 0.002, 128, 0.05, 9)
+        rule = hipq.bottleneck_tail_fusable(mid, widen, False, 0.04, 3, 0.09, 10)
+        assert rule == (divides or H * W >= 600), (H, W, rule)
+        mid.special(2)
+
+        def run(to):
+            return hipq.lib().hipq_bottleneck_tail_run(mid.handle, widen.handle, x, y, 0, 0.04, 3, 0.09, 10, 8, to, None, 0, None, None)
+        hipq.check(run(z))
+        assert [p for k, p in grids.items() if k in last.value.decode()] == [patch], (H, W, last.value)
+        assert (run(y) == 0) == divides, (H, W)
+
+
 def runtime():
     from nart_amd import art
     lib = os.path.join(ROOT, "nart_amd", "lib")
@@ -610,7 +636,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
