@@ -172,9 +172,10 @@ __device__ static inline uint32_t max_u8x4(uint32_t a, uint32_t b)
 bool make_add_params(float ia0, int iz0, float ia1, int iz1, float oa, int oz, int obits, AddParams *p);
 
 // Exact form of an add that has the fast one: the two terms of that lose up to 1.5 units of 2^-sh to their own shifts, which shows in the
-// result only where their exact sum lies that little above a multiple of 2^sh - for 98 of 100 pairs of scales in none of the 65 536
-// pairs of bytes.  Then x0*m0 + x1*m1 + k in 64 bits, its high word shifted by sh, is the result before the clamp: *p's m0, m1 and
-// sh become those, c0 and c1 the low and the high word of k.  False: there is no such form, *p is as it was.
+// result only where their exact sum lies that little above a multiple of 2^sh - where the sum's scale is larger than both operands', for
+// 98 of 100 pairs of scales in none of the 65 536 pairs of bytes; otherwise there is no such form.  Then the high word of x0*m0 + x1*m1 + k
+// in 64 bits is the result before the clamp: *p's m0 and m1 become those, sh 0, c0 and c1 the low and the high word of k.  False: *p is as
+// it was.
 bool make_add_exact(AddParams *p);
 
 } // namespace hipq

@@ -50,16 +50,15 @@ extern "C" void hipq_quant_scale(float x, int bits, uint32_t *mult, int *shift)
     *shift = s + bits - 1;
 }
 
-// The exact form's constants: with u = max(s0, s1) the sum of the terms is (x0 m0 2^(u-s0) + x1 m1 2^(u-s1) + const) / 2^u, scaled by a 2^k
-// that puts as much of the result as fits 32-bit multipliers into the high word.  For each x0 the x1 whose sum lies less than the lost
-// fractions, at most 3 * 2^(u-1), above a multiple of 2^(sh+u) are found in the sorted residues of the second term.
+// The exact form's constants: with u = max(s0, s1) the sum of the terms is (x0 m0 2^(u-s0) + x1 m1 2^(u-s1) + const) / 2^u, scaled so that its
+// high word is the result, which 32 bits hold the multipliers of where both ratios of scales are below one.  For each x0 the x1 whose
+// sum lies less than the lost fractions, at most 3 * 2^(u-1), above a multiple of 2^(sh+u) are found in the sorted residues of the second
+// term.
 static bool exact_form(hipq::AddParams *p)
 {
     const int u = std::max(p->s0, p->s1), d0 = u - p->s0, d1 = u - p->s1;
-    int k = 32 - u - p->sh;
-    while (k >= 0 && (((uint64_t)p->m0 << (d0 + k)) >> 32 || ((uint64_t)p->m1 << (d1 + k)) >> 32))
-        k--;
-    if (k < 0 || u + p->sh + k - 32 < 0 || u + p->sh > 40)
+    const int k = 32 - u - p->sh;
+    if (k < 0 || (uint64_t)p->m0 << (d0 + k) >> 32 || (uint64_t)p->m1 << (d1 + k) >> 32)
         return false;
     const int64_t mod = (int64_t)1 << (u + p->sh), rest = ((int64_t)p->cadd) << u;
     struct Term {
@@ -85,7 +84,7 @@ static bool exact_form(hipq::AddParams *p)
         }
     }
     const uint64_t at_zero = (((uint64_t)(int64_t)p->c0 << d0) + ((uint64_t)(int64_t)p->c1 << d1) + (uint64_t)rest) << k;
-    p->m0 <<= d0 + k, p->m1 <<= d1 + k, p->sh += u + k - 32;
+    p->m0 <<= d0 + k, p->m1 <<= d1 + k, p->sh = 0;
     p->c0 = (int32_t)(uint32_t)at_zero, p->c1 = (int32_t)(uint32_t)(at_zero >> 32);
     return true;
 }

@@ -163,6 +163,37 @@ def add_forms(pairs, took=None):
     return out
 
 
+def exact_adds_are_the_operator():
+    """The exact form of an add, wherever there is one, against the oracle's add over all 65 536 pairs of bytes: scales from an eighth of the
+    sum's to eight times it, any zero points.  Of the adds with a 32-bit form nearly all have one where both operands' scales are below
+    the sum's, otherwise none."""
+    import random
+    import numpy as np
+    from oracle import orc
+    rng = random.Random(11)
+    x0, x1 = (v.astype(np.uint8).reshape(1, 1, 256, 256) for v in np.indices((256, 256)))
+    a, b = x0.astype(np.uint64), x1.astype(np.uint64)
+    count = {True: [0, 0], False: [0, 0]}
+    for k in range(400):
+        r0, r1 = (2.0 ** rng.uniform(-3, 0 if k % 4 else 3) for _ in range(2))
+        if k % 8 == 1:
+            r1 = r0
+        alpha = float(np.float32(rng.uniform(0.01, 0.2)))
+        q = (float(np.float32(alpha * r0)), rng.choice((0, 255, rng.randrange(256))), float(np.float32(alpha * r1)), rng.choice((0, 255, rng.randrange(256))),
+             alpha, rng.choice((0, 255, rng.randrange(256))))
+        (plain, form), = add_forms([q])
+        kind = count[bool(np.float32(q[0]) / np.float32(alpha) < 1 and np.float32(q[2]) / np.float32(alpha) < 1)]
+        kind[0] += plain.fast
+        if form is None:
+            continue
+        kind[1] += 1
+        assert form.sh == 0
+        t = a * np.uint64(form.m0) + b * np.uint64(form.m1) + np.uint64((form.c1 & 0xffffffff) << 32 | (form.c0 & 0xffffffff))
+        got = np.clip((t >> np.uint64(32)).astype(np.uint32).view(np.int32), 0, 255)
+        assert np.array_equal(got, orc.add_u8(x0, x1, *q)), (q, int((got != orc.add_u8(x0, x1, *q)).sum()))
+    assert count[True][1] > 0.95 * count[True][0] and count[True][0] > 250 and count[False][0] > 50 and count[False][1] == 0, count
+
+
 def exact_adds_are_searched_for_once():
     """A launch asks for the exact form of its add each time: the forms of a network's adds are all remembered."""
     import random
@@ -681,7 +712,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
