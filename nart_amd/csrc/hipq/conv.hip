@@ -1318,6 +1318,7 @@ struct hipq_conv2d_plan {
     // tiles cannot take
     ResidentShape resident[2] = {}, narrow[2] = {};
     bool resident_named = false;           // by the caller (hipq_conv2d_plan_resident)
+    ResidentPairCosts pair_costs = {};     // of the same kernel with another layer in its launch
     StreamShape stream = {0, 0, 0}; // explicit shape of the streaming kernel (hipq_conv2d_plan_stream); mb = 0: built-in rule
     bool has_wzp;
     void *d_w = nullptr, *d_bias = nullptr, *d_q = nullptr;
@@ -1874,6 +1875,8 @@ static int plan_create(const hipq_conv2d_desc *dp, const uint8_t *w, const int32
         else
             p->name += "_perchannel";
     }
+    if (p->variant == kMfma)
+        conv_resident_pair_costs(a, &p->pair_costs);
     *plan_out = p;
     return 0;
 }
@@ -2571,19 +2574,18 @@ extern "C" int hipq_conv2d_run_add2(const hipq_conv2d_plan *p, const void *x, co
 
 // Two layers that do not depend on each other - a block's first layer and its projection shortcut - in one launch of
 // conv_resident_kernel's tiles
-static bool pair_shapes(const hipq_conv2d_plan *p, const hipq_conv2d_plan *q, ResidentShape *sp, ResidentShape *sq, double *us)
+static bool pair_shapes(const hipq_conv2d_plan *p, const hipq_conv2d_plan *q, ResidentShape *sp, ResidentShape *sq)
 {
     for (const hipq_conv2d_plan *l : {p, q})
         if (!l || l->variant != kMfma || !l->special || l->tile_selected || l->stream.mb || l->resident_named || l->has_wzp)
             return false;
-    return conv_resident_choose_pair(p->args, q->args, sp, sq, us);
+    return conv_resident_choose_pair(p->pair_costs, q->pair_costs, sp, sq);
 }
 
 extern "C" int hipq_conv2d_pair_fusable(const hipq_conv2d_plan *p, const hipq_conv2d_plan *q)
 {
     ResidentShape sp, sq;
-    double us;
-    if (!pair_shapes(p, q, &sp, &sq, &us))
+    if (!pair_shapes(p, q, &sp, &sq))
         return 0;
     if (p->special == 2)
         return 1;
@@ -2607,8 +2609,7 @@ extern "C" int hipq_conv2d_run_pair(const hipq_conv2d_plan *p, const void *x, in
     HIPQ_REQUIRE(!(relu && p->d.dtype != HIPQ_DTYPE_U8) && !(relu_q && q->d.dtype != HIPQ_DTYPE_U8),
                  "hipq_conv2d_run_pair: relu for uint8 plans only (op_quant_relu_run is a uint8 operator)");
     ResidentShape sp, sq;
-    double us;
-    HIPQ_REQUIRE(pair_shapes(p, q, &sp, &sq, &us), "hipq_conv2d_run_pair: these two plans (%s, %s) do not run in one launch: run hipq_conv2d_run "
+    HIPQ_REQUIRE(pair_shapes(p, q, &sp, &sq), "hipq_conv2d_run_pair: these two plans (%s, %s) do not run in one launch: run hipq_conv2d_run "
                  "twice", p->name.c_str(), q->name.c_str());
     ConvArgs a = p->args, b = q->args;
     a.x = static_cast<const uint8_t *>(x), a.y = static_cast<uint8_t *>(y);

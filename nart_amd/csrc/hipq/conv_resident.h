@@ -20,8 +20,14 @@ bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us);
 // the same among the shapes with 32 x 32 tiles, which not every launch of a plan can take: conv_resident_wide_applies
 bool conv_resident_wide_applies(const ConvArgs &a);
 bool conv_resident_choose_wide(const ConvArgs &a, ResidentShape *shape, double *us);
-// two layers that do not depend on each other in one launch: shapes for both; false: they do not run that way
-bool conv_resident_choose_pair(const ConvArgs &a, const ConvArgs &b, ResidentShape *sa, ResidentShape *sb, double *us);
+// two layers that do not depend on each other in one launch.  conv_resident_pair_costs: what each shape takes for a layer (a plan keeps
+// it: computing it takes longer than the rest of a launch); conv_resident_choose_pair: shapes for both; false: they do not run that way
+constexpr int kResidentShapes = 26;
+struct ResidentPairCosts {
+    double us[kResidentShapes]; // 0: not in this shape
+};
+void conv_resident_pair_costs(const ConvArgs &a, ResidentPairCosts *costs);
+bool conv_resident_choose_pair(const ResidentPairCosts &a, const ResidentPairCosts &b, ResidentShape *sa, ResidentShape *sb);
 void launch_conv_resident_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, const ResidentShape &t, hipStream_t st);
 void launch_conv_resident(const ConvArgs &a, const ResidentShape &s, hipStream_t st);
 

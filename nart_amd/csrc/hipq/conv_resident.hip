@@ -763,7 +763,7 @@ void launch_tile(const ConvArgs &a, const ResidentShape &s, hipStream_t st)
 namespace {
 
 // the shapes that are built (tiles of a wave: pixels by channels; waves: channel groups by shares of the reduction)
-constexpr ResidentShape kShapes[] = {{1, 1, 1, 8}, {1, 1, 1, 4}, {2, 1, 1, 8}, {2, 1, 1, 4}, {2, 2, 1, 8}, {2, 2, 1, 4}, {2, 2, 2, 4}, {2, 2, 2, 2}, {4, 1, 1, 8},
+constexpr ResidentShape kShapes[kResidentShapes] = {{1, 1, 1, 8}, {1, 1, 1, 4}, {2, 1, 1, 8}, {2, 1, 1, 4}, {2, 2, 1, 8}, {2, 2, 1, 4}, {2, 2, 2, 4}, {2, 2, 2, 2}, {4, 1, 1, 8},
                                      {4, 2, 1, 8}, {4, 2, 1, 4}, {4, 4, 1, 4}, {4, 4, 2, 4}, {4, 4, 2, 2}, {8, 2, 1, 2}, {1, 1, 2, 1}, {1, 1, 4, 1}, {2, 1, 4, 1},
                                      {2, 2, 2, 1}, {2, 2, 4, 1}, {4, 1, 4, 1}, {4, 2, 4, 1}, {4, 4, 2, 1}, {4, 4, 4, 1}, {8, 2, 2, 1}, {8, 2, 4, 1}};
 
@@ -933,23 +933,30 @@ void launch_pair(const ConvArgs &a, const ResidentShape &s, const ConvArgs &b, c
 
 } // namespace
 
-bool conv_resident_choose_pair(const ConvArgs &a, const ConvArgs &b, ResidentShape *sa, ResidentShape *sb, double *us)
+void conv_resident_pair_costs(const ConvArgs &a, ResidentPairCosts *costs)
 {
-    if (!pair_applies(a) || !pair_applies(b))
-        return false;
+    const bool applies = pair_applies(a);
+    for (int i = 0; i < kResidentShapes; i++) {
+        const ResidentShape &s = kShapes[i];
+        double t;
+        const bool padding = s.mb > 1 && 8 * s.mb >= (a.P + 15) / 16 * 16; // half of the rows
+        costs->us[i] = applies && s.mb * s.nb <= 8 && !padding && conv_resident_cost(a, s, &t) ? t : 0;
+    }
+}
+
+bool conv_resident_choose_pair(const ResidentPairCosts &a, const ResidentPairCosts &b, ResidentShape *sa, ResidentShape *sb)
+{
     double best = 1e30;
-    for (const ResidentShape &s : kShapes)
-        for (const ResidentShape &t : kShapes) {
-            double ta, tb;
-            if (s.mb != t.mb || s.nb != t.nb || s.nwc * s.ks != t.nwc * t.ks || s.mb * s.nb > 8 || !conv_resident_cost(a, s, &ta) || !conv_resident_cost(b, t, &tb)
-                || (s.mb > 1 && (8 * s.mb >= (a.P + 15) / 16 * 16 || 8 * s.mb >= (b.P + 15) / 16 * 16)))
+    for (int i = 0; i < kResidentShapes; i++)
+        for (int j = 0; a.us[i] > 0 && j < kResidentShapes; j++) {
+            const ResidentShape &s = kShapes[i], &t = kShapes[j];
+            if (!(b.us[j] > 0) || s.mb != t.mb || s.nb != t.nb || s.nwc * s.ks != t.nwc * t.ks)
                 continue;
             // the larger one's time, and half of what the smaller one takes beside its launch: its tiles share CUs
-            const double c = std::max(ta, tb) + 0.5 * (std::min(ta, tb) - 2.2);
+            const double c = std::max(a.us[i], b.us[j]) + 0.5 * (std::min(a.us[i], b.us[j]) - 2.2);
             if (c < best)
                 best = c, *sa = s, *sb = t;
         }
-    *us = best;
     return best < 1e30;
 }
 

@@ -138,6 +138,27 @@ def block_tails_keep_to_patches_that_divide_an_image():
         assert (run(y) == 0) == divides, (H, W)
 
 
+def a_pair_of_layers_is_launched_as_quickly_as_two():
+    """hipq_conv2d_run_pair and its predicate choose among what the plans keep: the call takes the host little more than two launches."""
+    import time
+    import numpy as np
+    from nart_amd import hipq
+    lib = hipq.lib()
+    a, b = (hipq.Conv2d((1, 128, 28, 28), np.full((256, 128, r, r), 129, np.uint8), None, r // 2, 2, 1, 0.05, 9, 0.002, 128, 0.05, 9) for r in (3, 1))
+
+    def best(f):
+        times = []
+        for _ in range(40):
+            t = time.perf_counter()
+            for _ in range(50):
+                f()
+            times.append(time.perf_counter() - t)
+        return min(times)
+    two = best(lambda: (lib.hipq_conv2d_run(a.handle, 4096, 8192, None, None), lib.hipq_conv2d_run(b.handle, 4096, 12288, None, None)))
+    pair = best(lambda: lib.hipq_conv2d_run_pair(a.handle, 4096, 0, 8192, b.handle, 4096, 0, 12288, None))
+    assert lib.hipq_conv2d_pair_fusable(a.handle, b.handle) and pair < 2.2 * two, (pair, two)
+
+
 def add_forms(pairs, took=None):
     """make_add_params and make_add_exact (csrc/hipq/common.h) for (alpha 0, zero point 0, alpha 1, zero point 1, alpha, zero point) of an
     add: its constants, and those of its exact form or None; took: called with the seconds that the latter took."""
@@ -712,7 +733,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
