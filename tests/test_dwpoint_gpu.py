@@ -12,9 +12,11 @@ from oracle import orc  # noqa: E402  (checker only)
 from nart_amd import hipq  # noqa: E402
 
 # channels, output channels, (N, H, W), stride: one slice and one tile; a half slice and partial tiles; more slices than waves; images
-# that a patch just fills, that it overhangs on two sides, and smaller than one; work-groups with idle waves (5 images)
+# that a patch just fills, that it overhangs on two sides, and smaller than one; work-groups with idle waves (5 images); six, seven and as
+# many waves as slices in a work-group
 CASES = [(32, 16, (5, 8, 8), 1), (32, 16, (5, 15, 16), 2), (80, 72, (3, 13, 11), 1), (80, 72, (3, 13, 11), 2), (560, 160, (2, 7, 7), 1),
-         (576, 320, (1, 7, 7), 1), (560, 160, (2, 14, 14), 2), (20, 20, (1, 3, 2), 1), (24, 200, (1, 3, 2), 2)]
+         (576, 320, (1, 7, 7), 1), (560, 160, (2, 14, 14), 2), (20, 20, (1, 3, 2), 1), (24, 200, (1, 3, 2), 2),
+         (192, 40, (2, 9, 10), 2), (224, 40, (1, 6, 9), 1), (512, 48, (1, 9, 9), 2)]
 SHAPES = ["4x8_n1", "4x8_n2", "4x8_n3", "4x8_n5", "8x8_n1", "8x8_n2", "8x8_n3", "narrow4x8_n1", "narrow4x8_n2", "narrow8x8_n1", "narrow8x8_n2"]
 
 
