@@ -444,16 +444,16 @@ void launch_shape(const ConvArgs &d, const ConvArgs &p, const PairShape &s, hipS
         hipLaunchKernelGGL((conv_dwpoint_narrow_kernel<S, PH, CT, false>), grid, block, v.lds, st, d, p, v.geo);
 }
 
-// Time by shape, in us, fitted to 420 pairs of layers (1 to 128 images of 3x3 to 128x128, 16 to 1024 channels to 12 to 400; nine in
-// ten within 18 % of the fit; the shape it picks takes 1.3 % more than the best one on average), narrow ones to 900.  Shared patches: a launch; per generation of resident work-groups its start, the waves' sums that meet in
-// LDS, and the tiles that a wave finishes; per slice that a wave takes its chain, alone and per wave on its SIMD; the slices per SIMD of the
-// chip.  Narrow ones: a launch; per patch that a wave takes its chain, alone and per wave on its SIMD; the patches, and their channel
-// tiles, per SIMD of the chip; generations.
+// Time by shape, in us, fitted to 3600 pairs of layers (1 to 128 images of 3x3 to 128x128, 16 to 1024 channels to 12 to 400; nine in
+// ten within 15 % of the fit; the shape it picks takes 0.8 % more than the best one on average), narrow ones to 900.  Shared patches: a
+// launch; per generation of resident work-groups its start; the slices per SIMD of the chip; per generation the output tiles that a wave finishes and
+// the multiplies of its slices; per CU the sums that meet in LDS, and the slices.  Narrow ones: a launch; per patch that a wave takes its
+// chain, alone and per wave on its SIMD; the patches, and their channel tiles, per SIMD of the chip; generations.
 double shape_cost(const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    static const double kShared[3][7] = {{2.473, 0.319, 0.738, 0.198, 0.805, 0.105, 0.304}, // 4x8, stride 1
-                                         {2.207, 1.202, 0.522, 0.501, 0.606, 0.143, 0.300}, // 8x8
-                                         {2.232, 0.727, 0.888, 0.240, 0.762, 0.207, 0.285}}; // 4x8, stride 2
+    static const double kShared[3][7] = {{2.932, 0.471, 0.142, 0.235, 0.117, 0.636, 0.280}, // 4x8, stride 1
+                                         {2.321, 1.496, 0.190, 0.256, 0.086, 0.429, 0.551}, // 8x8
+                                         {2.086, 1.572, 0.252, 0.219, 0.133, 0.468, 0.374}}; // 4x8, stride 2
     static const double kNarrow[3][6] = {{2.370, 0, 0.132, 0, 0.435, 0.557}, {2.379, 0.569, 0, 0, 0.794, 0.660}, {3.016, 0, 0.103, 0, 0.695, 0.155}};
     const PairShape &s = kShapes[shape];
     if ((d.stride_h == 2 && s.ph == 8) || (s.narrow && d.in_cs > 32))
@@ -464,8 +464,9 @@ double shape_cost(const ConvArgs &d, const ConvArgs &p, int shape)
     // work-groups that a CU holds
     const int held = s.narrow ? v.held : std::max(1, std::min((int)(160 * 1024 / v.lds), max_waves(pt, s.ct) / v.nw));
     const double gens = std::ceil(groups / (256 * held)), act = std::min((double)held, std::ceil(groups / 256)), steps = gens * v.rounds;
-    const double shared[7] = {1, gens, steps, steps * act * v.nw / 4, gens * act * v.nw * tiles * pt / 16, work * v.geo.nT,
-                              gens * ((s.ct * pt + v.nw - 1) / v.nw)};
+    const double cu = std::ceil(groups / 256);
+    const double shared[7] = {1, gens, work * v.geo.nT, gens * ((s.ct * pt + v.nw - 1) / v.nw), gens * v.rounds * s.ct * pt, cu * tiles * pt * v.nw / 16,
+                              cu * v.geo.nT / 4};
     const double narrow[6] = {1, steps, steps * act, work, work * tiles, gens};
     double t = 0;
     for (int i = 0; i < (s.narrow ? 6 : 7); i++)
@@ -529,14 +530,16 @@ double conv_dwpoint_us(const ConvArgs &d, const ConvArgs &p)
     return us;
 }
 
-// The two launches: their latencies, the bytes of the tensor between them, the products of the second and its output, its weights, less 0.07 (a tie stays apart); fitted to
-// the same pairs (nine in ten within 12 %).  Of the 420 this fuses 320, which take 0.75 of the two launches on average, 14 of them longer
-// (10.7 -> 13.2 us at most); of the other 100 it would have been faster for 14, by a tenth at most.
+// The two launches: their latencies, the bytes of the first one's input and of the tensor between them, the products of the second, its
+// output and its weights; fitted to the same pairs (nine in ten within 12 %), less 2 %: a tie stays apart.  Of the 3600 this fuses
+// 2680, which take 0.74 of the two launches on average, 45 of them more than 3 % longer (12.8 -> 16.6 us at most); it takes 0.8 % more
+// than the better of the two would each time.
 double conv_dwpoint_apart_us(const ConvArgs &d, const ConvArgs &p)
 {
-    const double mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6, in = d.in_cs * 1e-3, weights = (double)d.in_cs * p.out_cs * 1e-6;
-    return d.stride_h == 1 ? 6.10 + 0.580 * mid + 0.00154 * mid * p.out_cs + 0.216 * out + 0.254 * in + 2.171 * weights
-                           : 6.43 + 1.056 * mid + 0.00187 * mid * p.out_cs + 0.055 * out + 0.729 * weights;
+    const double in = (double)d.N * d.H * d.W * d.in_cs * 1e-6, mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6;
+    const double channels = d.in_cs * 1e-3, weights = (double)d.in_cs * p.out_cs * 1e-6;
+    return 0.98 * (d.stride_h == 1 ? 6.212 + 0.608 * mid + 0.00134 * mid * p.out_cs + 0.246 * out + 0.146 * channels + 2.299 * weights
+                                   : 6.527 + 0.088 * in + 0.611 * mid + 0.00210 * mid * p.out_cs + 0.249 * out + 1.328 * weights);
 }
 
 const char *conv_dwpoint_name(const ConvArgs &d, const ConvArgs &p, int wanted)

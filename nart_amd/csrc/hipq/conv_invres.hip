@@ -575,18 +575,20 @@ void launch_shape(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
 
 // ---- the shapes, and what each takes
 
-// Time by shape, in us, fitted to 626 blocks (1 to 128 images of 3x3 to 128x128, 16 to 160 channels widened 1 to 6 times; nine in ten
-// within 20 % of the fit).  A launch; for every generation of resident work-groups its start and end; for every
-// slice that a wave then takes its chain, alone and per k-step; the k-steps of the last layer that a wave takes, or a slice's channel tiles
-// where each wave has a patch; and per SIMD of the chip the slices and the patches, which share the vector units.  Chosen by this the
-// blocks take 0.6 % more than the best shape would on average, one in twenty more than 5 %.
+// Time by shape, in us, fitted to 2400 blocks (1 to 128 images of 3x3 to 128x128, 16 to 160 channels widened 1 to 6 times; nine in ten
+// within 15 % of the fit).  A launch; for every generation of resident work-groups its start and end, and the k-steps of the last layer
+// that a wave takes, or a slice's channel tiles where each wave has a patch; per SIMD of the chip the slices, and their output channel tiles;
+// per SIMD of a CU the slices, and their k-steps; the input's MB.  Chosen by this the blocks take 0.5 % more than the best shape would on
+// average, one in twenty more than 5 %.
 double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int shape)
 {
-    // launch, slice, k-steps of the last layer, slice x k-steps, slices per SIMD, generation, patches per SIMD
-    static const double kCost[2][kShapes][7] = {
-        {{3.871, 0, 0.105, 0.136, 0.567, 0.251, 0}, {3.926, 0.224, 0.165, 0.313, 0.722, 0, 0}, {4.572, 0.823, 0.229, 0.189, 1.044, 0, 0.084},
-         {4.108, 1.191, 0, 0.278, 0.418, 0, 0.956}, {3.607, 0.525, 0.070, 0.172, 0.303, 0, 0.607}, {4.523, 0.535, 0.214, 0.205, 0.965, 0.022, 0}},
-        {{3.673, 0.126, 0.117, 0.255, 0.559, 0, 0}, {3.956, 0.395, 0.209, 0.488, 0.827, 0, 0}, {}, {1.583, 1.003, 0.154, 0.139, 0.477, 2.009, 0.251}, {}, {}}};
+    // launch, generation, k-steps of the last layer, slices per SIMD, x channel tiles, slices of a CU's SIMD, x k-steps, MB
+    static const double kCost[2][kShapes][8] = {
+        {{3.871, 0.308, 0.029, 0.014, 0.084, 0.204, 0.059, 0.058}, {3.880, 0.462, 0.045, 0.111, 0.085, 0.446, 0.082, 0.142},
+         {4.348, 0.870, 0.000, 0.000, 0.335, 0.695, 0.165, 0.147}, {3.345, 0.960, 0.289, 0.000, 0.164, 0.839, 0.000, 0.189},
+         {3.049, 0.595, 0.219, 0.000, 0.052, 0.470, 0.000, 0.295}, {4.469, 0.556, 0.000, 0.027, 0.266, 0.667, 0.161, 0.054}},
+        {{4.046, 0.309, 0.028, 0.025, 0.060, 0.201, 0.096, 0.177}, {4.210, 0.527, 0.052, 0.015, 0.133, 0.535, 0.173, 0.238},
+         {}, {3.089, 0.703, 0.321, 0.000, 0.083, 0.833, 0.000, 0.169}, {}, {}}};
     const int s = d.stride_h;
     const Channels c = channels_of(e, p);
     if ((own(shape) && (c.nk > 2 || c.ct > 2)) || (shape == kOwn4 && s == 2) || ((shape == k8x8 || shape == k7x7) && (s == 2 || c.ct > 3)))
@@ -596,11 +598,11 @@ double shape_cost(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int s
         return 1e30;
     const int held = std::max(1, std::min((int)(160 * 1024 / v.lds), v.waves / ((v.nw + 3) / 4))); // work-groups of a CU, the first wave of each on the first SIMD
     const double gens = (double)((v.wgs + 256 * held - 1) / (256 * held)), steps = gens * v.rounds;
-    const double patches = (double)d.N * v.PY * v.PX;
+    const double work = (double)d.N * v.PY * v.PX * v.nT / 1024, slices = (double)((v.wgs + 255) / 256) * v.rounds * v.nw / 4;
     const double last = own(shape) ? steps * c.ct : gens * ((v.tiles * v.ks + v.nw - 1) / v.nw) * ((v.nT + v.ks - 1) / v.ks);
-    const double f[7] = {1, steps, last, steps * c.nk, patches * v.nT / 1024, gens, patches / 1024};
+    const double f[8] = {1, gens, last, work, work * ((p.out_cs + 31) / 32), slices, slices * c.nk, (double)e.P * e.in_cs * 1e-6};
     double t = 0;
-    for (int i = 0; i < 7; i++)
+    for (int i = 0; i < 8; i++)
         t += kCost[s - 1][shape][i] * f[i];
     return t;
 }
@@ -677,19 +679,22 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
         && e.N == d.N && e.OH == d.H && e.OW == d.W && (long long)e.P * e.in_cs < (1ll << 31);
 }
 
-// The three launches: their latencies, the hidden tensor's bytes at the output's resolution, the products of both 1x1 layers (nine in ten
-// within 10 %).  Of the 626 blocks 618 go the one launch's way by this, 2 of them more than 15 % slower than apart, none that stay apart
-// is more than 16 % slower.
+// The layers apart: the first one's latency, the last two by their own estimate (one launch where that is faster), the hidden tensor's
+// bytes, the products of both 1x1 layers, fitted to the same blocks (nine in ten within 11 %).  (A fit to the three launches, less what the
+// last two gain as one by the estimates of conv_dwpoint.hip, was 5 % low in the middle and 21 % at the ends: 64 -> 192 -> 16 on
+// 22 images of 31x28 went apart, 10.4 -> 12.7 us.)  Less 4 %: of the 2400 blocks 2240 go the one launch's way, 37 of them
+// more than 3 % slower than apart; on average a block takes 0.7 % more than the best choice would.
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;
-    double apart = d.stride_h == 1 ? 8.40 + 0.953 * narrow + 0.00326 * wide * e.in_cs + 0.00191 * narrow * p.out_cs
-                                         : 8.74 + 2.163 * narrow + 0.00291 * wide * e.in_cs + 0.00176 * narrow * p.out_cs;
-    if (conv_dwpoint_applies(d, p)) // the last two layers are one launch where that is faster
-        apart -= std::max(0.0, conv_dwpoint_apart_us(d, p) - conv_dwpoint_us(d, p));
+    double two = conv_dwpoint_apart_us(d, p);
+    if (conv_dwpoint_applies(d, p))
+        two = std::min(two, conv_dwpoint_us(d, p));
+    const double apart = d.stride_h == 1 ? 2.991 + 0.970 * two + 0.191 * wide + 0.00277 * wide * e.in_cs + 0.00083 * narrow * p.out_cs
+                                         : 2.875 + 0.993 * two + 0.195 * wide + 0.00315 * wide * e.in_cs + 0.00102 * narrow * p.out_cs;
     double us;
     choose_shape(e, d, p, -1, &us);
-    return us < apart;
+    return us < 0.96 * apart;
 }
 
 const char *conv_invres_name(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p, int wanted)

@@ -112,6 +112,22 @@ def a_plan_launches_the_kernel_that_it_names():
     assert len(seen) == len(names), seen
 
 
+def inverted_residual_blocks_run_as_one_where_that_is_faster():
+    """The built-in rule against blocks that were measured both ways (as one launch, and as the first layer and what is faster behind it):
+    it takes the one launch where that is clearly ahead."""
+    import numpy as np
+    from nart_amd import hipq
+    for n, ci, ch, co, h, w, one, apart in ((22, 64, 192, 16, 31, 28, 9.6, 13.0), (9, 80, 480, 16, 21, 22, 7.6, 12.8), (15, 40, 240, 24, 25, 22, 7.3, 12.5),
+                                            (92, 80, 480, 16, 5, 6, 7.5, 12.3), (17, 160, 480, 160, 5, 5, 7.2, 11.2), (5, 80, 480, 24, 29, 39, 7.8, 10.0),
+                                            (64, 24, 144, 24, 56, 56, 26.8, 39.5)):
+        plans = []
+        for C_, K, R, g in ((ci, ch, 1, 1), (ch, ch, 3, ch), (ch, co, 1, 1)):
+            plans.append(hipq.Conv2d((n, C_, h, w), np.full((K, C_ // g, R, R), 129, np.uint8), None, R // 2, 1, g, 0.05, 9, 0.002, 128, 0.05, 9))
+        assert hipq.inverted_residual_fusable(*plans), (n, ci, ch, co, h, w, one, apart)
+        for p in plans:
+            p.close()
+
+
 def block_tails_keep_to_patches_that_divide_an_image():
     """hipq_bottleneck_tail_run may write the sum over the residual wherever some patch shape divides the image, also where another would
     need as many overlapping patches or fewer, and takes 128 channels by rule on such images however few their pixels; where none
@@ -733,7 +749,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
