@@ -2423,7 +2423,7 @@ extern "C" int hipq_inverted_residual_run(const hipq_conv2d_plan *pe, const hipq
 extern "C" int hipq_inverted_residual_select(hipq_conv2d_plan *pp, int shape)
 {
     clear_error();
-    HIPQ_REQUIRE(pp && shape >= -1 && shape <= 5, "hipq_inverted_residual_select: null plan, or shape %d outside -1..4", shape);
+    HIPQ_REQUIRE(pp && shape >= -1 && shape <= 5, "hipq_inverted_residual_select: null plan, or shape %d outside -1..5", shape);
     pp->invres_shape = shape;
     return 0;
 }

@@ -128,6 +128,17 @@ def inverted_residual_blocks_run_as_one_where_that_is_faster():
             p.close()
 
 
+def a_patch_shape_out_of_range_names_the_range():
+    import numpy as np
+    from nart_amd import hipq
+    p = hipq.Conv2d((1, 32, 8, 8), np.full((16, 32, 1, 1), 129, np.uint8), None, 0, 1, 1, 0.05, 9, 0.002, 128, 0.05, 9)
+    for shape in range(-1, 6):
+        hipq.inverted_residual_select(p, shape)
+    for shape in (-2, 6):
+        with pytest.raises(hipq.HipqError, match="shape %d outside -1..5" % shape):
+            hipq.inverted_residual_select(p, shape)
+
+
 def block_tails_keep_to_patches_that_divide_an_image():
     """hipq_bottleneck_tail_run may write the sum over the residual wherever some patch shape divides the image, also where another would
     need as many overlapping patches or fewer, and takes 128 channels by rule on such images however few their pixels; where none
@@ -749,7 +760,7 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+CASES = [a_patch_shape_out_of_range_names_the_range, inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
          a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
          operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
          layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
