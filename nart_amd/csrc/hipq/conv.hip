@@ -1505,10 +1505,12 @@ static double stream_us(const hipq_conv2d_plan *p, const StreamShape &s)
     return 2.56 + (double)((wgs + kCUs - 1) / kCUs) * ((point ? 0.0147 : 0.0233) * (s.mb + s.nb) * a.nslab + 0.193 * s.mb * s.nb + (point ? 0 : 0.34) + (p->d_q ? 0.32 : 0));
 }
 
-// Which shape, if any, the built-in rule takes it in.  The margins, set by hand, are what keeps layers from getting slower where both fits
-// are a few per cent off: of 220 layers that the fits have not seen 69 change kernel and take 0.76 of the time on average, one of them
-// 8 % more (7.1 -> 7.6 us).  Layers that have a kernel of their own keep it, without a comparison, and so do the two classes that
-// stream_applies keeps out.
+// Which shape, if any, the built-in rule takes it in.  With one scale the margins, set by hand, are what keeps layers from getting slower where
+// both fits are a few per cent off: of 220 layers that the fits have not seen 69 change kernel and take 0.76 of the time on average, one
+// of them 8 % more (7.1 -> 7.6 us).  With a scale per channel or a signed range the cheaper fit decides: of 1000 such layers that the fits
+// have not seen it takes another kernel or shape for 263 than margins of 0.75 to 0.95 and the fits before, which took 1.09 times as
+// long on those; 26 of them take more than 3 % longer (16.1 -> 20.5 us at worst), 181 less (8.4 -> 5.2).  Layers that have a kernel of
+// their own keep it, without a comparison, and so do the two classes that stream_applies keeps out.
 static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &a, ResidentShape *narrow)
 {
     ResidentShape s = {0, 0, 0, 0}, wide = {0, 0, 0, 0};
@@ -1519,7 +1521,8 @@ static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &
         return {0, 0, 0, 0};
     StreamShape ss;
     const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1, halo = !streams && halo_applies(p);
-    const double now = streams ? stream_us(p, ss) : tile_us(p), margin = streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
+    const bool channels = a.qmult != nullptr || a.lo < 0;
+    const double now = streams ? stream_us(p, ss) : tile_us(p), margin = channels ? 1 : streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
     // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.2 us streamed, 7.6 with resident rows; 128
     // rows 9.9 against 9.1.  A 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 7.5
     // against 8.2 us in its best shape
@@ -1530,12 +1533,10 @@ static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &
     // With 32 x 32 tiles, for layers with work for every SIMD, against whichever of the others it would be.  The halo kernel keeps its layers of
     // few pixels, as above; a 1x1 layer with a stride would fill LDS with pixels that nobody reads, and one with one scale has no
     // requantisation to gain by (136 -> 135 channels, 15 images of 94x81, 15.8 us in tiles and 19.1 here; 641 -> 443, 7 of 32x33, 8.4
-    // and 9.0).  The margins leave out what the fits cannot tell apart: of 900 layers 44 change kernel, from 0.96 to 1.42 times as fast,
-    // 1.17 on average.  Scales per channel and signed ranges, which the other kernels requantise in twice the instructions, gain 1.05 to 1.75
-    // times down to the line; what the fit gives the 16 x 16 tiles for those is a sixth below what they measure (96 -> 200 channels
-    // on 25 125 pixels: 10.8 us estimated, 14.2 measured, 12.4 here), so that their line lies as much higher.
-    const bool few = halo && a.P <= 8192, channels = a.qmult != nullptr || a.lo < 0;
-    const double line = !channels ? 0.88 : s.mb && s.ks == 1 ? 1.08 : 0.97;
+    // and 9.0).  With one scale 0.88 leaves out what the fits cannot tell apart.  Scales per channel and signed ranges, which the other kernels
+    // requantise in twice the instructions, are decided by the fits alone.
+    const bool few = halo && a.P <= 8192;
+    const double line = channels ? 1 : 0.88;
     if (!few && !(streams && fc && ss.mb < 4) && !(point && (!channels || a.stride_h > 1 || a.stride_w > 1)) && conv_resident_choose_wide(a, &wide, &wide_us)
         && wide_us < line * us)
         return wide;

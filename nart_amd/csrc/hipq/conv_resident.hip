@@ -778,60 +778,84 @@ bool wide_applies(const ConvArgs &a)
         && (a.res == nullptr || (!channels && a.addq.fast && a.addq.hi == 255));
 }
 
-// Microseconds of a launch of the 32 x 32 form, fitted to 4900 launches: 400 layers of 300 000 to 24 million outputs in the shapes that
-// fit LDS (nine in ten within 20 % of the fit).  A launch; for every generation of resident work-groups its start and end, and per step and per
-// tile of a wave its chain; per CU the multiplies, those of them that are of channels the layer has, the pixels' KB, the weights'
-// KB and the tiles; the tensors' MB.
+// Microseconds of a launch.  Layers with one scale and no sign, and those that go through the general requantisation (kAny), in the 16 x 16
+// form: fitted to 12 000 launches, 490 layers of 1 to 200 000 pixels and 16 to 8192 channels in every shape that fits LDS (half of them
+// within 8 % of the fit, nine in ten within 18); in the 32 x 32 form to 4900, 400 layers of 300 000 to 24 million outputs (nine in ten within
+// 20 %).  Layers with a scale per channel or a signed range, whose requantisation takes twice the instructions, in both forms: fitted to
+// 2200 layers of 300 to 24 million outputs in every shape that takes less than twice the best one's time (nine in ten within 17 %); of the
+// shapes that fit LDS, the one that this picks for them takes 2 % more than the best on average (8 % by the other layers' terms, which spread 300
+// work-groups evenly over 256 CUs).
+
+// the 32 x 32 form.  A launch; for every generation of resident work-groups its start and end, and per step and per tile of a wave its
+// chain; per CU the multiplies, those of them that are of channels the layer has, the pixels' KB, the weights' KB and the tiles; the
+// tensors' MB
 double wide_cost(const ConvArgs &a, const ResidentShape &s)
 {
-    static const double kCost[2][2][11] = {
-        {{2.684, 1.019, 0.0112, 0.0036, 0.0133, 0.0203, 0.0325, 0.0271, 0.0332, 0.1241, 0.0001},  // a step lies in one tap: one scale,
-         {2.603, 1.107, 0.0121, 0.0056, 0.0073, 0.0099, 0.0276, 0.0590, 0.0564, 0.1477, 0.0019}}, // channels' scales or signed
-        {{2.888, 0.662, 0.0096, 0.0086, 0.0053, 0.0244, 0.0675, 0.0426, 0.0265, 0.1094, 0.0000},  // it does not
-         {3.216, 0.311, 0.0077, 0.0000, 0.0125, 0.0128, 0.0613, 0.0918, 0.0454, 0.1694, 0.0038}}};
-    const bool channels = a.qmult != nullptr || a.lo < 0;
-    const double *const k = kCost[a.in_cs % 32 != 0][channels];
+    static const double kCost[2][11] = {{2.684, 1.019, 0.0112, 0.0036, 0.0133, 0.0203, 0.0325, 0.0271, 0.0332, 0.1241, 0.0001},  // a step lies in one tap,
+                                        {2.888, 0.662, 0.0096, 0.0086, 0.0053, 0.0244, 0.0675, 0.0426, 0.0265, 0.1094, 0.0000}}; // it does not
+    // channels' scales or a signed range: a launch; generation, tile x step, step, tile, KB of pixels / wave; CU's multiplies, tiles, those with a
+    // scale per channel, KB of pixels, weights; MB
+    static const double kChannelCost[2][12] = {{2.07, 1.24, 0.0123, 0.0172, 0.167, 0.0383, 0.0111, 0.0245, 0.0319, 0.00110, 0.00485, 0.129},
+                                               {2.68, 0.248, 0.00765, 0.0490, 0.175, 0.0341, 0.00956, 0.0295, 0.0310, 0.00769, 0.00628, 0.106}};
+    const bool channels = a.qmult != nullptr || a.lo < 0, pieces = a.in_cs % 32 != 0;
     const int mt = s.mb / 2, nt = s.nb / 2, nw = s.nwc, steps = (a.Ktot + 31) / 32, ct = (a.out_cs + 31) / 32;
     const int groups = (a.out_cs + 16 * s.nb * nw - 1) / (16 * s.nb * nw);
     const double wgs = (double)((a.P + 16 * s.mb - 1) / (16 * s.mb)) * groups;
     const int waves = mt * nt == 8 || (mt * nt == 4 && (nt == 2 || channels)) ? 2 : mt * nt == 4 || channels ? 3 : 4; // of a SIMD, by their registers
-    const int held = std::max(1, std::min(160 * 1024 / lds_bytes(a, s), 4 * waves / nw));
+    // five and six waves: two of a work-group on one SIMD, none left for two of the next (the fit was a quarter low with two work-groups)
+    const int held = std::max(1, std::min(160 * 1024 / lds_bytes(a, s), channels && nw > 4 ? waves / 2 : 4 * waves / nw));
     const double gens = std::ceil(wgs / (256.0 * held)), cu = std::max(1.0, wgs / 256), most = std::ceil(wgs / 256), used = (double)std::min(nw * nt * groups, ct) / groups;
     const double region = 1e-3 * region_rows(a, s.mb) * lds_row(a), mb = 1e-6 * ((double)a.P * a.out_cs + (double)a.N * a.H * a.W * a.in_cs);
-    return k[0] + gens * (k[1] + steps * (k[2] * mt * nt + k[6]) + k[9] * mt * nt) + most * (0.25 * steps * mt * (k[3] * nt * nw + k[4] * used) + k[8] * nw * mt * nt)
+    const double tiles = most * nw * mt * nt;
+    if (channels) {
+        const double *const k = kChannelCost[pieces];
+        return k[0] + gens * (k[1] + steps * (k[2] * mt * nt + k[3]) + k[4] * mt * nt + k[5] * region / nw)
+               + most * (0.25 * k[6] * steps * mt * nt * nw + k[9] * region) + tiles * (k[7] + (a.qmult != nullptr ? k[8] : 0)) + cu * k[10] * steps * nt * nw + k[11] * mb;
+    }
+    const double *const k = kCost[pieces];
+    return k[0] + gens * (k[1] + steps * (k[2] * mt * nt + k[6]) + k[9] * mt * nt) + most * 0.25 * steps * mt * (k[3] * nt * nw + k[4] * used) + tiles * k[8]
            + cu * (k[5] * region + k[10] * steps * nt * nw) + k[7] * mb;
 }
 
-// Microseconds of a launch in one shape, fitted to 12 000 launches: 490 layers of 1 to 200 000 pixels and 16 to 8192 channels in every
-// shape that fits LDS (half of them within 8 % of the fit, nine in ten within 18).  A launch; for every generation of
-// resident work-groups its start and end; for every slab that a wave takes its chain, alone and per pixel tile; per CU the weight and
-// the pixel bytes that it pulls, the output tiles, the partial sums, the pixels that its waves locate.
+// The 16 x 16 form.  A launch; for every generation of resident work-groups its start and end; for every slab that a wave takes its chain,
+// alone and per pixel tile; per CU the weight and the pixel bytes that it pulls, the output tiles, the partial sums, the pixels that its
+// waves locate.
 double shape_cost(const ConvArgs &a, const ResidentShape &s)
 {
     if (s.ks == 0)
         return wide_cost(a, s);
     // launch, generation, slab, slab x pixel tile, KB of weights, KB of pixels, output tile, partial tile, pixel tile of a SIMD
-    static const double kCost[2][5][9] = {
+    static const double kCost[2][4][9] = {
         {{2.505, 0.101, 0.0027, 0.0142, 0.0086, 0.0295, 0.0156, 0, 0},        // whole reductions: 1x1,
          {2.160, 1.013, 0.0079, 0.0177, 0.0083, 0.0270, 0.0302, 0, 0},        // a slab lies in one tap,
          {2.391, 0.560, 0.0304, 0.0198, 0.0065, 0.0286, 0.0260, 0, 0},        // it does not,
-         {2.443, 0.648, 0.0203, 0.0237, 0.0074, 0.0206, 0.0261, 0, 0.0370},   // channels' scales or signed,
          {3.521, 0, 0.0101, 0.0550, 0.0058, 0.0237, 0.0668, 0, 0}},           // weight zero points and the rest
         {{2.279, 0.502, 0, 0.0220, 0.0095, 0.0147, 0.0306, 0.0085, 0},        // shared ones
          {2.225, 0.842, 0, 0.0263, 0.0105, 0.0103, 0.0355, 0.0063, 0.0607},
          {2.243, 0.689, 0.0235, 0.0264, 0.0095, 0.0115, 0.0211, 0.0096, 0.0663},
-         {2.274, 0.845, 0.0263, 0.0282, 0.0089, 0.0118, 0.0244, 0.0133, 0.0471},
          {2.438, 0.885, 0.0024, 0.0643, 0.0097, 0.0067, 0.0459, 0.0143, 0.0591}}};
-    const bool any = a.bwz != 0 || !(a.qmult != nullptr ? a.fastch : a.fastq);
-    const double *const k = kCost[s.ks > 1][any ? 4 : a.qmult != nullptr || a.lo < 0 ? 3 : point(a) ? 0 : a.in_cs % 64 == 0 ? 1 : 2];
+    // channels' scales or a signed range, whole and shared reductions: a launch; generation, slab, slab of 128 pixels (two slabs of weights ahead
+    // instead of four), slab x pixel tile, tile, the same with a scale per channel; of the CU with the most work-groups KB of pixels,
+    // multiplies of a SIMD, pixel tiles of a SIMD, output tiles; KB of weights; MB
+    static const double kChannelCost[2][13] = {{2.64, 0.425, 0.0384, 0.0206, 0.00621, 0.0731, 0.0420, 0.0134, 0.00404, 0.0731, 0, 0.00751, 0.146},
+                                               {2.57, 0.542, 0.0642, 0.173, 0, 0.0331, 0.0164, 0.0104, 0.00666, 0.103, 0.0235, 0.00688, 0.0445}};
     const int nw = s.nwc * s.ks, lds = lds_bytes(a, s);
     const double wgs = (double)((a.P + 16 * s.mb - 1) / (16 * s.mb)) * ((a.out_cs + 16 * s.nb * s.nwc - 1) / (16 * s.nb * s.nwc));
     const int regs = 4 * s.mb * s.nb + 4 * s.nb * (s.nb == 1 ? (s.mb == 1 ? 9 : 8) : s.nb == 2 && s.mb < 8 ? 6 : 4) + 8 * s.mb + 40;
     const int waves = std::max(1, std::min(8, 512 / regs)); // of a SIMD
     const int held = std::max(1, std::min(160 * 1024 / lds, 4 * waves / nw));
     const double gens = std::ceil(wgs / (256.0 * held)), per = (a.nslab + s.ks - 1) / s.ks, cu = std::max(1.0, wgs / 256);
-    return k[0] + gens * (k[1] + per * (k[2] + k[3] * s.mb)) + cu * (k[4] * 1.024 * a.nslab * s.nb * s.nwc + k[5] * 1e-3 * region_rows(a, s.mb) * lds_row(a)
-           + k[6] * s.mb * s.nb * s.nwc + (s.ks > 1 ? k[7] * nw * s.mb * s.nb : 0) + k[8] * 0.25 * nw * s.mb);
+    const double region = 1e-3 * region_rows(a, s.mb) * lds_row(a), weights = 1.024 * a.nslab * s.nb * s.nwc;
+    const bool any = a.bwz != 0 || !(a.qmult != nullptr ? a.fastch : a.fastq), channels = a.qmult != nullptr || a.lo < 0;
+    if (channels && !any) {
+        const double *const k = kChannelCost[s.ks > 1];
+        const double most = std::ceil(wgs / 256), mb = 1e-6 * ((double)a.P * a.out_cs + (double)a.N * a.H * a.W * a.in_cs);
+        return k[0] + gens * (k[1] + per * (k[2] + (s.mb == 8 ? k[3] : 0) + k[4] * s.mb) + s.mb * s.nb * (k[5] + (a.qmult != nullptr ? k[6] : 0)))
+               + most * (k[7] * region + 0.25 * nw * s.mb * (k[8] * per * s.nb + k[9]) + k[10] * s.mb * s.nb * s.nwc) + cu * k[11] * weights + k[12] * mb;
+    }
+    const double *const k = kCost[s.ks > 1][any ? 3 : point(a) ? 0 : a.in_cs % 64 == 0 ? 1 : 2];
+    return k[0] + gens * (k[1] + per * (k[2] + k[3] * s.mb)) + cu * (k[4] * weights + k[5] * region + k[6] * s.mb * s.nb * s.nwc
+           + (s.ks > 1 ? k[7] * nw * s.mb * s.nb : 0) + k[8] * 0.25 * nw * s.mb);
 }
 
 } // namespace

@@ -128,6 +128,22 @@ def inverted_residual_blocks_run_as_one_where_that_is_faster():
             p.close()
 
 
+def layers_with_channel_scales_take_the_faster_shape():
+    """The built-in rule against layers with a scale per channel or a signed range that were measured in two kernels or shapes, a fifth
+    apart and more: not the slower one, whatever the neighbouring sizes take."""
+    import numpy as np
+    from nart_amd import hipq
+    for n, c, h, w, k, r, i8, pc, fast, slow in ((5, 96, 75, 67, 192, 3, True, True, 11.1, ("resident_64x192", 13.8)), (5, 96, 75, 67, 160, 3, True, True, 10.8, ("resident_64x160", 12.9)),
+                                                 (13, 41, 65, 53, 32, 3, True, True, 5.2, ("resident_128x32", 8.4)), (22, 18, 41, 43, 18, 3, False, True, 5.5, ("resident_128x32", 7.8)),
+                                                 (9, 23, 70, 58, 21, 3, False, True, 5.4, ("resident_128x32", 7.7)), (3, 124, 16, 17, 156, 1, False, True, 3.3, ("64x64", 4.7)),
+                                                 (1, 29, 11, 9, 967, 1, True, True, 3.1, ("64x64", 4.4)), (5, 96, 75, 67, 200, 3, True, True, 12.1, ("resident_64x256", 14.2))):
+        wt = np.full((k, c, r, r), 1 if i8 else 129, np.int8 if i8 else np.uint8)
+        p = hipq.Conv2d((n, c, h, w), wt, None, r // 2, 1, 1, 0.02, 0 if i8 else 128, np.linspace(0.003, 0.007, k).astype(np.float32) if pc else 0.005, 0 if i8 else 128,
+                        0.02, 0 if i8 else 120, obits=7 if i8 else 8, dtype=hipq.DTYPE_I8 if i8 else hipq.DTYPE_U8)
+        assert p.kernel.split("_i8_")[1].replace("_signed", "").replace("_perchannel", "") != slow[0], (p.kernel, n, c, h, w, k, fast, slow)
+        p.close()
+
+
 def a_patch_shape_out_of_range_names_the_range():
     import numpy as np
     from nart_amd import hipq
@@ -760,11 +776,14 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [a_patch_shape_out_of_range_names_the_range, inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster, a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
-         a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
-         operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
-         layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
-         a_pass_that_cannot_be_recorded_runs_its_operators,
+CASES = [inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster,
+         a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once,
+         block_tails_keep_to_patches_that_divide_an_image, layers_with_channel_scales_take_the_faster_shape,
+         a_patch_shape_out_of_range_names_the_range, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names,
+         fused_block_follows_the_scales_of_its_operators, a_chain_of_separable_layers_is_divided_blocks_first,
+         blocks_are_decided_again_for_recorded_passes, operators_run_one_by_one_launch_themselves,
+         two_parades_of_one_input_launch_their_own_layers, layers_run_together_only_where_their_memories_allow,
+         layers_computed_ahead_follow_their_tensors, a_pass_that_cannot_be_recorded_runs_its_operators,
          records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
          a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
          operators_of_two_workspaces_wait_for_each_other]
