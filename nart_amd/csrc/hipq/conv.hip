@@ -1521,7 +1521,7 @@ static ResidentShape choose_resident(const hipq_conv2d_plan *p, const ConvArgs &
         return {0, 0, 0, 0};
     StreamShape ss;
     const bool streams = stream_applies(p, &ss), point = a.R == 1 && a.S == 1, fc = point && a.H == 1 && a.W == 1, halo = !streams && halo_applies(p);
-    const bool channels = a.qmult != nullptr || a.lo < 0;
+    const bool channels = conv_resident_channels(a);
     const double now = streams ? stream_us(p, ss) : tile_us(p), margin = channels ? 1 : streams ? 0.95 : fc || (now < 8 && !point) ? 0.85 : 0.75;
     // a fully-connected layer on a few rows is nothing but its weights: 64 x 4096 x 4096 7.2 us streamed, 7.6 with resident rows; 128
     // rows 9.9 against 9.1.  A 1x1 layer on many pixels or with a stride has little to keep: 128 -> 512 channels on 18 432 pixels 7.5

@@ -20,6 +20,8 @@ bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us);
 // the same among the shapes with 32 x 32 tiles, which not every launch of a plan can take: conv_resident_wide_applies
 bool conv_resident_wide_applies(const ConvArgs &a);
 bool conv_resident_choose_wide(const ConvArgs &a, ResidentShape *shape, double *us);
+// a scale per channel or a signed range in the one-multiply requantisation: layers that have a fit of their own
+bool conv_resident_channels(const ConvArgs &a);
 // two layers that do not depend on each other in one launch.  conv_resident_pair_costs: what each shape takes for a layer (a plan keeps
 // it: computing it takes longer than the rest of a launch); conv_resident_choose_pair: shapes for both; false: they do not run that way
 constexpr int kResidentShapes = 26;

@@ -797,7 +797,7 @@ double wide_cost(const ConvArgs &a, const ResidentShape &s)
     // scale per channel, KB of pixels, weights; MB
     static const double kChannelCost[2][12] = {{2.07, 1.24, 0.0123, 0.0172, 0.167, 0.0383, 0.0111, 0.0245, 0.0319, 0.00110, 0.00485, 0.129},
                                                {2.68, 0.248, 0.00765, 0.0490, 0.175, 0.0341, 0.00956, 0.0295, 0.0310, 0.00769, 0.00628, 0.106}};
-    const bool channels = a.qmult != nullptr || a.lo < 0, pieces = a.in_cs % 32 != 0;
+    const bool channels = conv_resident_channels(a), pieces = a.in_cs % 32 != 0;
     const int mt = s.mb / 2, nt = s.nb / 2, nw = s.nwc, steps = (a.Ktot + 31) / 32, ct = (a.out_cs + 31) / 32;
     const int groups = (a.out_cs + 16 * s.nb * nw - 1) / (16 * s.nb * nw);
     const double wgs = (double)((a.P + 16 * s.mb - 1) / (16 * s.mb)) * groups;
@@ -846,8 +846,8 @@ double shape_cost(const ConvArgs &a, const ResidentShape &s)
     const int held = std::max(1, std::min(160 * 1024 / lds, 4 * waves / nw));
     const double gens = std::ceil(wgs / (256.0 * held)), per = (a.nslab + s.ks - 1) / s.ks, cu = std::max(1.0, wgs / 256);
     const double region = 1e-3 * region_rows(a, s.mb) * lds_row(a), weights = 1.024 * a.nslab * s.nb * s.nwc;
-    const bool any = a.bwz != 0 || !(a.qmult != nullptr ? a.fastch : a.fastq), channels = a.qmult != nullptr || a.lo < 0;
-    if (channels && !any) {
+    const bool any = a.bwz != 0 || !(a.qmult != nullptr ? a.fastch : a.fastq);
+    if (conv_resident_channels(a)) {
         const double *const k = kChannelCost[s.ks > 1];
         const double most = std::ceil(wgs / 256), mb = 1e-6 * ((double)a.P * a.out_cs + (double)a.N * a.H * a.W * a.in_cs);
         return k[0] + gens * (k[1] + per * (k[2] + (s.mb == 8 ? k[3] : 0) + k[4] * s.mb) + s.mb * s.nb * (k[5] + (a.qmult != nullptr ? k[6] : 0)))
@@ -895,6 +895,8 @@ bool conv_resident_choose(const ConvArgs &a, ResidentShape *shape, double *us)
 }
 
 bool conv_resident_wide_applies(const ConvArgs &a) { return wide_applies(a); }
+
+bool conv_resident_channels(const ConvArgs &a) { return a.bwz == 0 && (a.qmult != nullptr ? a.fastch : a.lo < 0 && a.fastq); }
 
 bool conv_resident_choose_wide(const ConvArgs &a, ResidentShape *shape, double *us)
 {
