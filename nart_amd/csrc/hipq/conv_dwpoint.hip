@@ -530,16 +530,19 @@ double conv_dwpoint_us(const ConvArgs &d, const ConvArgs &p)
     return us;
 }
 
-// The two launches: their latencies, the bytes of the first one's input and of the tensor between them, the products of the second, its
-// output and its weights; fitted to the same pairs (nine in ten within 12 %), less 2 %: a tie stays apart.  Of the 3600 this fuses
-// 2680, which take 0.74 of the two launches on average, 45 of them more than 3 % longer (12.8 -> 16.6 us at most); it takes 0.8 % more
-// than the better of the two would each time.
+// The two launches: their latencies, the bytes of the tensor between them, the products of the second, its output, channels and weights,
+// and what the tile kernel's two groups of waves add where they keep a 1x1 layer with a partial last slab (an even number of at least 8);
+// fitted to 2200 further pairs (nine in ten within 10 %), by 6 % more: the fit above is 8 % above what these measure, and a tie stays apart.
+// Of the 2200 this fuses 1796, 20 of them more than 3 % longer (1.3 times at most), and leaves 18 apart that are more than 3 % faster
+// as one, where the fit before, which did not tell the partial slabs, left 80 (878 -> 14 channels on five images of 5x4: 8.4 us, 6.1);
+// it takes 0.5 % more than the better of the two would each time, before 1.0.
 double conv_dwpoint_apart_us(const ConvArgs &d, const ConvArgs &p)
 {
-    const double in = (double)d.N * d.H * d.W * d.in_cs * 1e-6, mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6;
+    const double mid = (double)p.P * d.in_cs * 1e-6, out = (double)p.P * p.out_cs * 1e-6;
     const double channels = d.in_cs * 1e-3, weights = (double)d.in_cs * p.out_cs * 1e-6;
-    return 0.98 * (d.stride_h == 1 ? 6.212 + 0.608 * mid + 0.00134 * mid * p.out_cs + 0.246 * out + 0.146 * channels + 2.299 * weights
-                                   : 6.527 + 0.088 * in + 0.611 * mid + 0.00210 * mid * p.out_cs + 0.249 * out + 1.328 * weights);
+    const bool partial = d.in_cs % 64 != 0 && p.nslab >= 8 && p.nslab % 2 == 0;
+    return d.stride_h == 1 ? 5.92 + 0.669 * mid + 0.00187 * mid * p.out_cs + 0.237 * out + 0.263 * channels + 2.75 * weights + (partial ? 0.172 + 0.1425 * p.nslab : 0)
+                           : 6.33 + 1.05 * mid + 0.00243 * mid * p.out_cs + 0.205 * out + 0.158 * channels + 1.62 * weights + (partial ? 0.305 + 0.14 * p.nslab : 0);
 }
 
 const char *conv_dwpoint_name(const ConvArgs &d, const ConvArgs &p, int wanted)

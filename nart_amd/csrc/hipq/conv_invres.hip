@@ -682,8 +682,9 @@ bool conv_invres_applies(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p
 // The layers apart: the first one's latency, the last two by their own estimate (one launch where that is faster), the hidden tensor's
 // bytes, the products of both 1x1 layers, fitted to the same blocks (nine in ten within 11 %).  (A fit to the three launches, less what the
 // last two gain as one by the estimates of conv_dwpoint.hip, was 5 % low in the middle and 21 % at the ends: 64 -> 192 -> 16 on
-// 22 images of 31x28 went apart, 10.4 -> 12.7 us.)  Less 4 %: of the 2400 blocks 2240 go the one launch's way, 37 of them
-// more than 3 % slower than apart; on average a block takes 0.7 % more than the best choice would.
+// 22 images of 31x28 went apart, 10.4 -> 12.7 us.)  Less 4 %: of 900 blocks that no fit has seen 852 go the one launch's way, 8 of
+// them more than 3 % slower than apart; 12 of the others would be more than 3 % faster; on average a block takes 0.3 % more than the best
+// choice would.
 bool conv_invres_preferred(const ConvArgs &e, const ConvArgs &d, const ConvArgs &p)
 {
     const double wide = (double)e.P * d.in_cs * 1e-6, narrow = (double)p.P * d.in_cs * 1e-6;

@@ -128,6 +128,21 @@ def inverted_residual_blocks_run_as_one_where_that_is_faster():
             p.close()
 
 
+def depthwise_pairs_run_as_one_where_that_is_faster():
+    """The built-in rule against pairs of layers that were measured both ways, a tenth apart and more (a tie: 960 -> 320 channels at 7x7,
+    64 images, 9.6 us and 10.2, where the network around it gains 4)."""
+    import numpy as np
+    from nart_amd import hipq
+    for n, h, w, c, k, stride, one, apart in ((64, 7, 7, 960, 320, 1, 9.6, 10.2), (64, 7, 7, 768, 320, 1, 8.0, 9.1), (64, 7, 7, 960, 160, 1, 8.3, 10.1), (5, 5, 4, 878, 14, 1, 6.1, 8.4),
+                                              (13, 17, 18, 708, 38, 2, 6.5, 8.9), (10, 47, 38, 454, 56, 1, 10.1, 13.6), (128, 7, 7, 960, 320, 1, 16.6, 14.2), (64, 10, 10, 960, 320, 1, 23.6, 14.0),
+                                              (64, 7, 7, 512, 512, 1, 12.0, 8.6)):
+        oh, ow = (h - 1) // stride + 1, (w - 1) // stride + 1
+        depthwise = hipq.Conv2d((n, c, h, w), np.full((c, 1, 3, 3), 129, np.uint8), None, 1, stride, c, 0.05, 9, 0.002, 128, 0.05, 9)
+        point = hipq.Conv2d((n, c, oh, ow), np.full((k, c, 1, 1), 129, np.uint8), None, 0, 1, 1, 0.05, 9, 0.002, 128, 0.05, 9)
+        assert hipq.depthwise_point_fusable(depthwise, point) is (one < apart), (n, h, w, c, k, stride, one, apart)
+        depthwise.close(), point.close()
+
+
 def layers_with_channel_scales_take_the_faster_shape():
     """The built-in rule against layers with a scale per channel or a signed range that were measured in two kernels or shapes, a fifth
     apart and more: not the slower one, whatever the neighbouring sizes take."""
@@ -776,17 +791,17 @@ def operators_of_two_workspaces_wait_for_each_other():
     assert replays.value >= 4
 
 
-CASES = [inverted_residual_add_needs_equal_shapes, inverted_residual_blocks_run_as_one_where_that_is_faster,
-         a_pair_of_layers_is_launched_as_quickly_as_two, exact_adds_are_the_operator, exact_adds_are_searched_for_once,
-         block_tails_keep_to_patches_that_divide_an_image, layers_with_channel_scales_take_the_faster_shape,
-         a_patch_shape_out_of_range_names_the_range, a_chained_add_names_its_kernels, a_plan_launches_the_kernel_that_it_names,
-         fused_block_follows_the_scales_of_its_operators, a_chain_of_separable_layers_is_divided_blocks_first,
-         blocks_are_decided_again_for_recorded_passes, operators_run_one_by_one_launch_themselves,
-         two_parades_of_one_input_launch_their_own_layers, layers_run_together_only_where_their_memories_allow,
-         layers_computed_ahead_follow_their_tensors, a_pass_that_cannot_be_recorded_runs_its_operators,
-         records_are_taken_again_after_many_changes, an_output_that_nobody_reads_is_not_copied_back,
-         a_write_waits_for_the_copy_back_that_fills_the_same_mirror, a_write_waits_for_every_stream_that_reads_the_array,
-         operators_of_two_workspaces_wait_for_each_other]
+CASES = [depthwise_pairs_run_as_one_where_that_is_faster, inverted_residual_add_needs_equal_shapes,
+         inverted_residual_blocks_run_as_one_where_that_is_faster, a_pair_of_layers_is_launched_as_quickly_as_two,
+         exact_adds_are_the_operator, exact_adds_are_searched_for_once, block_tails_keep_to_patches_that_divide_an_image,
+         layers_with_channel_scales_take_the_faster_shape, a_patch_shape_out_of_range_names_the_range, a_chained_add_names_its_kernels,
+         a_plan_launches_the_kernel_that_it_names, fused_block_follows_the_scales_of_its_operators,
+         a_chain_of_separable_layers_is_divided_blocks_first, blocks_are_decided_again_for_recorded_passes,
+         operators_run_one_by_one_launch_themselves, two_parades_of_one_input_launch_their_own_layers,
+         layers_run_together_only_where_their_memories_allow, layers_computed_ahead_follow_their_tensors,
+         a_pass_that_cannot_be_recorded_runs_its_operators, records_are_taken_again_after_many_changes,
+         an_output_that_nobody_reads_is_not_copied_back, a_write_waits_for_the_copy_back_that_fills_the_same_mirror,
+         a_write_waits_for_every_stream_that_reads_the_array, operators_of_two_workspaces_wait_for_each_other]
 
 
 @pytest.fixture(scope="module")
