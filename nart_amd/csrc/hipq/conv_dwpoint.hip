@@ -13,14 +13,14 @@
 // The waves of a work-group split the channels of one patch and add their partial sums up in LDS, or, where there are many patches and
 // one slice, every wave has patches of its own.  Output channel tiles are divided into groups: each group computes the depthwise
 // layer again, which costs less than idle CUs, and spreads a 7x7 image over more CUs.
-// What bounds it: many patches of few channels - memory and vector issue (the requantisations: 44 % of a CU's busy time at 4 clocks an
-// instruction, matrix cores 14 %); few pixels of many channels - the chain launch, region, slices, sum, in which a CU's vector units (29
-// to 35 %) and matrix cores (4 to 7 %) take turns and mostly wait.
-// Measured, the two launches -> this one (back to back and warm): 32 -> 16 channels at 112x112, 64 images: 24.8 -> 14.7 us (38 MB of
-// input and output), 1 image: 5.2 -> 3.0; 64 -> 128 at 56x56, stride 2, 1 image: 6.1 -> 4.1; 192 -> 64 at 28x28, stride 2, 6 images:
-// 5.5 -> 4.3; 960 -> 160 at 7x7, 64 images: 10.6 -> 9.1, 1 image: 6.6 -> 6.8 (there the two launches stay).  A shared patch's biases,
-// residual and the place where its sums meet are ready before them: 1.1 to 1.4 times as fast as with the three in the chain (960 ->
-// 320, 64 images, 11.2 -> 9.2).
+// What bounds it: many patches of few channels - memory and vector issue (the requantisations: 45 % of a CU's busy time at 4 clocks an
+// instruction, matrix cores 14 %); few pixels of many channels - the chain launch, region, slices, sum, in which a CU's vector units (28
+// to 34 %) and matrix cores (7 to 8 %) take turns and mostly wait.
+// Measured, the two launches -> this one (back to back, three sets of tensors in turn): 32 -> 16 channels at 112x112, 64 images: 24.6 -> 15.7
+// us (38 MB of input and output), 1 image: 5.6 -> 3.4; 64 -> 128 at 56x56, stride 2, 1 image: 6.5 -> 3.8; 192 -> 64 at 28x28, stride 2,
+// 6 images: 5.8 -> 4.3; 960 -> 160 at 7x7, 64 images: 10.0 -> 8.3, 1 image: 6.0 -> 6.3 (the rule takes it for a tie).  A shared patch's
+// biases, residual and the place where its sums meet are ready before them: 1.1 to 1.4 times as fast as with the three in the chain (960 ->
+// 320, 64 images, 11.2 -> 9.4).
 // Requirements (checked by the host): uint8 tensors, weight zero points 128, per-tensor scales, one-multiply requantisations.
 #include "conv_dwpoint.h"
 

@@ -36,9 +36,9 @@
 // 32 -> 192 -> 32 at 28x28.
 // A work-group's first instructions count: its pixels, its waves' weights and biases of all layers are under way before the first wait,
 // with quotients from the host (0.6 us of each block; until then the weights followed the pixels).
-// What bounds it, at batch 64: with a patch per wave vector issue first (the requantisations; 54 % of a CU's busy time at 4 clocks an
+// What bounds it, at batch 64: with a patch per wave vector issue first (the requantisations; 57 to 60 % of a CU's busy time at 4 clocks an
 // instruction, matrix cores 9 to 10 %).  With a shared patch the chain of a wave, region - expand - LDS - depthwise - LDS -
-// project, a slice after the other, with three waves a SIMD.
+// project, a slice after the other, with three waves a SIMD (vector issue 32 to 38 %, matrix cores 4 to 9 %).
 // Measured, the three launches -> this one (batch 64, launches back to back, random bytes): 24 -> 144 -> 24 at 56x56: 39.5 -> 26.8 us;
 // 32 -> 192 -> 32 at 28x28: 18.4 -> 12.2; 64 -> 384 -> 64 at 14x14: 14.7 -> 9.4; 96 -> 576 -> 96: 18.1 -> 12.8; 160 -> 960 -> 160 at 7x7: 15.1 -> 14.0;
 // batch 1, 24 -> 144 -> 24: 10.4 -> 5.8.

@@ -782,7 +782,7 @@ bool wide_applies(const ConvArgs &a)
 // form: fitted to 12 000 launches, 490 layers of 1 to 200 000 pixels and 16 to 8192 channels in every shape that fits LDS (half of them
 // within 8 % of the fit, nine in ten within 18); in the 32 x 32 form to 4900, 400 layers of 300 000 to 24 million outputs (nine in ten within
 // 20 %).  Layers with a scale per channel or a signed range, whose requantisation takes twice the instructions, in both forms: fitted to
-// 2200 layers of 300 to 24 million outputs in every shape that takes less than twice the best one's time (nine in ten within 17 %); of the
+// 2200 layers of 10 outputs to 25 million in every shape that takes less than twice the best one's time (nine in ten within 17 %); of the
 // shapes that fit LDS, the one that this picks for them takes 2 % more than the best on average (8 % by the other layers' terms, which spread 300
 // work-groups evenly over 256 CUs).
 
